@@ -231,9 +231,24 @@ cra::Docs group_table(const Plan& pl, int g) {
   return t;
 }
 
-size_t workspace_bytes(const cra_problem* p, const Plan& pl, int* nchunk) {
-  return cra::bwd_workspace_bytes(p->D, p->B, p->H_q, p->H_kv, p->S, pl.n, pl.len.data(),
-                                  pl.W.data(), pl.rpb.data(), pl.G, device_cus(), nchunk);
+cra::ChunkPlan chunk_plan(const cra_problem* p, const Plan& pl) {
+  return cra::plan_chunks(p->D, p->B, p->H_kv, pl.n, pl.len.data(), pl.W.data(), pl.rpb.data(),
+                          device_cus());
+}
+
+// The same documents with at most `cap` chunks each (one document: the
+// allocation-free entry point fits the partials into its fixed scratch).
+cra::ChunkPlan cap_chunks(const Plan& pl, cra::ChunkPlan c, int cap) {
+  if (cap > 0 && c.nchunk > cap) {
+    c.nchunk = cap;
+    c.chunk_len = cra::chunk_len_for(pl.len[0], cap);
+    c.part_rows = cap * pl.G;
+  }
+  return c;
+}
+
+size_t workspace_bytes(const cra_problem* p, const cra::ChunkPlan& c) {
+  return cra::bwd_workspace_layout(p->D, p->B, p->H_q, p->H_kv, p->S, c.part_rows);
 }
 
 int build_global_impl(const cra_problem* p, const Plan& pl, cra_tensor k, cra_tensor v,
@@ -327,12 +342,8 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   if (int e = check_buf("glob_k", glob_k)) return e;
   if (int e = check_buf("glob_v", glob_v)) return e;
   if (pl.any_relay && !relay_src) return fail(CRA_E_INVALID, "relay_src is NULL with relay on");
-  int nchunk = 0;
-  size_t need = workspace_bytes(p, pl, &nchunk);
-  if (nchunk_cap > 0 && nchunk > nchunk_cap) {
-    nchunk = nchunk_cap;
-    need = cra::bwd_workspace_layout(p->D, p->B, p->H_q, p->H_kv, p->S, pl.G, nchunk);
-  }
+  const cra::ChunkPlan chunks = cap_chunks(pl, chunk_plan(p, pl), nchunk_cap);
+  const size_t need = workspace_bytes(p, chunks);
   if (need > 0 && (!workspace || workspace_bytes_given < need))
     return fail(CRA_E_WORKSPACE, "workspace of %zu bytes needed, %zu given", need,
                 workspace ? workspace_bytes_given : (size_t)0);
@@ -355,7 +366,8 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   a.NB = (int)pl.NB;
   a.G = pl.G;
   a.scale = p->scale;
-  a.nchunk = nchunk;
+  a.chunk_len = chunks.chunk_len;
+  a.nchunk = chunks.nchunk;
   // workspace carve-up: delta and nlse2 [B*Hq*S] fp32 each, then the
   // global-row partials
   char* ws = static_cast<char*>(workspace);
@@ -364,9 +376,16 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   a.nlse2 = reinterpret_cast<float*>(ws + delta_bytes);
   a.gpart = reinterpret_cast<float*>(ws + 2 * delta_bytes);
   a.dalpha = dalpha;
+  std::vector<int> pofs(pl.n);  // partial rows before each document, in layout order
+  for (int d = 0, s = 0; d < pl.n; ++d) {
+    pofs[d] = s;
+    s += cra::num_chunks(pl.len[d], chunks.chunk_len) *
+         cra::doc_rows(pl.len[d], pl.W[d], pl.rpb[d]);
+  }
   for (int g = 0; g < num_groups(pl); ++g) {
     a.group = g;
     a.docs = group_table(pl, g);
+    for (int i = 0; i < a.docs.n; ++i) a.docs.pofs[i] = pofs[pl.order[g * cra::kMaxDocs + i]];
     hipError_t e = cra::launch_bwd(p->dtype, p->D, a, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "cra_bwd launch");
   }
@@ -460,8 +479,7 @@ int cra_fwd_persistent(const cra_problem* p, cra_tensor q, cra_tensor k, cra_ten
 size_t cra_bwd_workspace_bytes(const cra_problem* p) {
   Plan pl;
   if (plan_plain(p, &pl)) return 0;
-  int nchunk = 0;
-  return workspace_bytes(p, pl, &nchunk);
+  return workspace_bytes(p, chunk_plan(p, pl));
 }
 
 int cra_bwd(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cra_tensor o,
@@ -480,13 +498,12 @@ int cra_bwd_noalloc(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor
                     cra_tensor dk, cra_tensor dv, float* dalpha, void* stream) {
   Plan pl;
   if (int e = plan_plain(p, &pl)) return e;
-  int nchunk = 0;
-  const size_t planned = workspace_bytes(p, pl, &nchunk);
+  const size_t planned = workspace_bytes(p, chunk_plan(p, pl));
   int cap = 0;  // keep the planned chunks if they fit: then results equal cra_bwd's bit for bit
   if (planned > (size_t)CRA_NOALLOC_SCRATCH_BYTES) {
-    const size_t one = cra::bwd_workspace_layout(p->D, p->B, p->H_q, p->H_kv, p->S, pl.G, 1);
+    const size_t one = cra::bwd_workspace_layout(p->D, p->B, p->H_q, p->H_kv, p->S, pl.G);
     const size_t per_chunk = one - cra::bwd_workspace_layout(p->D, p->B, p->H_q, p->H_kv, p->S,
-                                                             pl.G, 0);
+                                                             0);
     if (one > (size_t)CRA_NOALLOC_SCRATCH_BYTES)
       return fail(CRA_E_WORKSPACE,
                   "cra_bwd_noalloc: this problem needs %zu bytes of workspace even with one "
@@ -529,8 +546,7 @@ int cra_fwd_varlen(const cra_problem* p, const cra_docs* docs, cra_tensor q, cra
 size_t cra_bwd_workspace_bytes_varlen(const cra_problem* p, const cra_docs* docs) {
   Plan pl;
   if (plan_varlen(p, docs, &pl)) return 0;
-  int nchunk = 0;
-  return workspace_bytes(p, pl, &nchunk);
+  return workspace_bytes(p, chunk_plan(p, pl));
 }
 
 int cra_bwd_varlen(const cra_problem* p, const cra_docs* docs, cra_tensor q, cra_tensor k,

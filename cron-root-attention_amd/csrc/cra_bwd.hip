@@ -23,6 +23,7 @@
 //                        writes dK/dV once.
 // No atomics: every output row has exactly one writer and the partial sums
 // are reduced in a fixed order, so two runs give identical bits.
+#include <algorithm>
 #include <type_traits>
 
 #include "cra_common.hpp"
@@ -71,7 +72,7 @@ __device__ __forceinline__ void store4(T* p, const f32x4& v, float mul) {
 }
 
 // First query that sees packed global row gr (inverse of glob_prefix).
-__device__ __forceinline__ int glob_row_first_query(int gr, int W, int rpb) {
+__host__ __device__ inline int glob_row_first_query(int gr, int W, int rpb) {
   const int r = gr / rpb;
   return (gr - r * rpb) == 0 ? r * W + W : (r + 1) * W + W - 1;
 }
@@ -380,8 +381,9 @@ __global__ __launch_bounds__(256) void dkdv_kernel(BwdArgs a) {
   const int bhk = blockIdx.x % nbh;
   const int rest = blockIdx.x / nbh;
   const Doc dc = find_doc(a.docs, rest);
-  const int chunk = GLOB ? dc.item % a.nchunk : 0;
-  const int tile = GLOB ? dc.item / a.nchunk : dc.item;
+  const int nck = GLOB ? num_chunks(dc.len, a.chunk_len) : 1;
+  const int tile = GLOB ? dc.item / nck : dc.item;
+  const int chunk = GLOB ? dc.item - tile * nck : 0;
   const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
   const int grp = a.Hq / a.Hkv;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -432,9 +434,8 @@ __global__ __launch_bounds__(256) void dkdv_kernel(BwdArgs a) {
   const bool active = kw < nrows;
   int q_lo, q_hi, wq_lo, wq_hi;
   if (GLOB) {
-    const int chunk_len = chunk_len_for(S, a.nchunk);
-    const int c_lo = chunk * chunk_len;
-    const int c_hi = min(S, c_lo + chunk_len);
+    const int c_lo = chunk * a.chunk_len;
+    const int c_hi = min(S, c_lo + a.chunk_len);
     q_lo = max(c_lo, glob_row_first_query(k0, W, rpb));
     q_hi = c_hi;
     wq_lo = active ? max(c_lo, glob_row_first_query(kw, W, rpb)) : S;
@@ -495,7 +496,7 @@ __global__ __launch_bounds__(256) void dkdv_kernel(BwdArgs a) {
 
   // Epilogue. Lane owns key row kw + 16kb + l16, dims 16db + 4g .. +4.
   if (GLOB) {
-    float* part = a.gpart + (((int64_t)chunk * nbh + bhk) * a.G + dc.gofs) * 2 * D;
+    float* part = a.gpart + part_row(dc, chunk, nbh, bhk, 0) * 2 * D;
 #pragma unroll
     for (int kb = 0; kb < NB; ++kb) {
       const int row = kw + 16 * kb + l16;
@@ -539,7 +540,7 @@ __global__ __launch_bounds__(256) void dkdv_kernel(BwdArgs a) {
     }
     // the chunk partials of the global rows are summed into chunk 0
     for (int m = 0; m < nm; ++m) {
-      const float* pk = a.gpart + ((int64_t)bhk * a.G + dc.gofs + grow[m]) * 2 * D;
+      const float* pk = a.gpart + part_row(dc, 0, nbh, bhk, grow[m]) * 2 * D;
 #pragma unroll
       for (int db = 0; db < Tr::kDB; ++db) {
         dka[db][kb] += *reinterpret_cast<const f32x4*>(pk + 16 * db + 4 * g) * gsc[m];
@@ -565,18 +566,17 @@ __global__ __launch_bounds__(256) void gsum_kernel(BwdArgs a) {
   const int nbh = a.B * a.Hkv;
   const int bhk = blockIdx.x % nbh;
   const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
-  const int rows = (dc.len + dc.W - 1) / dc.W * dc.rpb;
+  const int rows = doc_rows(dc.len, dc.W, dc.rpb);
   const int e = dc.item * 256 + (int)threadIdx.x;
   if (e >= rows * kVec) return;
   // Chunks [c_lo, c_hi) hold queries that see the row; the global-row
   // kernel wrote no partial for the others (their workgroups had no query
   // that sees the tile), so they are skipped rather than read.
-  const int L = chunk_len_for(dc.len, a.nchunk);
   const int first = glob_row_first_query(e / kVec, dc.W, dc.rpb);
-  const int c_lo = first / L;
-  const int c_hi = first < dc.len ? min(a.nchunk, (dc.len + L - 1) / L) : c_lo;
-  float* p0 = a.gpart + ((int64_t)bhk * a.G + dc.gofs) * 2 * D + 4 * (int64_t)e;
-  const int64_t cstride = (int64_t)nbh * a.G * 2 * D;
+  const int c_lo = first / a.chunk_len;
+  const int c_hi = first < dc.len ? num_chunks(dc.len, a.chunk_len) : c_lo;
+  float* p0 = a.gpart + part_row(dc, 0, nbh, bhk, 0) * 2 * D + 4 * (int64_t)e;
+  const int64_t cstride = (int64_t)nbh * rows * 2 * D;
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int c = c_lo; c < c_hi; ++c) acc += *reinterpret_cast<const f32x4*>(p0 + c * cstride);
   *reinterpret_cast<f32x4*>(p0) = acc;
@@ -599,13 +599,16 @@ __global__ __launch_bounds__(256) void dalpha_kernel(BwdArgs a) {
     for (int doc = 0; doc < a.docs.n; ++doc) {
       const int rpb = a.docs.rpb[doc];
       if (rpb == 1) continue;  // no relay rows in this document
-      const int nrel = (a.docs.len[doc] + a.docs.W[doc] - 1) / a.docs.W[doc] * a.top_k;
+      const int rows = doc_rows(a.docs.len[doc], a.docs.W[doc], rpb);
+      const int nrel = rows / rpb * a.top_k;
+      const int64_t part = (int64_t)a.docs.pofs[doc] * nbh + (int64_t)bhk * rows;  // summed chunks
+      const int64_t gofs = a.docs.gofs[doc];
       for (int e = tid; e < nrel * D; e += 256) {
         const int t = e / D, d = e % D;
-        const int row = a.docs.gofs[doc] + (t / a.top_k) * rpb + 1 + t % a.top_k;
-        const float* pk = a.gpart + ((int64_t)bhk * a.G + row) * 2 * D;  // summed chunks
-        const float dk = pk[d], dv = pk[D + d];
-        acc += dk * to_f32(gk[(int64_t)row * D + d]) + dv * to_f32(gv[(int64_t)row * D + d]);
+        const int row = (t / a.top_k) * rpb + 1 + t % a.top_k;
+        const float* pk = a.gpart + (part + row) * 2 * D;
+        const int64_t ge = (gofs + row) * D + d;
+        acc += pk[d] * to_f32(gk[ge]) + pk[D + d] * to_f32(gv[ge]);
       }
     }
   }
@@ -1069,8 +1072,9 @@ void dkdv2_kernel(BwdArgs a) {
   const int bhk = item % nbh;
   const int rest = item / nbh;
   const Doc dc = find_doc(a.docs, rest);
-  const int chunk = GLOB ? dc.item % a.nchunk : 0;
-  const int tile = GLOB ? dc.item / a.nchunk : dc.item;
+  const int nck = GLOB ? num_chunks(dc.len, a.chunk_len) : 1;
+  const int tile = GLOB ? dc.item / nck : dc.item;
+  const int chunk = GLOB ? dc.item - tile * nck : 0;
   const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
   const int grp = a.Hq / a.Hkv;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -1098,9 +1102,8 @@ void dkdv2_kernel(BwdArgs a) {
   // query interval of the workgroup; per-key intervals for the masks
   int q_lo, q_hi;
   if (GLOB) {
-    const int chunk_len = chunk_len_for(S, a.nchunk);
-    const int c_lo = chunk * chunk_len;
-    q_hi = min(S, c_lo + chunk_len);
+    const int c_lo = chunk * a.chunk_len;
+    q_hi = min(S, c_lo + a.chunk_len);
     q_lo = max(c_lo, glob_row_first_query(k0, W, rpb));
     // no query of this chunk sees the tile's rows: gsum_kernel skips the
     // chunk for them (with a single chunk the zeros are written instead)
@@ -1247,7 +1250,7 @@ void dkdv2_kernel(BwdArgs a) {
   }
 
   if (GLOB) {
-    float* part = a.gpart + (((int64_t)chunk * nbh + bhk) * a.G + dc.gofs) * 2 * D;
+    float* part = a.gpart + part_row(dc, chunk, nbh, bhk, 0) * 2 * D;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const int row = kw + 16 * kb + l16;
@@ -1289,7 +1292,7 @@ void dkdv2_kernel(BwdArgs a) {
     }
     // the chunk partials of the global rows are summed into chunk 0
     for (int m = 0; m < nm; ++m) {
-      const float* pk = a.gpart + ((int64_t)bhk * a.G + dc.gofs + grow[m]) * 2 * D;
+      const float* pk = a.gpart + part_row(dc, 0, nbh, bhk, grow[m]) * 2 * D;
 #pragma unroll
       for (int db = 0; db < D / 16; ++db) {
         dka[db][kb] += *reinterpret_cast<const f32x4*>(pk + 16 * db + 4 * g) * gsc[m];
@@ -1343,6 +1346,34 @@ constexpr int kDqWPE = 2;   // dQ waves per SIMD (register budget)
 constexpr int kDkdvGlobBQ = 128;
 constexpr int kDkdvLocalBQ = 32;
 
+// The global-row kernel's second geometry: 4-wave workgroups of 64 rows with
+// 32-query tiles (the local kernel's: 33 KB of LDS, 3 workgroups per CU at
+// D = 128), for problems of few packed rows. A workgroup of 192 rows then
+// leaves most waves without a visible row in the early chunks (at G = 192
+// all rows are one tile, and half of its wave slots idle), and one workgroup
+// per CU makes the last round coarse; against that, 64-row tiles sweep the
+// queries once per 64 rows. Kernel time, 192-row / 64-row workgroups, D = 128
+// (H: query / kv heads):
+//   B=2 H=32/32 S=4096   (G =  192)   72 /   51 us
+//   B=1 H=16/4  S=16000  (G =  381)  112 /   82 us
+//   B=1 H=16/16 S=32768  (G =  546)  210 /  213 us;  H=32/4  516 / 402 us
+//   B=1 H=16/16 S=65536  (G =  768)  557 /  523 us
+//   B=1 H=16/16 S=131072 (G = 1086) 1373 / 1550 us
+// Below D = 128 the first geometry is 128 rows with two workgroups per CU
+// and loses less: H=8 S=16384 (G = 384) 31 / 27 us, H=12 S=8192 (G = 273)
+// 20.6 / 21.1, S=32768 (G = 546) 96 / 96, S=65536 (G = 768) 227 / 242 us.
+constexpr int kNarrowWaves = 4, kNarrowBQ = 32;
+template <int D>
+constexpr int kNarrowMaxRows = D == 128 ? 768 : 384;
+
+template <int D>
+bool narrow_glob(const BwdArgs& a) {
+  int most = 0;
+  for (int d = 0; d < a.docs.n; ++d)
+    most = std::max(most, doc_rows(a.docs.len[d], a.docs.W[d], a.docs.rpb[d]));
+  return most <= kNarrowMaxRows<D>;
+}
+
 // The gfx950-tiled kernels (dq2, dkdv2) serve fp16/bf16 up to D = 128; the
 // generic kernels serve fp32 and every dtype at D = 256.
 template <typename T, int D>
@@ -1367,11 +1398,12 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   BwdArgs aq = a, ag = a, al = a;
   constexpr int kQM = kTiled ? 16 * kDqWaves * kDqQB : Tr::kBM;  // dQ queries per workgroup
   set_items(aq.docs, [&](int d) { return (a.docs.len[d] + kQM - 1) / kQM; });
-  constexpr int kGK = kTiled ? 16 * kDkdvGlobWaves<D> * kDkdvKB : Tr::kBK;   // rows per workgroup
+  const bool narrow = kTiled && narrow_glob<D>(a);
+  const int kGK = !kTiled ? Tr::kBK : narrow ? 16 * kNarrowWaves : 16 * kDkdvGlobWaves<D> * kDkdvKB;
   constexpr int kLK = kTiled ? 16 * kDkdvLocalWaves * kDkdvLocalKB<D> : Tr::kBK;
   set_items(ag.docs, [&](int d) {
-    const int g = (a.docs.len[d] + a.docs.W[d] - 1) / a.docs.W[d] * a.docs.rpb[d];
-    return (g + kGK - 1) / kGK * a.nchunk;
+    return (doc_rows(a.docs.len[d], a.docs.W[d], a.docs.rpb[d]) + kGK - 1) / kGK *
+           num_chunks(a.docs.len[d], a.chunk_len);
   });
   set_items(al.docs, [&](int d) { return (a.docs.len[d] + kLK - 1) / kLK; });
   const int nq = aq.docs.item0[a.docs.n], ng = ag.docs.item0[a.docs.n];
@@ -1387,8 +1419,12 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   if constexpr (kTiled) {
     hipLaunchKernelGGL((dq2_kernel<T, D, kDqWaves, kDqQB, kDqBN, kDqWPE>), dim3(gq),
                        dim3(64 * kDqWaves), 0, st, aq);
-    hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kDkdvGlobWaves<D>, kDkdvKB, kDkdvGlobBQ>),
-                       dim3(ng * a.B * a.Hkv), dim3(64 * kDkdvGlobWaves<D>), 0, st, ag);
+    if (narrow)
+      hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kNarrowWaves, kDkdvKB, kNarrowBQ>),
+                         dim3(ng * a.B * a.Hkv), dim3(64 * kNarrowWaves), 0, st, ag);
+    else
+      hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kDkdvGlobWaves<D>, kDkdvKB, kDkdvGlobBQ>),
+                         dim3(ng * a.B * a.Hkv), dim3(64 * kDkdvGlobWaves<D>), 0, st, ag);
   } else {
     hipLaunchKernelGGL((dq_kernel<T, D, NB>), dim3(nq * a.B * a.Hq), dim3(256), 0, st, aq);
     hipLaunchKernelGGL((dkdv_kernel<T, D, NB, true>), dim3(ng * a.B * a.Hkv), dim3(256), 0, st,
@@ -1397,8 +1433,7 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   if (a.nchunk > 1) {
     BwdArgs as = a;
     set_items(as.docs, [&](int d) {
-      const int g = (a.docs.len[d] + a.docs.W[d] - 1) / a.docs.W[d] * a.docs.rpb[d];
-      return (g * (2 * D / 4) + 255) / 256;
+      return (doc_rows(a.docs.len[d], a.docs.W[d], a.docs.rpb[d]) * (2 * D / 4) + 255) / 256;
     });
     hipLaunchKernelGGL((gsum_kernel<D>), dim3(as.docs.item0[a.docs.n] * a.B * a.Hkv), dim3(256),
                        0, st, as);
@@ -1426,10 +1461,10 @@ hipError_t launch_T(int D, const BwdArgs& a, hipStream_t st) {
 
 }  // namespace
 
-size_t bwd_workspace_bytes(int D, int B, int Hq, int Hkv, int S, int n, const int* len,
-                           const int* W, const int* rpb, int64_t G, int cus, int* nchunk) {
+ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len,
+                      const int* W, const int* rpb, int cus) {
   // Query chunks of the global-row kernel: each document's query range is
-  // cut into the same number of chunks (multiples of 64 queries), one
+  // cut into chunks of chunk_len queries (a multiple of 64), one
   // workgroup per (row tile, chunk). More chunks balance the uneven
   // workgroups better (a late row tile sees only the last queries) and
   // shorten the last round; each chunk costs a partial dK/dV of its rows,
@@ -1452,26 +1487,58 @@ size_t bwd_workspace_bytes(int D, int B, int Hq, int Hkv, int S, int n, const in
   int64_t row_tiles = 0;
   int max_len = 1;
   for (int d = 0; d < n; ++d) {
-    const int64_t g = (int64_t)(len[d] + W[d] - 1) / W[d] * rpb[d];
-    row_tiles += (g + rows - 1) / rows;
+    row_tiles += (doc_rows(len[d], W[d], rpb[d]) + rows - 1) / rows;
     if (len[d] > max_len) max_len = len[d];
   }
   const int64_t base = row_tiles * B * Hkv;
+  ChunkPlan c{};
+  if (n > 1) {
+    // Several documents: chunks of one length, so that a long document gets
+    // more of them than a short one. The sweeps (visible queries x heads of
+    // the kv group, per 64-row tile) are cut into about three pieces per CU,
+    // the 64-row kernel's resident workgroups. (With the same number of
+    // chunks for every document the longest document's workgroups ran alone
+    // at the end: 16 documents of 1 to 9001 tokens, H=16/4 D=128, 237 us in
+    // the global-row kernel and 7 in gsum_kernel; with this rule and 64-row
+    // tiles 78 + 12, with 0.75 / 1.5 / 2 times as many pieces 78 + 10, 74 +
+    // 14 and 82 + 20.)
+    double sweeps = 0;
+    for (int d = 0; d < n; ++d) {
+      const int g = doc_rows(len[d], W[d], rpb[d]);
+      for (int t = 0; t < g; t += 64)
+        sweeps += std::max(0, len[d] - glob_row_first_query(t, W[d], rpb[d]));
+    }
+    sweeps *= (double)B * Hkv;
+    const double pieces = 3.0 * (cus > 0 ? cus : 256);
+    const double L = std::min(std::max(sweeps / pieces, 64.0), 6144.0);
+    c.chunk_len = chunk_len_for((int)L, 1);
+    for (;;) {
+      c.part_rows = 0;
+      for (int d = 0; d < n; ++d)
+        c.part_rows += (int64_t)num_chunks(len[d], c.chunk_len) * doc_rows(len[d], W[d], rpb[d]);
+      if (c.part_rows < ((int64_t)1 << 31)) break;  // pofs is 32-bit
+      c.chunk_len *= 2;
+    }
+    c.nchunk = num_chunks(max_len, c.chunk_len);
+    return c;
+  }
   int64_t nc = (3 * slots + 2 * base - 1) / (2 * base);  // 1.5 rounds of workgroups
   const int64_t by_len = (max_len + 6143) / 6144;
   if (nc < by_len) nc = by_len;
   const int64_t max_nc = (max_len + 255) / 256;
   if (nc > max_nc) nc = max_nc;
   if (nc < 1) nc = 1;
-  *nchunk = (int)nc;
-  return bwd_workspace_layout(D, B, Hq, Hkv, S, G, (int)nc);
+  c.nchunk = (int)nc;
+  c.chunk_len = chunk_len_for(max_len, c.nchunk);
+  c.part_rows = nc * doc_rows(len[0], W[0], rpb[0]);
+  return c;
 }
 
-size_t bwd_workspace_layout(int D, int B, int Hq, int Hkv, int S, int64_t G, int nchunk) {
+size_t bwd_workspace_layout(int D, int B, int Hq, int Hkv, int S, int64_t part_rows) {
   // Delta (2-byte path: -Delta) and -lse * log2(e) per query, then the chunk
   // partials
   const size_t delta = (((size_t)B * Hq * S * 4) + 255) / 256 * 256;
-  const size_t part = (size_t)nchunk * B * Hkv * G * 2 * D * 4;
+  const size_t part = (size_t)part_rows * B * Hkv * 2 * D * 4;
   return 2 * delta + part;
 }
 

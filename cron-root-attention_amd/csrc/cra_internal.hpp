@@ -21,19 +21,21 @@ struct Docs {
   int rpb[kMaxDocs];   // packed global rows per block: 1 + top_k with relay, else 1
   int gofs[kMaxDocs];  // first packed global row
   int bofs[kMaxDocs];  // first block (relay_src rows)
+  int pofs[kMaxDocs];  // backward: first row of the global-row partials, per (b, kv head)
   int item0[kMaxDocs + 1];
 };
 
 // One document, resolved for a work item.
 struct Doc {
-  int off, len, W, rpb, gofs, bofs;
+  int off, len, W, rpb, gofs, bofs, pofs;
   int item;  // work item index within the document
 };
 
 __device__ __forceinline__ Doc find_doc(const Docs& t, int item) {
   int d = 0;
   for (int i = 1; i < t.n; ++i) d += item >= t.item0[i];  // item0 is non-decreasing
-  return Doc{t.off[d], t.len[d], t.W[d], t.rpb[d], t.gofs[d], t.bofs[d], item - t.item0[d]};
+  return Doc{t.off[d], t.len[d], t.W[d], t.rpb[d], t.gofs[d], t.bofs[d], t.pofs[d],
+             item - t.item0[d]};
 }
 
 // XCD-aware work order for launches of nbh heads x nt tiles (one document)
@@ -153,7 +155,7 @@ struct BwdArgs {
   void* dv;
   float* delta;    // [B, Hq, S] rowsum(o * do); 2-byte path: stored negated
   float* nlse2;    // [B, Hq, S] 2-byte path: -lse * log2(e)
-  float* gpart;    // [nchunk, B, Hkv, G, 2, D] fp32 partial dK/dV of the global rows
+  float* gpart;    // fp32 partial dK/dV of the global rows (part_row)
   float* dalpha;   // [Hkv] or null
   int64_t qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, osb, osh, oss;
   int64_t dosb, dosh, doss, dqsb, dqsh, dqss, dksb, dksh, dkss, dvsb, dvsh, dvss;
@@ -162,7 +164,8 @@ struct BwdArgs {
   int NB;          // blocks of all documents (rows of relay_src per head)
   int64_t G;       // packed global rows of all documents, per head
   float scale;
-  int nchunk;      // query chunks per document of the global-row kernel
+  int chunk_len;   // queries per chunk of the global-row kernel
+  int nchunk;      // most query chunks of a document
   int group;       // 0: first launch of a call (fp32: computes Delta; writes dalpha);
                    // later document groups of the call add to dalpha
   int xcd_nt;      // > 0: XCD-aware order (xcd_item) over this many tiles per head
@@ -186,6 +189,22 @@ __host__ __device__ inline int chunk_len_for(int len, int nchunk) {
   return (c + 63) / 64 * 64;
 }
 
+// Query chunks of a document of length len.
+__host__ __device__ inline int num_chunks(int len, int chunk_len) {
+  return (len + chunk_len - 1) / chunk_len;
+}
+
+// Packed global rows of a document.
+__host__ __device__ inline int doc_rows(int len, int W, int rpb) { return (len + W - 1) / W * rpb; }
+
+// Partial dK/dV of global row `row` of a document from query chunk `chunk`:
+// row index into gpart ([2, D] each). A document's partials are
+// [chunks, B * Hkv, rows], behind those of the documents before it.
+__device__ __forceinline__ int64_t part_row(const Doc& dc, int chunk, int nbh, int bhk, int row) {
+  const int rows = doc_rows(dc.len, dc.W, dc.rpb);
+  return (int64_t)dc.pofs * nbh + ((int64_t)chunk * nbh + bhk) * rows + row;
+}
+
 // Compiled tile geometry (dtype 0 f16, 1 bf16, 2 f32; D 32/64/128): the forward's
 // {waves, queries, key rows per tile} and the backward's {waves, rows, tile} of
 // dQ, global-row dK/dV and local dK/dV. Returns false for an unbuilt (dtype, D).
@@ -196,15 +215,19 @@ bool bwd_tile_config(int dtype, int D, int out[9]);
 hipError_t launch_build_global(int dtype, int D, const GlobalArgs& a, int B, hipStream_t st);
 hipError_t launch_fwd(int dtype, int D, const FwdArgs& a, hipStream_t st);
 hipError_t launch_bwd(int dtype, int D, const BwdArgs& a, hipStream_t st);
-// Workspace of the backward for n documents of lengths len[], windows W[]
-// and packed rows per block rpb[] (G packed rows per head in total) on a
-// device with `cus` compute units; *nchunk receives the query chunks per
-// document of the global-row kernel.
-size_t bwd_workspace_bytes(int D, int B, int Hq, int Hkv, int S, int n, const int* len,
-                           const int* W, const int* rpb, int64_t G, int cus, int* nchunk);
-// Workspace of the backward with nchunk query chunks: Delta and -lse*log2(e),
-// [B*Hq*S] fp32 each (rounded up to 256 bytes), then the partials
-// [nchunk, B, Hkv, G, 2, D] fp32.
-size_t bwd_workspace_layout(int D, int B, int Hq, int Hkv, int S, int64_t G, int nchunk);
+// Query chunks of the global-row kernel and its fp32 partials for n documents
+// of lengths len[], windows W[] and packed rows per block rpb[] on a device
+// with `cus` compute units.
+struct ChunkPlan {
+  int chunk_len;      // queries per chunk (multiple of 64)
+  int nchunk;         // most chunks of a document
+  int64_t part_rows;  // partial rows per (b, kv head), all documents
+};
+ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len, const int* W,
+                      const int* rpb, int cus);
+// Workspace of the backward: Delta and -lse*log2(e), [B*Hq*S] fp32 each
+// (rounded up to 256 bytes), then the partials, part_rows * B * Hkv rows of
+// [2, D] fp32.
+size_t bwd_workspace_layout(int D, int B, int Hq, int Hkv, int S, int64_t part_rows);
 
 }  // namespace cra
