@@ -560,6 +560,10 @@ __global__ __launch_bounds__(256) void dkdv_kernel(BwdArgs a) {
 // (one float4 per thread; work items: the documents' rows x 2D / 4 / 256).
 // Only chunks with a query that sees the row are read.
 // ---------------------------------------------------------------------------
+// kGsumU partials' loads are in flight together (past the last chunk that
+// chunk is read again and left out): one at a time, the sum is a chain of
+// memory latencies
+constexpr int kGsumU = 8;
 template <int D>
 __global__ __launch_bounds__(256) void gsum_kernel(BwdArgs a) {
   constexpr int kVec = 2 * D / 4;  // float4 per row (dK and dV)
@@ -578,7 +582,15 @@ __global__ __launch_bounds__(256) void gsum_kernel(BwdArgs a) {
   float* p0 = a.gpart + part_row(dc, 0, nbh, bhk, 0) * 2 * D + 4 * (int64_t)e;
   const int64_t cstride = (int64_t)nbh * rows * 2 * D;
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int c = c_lo; c < c_hi; ++c) acc += *reinterpret_cast<const f32x4*>(p0 + c * cstride);
+  for (int c = c_lo; c < c_hi; c += kGsumU) {
+    f32x4 x[kGsumU];
+#pragma unroll
+    for (int u = 0; u < kGsumU; ++u)
+      x[u] = *reinterpret_cast<const f32x4*>(p0 + min(c + u, c_hi - 1) * cstride);
+#pragma unroll
+    for (int u = 0; u < kGsumU; ++u)
+      if (c + u < c_hi) acc += x[u];
+  }
   *reinterpret_cast<f32x4*>(p0) = acc;
 }
 
@@ -586,8 +598,12 @@ __global__ __launch_bounds__(256) void gsum_kernel(BwdArgs a) {
 // 4. d(relay_log_scale)[hk] = sum over b and relay rows of dRK.RK + dRV.RV
 // (reference core.py:3363-3366), one workgroup per kv head, fixed order.
 // ---------------------------------------------------------------------------
+// 1024 threads with four elements each per step, four rows' loads in flight:
+// the sum is latency-bound (one element per thread and step of a 256-thread
+// workgroup took 66 us at B=1 H_kv=4 S=8191 D=256, this one 9.8 us).
 template <typename T, int D>
-__global__ __launch_bounds__(256) void dalpha_kernel(BwdArgs a) {
+__global__ __launch_bounds__(1024) void dalpha_kernel(BwdArgs a) {
+  constexpr int kVec = D / 4;  // four-element groups per row
   const int hk = blockIdx.x;
   const int tid = threadIdx.x;
   const int nbh = a.B * a.Hkv;
@@ -603,19 +619,25 @@ __global__ __launch_bounds__(256) void dalpha_kernel(BwdArgs a) {
       const int nrel = rows / rpb * a.top_k;
       const int64_t part = (int64_t)a.docs.pofs[doc] * nbh + (int64_t)bhk * rows;  // summed chunks
       const int64_t gofs = a.docs.gofs[doc];
-      for (int e = tid; e < nrel * D; e += 256) {
-        const int t = e / D, d = e % D;
+#pragma unroll 4
+      for (int e = tid; e < nrel * kVec; e += 1024) {
+        const int t = e / kVec, d = e % kVec * 4;
         const int row = (t / a.top_k) * rpb + 1 + t % a.top_k;
-        const float* pk = a.gpart + (part + row) * 2 * D;
-        const int64_t ge = (gofs + row) * D + d;
-        acc += pk[d] * to_f32(gk[ge]) + pk[D + d] * to_f32(gv[ge]);
+        const float* pk = a.gpart + (part + row) * 2 * D + d;
+        const f32x4 dk = *reinterpret_cast<const f32x4*>(pk);
+        const f32x4 dv = *reinterpret_cast<const f32x4*>(pk + D);
+        T ek[4], ev[4];
+        __builtin_memcpy(ek, gk + (gofs + row) * D + d, sizeof(ek));
+        __builtin_memcpy(ev, gv + (gofs + row) * D + d, sizeof(ev));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc += dk[i] * to_f32(ek[i]) + dv[i] * to_f32(ev[i]);
       }
     }
   }
-  __shared__ float red[256];
+  __shared__ float red[1024];
   red[tid] = acc;
   __syncthreads();
-  for (int off = 128; off >= 1; off >>= 1) {
+  for (int off = 512; off >= 1; off >>= 1) {
     if (tid < off) red[tid] += red[tid + off];
     __syncthreads();
   }
@@ -1438,7 +1460,7 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((gsum_kernel<D>), dim3(as.docs.item0[a.docs.n] * a.B * a.Hkv), dim3(256),
                        0, st, as);
   }
-  if (a.dalpha) hipLaunchKernelGGL((dalpha_kernel<T, D>), dim3(a.Hkv), dim3(256), 0, st, a);
+  if (a.dalpha) hipLaunchKernelGGL((dalpha_kernel<T, D>), dim3(a.Hkv), dim3(1024), 0, st, a);
   if constexpr (kTiled)
     hipLaunchKernelGGL((dkdv2_kernel<T, D, false, kDkdvLocalWaves, kDkdvLocalKB<D>, kDkdvLocalBQ>),
                        dim3(gl), dim3(64 * kDkdvLocalWaves), 0, st, al);
