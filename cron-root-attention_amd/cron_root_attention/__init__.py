@@ -41,8 +41,9 @@ def calibrate(H: int = 8, D: int = 64, dtype=None, S: int = 4096, verbose: bool 
         v = _torch.randn(1, H, S, D, device=dev, dtype=dtype, requires_grad=True)
         cron_root_attention_v14(q, k, v).sum().backward()
         _torch.cuda.synchronize(dev)
-    # the gfx950-tiled kernels (fp16/bf16 up to D = 128) double-buffer their
-    # streamed tiles in LDS; the generic ones (fp32, D = 256) stage one tile
+    # fp16/bf16 up to D = 128 double-buffer their streamed tiles in LDS; fp32
+    # stages one tile, and so does D = 256 (fp16/bf16: K and V in turn, each
+    # filled while the other is in use)
     stages = 2 if (dtype != _torch.float32 and Dp <= 128) else 1
     cfg = {"fwd": (t["fwd_waves"], stages), "bwd": (t["dq_waves"], stages)}
     if verbose:

@@ -651,10 +651,19 @@ __global__ __launch_bounds__(1024) void dalpha_kernel(BwdArgs a) {
 // computed; transposed operands (K^T for dQ, Q^T and dO^T for dK/dV) are
 // read with ds_read_b64_tr_b16 from the same row-major tiles.
 // ---------------------------------------------------------------------------
+// Lane offsets; at D = 256 the upper half of a row lies 256 bytes behind the
+// lower half (the swizzle permutes 16 chunks): an immediate of the read.
 template <int D>
 struct LaneOffs {
-  int row[D / 32];  // row fragment, chunk 4c + g, row lane%16
-  int tr[D / 16];   // transposed fragment, columns 16 db ..
+  static constexpr int kD = D < 128 ? D : 128;
+  int row[kD / 32];  // row fragment, chunk 4c + g, row lane%16
+  int tr[kD / 16];   // transposed fragment, columns 16 db ..
+  __device__ __forceinline__ int row_at(int c) const {
+    return row[c % (kD / 32)] + c / (kD / 32) * 256;
+  }
+  __device__ __forceinline__ int tr_at(int db) const {
+    return tr[db % (kD / 16)] + db / (kD / 16) * 256;
+  }
 };
 
 template <int D>
@@ -663,9 +672,9 @@ __device__ __forceinline__ LaneOffs<D> lane_offs(int lane) {
   LaneOffs<D> o;
   const int g = lane >> 4;
 #pragma unroll
-  for (int c = 0; c < D / 32; ++c) o.row[c] = Tile::row_lane_off(lane, 4 * c + g);
+  for (int c = 0; c < o.kD / 32; ++c) o.row[c] = Tile::row_lane_off(lane, 4 * c + g);
 #pragma unroll
-  for (int db = 0; db < D / 16; ++db) o.tr[db] = Tile::tr_lane_off(lane, 16 * db);
+  for (int db = 0; db < o.kD / 16; ++db) o.tr[db] = Tile::tr_lane_off(lane, 16 * db);
   return o;
 }
 
@@ -673,6 +682,90 @@ __device__ __forceinline__ LaneOffs<D> lane_offs(int lane) {
 // tile, in 32-key halves: S = K . Q^T and dP - Delta = V . dO^T - Delta (key
 // on rows; the products accumulate onto -Delta, so no subtraction per
 // element), dS = P * (dP - Delta), dQ^T += K^T . dS^T.
+//
+// dq2_ds: dS of 32-key half kc.
+template <typename T, int D, int QB, int BN, bool MASK>
+__device__ __forceinline__ void dq2_ds(const char* tK, const char* tV, int kc,
+                                       const LaneOffs<D>& lo, const Frag<T> (&qf)[QB][D / 32],
+                                       const Frag<T> (&df)[QB][D / 32], const float (&lse2)[QB],
+                                       const float (&ndl)[QB], float c2, int g,
+                                       const TileMask<QB>& mk, Frag<T> (&dsf)[QB]) {
+  using Tile = SwzTile<D, BN>;
+  constexpr int NC = D / 32;
+  float ds[2][QB][4];  // [h][qb][r]
+  // K and V row fragments are read two steps ahead of their MFMAs; fences
+  // keep the compiler from moving the reads next to their uses
+  constexpr int NT = 2 * NC;
+  auto row_kv = [&](int t, Frag<T>& k_, Frag<T>& v_) {
+    const int kn = 2 * kc + t / NC, cn = t % NC;
+    k_ = Tile::template row_frag_at<T>(tK + kn * Tile::kBlk16 + lo.row_at(cn));
+    v_ = Tile::template row_frag_at<T>(tV + kn * Tile::kBlk16 + lo.row_at(cn));
+  };
+  Frag<T> kf[3], vf[3];
+  row_kv(0, kf[0], vf[0]);
+  row_kv(1, kf[1], vf[1]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    f32x4 sc[QB], dp[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      sc[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      dp[qb] = f32x4{ndl[qb], ndl[qb], ndl[qb], ndl[qb]};
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int t = h * NC + c;
+      if (t + 2 < NT) row_kv(t + 2, kf[(t + 2) % 3], vf[(t + 2) % 3]);
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        sc[qb] = mma(sc[qb], kf[t % 3], qf[qb][c]);
+        dp[qb] = mma(dp[qb], vf[t % 3], df[qb][c]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int kb = 2 * kc + h;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int ko = 16 * kb + 4 * g + r;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        float x = fmaf(sc[qb][r], c2, -lse2[qb]);
+        if (MASK && !mk.ok(ko, qb)) x = -__builtin_huge_valf();
+        ds[h][qb][r] = __builtin_amdgcn_exp2f(x) * dp[qb][r];
+      }
+    }
+  }
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const float v8[8] = {ds[0][qb][0], ds[0][qb][1], ds[0][qb][2], ds[0][qb][3],
+                         ds[1][qb][0], ds[1][qb][1], ds[1][qb][2], ds[1][qb][3]};
+    dsf[qb] = pack8<T>(v8);
+  }
+}
+
+// dQ^T += K^T . dS^T of 32-key half kc; transposed K fragments two steps ahead.
+template <typename T, int D, int QB, int BN>
+__device__ __forceinline__ void dq2_acc(const char* tK, int kc, const LaneOffs<D>& lo,
+                                        const Frag<T> (&dsf)[QB], f32x4 (&dqa)[D / 16][QB]) {
+  using Tile = SwzTile<D, BN>;
+  Frag<T> kt[3];
+  auto tr_k = [&](int db) {
+    const char* pa = tK + (2 * kc) * Tile::kBlk16 + lo.tr_at(db);
+    return Tile::template tr_frag_at<T>(pa, pa + Tile::kBlk16);
+  };
+  kt[0] = tr_k(0);
+  kt[1] = tr_k(1);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) {
+    if (db + 2 < D / 16) kt[(db + 2) % 3] = tr_k(db + 2);
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) dqa[db][qb] = mma(dqa[db][qb], kt[db % 3], dsf[qb]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 template <typename T, int D, int QB, int BN, bool MASK>
 __device__ __forceinline__ void dq2_tile(const char* tK, const char* tV, const LaneOffs<D>& lo,
                                          const Frag<T> (&qf)[QB][D / 32],
@@ -680,79 +773,13 @@ __device__ __forceinline__ void dq2_tile(const char* tK, const char* tV, const L
                                          f32x4 (&dqa)[D / 16][QB], const float (&lse2)[QB],
                                          const float (&ndl)[QB], float c2, int g,
                                          const TileMask<QB>& mk, bool half0, bool half1) {
-  using Tile = SwzTile<D, BN>;
-  constexpr int NC = D / 32;
 #pragma unroll
   for (int kc = 0; kc < BN / 32; ++kc) {
     // masked tiles: a 32-key half with no key visible to the wave is skipped
     if (MASK && !(kc ? half1 : half0)) continue;
-    float ds[2][QB][4];  // [h][qb][r]
-    // K and V row fragments are read two steps ahead of their MFMAs; fences
-    // keep the compiler from moving the reads next to their uses
-    constexpr int NT = 2 * NC;
-    auto row_kv = [&](int t, Frag<T>& k_, Frag<T>& v_) {
-      const int kn = 2 * kc + t / NC, cn = t % NC;
-      k_ = Tile::template row_frag_at<T>(tK + kn * Tile::kBlk16 + lo.row[cn]);
-      v_ = Tile::template row_frag_at<T>(tV + kn * Tile::kBlk16 + lo.row[cn]);
-    };
-    Frag<T> kf[3], vf[3];
-    row_kv(0, kf[0], vf[0]);
-    row_kv(1, kf[1], vf[1]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      f32x4 sc[QB], dp[QB];
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) {
-        sc[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        dp[qb] = f32x4{ndl[qb], ndl[qb], ndl[qb], ndl[qb]};
-      }
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const int t = h * NC + c;
-        if (t + 2 < NT) row_kv(t + 2, kf[(t + 2) % 3], vf[(t + 2) % 3]);
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb) {
-          sc[qb] = mma(sc[qb], kf[t % 3], qf[qb][c]);
-          dp[qb] = mma(dp[qb], vf[t % 3], df[qb][c]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      const int kb = 2 * kc + h;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int ko = 16 * kb + 4 * g + r;
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb) {
-          float x = fmaf(sc[qb][r], c2, -lse2[qb]);
-          if (MASK && !mk.ok(ko, qb)) x = -__builtin_huge_valf();
-          ds[h][qb][r] = __builtin_amdgcn_exp2f(x) * dp[qb][r];
-        }
-      }
-    }
     Frag<T> dsf[QB];
-#pragma unroll
-    for (int qb = 0; qb < QB; ++qb) {
-      const float v8[8] = {ds[0][qb][0], ds[0][qb][1], ds[0][qb][2], ds[0][qb][3],
-                           ds[1][qb][0], ds[1][qb][1], ds[1][qb][2], ds[1][qb][3]};
-      dsf[qb] = pack8<T>(v8);
-    }
-    // transposed K fragments, also two steps ahead
-    Frag<T> kt[3];
-    auto tr_k = [&](int db) {
-      const char* pa = tK + (2 * kc) * Tile::kBlk16 + lo.tr[db];
-      return Tile::template tr_frag_at<T>(pa, pa + Tile::kBlk16);
-    };
-    kt[0] = tr_k(0);
-    kt[1] = tr_k(1);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int db = 0; db < D / 16; ++db) {
-      if (db + 2 < D / 16) kt[(db + 2) % 3] = tr_k(db + 2);
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) dqa[db][qb] = mma(dqa[db][qb], kt[db % 3], dsf[qb]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    dq2_ds<T, D, QB, BN, MASK>(tK, tV, kc, lo, qf, df, lse2, ndl, c2, g, mk, dsf);
+    dq2_acc<T, D, QB, BN>(tK, kc, lo, dsf, dqa);
   }
 }
 
@@ -940,6 +967,154 @@ void dq2_kernel(BwdArgs a) {
   }
 }
 
+// dQ of the 2-byte types at head dim 256: 4 waves of 16 queries (Q, dO and dQ
+// take 128 registers of a wave per 16 queries), 32-key tiles. V is staged one
+// tile at a time and K two, 48 KB of LDS per workgroup: the next K arrives
+// during this tile's S and dP, the next V during its K^T . dS^T. Bound by
+// LDS reads (one K, V or K^T fragment per MFMA: at most about 60% MFMA-busy)
+// and 2 waves per SIMD (216 VGPRs). B=1 H=8 S=32768 fp16: 318 us, where
+// dq_kernel (tiles through registers, V and K^T stored transposed by 2-byte
+// LDS writes, one stage) took 478 us and delta_kernel before it 46 us.
+constexpr int kWideWaves = 4, kWideBN = 32;
+template <typename T, int D>
+__global__ __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(2)))
+void dq_wide_kernel(BwdArgs a) {
+  constexpr int NW = kWideWaves, BN = kWideBN, kBM = 16 * NW;
+  using Tile = SwzTile<D, BN>;
+  __shared__ __attribute__((aligned(1024))) char sK0[Tile::kBytes];
+  __shared__ __attribute__((aligned(1024))) char sK1[Tile::kBytes];
+  __shared__ __attribute__((aligned(1024))) char sV[Tile::kBytes];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int nbh = a.B * a.Hq;
+  const int bh = blockIdx.x % nbh;
+  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
+  const int b = bh / a.Hq, h = bh % a.Hq;
+  const int hk = h / (a.Hq / a.Hkv);
+  const int m0 = tile * kBM;
+  const int q0 = m0 + wave * 16;
+  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+
+  const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
+  const T* dop =
+      static_cast<const T*>(a.dout) + b * a.dosb + h * a.dosh + (int64_t)dc.off * a.doss;
+  const T* opp = static_cast<const T*>(a.o) + b * a.osb + h * a.osh + (int64_t)dc.off * a.oss;
+  const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
+  const T* vp = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
+  const int64_t row_bh = (int64_t)bh * a.S + dc.off;
+  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
+  const T* gkp = static_cast<const T*>(a.gk) + gbase;
+  const T* gvp = static_cast<const T*>(a.gv) + gbase;
+
+  const int lo_k = max(0, m0 - W + 1);
+  const int hi = min(S, m0 + kBM);
+  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int nloc = (hi - lo_k + BN - 1) / BN;
+  const int nglob = (gmax + BN - 1) / BN;
+  const int ntot = nloc + nglob;
+  using Fill = typename Tile::template Fill<NW>;
+  const int kbytes = (int)(a.kss * 2), vbytes = (int)(a.vss * 2);
+  const __amdgpu_buffer_rsrc_t rk = make_rsrc(kp, (uint32_t)((hi - 1) * kbytes + D * 2));
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(vp, (uint32_t)((hi - 1) * vbytes + D * 2));
+  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gkp, (uint32_t)(gmax * D * 2));
+  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gvp, (uint32_t)(gmax * D * 2));
+  const int fk = Fill::lane_off(wave, lane, kbytes);
+  const int fv = Fill::lane_off(wave, lane, vbytes);
+  const int fg = Fill::lane_off(wave, lane, D * 2);
+  // global tiles first, then the local window from its highest tile down
+  auto row0 = [&](int it) { return it >= nglob ? lo_k + (nloc - 1 - (it - nglob)) * BN : it * BN; };
+  auto issue_k = [&](int it, char* dst) {
+    if (it >= nglob)
+      Fill::load(dst, rk, fk, kbytes, row0(it), wave);
+    else
+      Fill::load(dst, rgk, fg, D * 2, row0(it), wave);
+  };
+  auto issue_v = [&](int it) {
+    if (it >= nglob)
+      Fill::load(sV, rv, fv, vbytes, row0(it), wave);
+    else
+      Fill::load(sV, rgv, fg, D * 2, row0(it), wave);
+  };
+  issue_k(0, sK0);
+  issue_v(0);
+
+  const LaneOffs<D> lo = lane_offs<D>(lane);
+  // Delta = rowsum(O * dO) of the wave's queries, stored negated with
+  // -lse * log2(e) for the dK/dV kernels (see dq2_kernel). Rows past the
+  // document read its last row; their results are never stored.
+  Frag<T> qf[1][D / 32], df[1][D / 32];
+  const int qi = q0 + l16;
+  const int qr = min(qi, S - 1);
+  const bool ok = qi < S;
+  const float lse2[1] = {ok ? a.lse[row_bh + qr] * kLog2e : 0.f};
+  float od = 0.f;
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    qf[0][c] = lds_frag_row<T>(qp + (int64_t)qr * a.qss + 32 * c + 8 * g);
+    df[0][c] = lds_frag_row<T>(dop + (int64_t)qr * a.doss + 32 * c + 8 * g);
+    const Frag<T> of = lds_frag_row<T>(opp + (int64_t)qr * a.oss + 32 * c + 8 * g);
+    const T* eo = reinterpret_cast<const T*>(of.w);
+    const T* ed = reinterpret_cast<const T*>(df[0][c].w);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) od = fmaf(to_f32(eo[i]), to_f32(ed[i]), od);
+  }
+  od += __shfl_xor(od, 16);
+  od += __shfl_xor(od, 32);
+  const float ndl[1] = {-od};
+  if (ok && g == 0) {
+    a.delta[row_bh + qi] = -od;
+    a.nlse2[row_bh + qi] = -lse2[0];
+  }
+  const float c2 = a.scale * kLog2e;
+  f32x4 dqa[D / 16][1];
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) dqa[db][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const bool active = q0 < S;
+  const int q_last = min(q0 + 16, S) - 1;
+  const int w_lo = max(0, q0 - W + 1);
+  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
+  const int glen = glob_prefix(qi, W, rpb);
+
+  auto step = [&](auto buf_c, int it) {
+    char(&cur)[Tile::kBytes] = decltype(buf_c)::value ? sK1 : sK0;
+    char(&nxt)[Tile::kBytes] = decltype(buf_c)::value ? sK0 : sK1;
+    wait_vmem();
+    __syncthreads();  // this tile's K and V landed; every wave is done with the other K
+    if (it + 1 < ntot) issue_k(it + 1, nxt);
+    const bool loc = it >= nglob;
+    const int ts = row0(it);
+    const bool work = active && (loc ? (ts <= q_last && ts + BN - 1 >= w_lo) : ts < wg_hi);
+    Frag<T> dsf[1];
+    if (work) {
+      const bool full = loc ? (ts >= q_last - W + 1 && ts + BN - 1 <= q0) : ts + BN <= wg_lo;
+      TileMask<1> mk;
+      mk.hi[0] = loc ? qi - ts : glen - 1 - ts;
+      mk.span[0] = loc ? (unsigned)(W - 1) : 0x7fffffffu;
+      if (full)
+        dq2_ds<T, D, 1, BN, false>(cur, sV, 0, lo, qf, df, lse2, ndl, c2, g, mk, dsf);
+      else
+        dq2_ds<T, D, 1, BN, true>(cur, sV, 0, lo, qf, df, lse2, ndl, c2, g, mk, dsf);
+    }
+    __syncthreads();  // every wave is done with this tile's V
+    if (it + 1 < ntot) issue_v(it + 1);
+    if (work) dq2_acc<T, D, 1, BN>(cur, 0, lo, dsf, dqa);
+  };
+  for (int it = 0; it < ntot; it += 2) {
+    step(std::integral_constant<int, 0>{}, it);
+    if (it + 1 < ntot) step(std::integral_constant<int, 1>{}, it + 1);
+  }
+
+  if (!active || qi >= S) return;
+  T* row = static_cast<T*>(a.dq) + b * a.dqsb + h * a.dqsh + (int64_t)(dc.off + qi) * a.dqss;
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) store4<T>(row + 16 * db + 4 * g, dqa[db][0], a.scale);
+}
+
 // Key-centric dK/dV: each wave owns KB blocks of 16 key rows (rows of k/v,
 // or packed global rows with GLOB), B operands in registers; query tiles of
 // BQ rows of Q and dO stream through LDS with their -lse * log2(e) (sL) and
@@ -965,8 +1140,8 @@ __device__ __forceinline__ void dkdv2_tile(const char* tQ, const char* tO, const
     constexpr int NC = D / 32, NT = 2 * NC;
     auto row_qo = [&](int t, Frag<T>& q_, Frag<T>& o_) {
       const int qn = 2 * qs + t / NC, cn = t % NC;
-      q_ = Tile::template row_frag_at<T>(tQ + qn * Tile::kBlk16 + lo.row[cn]);
-      o_ = Tile::template row_frag_at<T>(tO + qn * Tile::kBlk16 + lo.row[cn]);
+      q_ = Tile::template row_frag_at<T>(tQ + qn * Tile::kBlk16 + lo.row_at(cn));
+      o_ = Tile::template row_frag_at<T>(tO + qn * Tile::kBlk16 + lo.row_at(cn));
     };
     Frag<T> qa[PF + 1], oa[PF + 1];
 #pragma unroll
@@ -1044,8 +1219,8 @@ __device__ __forceinline__ void dkdv2_tile(const char* tQ, const char* tO, const
     // each transposed Q/dO fragment pair serves every key block of the wave
     Frag<T> ot[PF + 1], qt[PF + 1];
     auto tr_pair = [&](int db, Frag<T>& o_, Frag<T>& q_) {
-      const char* po = tO + (2 * qs) * Tile::kBlk16 + lo.tr[db];
-      const char* pq = tQ + (2 * qs) * Tile::kBlk16 + lo.tr[db];
+      const char* po = tO + (2 * qs) * Tile::kBlk16 + lo.tr_at(db);
+      const char* pq = tQ + (2 * qs) * Tile::kBlk16 + lo.tr_at(db);
       o_ = Tile::template tr_frag_at<T>(po, po + Tile::kBlk16);
       q_ = Tile::template tr_frag_at<T>(pq, pq + Tile::kBlk16);
     };
@@ -1067,10 +1242,15 @@ __device__ __forceinline__ void dkdv2_tile(const char* tQ, const char* tO, const
 
 // NW waves of KB key blocks each cover the workgroup's 16 * NW * KB key
 // rows; query tiles of BQ rows. At most 168 VGPRs: 3 waves per SIMD (the
-// global-row kernel below D = 128: at most 128, 4 waves per SIMD).
+// global-row kernel below D = 128: at most 128, 4 waves per SIMD). At D = 256
+// the accumulators and the resident K/V fragments take 192 registers of a
+// 16-row wave: 256 VGPRs (2-10 spilled), 2 waves per SIMD, 4-wave workgroups
+// with 32-query tiles (66 KB of LDS, two per CU). B=1 H=8 S=32768 fp16:
+// global rows 215 us, local 306 us; dkdv_kernel (one LDS stage, transposed
+// tiles written by 2-byte LDS stores) took 720 and 638 us.
 template <typename T, int D, bool GLOB, int NW, int KB, int BQ>
 __global__ __launch_bounds__(64 * NW)
-__attribute__((amdgpu_waves_per_eu(GLOB && D < 128 ? 4 : 3)))
+__attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : GLOB && D < 128 ? 4 : 3)))
 void dkdv2_kernel(BwdArgs a) {
   using Tile = SwzTile<D, BQ>;
   constexpr int kKW = 16 * KB, kBK = NW * kKW, kBQ = BQ;
@@ -1351,11 +1531,11 @@ void dkdv2_kernel(BwdArgs a) {
 // tiles. Config 4 training (B=1 H=12 D=64) 1.2-1.7% faster at S = 8192,
 // 32768 and 131072 (three alternating runs).
 template <int D>
-constexpr int kDkdvGlobWaves = D == 128 ? 12 : 8;
+constexpr int kDkdvGlobWaves = D > 128 ? 4 : D == 128 ? 12 : 8;
 constexpr int kDkdvLocalWaves = 4;
 constexpr int kDkdvKB = 1;  // 16-key blocks per wave (global-row kernel)
 template <int D>
-constexpr int kDkdvLocalKB = D == 128 ? 1 : 2;  // local kernel
+constexpr int kDkdvLocalKB = D >= 128 ? 1 : 2;  // local kernel
 constexpr int kDqWaves = 4;
 constexpr int kDqQB = 2;    // 16-query blocks per dQ wave
 constexpr int kDqBN = 64;   // key rows per dQ tile
@@ -1365,7 +1545,8 @@ constexpr int kDqWPE = 2;   // dQ waves per SIMD (register budget)
 // a CU; with 64-row tiles only two fit. The global-row kernel (one 12-wave
 // workgroup per CU, 130 KB of LDS) takes 128-row tiles: one barrier per 128
 // queries instead of 64 (backward 1.7% faster).
-constexpr int kDkdvGlobBQ = 128;
+template <int D>
+constexpr int kDkdvGlobBQ = D > 128 ? 32 : 128;
 constexpr int kDkdvLocalBQ = 32;
 
 // The global-row kernel's second geometry: 4-wave workgroups of 64 rows with
@@ -1386,7 +1567,7 @@ constexpr int kDkdvLocalBQ = 32;
 // 20.6 / 21.1, S=32768 (G = 546) 96 / 96, S=65536 (G = 768) 227 / 242 us.
 constexpr int kNarrowWaves = 4, kNarrowBQ = 32;
 template <int D>
-constexpr int kNarrowMaxRows = D == 128 ? 768 : 384;
+constexpr int kNarrowMaxRows = D > 128 ? 0 : D == 128 ? 768 : 384;
 
 template <int D>
 bool narrow_glob(const BwdArgs& a) {
@@ -1396,10 +1577,10 @@ bool narrow_glob(const BwdArgs& a) {
   return most <= kNarrowMaxRows<D>;
 }
 
-// The gfx950-tiled kernels (dq2, dkdv2) serve fp16/bf16 up to D = 128; the
-// generic kernels serve fp32 and every dtype at D = 256.
+// The gfx950-tiled kernels (dq2 and dq_wide, dkdv2) serve fp16/bf16, the
+// generic kernels fp32.
 template <typename T, int D>
-constexpr bool kTiledBwd = sizeof(T) == 2 && D <= 128;
+constexpr bool kTiledBwd = sizeof(T) == 2;
 template <int D>
 constexpr int kGenericNB = D > 128 ? 1 : 2;
 
@@ -1418,7 +1599,7 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   // chunks (global dK/dV), key tiles (local dK/dV), each of its kernel's
   // workgroup size
   BwdArgs aq = a, ag = a, al = a;
-  constexpr int kQM = kTiled ? 16 * kDqWaves * kDqQB : Tr::kBM;  // dQ queries per workgroup
+  constexpr int kQM = !kTiled ? Tr::kBM : D > 128 ? 16 * kWideWaves : 16 * kDqWaves * kDqQB;  // dQ queries per workgroup
   set_items(aq.docs, [&](int d) { return (a.docs.len[d] + kQM - 1) / kQM; });
   const bool narrow = kTiled && narrow_glob<D>(a);
   const int kGK = !kTiled ? Tr::kBK : narrow ? 16 * kNarrowWaves : 16 * kDkdvGlobWaves<D> * kDkdvKB;
@@ -1439,13 +1620,16 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   const int gq = xq ? xcd_grid(a.B * a.Hq, nq) : nq * a.B * a.Hq;
   const int gl = xl ? xcd_grid(a.B * a.Hkv, nl) : nl * a.B * a.Hkv;
   if constexpr (kTiled) {
-    hipLaunchKernelGGL((dq2_kernel<T, D, kDqWaves, kDqQB, kDqBN, kDqWPE>), dim3(gq),
-                       dim3(64 * kDqWaves), 0, st, aq);
-    if (narrow)
+    if constexpr (D > 128)
+      hipLaunchKernelGGL((dq_wide_kernel<T, D>), dim3(gq), dim3(64 * kWideWaves), 0, st, aq);
+    else
+      hipLaunchKernelGGL((dq2_kernel<T, D, kDqWaves, kDqQB, kDqBN, kDqWPE>), dim3(gq),
+                         dim3(64 * kDqWaves), 0, st, aq);
+    if (D <= 128 && narrow)
       hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kNarrowWaves, kDkdvKB, kNarrowBQ>),
                          dim3(ng * a.B * a.Hkv), dim3(64 * kNarrowWaves), 0, st, ag);
     else
-      hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kDkdvGlobWaves<D>, kDkdvKB, kDkdvGlobBQ>),
+      hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kDkdvGlobWaves<D>, kDkdvKB, kDkdvGlobBQ<D>>),
                          dim3(ng * a.B * a.Hkv), dim3(64 * kDkdvGlobWaves<D>), 0, st, ag);
   } else {
     hipLaunchKernelGGL((dq_kernel<T, D, NB>), dim3(nq * a.B * a.Hq), dim3(256), 0, st, aq);
@@ -1500,8 +1684,8 @@ ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len,
   //   B=1 H=12 D=64 S=8192 / 32768 / 131072: 22 / 13 / 22 chunks
   //   B=2 H=32 D=128 S=4096: 6 (the previous rule's 16 was 12% slower)
   //   B=1 H=8 D=64 S=16384: 32 (64 was 10% slower)
-  // (D = 256 runs the generic global-row kernel: 64 rows per 4-wave
-  // workgroup, two workgroups per CU by their 71 KB of LDS)
+  // (D = 256: 64 rows per 4-wave workgroup, two workgroups per CU by their
+  // 66 KB of LDS)
   const int rows = D > 128    ? BwdTraits<f16, 256, 1>::kBK
                    : D == 128 ? 16 * kDkdvGlobWaves<128> * kDkdvKB
                               : 16 * kDkdvGlobWaves<64> * kDkdvKB;
@@ -1580,7 +1764,7 @@ bool bwd_tile_config(int dtype, int D, int out[9]) {
     const int gw = D == 128 ? kDkdvGlobWaves<128> : kDkdvGlobWaves<64>;
     const int lkb = D == 128 ? kDkdvLocalKB<128> : kDkdvLocalKB<64>;
     const int v[9] = {kDqWaves,        16 * kDqWaves * kDqQB,        kDqBN,
-                      gw,              16 * gw * kDkdvKB,            kDkdvGlobBQ,
+                      gw,              16 * gw * kDkdvKB,            kDkdvGlobBQ<128>,
                       kDkdvLocalWaves, 16 * kDkdvLocalWaves * lkb,   kDkdvLocalBQ};
     for (int i = 0; i < 9; ++i) out[i] = v[i];
   }

@@ -221,13 +221,14 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 template <int D, int ROWS>
 struct SwzTile {
-  static_assert(D == 32 || D == 64 || D == 128, "head dim");
+  static_assert(D == 32 || D == 64 || D == 128 || D == 256, "head dim");
   static constexpr int kCPR = D / 8;      // 16-byte chunks per row
-  static constexpr int kRPL = 128 / D;    // rows sharing one 256-byte line
+  static constexpr int kRPL = D < 128 ? 128 / D : 1;  // rows sharing one 256-byte line
+  static constexpr int kSwz = kCPR < 16 ? kCPR : 16;  // chunks the swizzle permutes
   static constexpr int kBytes = ROWS * D * 2;
   static constexpr int kInstr = ROWS * kCPR / 64;  // 1 KB global_load_lds per instruction
 
-  __device__ __forceinline__ static int swz(int row) { return (row / kRPL) % kCPR; }
+  __device__ __forceinline__ static int swz(int row) { return (row / kRPL) % kSwz; }
   // byte offset of logical 16-byte chunk `chunk` of `row`
   __device__ __forceinline__ static int off(int row, int chunk) {
     return row * (D * 2) + ((chunk ^ swz(row)) << 4);
@@ -238,13 +239,15 @@ struct SwzTile {
   // wave's successive instructions are kRowStep rows apart. kRowStep is a
   // multiple of the swizzle period, so a lane's in-row chunk is the same for
   // all of its instructions and its offset is one precomputed VGPR plus a
-  // wave-uniform row offset.
+  // wave-uniform row offset. At D = 256 with 4 waves it is half the period:
+  // every other instruction takes the chunk with bit 3 flipped (kAlt).
   template <int NWAVES>
   struct Fill {
     static constexpr int kPer = (kInstr + NWAVES - 1) / NWAVES;
     static constexpr int kRowsPerInstr = 64 / kCPR;
     static constexpr int kRowStep = NWAVES * kRowsPerInstr;
-    static_assert(kPer == 1 || (kRowStep % kRPL == 0 && (kRowStep / kRPL) % kCPR == 0),
+    static constexpr bool kAlt = kPer > 1 && D == 256 && kRowStep == 8;
+    static_assert(kPer == 1 || kAlt || (kRowStep % kRPL == 0 && (kRowStep / kRPL) % kSwz == 0),
                   "swizzle must repeat every instruction step");
 
     // Lane's byte offset for its first instruction, relative to tile row 0 of
@@ -264,12 +267,18 @@ struct SwzTile {
       // from reads of the other buffer and waits for it before them.
       static_assert((NWAVES & (NWAVES - 1)) == 0, "power-of-two wave count");
       const int w = __builtin_amdgcn_readfirstlane(wave) & (NWAVES - 1);
+      int alt = 0;  // byte distance of the flipped chunk
+      if (kAlt) {
+        const int lane = threadIdx.x & 63;
+        alt = (((lane % kCPR) ^ swz(wave * kRowsPerInstr + lane / kCPR)) & 8) ? -128 : 128;
+      }
 #pragma unroll
       for (int t0 = 0; t0 < kPer; ++t0) {
         const int t = t0 * NWAVES + w;
         if (kInstr % NWAVES != 0 && t >= kInstr) break;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, CRA_LDS(lds + t * 1024), 16,
-                                                 lane_off + (row0 + t0 * kRowStep) * row_bytes,
+                                                 lane_off + (row0 + t0 * kRowStep) * row_bytes +
+                                                     (kAlt && t0 % 2 ? alt : 0),
                                                  0, 0, 0);
       }
     }
@@ -283,7 +292,7 @@ struct SwzTile {
     return f;
   }
 
-  // The swizzle repeats every 16 rows (16 / kRPL is a multiple of kCPR), so
+  // The swizzle repeats every 16 rows (16 / kRPL is a multiple of kSwz), so
   // for rows 16*blk + r the offset is blk * 16 * row_bytes + lane_off(r, ..):
   // lane-constant parts are computed once and the block term folds into the
   // instruction's immediate offset.

@@ -276,16 +276,31 @@ void fwd_kernel(FwdArgs a) {
 #define CRA_FWD_PF 3
 #endif
 
+// Lane offsets into the swizzled tiles. The swizzle permutes 16 chunks (256
+// bytes) of a row, so at D = 256 the upper half of a row is 256 bytes behind
+// the lower half: an immediate of the read, no further register.
 template <int D>
 struct Fwd2Lane {
-  int k[D / 32];   // K row fragment, chunk 4c + g, row lane%16
-  int v[D / 16];   // V^T fragment, columns 16 db ..
+  static constexpr int kD = D < 128 ? D : 128;
+  int k[kD / 32];   // K row fragment, chunk 4c + g, row lane%16
+  int v[kD / 16];   // V^T fragment, columns 16 db ..
+  __device__ __forceinline__ void init(int lane) {
+    using Tile = SwzTile<D, 64>;
+#pragma unroll
+    for (int c = 0; c < kD / 32; ++c) k[c] = Tile::row_lane_off(lane, 4 * c + (lane >> 4));
+#pragma unroll
+    for (int db = 0; db < kD / 16; ++db) v[db] = Tile::tr_lane_off(lane, 16 * db);
+  }
+  __device__ __forceinline__ int k_at(int c) const { return k[c % (kD / 32)] + c / (kD / 32) * 256; }
+  __device__ __forceinline__ int v_at(int db) const {
+    return v[db % (kD / 16)] + db / (kD / 16) * 256;
+  }
 };
 
-template <typename T, int D, int BN>
+template <typename T, int D, int BN, int QB>
 __device__ __forceinline__ void tile_scores(const char* tK, const Fwd2Lane<D>& lo,
-                                            const Frag<T> (&qf)[2][D / 32], int kc,
-                                            f32x4 (&s)[2][2]) {
+                                            const Frag<T> (&qf)[QB][D / 32], int kc,
+                                            f32x4 (&s)[2][QB]) {
   using Tile = SwzTile<D, BN>;
   constexpr int NC = D / 32, NK = 2 * NC;
   // K fragments are read CRA_FWD_PF steps ahead of the MFMAs that use them; fences
@@ -294,7 +309,7 @@ __device__ __forceinline__ void tile_scores(const char* tK, const Fwd2Lane<D>& l
   // each MFMA's accumulator was last written four MFMAs earlier (key block
   // major, two apart, measured 0.5% slower).
   auto k_frag = [&](int t) {
-    return Tile::template row_frag_at<T>(tK + (2 * kc + t % 2) * Tile::kBlk16 + lo.k[t / 2]);
+    return Tile::template row_frag_at<T>(tK + (2 * kc + t % 2) * Tile::kBlk16 + lo.k_at(t / 2));
   };
   constexpr int PF = CRA_FWD_PF < NK ? CRA_FWD_PF : NK;
   Frag<T> kf[PF + 1];
@@ -305,22 +320,24 @@ __device__ __forceinline__ void tile_scores(const char* tK, const Fwd2Lane<D>& l
   for (int t = 0; t < NK; ++t) {
     if (t + PF < NK) kf[(t + PF) % (PF + 1)] = k_frag(t + PF);
     const int h = t % 2, c = t / 2;
-    if (c == 0) s[h][0] = s[h][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    s[h][0] = mma(s[h][0], kf[t % (PF + 1)], qf[0][c]);
-    s[h][1] = mma(s[h][1], kf[t % (PF + 1)], qf[1][c]);
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      if (c == 0) s[h][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      s[h][qb] = mma(s[h][qb], kf[t % (PF + 1)], qf[qb][c]);
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
 // O^T += V^T . P^T for 32-key half kh: transposed V fragments read
 // CRA_FWD_PF steps ahead of the MFMAs that use them.
-template <typename T, int D, int BN>
+template <typename T, int D, int BN, int QB>
 __device__ __forceinline__ void pv_half(const char* tV, int kh, const Fwd2Lane<D>& lo,
-                                        const Frag<T> (&pf)[2], f32x4 (&acc)[D / 16][2]) {
+                                        const Frag<T> (&pf)[QB], f32x4 (&acc)[D / 16][QB]) {
   using Tile = SwzTile<D, BN>;
   constexpr int NDB = D / 16;
   auto tr_v = [&](int db) {
-    const char* pa = tV + (2 * kh) * Tile::kBlk16 + lo.v[db];
+    const char* pa = tV + (2 * kh) * Tile::kBlk16 + lo.v_at(db);
     return Tile::template tr_frag_at<T>(pa, pa + Tile::kBlk16);
   };
   constexpr int PF = CRA_FWD_PF < NDB ? CRA_FWD_PF : NDB;
@@ -331,8 +348,8 @@ __device__ __forceinline__ void pv_half(const char* tV, int kh, const Fwd2Lane<D
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
     if (db + PF < NDB) vt[(db + PF) % (PF + 1)] = tr_v(db + PF);
-    acc[db][0] = mma(acc[db][0], vt[db % (PF + 1)], pf[0]);
-    acc[db][1] = mma(acc[db][1], vt[db % (PF + 1)], pf[1]);
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) acc[db][qb] = mma(acc[db][qb], vt[db % (PF + 1)], pf[qb]);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -362,9 +379,9 @@ __device__ __forceinline__ float half_sum(const Frag<T>& pk, const Frag<T>& one)
 // Exponentials of one 32-key half (8 per lane and query block) against the
 // running maximum, rounded to the input type, and the sum of the rounded
 // values over the half's 32 keys (the P.V operand and its normaliser).
-template <typename T, bool MASK>
-__device__ __forceinline__ void half_exp(f32x4 (&s)[2][2], int kc, int qb, float c2, float m,
-                                         int g, const TileMask<2>& mk, const Frag<T>& one,
+template <typename T, bool MASK, int QB>
+__device__ __forceinline__ void half_exp(f32x4 (&s)[2][QB], int kc, int qb, float c2, float m,
+                                         int g, const TileMask<QB>& mk, const Frag<T>& one,
                                          Frag<T>& pk, float& ps) {
   float pv[8];
 #pragma unroll
@@ -383,10 +400,10 @@ __device__ __forceinline__ void half_exp(f32x4 (&s)[2][2], int kc, int qb, float
 // first visible keys and whenever a score exceeds the running maximum by
 // enough to push a sum of 8 rounded terms past kSumMax (inf and NaN sums
 // included).
-template <typename T, int D>
-__device__ __forceinline__ void half_rescale(f32x4 (&s)[2][2], int qb, float c2,
-                                             f32x4 (&acc)[D / 16][2], float (&m_run)[2],
-                                             float (&l_run)[2], const Frag<T>& one, Frag<T>& pk,
+template <typename T, int D, int QB>
+__device__ __forceinline__ void half_rescale(f32x4 (&s)[2][QB], int qb, float c2,
+                                             f32x4 (&acc)[D / 16][QB], float (&m_run)[QB],
+                                             float (&l_run)[QB], const Frag<T>& one, Frag<T>& pk,
                                              float& ps) {
   float mx = -__builtin_huge_valf();
 #pragma unroll
@@ -429,7 +446,7 @@ __device__ __forceinline__ void attend_tile2(const char* tK, const char* tV, con
   using Tile = SwzTile<D, BN>;
   constexpr int kHalves = BN / 32;
   f32x4 s[kHalves][2][2];
-  tile_scores<T, D, BN>(tK, lo, qf, 0, s[0]);
+  tile_scores<T, D, BN, 2>(tK, lo, qf, 0, s[0]);
   Frag<T> pf[2];
 #pragma unroll
   for (int kc = 0; kc < kHalves; ++kc) {
@@ -437,18 +454,18 @@ __device__ __forceinline__ void attend_tile2(const char* tK, const char* tV, con
     float ps[2];
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb)
-      half_exp<T, MASK>(s[kc], kc, qb, c2, m_run[qb], g, mk, one, pn[qb], ps[qb]);
-    if (kc > 0) pv_half<T, D, BN>(tV, kc - 1, lo, pf, acc);  // beside this half's exponentials
-    if (kc + 1 < kHalves) tile_scores<T, D, BN>(tK, lo, qf, kc + 1, s[kc + 1]);
+      half_exp<T, MASK, 2>(s[kc], kc, qb, c2, m_run[qb], g, mk, one, pn[qb], ps[qb]);
+    if (kc > 0) pv_half<T, D, BN, 2>(tV, kc - 1, lo, pf, acc);  // beside this half's exponentials
+    if (kc + 1 < kHalves) tile_scores<T, D, BN, 2>(tK, lo, qf, kc + 1, s[kc + 1]);
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       if (__any(!(ps[qb] <= kSumMax)))
-        half_rescale<T, D>(s[kc], qb, c2, acc, m_run, l_run, one, pn[qb], ps[qb]);
+        half_rescale<T, D, 2>(s[kc], qb, c2, acc, m_run, l_run, one, pn[qb], ps[qb]);
       l_run[qb] += ps[qb];
       pf[qb] = pn[qb];
     }
   }
-  pv_half<T, D, BN>(tV, kHalves - 1, lo, pf, acc);
+  pv_half<T, D, BN, 2>(tV, kHalves - 1, lo, pf, acc);
 }
 
 // One 32-key half kc of a masked tile, for tiles whose other half has no
@@ -461,19 +478,19 @@ __device__ __forceinline__ void attend_half(const char* tK, const char* tV, int 
                                             const TileMask<2>& mk, const Frag<T>& one) {
   using Tile = SwzTile<D, BN>;
   f32x4 s[2][2];
-  tile_scores<T, D, BN>(tK, lo, qf, kc, s);
+  tile_scores<T, D, BN, 2>(tK, lo, qf, kc, s);
   float ps[2];
   Frag<T> pf[2];
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb)
-    half_exp<T, true>(s, kc, qb, c2, m_run[qb], g, mk, one, pf[qb], ps[qb]);
+    half_exp<T, true, 2>(s, kc, qb, c2, m_run[qb], g, mk, one, pf[qb], ps[qb]);
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
     if (__any(!(ps[qb] <= kSumMax)))
-      half_rescale<T, D>(s, qb, c2, acc, m_run, l_run, one, pf[qb], ps[qb]);
+      half_rescale<T, D, 2>(s, qb, c2, acc, m_run, l_run, one, pf[qb], ps[qb]);
     l_run[qb] += ps[qb];
   }
-  pv_half<T, D, BN>(tV, kc, lo, pf, acc);
+  pv_half<T, D, BN, 2>(tV, kc, lo, pf, acc);
 }
 
 // NW waves of 32 queries share each K/V tile of BN = 64 rows (2 x 32 KB
@@ -555,11 +572,7 @@ __device__ __forceinline__ void fwd2_item(const FwdArgs& a, const int item, FwdS
   issue(0, stage0[0]);
 
   Fwd2Lane<D> lo;
-#pragma unroll
-  for (int c = 0; c < D / 32; ++c) lo.k[c] = Tile::row_lane_off(lane, 4 * c + g);
-#pragma unroll
-  for (int db = 0; db < D / 16; ++db) lo.v[db] = Tile::tr_lane_off(lane, 16 * db);
-
+  lo.init(lane);
   Frag<T> qf[2][D / 32];
   int qi[2];
 #pragma unroll
@@ -685,6 +698,142 @@ void fwd2_persistent_kernel(FwdArgs a) {
   }
 }
 
+// fp16/bf16 forward at head dim 256: 4 waves of 16 queries (two blocks per
+// wave would hold 192 registers of accumulators and Q operands), 32-key tiles.
+// K and V are staged in turn, one tile of each in LDS: while a tile's scores
+// and softmax are computed its V is on the way, and the next tile's K during
+// P.V, so 32 KB of LDS per workgroup hide the fills and three workgroups (3
+// waves per SIMD at 168 VGPRs) share a CU. Bound by LDS reads: a K or V
+// fragment serves one MFMA, which caps MFMA-busy at about 60%. B=1 H=8
+// S=32768 fp16: 214 us (562 effective TFLOP/s); fwd_kernel (tiles through
+// registers, V stored transposed by 2-byte LDS writes) took 470 us.
+constexpr int kWideWaves = 4, kWideBN = 32;
+template <typename T, int D>
+__global__ __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(3)))
+void fwd_wide_kernel(FwdArgs a) {
+  constexpr int NW = kWideWaves, BN = kWideBN, kBM = 16 * NW;
+  using Tile = SwzTile<D, BN>;
+  __shared__ __attribute__((aligned(1024))) char sK[Tile::kBytes];
+  __shared__ __attribute__((aligned(1024))) char sV[Tile::kBytes];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int nbh = a.B * a.Hq;
+  const int bh = blockIdx.x % nbh;
+  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
+  const int b = bh / a.Hq, h = bh % a.Hq;
+  const int hk = h / (a.Hq / a.Hkv);
+  const int m0 = tile * kBM;
+  const int q0 = m0 + wave * 16;
+  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+
+  const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
+  const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
+  const T* vp = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
+  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
+  const T* gkp = static_cast<const T*>(a.gk) + gbase;
+  const T* gvp = static_cast<const T*>(a.gv) + gbase;
+
+  const int lo_k = max(0, m0 - W + 1);
+  const int hi = min(S, m0 + kBM);
+  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int nloc = (a.phases & 1) ? (hi - lo_k + BN - 1) / BN : 0;
+  const int nglob = (a.phases & 2) ? (gmax + BN - 1) / BN : 0;
+  const int ntot = nloc + nglob;
+  using Fill = typename Tile::template Fill<NW>;
+  const int kbytes = (int)(a.kss * 2), vbytes = (int)(a.vss * 2);
+  const __amdgpu_buffer_rsrc_t rk = make_rsrc(kp, (uint32_t)((hi - 1) * kbytes + D * 2));
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(vp, (uint32_t)((hi - 1) * vbytes + D * 2));
+  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gkp, (uint32_t)(gmax * D * 2));
+  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gvp, (uint32_t)(gmax * D * 2));
+  const int fk = Fill::lane_off(wave, lane, kbytes);
+  const int fv = Fill::lane_off(wave, lane, vbytes);
+  const int fg = Fill::lane_off(wave, lane, D * 2);
+  // global tiles first, then the local window from its highest tile down
+  auto row0 = [&](int it) { return it >= nglob ? lo_k + (nloc - 1 - (it - nglob)) * BN : it * BN; };
+  auto issue_k = [&](int it) {
+    if (it >= nglob)
+      Fill::load(sK, rk, fk, kbytes, row0(it), wave);
+    else
+      Fill::load(sK, rgk, fg, D * 2, row0(it), wave);
+  };
+  auto issue_v = [&](int it) {
+    if (it >= nglob)
+      Fill::load(sV, rv, fv, vbytes, row0(it), wave);
+    else
+      Fill::load(sV, rgv, fg, D * 2, row0(it), wave);
+  };
+  if (ntot > 0) issue_k(0);
+
+  Fwd2Lane<D> lo;
+  lo.init(lane);
+  Frag<T> qf[1][D / 32];
+  const int qi = q0 + l16;
+  const int qr = min(qi, S - 1);  // queries past the document are never stored
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c)
+    qf[0][c] = lds_frag_row<T>(qp + (int64_t)qr * a.qss + 32 * c + 8 * g);
+  const float c2 = a.scale * kLog2e;
+  float m_run[1] = {-__builtin_huge_valf()}, l_run[1] = {0.f};
+  f32x4 acc[D / 16][1];
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) acc[db][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const bool active = q0 < S;
+  const int q_last = min(q0 + 16, S) - 1;
+  const int w_lo = max(0, q0 - W + 1);
+  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
+  const int glen = glob_prefix(qi, W, rpb);
+  const Frag<T> one = ones_frag<T>();
+
+  for (int it = 0; it < ntot; ++it) {
+    wait_vmem();
+    __syncthreads();  // K of this tile landed; every wave is done with the previous V
+    issue_v(it);
+    const bool loc = it >= nglob;
+    const int ts = row0(it);
+    const bool work = active && (loc ? (ts <= q_last && ts + BN - 1 >= w_lo) : ts < wg_hi);
+    Frag<T> pf[1];
+    if (work) {
+      const bool full = loc ? (ts >= q_last - W + 1 && ts + BN - 1 <= q0) : ts + BN <= wg_lo;
+      TileMask<1> mk;
+      mk.hi[0] = loc ? qi - ts : glen - 1 - ts;
+      mk.span[0] = loc ? (unsigned)(W - 1) : 0x7fffffffu;
+      f32x4 s[2][1];
+      tile_scores<T, D, BN, 1>(sK, lo, qf, 0, s);
+      float ps;
+      if (full)
+        half_exp<T, false, 1>(s, 0, 0, c2, m_run[0], g, mk, one, pf[0], ps);
+      else
+        half_exp<T, true, 1>(s, 0, 0, c2, m_run[0], g, mk, one, pf[0], ps);
+      if (__any(!(ps <= kSumMax)))
+        half_rescale<T, D, 1>(s, 0, c2, acc, m_run, l_run, one, pf[0], ps);
+      l_run[0] += ps;
+    }
+    wait_vmem();
+    __syncthreads();  // V landed; every wave is done with this tile's K
+    if (it + 1 < ntot) issue_k(it + 1);
+    if (work) pv_half<T, D, BN, 1>(sV, 0, lo, pf, acc);
+  }
+
+  if (!active || qi >= S) return;
+  T* orow = static_cast<T*>(a.o) + b * a.osb + h * a.osh + (int64_t)(dc.off + qi) * a.oss;
+  const float l = fmaxf(l_run[0], 1e-6f);
+  const float inv = __builtin_amdgcn_rcpf(l);  // its 1-ulp error is invisible in the 2-byte O
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) {
+    T e[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) e[r] = from_f32<T>(acc[db][0][r] * inv);
+    *reinterpret_cast<uint2*>(orow + 16 * db + 4 * g) = *reinterpret_cast<const uint2*>(e);
+  }
+  if (g == 0)
+    a.lse[(int64_t)bh * a.S + dc.off + qi] = (m_run[0] + __builtin_amdgcn_logf(l)) * kLn2;
+}
+
 // Resident workgroups of `kern` on the current device (CUs x workgroups per
 // CU), looked up once per device and instantiation: the persistent launch
 // serves small problems, where per-call host queries would cost more than
@@ -715,17 +864,21 @@ hipError_t resident_slots(K kern, int threads, int* out) {
 // measured 4% slower at D = 128: the wider local window adds key tiles.
 constexpr int kFwdWaves = 4;
 
-// Head dim 256, every dtype: the generic forward with 16 queries per wave
-// (64 per workgroup). A persistent request runs the same tiled kernel (the
-// work-queue form is built for the gfx950-tiled kernel only; the results
+// Head dim 256: 16 queries per wave, 64 per workgroup; the 2-byte types on
+// fwd_wide_kernel, fp32 on the generic kernel. A persistent request runs the
+// same tiled kernel (the work-queue form is built for fwd2 only; the results
 // are the same function of the inputs).
 template <typename T>
 hipError_t launch_wide(const FwdArgs& a, hipStream_t st) {
   using Tr = FwdTraits<T, 256, 1>;
+  static_assert(Tr::kBM == 16 * kWideWaves, "one workgroup size at head dim 256");
   FwdArgs b = a;
   set_items(b.docs, [&](int d) { return (b.docs.len[d] + Tr::kBM - 1) / Tr::kBM; });
   const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq);
-  hipLaunchKernelGGL((fwd_kernel<T, 256, 1>), grid, dim3(Tr::kThreads), 0, st, b);
+  if constexpr (sizeof(T) == 2)
+    hipLaunchKernelGGL((fwd_wide_kernel<T, 256>), grid, dim3(Tr::kThreads), 0, st, b);
+  else
+    hipLaunchKernelGGL((fwd_kernel<T, 256, 1>), grid, dim3(Tr::kThreads), 0, st, b);
   return hipGetLastError();
 }
 
