@@ -9,15 +9,14 @@
 // dQ_i += scale dS k_j, dK_j += scale dS q_i, dV_j += P dO_i.
 //
 // This build keeps every accumulation in fp32 and rounds once:
-//   1. delta_kernel      Delta = rowsum(O * dO)  (fp32 inputs; for fp16/bf16
-//                        dq2_kernel computes Delta of its queries and stores
-//                        -Delta and -lse * log2(e) for the dK/dV kernels)
-//   2. dq_kernel         query-centric: local band + global prefix -> dQ
-//   3. dkdv_kernel<GLOB> packed global rows (strided + relay), query range
-//                        split in chunks -> fp32 partials in the workspace
-//   3b. gsum_kernel      sums the chunk partials of each global row
+//   1. dq2_kernel        query-centric: local band + global prefix -> dQ; it
+//      (dq_wide, dq_f32) also forms Delta = rowsum(O * dO) of its queries and
+//                        stores -Delta and -lse * log2(e) for the dK/dV kernels
+//   2. dkdv2_kernel<GLOB> packed global rows (strided + relay), query range
+//      (dkdv_f32)        split in chunks -> fp32 partials in the workspace
+//   3. gsum_kernel       sums the chunk partials of each global row
 //   4. dalpha_kernel     (optional) gradient of the relay log-scale
-//   5. dkdv_kernel<LOC>  key-centric local band; its epilogue adds the
+//   5. dkdv2_kernel<LOC> key-centric local band; its epilogue adds the
 //                        summed partials of the global rows whose source is
 //                        the key row (strided row r*W, relay source rows) and
 //                        writes dK/dV once.
@@ -32,27 +31,6 @@
 namespace cra {
 
 namespace {
-
-// Geometry of the generic (non-gfx950-tiled) kernels: the fp32 path, and
-// every dtype at head dim 256. NB = 16-row blocks per wave (queries for dQ,
-// keys for dK/dV): two below D = 256; one at D = 256, where two would hold
-// 256 VGPRs of accumulators and operands per wave.
-template <typename T, int D, int NB = 2>
-struct BwdTraits {
-  static constexpr int kThreads = 256;
-  static constexpr bool kSmallTiles = sizeof(T) == 4 || D > 128;
-  static constexpr int kQW = 16 * NB;                   // dq: queries per wave
-  static constexpr int kBM = 4 * kQW;                   // dq: queries per workgroup
-  static constexpr int kBN = kSmallTiles ? 32 : 64;     // dq: key rows per tile
-  static constexpr int kKW = 16 * NB;                   // dkdv: key rows per wave
-  static constexpr int kBK = 4 * kKW;                   // dkdv: key rows per workgroup
-  static constexpr int kBQ = kSmallTiles ? 32 : 64;     // dkdv: queries per tile
-  static constexpr int kDC = D / 32;
-  static constexpr int kDB = D / 16;
-  static constexpr int kLD = D + 16 / (int)sizeof(T);
-  static constexpr int kLDTN = kBN + 4;
-  static constexpr int kLDTQ = kBQ + 4;
-};
 
 template <typename T>
 __device__ __forceinline__ void zero_frag(Frag<T>& f) {
@@ -78,485 +56,7 @@ __host__ __device__ inline int glob_row_first_query(int gr, int W, int rpb) {
 }
 
 // ---------------------------------------------------------------------------
-// 1. Delta = rowsum(O * dO)
-// ---------------------------------------------------------------------------
-template <typename T, int D>
-__global__ __launch_bounds__(256) void delta_kernel(BwdArgs a) {
-  constexpr int kLPR = D / 8;
-  constexpr int kRows = 256 / kLPR;
-  const int bh = blockIdx.y;
-  const int b = bh / a.Hq, h = bh % a.Hq;
-  const int tid = threadIdx.x;
-  const int li = tid % kLPR;
-  const int row = blockIdx.x * kRows + tid / kLPR;
-  float acc = 0.f;
-  if (row < a.S) {
-    const Frag<T> o = lds_frag_row<T>(static_cast<const T*>(a.o) + b * a.osb + h * a.osh +
-                                      (int64_t)row * a.oss + li * 8);
-    const Frag<T> d = lds_frag_row<T>(static_cast<const T*>(a.dout) + b * a.dosb + h * a.dosh +
-                                      (int64_t)row * a.doss + li * 8);
-    const T* eo = reinterpret_cast<const T*>(o.w);
-    const T* ed = reinterpret_cast<const T*>(d.w);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc += to_f32(eo[i]) * to_f32(ed[i]);
-  }
-#pragma unroll
-  for (int off = kLPR / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
-  if (row < a.S && li == 0) a.delta[(int64_t)bh * a.S + row] = acc;
-}
-
-// ---------------------------------------------------------------------------
-// 2. dQ, query-centric (mirror of the forward's tiling)
-// ---------------------------------------------------------------------------
-template <typename T, int D, int NB, bool MASK, typename Valid>
-__device__ __forceinline__ void dq_tile(const T* sK, const T* sV, const T* sKt,
-                                        const Frag<T> (&qf)[NB][BwdTraits<T, D, NB>::kDC],
-                                        const Frag<T> (&df)[NB][BwdTraits<T, D, NB>::kDC],
-                                        f32x4 (&dqa)[BwdTraits<T, D, NB>::kDB][NB],
-                                        const float (&lse2)[NB], const float (&dl)[NB], float c2,
-                                        int l16, int g, Valid valid) {
-  using Tr = BwdTraits<T, D, NB>;
-  constexpr int kKB = Tr::kBN / 16, kKC = Tr::kBN / 32;
-  Frag<T> dsf[kKC][NB];
-  float ds[kKB][NB][4];
-#pragma unroll
-  for (int kb = 0; kb < kKB; ++kb) {
-    f32x4 sc[NB], dp[NB];
-#pragma unroll
-    for (int qb = 0; qb < NB; ++qb) sc[qb] = dp[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < Tr::kDC; ++c) {
-      const Frag<T> kf = lds_frag_row<T>(sK + (16 * kb + l16) * Tr::kLD + 32 * c + 8 * g);
-      const Frag<T> vf = lds_frag_row<T>(sV + (16 * kb + l16) * Tr::kLD + 32 * c + 8 * g);
-#pragma unroll
-      for (int qb = 0; qb < NB; ++qb) sc[qb] = mma(sc[qb], kf, qf[qb][c]);
-#pragma unroll
-      for (int qb = 0; qb < NB; ++qb) dp[qb] = mma(dp[qb], vf, df[qb][c]);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int ko = 16 * kb + 4 * g + r;
-#pragma unroll
-      for (int qb = 0; qb < NB; ++qb) {
-        float x = sc[qb][r] * c2 - lse2[qb];
-        if (MASK && !valid(ko, qb)) x = -__builtin_huge_valf();
-        ds[kb][qb][r] = __builtin_amdgcn_exp2f(x) * (dp[qb][r] - dl[qb]);
-      }
-    }
-  }
-#pragma unroll
-  for (int kc = 0; kc < kKC; ++kc) {
-#pragma unroll
-    for (int qb = 0; qb < NB; ++qb) {
-      const float v8[8] = {ds[2 * kc][qb][0],     ds[2 * kc][qb][1],     ds[2 * kc][qb][2],
-                           ds[2 * kc][qb][3],     ds[2 * kc + 1][qb][0], ds[2 * kc + 1][qb][1],
-                           ds[2 * kc + 1][qb][2], ds[2 * kc + 1][qb][3]};
-      dsf[kc][qb] = pack8<T>(v8);
-    }
-  }
-#pragma unroll
-  for (int db = 0; db < Tr::kDB; ++db) {
-    const T* row = sKt + (16 * db + l16) * Tr::kLDTN;
-#pragma unroll
-    for (int kc = 0; kc < kKC; ++kc) {
-      const Frag<T> kt = lds_frag_2x4<T>(row + 32 * kc + 4 * g, row + 32 * kc + 16 + 4 * g);
-#pragma unroll
-      for (int qb = 0; qb < NB; ++qb) dqa[db][qb] = mma(dqa[db][qb], kt, dsf[kc][qb]);
-    }
-  }
-}
-
-template <typename T, int D, int NB>
-__global__ __launch_bounds__(256) void dq_kernel(BwdArgs a) {
-  using Tr = BwdTraits<T, D, NB>;
-  __shared__ __attribute__((aligned(16))) T sK[Tr::kBN * Tr::kLD];
-  __shared__ __attribute__((aligned(16))) T sV[Tr::kBN * Tr::kLD];
-  __shared__ __attribute__((aligned(16))) T sKt[D * Tr::kLDTN];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int l16 = lane & 15, g = lane >> 4;
-  const int nbh = a.B * a.Hq;
-  const int bh = blockIdx.x % nbh;
-  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
-  const int tile = (dc.len + Tr::kBM - 1) / Tr::kBM - 1 - dc.item;  // heaviest first
-  const int b = bh / a.Hq, h = bh % a.Hq;
-  const int hk = h / (a.Hq / a.Hkv);
-  const int m0 = tile * Tr::kBM;
-  const int q0 = m0 + wave * Tr::kQW;
-  const int S = dc.len, W = dc.W, rpb = dc.rpb;
-
-  const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
-  const T* dop =
-      static_cast<const T*>(a.dout) + b * a.dosb + h * a.dosh + (int64_t)dc.off * a.doss;
-  const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
-  const T* vp = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
-  const float* lse = a.lse + (int64_t)bh * a.S + dc.off;
-  const float* delta = a.delta + (int64_t)bh * a.S + dc.off;
-  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
-  const T* gkp = static_cast<const T*>(a.gk) + gbase;
-  const T* gvp = static_cast<const T*>(a.gv) + gbase;
-
-  Frag<T> qf[NB][Tr::kDC], df[NB][Tr::kDC];
-  int qi[NB];
-  float lse2[NB], dl[NB];
-#pragma unroll
-  for (int qb = 0; qb < NB; ++qb) {
-    qi[qb] = q0 + 16 * qb + l16;
-    const bool ok = qi[qb] < S;
-    lse2[qb] = ok ? lse[qi[qb]] * kLog2e : 0.f;
-    dl[qb] = ok ? delta[qi[qb]] : 0.f;
-#pragma unroll
-    for (int c = 0; c < Tr::kDC; ++c) {
-      if (ok) {
-        qf[qb][c] = lds_frag_row<T>(qp + (int64_t)qi[qb] * a.qss + 32 * c + 8 * g);
-        df[qb][c] = lds_frag_row<T>(dop + (int64_t)qi[qb] * a.doss + 32 * c + 8 * g);
-      } else {
-        zero_frag(qf[qb][c]);
-        zero_frag(df[qb][c]);
-      }
-    }
-  }
-  const float c2 = a.scale * kLog2e;
-  f32x4 dqa[Tr::kDB][NB];
-#pragma unroll
-  for (int db = 0; db < Tr::kDB; ++db)
-#pragma unroll
-    for (int qb = 0; qb < NB; ++qb) dqa[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const bool active = q0 < S;
-  const int q_last = min(q0 + Tr::kQW, S) - 1;
-  TileStage<T, D, Tr::kBN, Tr::kThreads> stk, stv;
-
-  const int lo = max(0, m0 - W + 1);
-  const int hi = min(S, m0 + Tr::kBM);
-  const int w_lo = max(0, q0 - W + 1);
-  for (int ts = lo; ts < hi; ts += Tr::kBN) {
-    stk.load(kp, a.kss, ts, 0, hi, tid);
-    stv.load(vp, a.vss, ts, 0, hi, tid);
-    __syncthreads();
-    stk.template store_rows<Tr::kLD>(sK, tid);
-    stk.template store_cols<Tr::kLDTN>(sKt, tid);
-    stv.template store_rows<Tr::kLD>(sV, tid);
-    __syncthreads();
-    if (active && ts <= q_last && ts + Tr::kBN - 1 >= w_lo) {
-      const bool full = ts >= q_last - W + 1 && ts + Tr::kBN - 1 <= q0;
-      auto valid = [&](int ko, int qb) {
-        const int j = ts + ko;
-        return j <= qi[qb] && j >= qi[qb] - W + 1;
-      };
-      if (full)
-        dq_tile<T, D, NB, false>(sK, sV, sKt, qf, df, dqa, lse2, dl, c2, l16, g, valid);
-      else
-        dq_tile<T, D, NB, true>(sK, sV, sKt, qf, df, dqa, lse2, dl, c2, l16, g, valid);
-    }
-  }
-
-  const int gmax = glob_prefix(hi - 1, W, rpb);
-  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
-  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
-  int glen[NB];
-#pragma unroll
-  for (int qb = 0; qb < NB; ++qb) glen[qb] = glob_prefix(qi[qb], W, rpb);
-  for (int ts = 0; ts < gmax; ts += Tr::kBN) {
-    stk.load(gkp, D, ts, 0, gmax, tid);
-    stv.load(gvp, D, ts, 0, gmax, tid);
-    __syncthreads();
-    stk.template store_rows<Tr::kLD>(sK, tid);
-    stk.template store_cols<Tr::kLDTN>(sKt, tid);
-    stv.template store_rows<Tr::kLD>(sV, tid);
-    __syncthreads();
-    if (active && ts < wg_hi) {
-      auto valid = [&](int ko, int qb) { return ts + ko < glen[qb]; };
-      if (ts + Tr::kBN <= wg_lo)
-        dq_tile<T, D, NB, false>(sK, sV, sKt, qf, df, dqa, lse2, dl, c2, l16, g, valid);
-      else
-        dq_tile<T, D, NB, true>(sK, sV, sKt, qf, df, dqa, lse2, dl, c2, l16, g, valid);
-    }
-  }
-
-  T* dqp = static_cast<T*>(a.dq) + b * a.dqsb + h * a.dqsh + (int64_t)dc.off * a.dqss;
-#pragma unroll
-  for (int qb = 0; qb < NB; ++qb) {
-    if (!active || qi[qb] >= S) continue;
-    T* row = dqp + (int64_t)qi[qb] * a.dqss;
-#pragma unroll
-    for (int db = 0; db < Tr::kDB; ++db) store4<T>(row + 16 * db + 4 * g, dqa[db][qb], a.scale);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 3/5. dK, dV, key-centric. GLOB: the keys are packed global rows and the
-// result is an fp32 partial per query chunk; LOC: the keys are rows of k/v,
-// the queries their local band, and the epilogue folds in the global rows.
-// ---------------------------------------------------------------------------
-template <typename T, int D, int NB, bool GLOB, bool MASK>
-__device__ __forceinline__ void dkdv_tile(const T* sQ, const T* sO, const T* sQt, const T* sOt,
-                                          const float* sL, const float* sDl, const int* sGl,
-                                          const Frag<T> (&kf)[NB][BwdTraits<T, D, NB>::kDC],
-                                          const Frag<T> (&vf)[NB][BwdTraits<T, D, NB>::kDC],
-                                          f32x4 (&dka)[BwdTraits<T, D, NB>::kDB][NB],
-                                          f32x4 (&dva)[BwdTraits<T, D, NB>::kDB][NB], float c2,
-                                          int l16, int g, int ts, int kw, int W, int q_hi) {
-  using Tr = BwdTraits<T, D, NB>;
-  constexpr int kQS = Tr::kBQ / 32;  // 32-query steps per tile
-#pragma unroll
-  for (int qs = 0; qs < kQS; ++qs) {
-    float p[2][NB][4], ds[2][NB][4];  // [query block][key block][r]
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
-      const int qo = 32 * qs + 16 * qb;
-      f32x4 sc[NB], dd[NB];
-#pragma unroll
-      for (int kb = 0; kb < NB; ++kb) sc[kb] = dd[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < Tr::kDC; ++c) {
-        const Frag<T> qa = lds_frag_row<T>(sQ + (qo + l16) * Tr::kLD + 32 * c + 8 * g);
-        const Frag<T> oa = lds_frag_row<T>(sO + (qo + l16) * Tr::kLD + 32 * c + 8 * g);
-#pragma unroll
-        for (int kb = 0; kb < NB; ++kb) sc[kb] = mma(sc[kb], qa, kf[kb][c]);
-#pragma unroll
-        for (int kb = 0; kb < NB; ++kb) dd[kb] = mma(dd[kb], oa, vf[kb][c]);
-      }
-      const f32x4 lq = *reinterpret_cast<const f32x4*>(sL + qo + 4 * g);
-      const f32x4 dq = *reinterpret_cast<const f32x4*>(sDl + qo + 4 * g);
-      int gq[4] = {0, 0, 0, 0};
-      if (GLOB && MASK) {
-        const int4 t4 = *reinterpret_cast<const int4*>(sGl + qo + 4 * g);
-        gq[0] = t4.x; gq[1] = t4.y; gq[2] = t4.z; gq[3] = t4.w;
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int qabs = ts + qo + 4 * g + r;
-#pragma unroll
-        for (int kb = 0; kb < NB; ++kb) {
-          float x = sc[kb][r] * c2 - lq[r];
-          if (MASK) {
-            const int j = kw + 16 * kb + l16;
-            const bool vis = GLOB ? (qabs < q_hi && j < gq[r])
-                                  : (qabs < q_hi && j <= qabs && j >= qabs - W + 1);
-            if (!vis) x = -__builtin_huge_valf();
-          }
-          p[qb][kb][r] = __builtin_amdgcn_exp2f(x);
-          ds[qb][kb][r] = p[qb][kb][r] * (dd[kb][r] - dq[r]);
-        }
-      }
-    }
-#pragma unroll
-    for (int kb = 0; kb < NB; ++kb) {
-      const float pv[8] = {p[0][kb][0], p[0][kb][1], p[0][kb][2], p[0][kb][3],
-                           p[1][kb][0], p[1][kb][1], p[1][kb][2], p[1][kb][3]};
-      const float dv8[8] = {ds[0][kb][0], ds[0][kb][1], ds[0][kb][2], ds[0][kb][3],
-                            ds[1][kb][0], ds[1][kb][1], ds[1][kb][2], ds[1][kb][3]};
-      const Frag<T> pf = pack8<T>(pv);
-      const Frag<T> sf = pack8<T>(dv8);
-#pragma unroll
-      for (int db = 0; db < Tr::kDB; ++db) {
-        const T* orow = sOt + (16 * db + l16) * Tr::kLDTQ + 32 * qs;
-        const T* qrow = sQt + (16 * db + l16) * Tr::kLDTQ + 32 * qs;
-        const Frag<T> ot = lds_frag_2x4<T>(orow + 4 * g, orow + 16 + 4 * g);
-        const Frag<T> qt = lds_frag_2x4<T>(qrow + 4 * g, qrow + 16 + 4 * g);
-        dva[db][kb] = mma(dva[db][kb], ot, pf);
-        dka[db][kb] = mma(dka[db][kb], qt, sf);
-      }
-    }
-  }
-}
-
-template <typename T, int D, int NB, bool GLOB>
-__global__ __launch_bounds__(256) void dkdv_kernel(BwdArgs a) {
-  using Tr = BwdTraits<T, D, NB>;
-  __shared__ __attribute__((aligned(16))) T sQ[Tr::kBQ * Tr::kLD];
-  __shared__ __attribute__((aligned(16))) T sO[Tr::kBQ * Tr::kLD];
-  __shared__ __attribute__((aligned(16))) T sQt[D * Tr::kLDTQ];
-  __shared__ __attribute__((aligned(16))) T sOt[D * Tr::kLDTQ];
-  __shared__ __attribute__((aligned(16))) float sL[Tr::kBQ];
-  __shared__ __attribute__((aligned(16))) float sDl[Tr::kBQ];
-  __shared__ __attribute__((aligned(16))) int sGl[Tr::kBQ];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int l16 = lane & 15, g = lane >> 4;
-  const int nbh = a.B * a.Hkv;
-  const int bhk = blockIdx.x % nbh;
-  const int rest = blockIdx.x / nbh;
-  const Doc dc = find_doc(a.docs, rest);
-  const int nck = GLOB ? num_chunks(dc.len, a.chunk_len) : 1;
-  const int tile = GLOB ? dc.item / nck : dc.item;
-  const int chunk = GLOB ? dc.item - tile * nck : 0;
-  const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
-  const int grp = a.Hq / a.Hkv;
-  const int S = dc.len, W = dc.W, rpb = dc.rpb;
-  const bool relay = rpb > 1;
-  const int nrows = GLOB ? (S + W - 1) / W * rpb : S;  // keys: global rows or rows
-  const int k0 = tile * Tr::kBK;
-  const int kw = k0 + wave * Tr::kKW;
-
-  const T* kbase;
-  const T* vbase;
-  int64_t kstride, vstride;
-  if (GLOB) {
-    const int64_t gb = ((int64_t)bhk * a.G + dc.gofs) * D;
-    kbase = static_cast<const T*>(a.gk) + gb;
-    vbase = static_cast<const T*>(a.gv) + gb;
-    kstride = D;
-    vstride = D;
-  } else {
-    kbase = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
-    vbase = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
-    kstride = a.kss;
-    vstride = a.vss;
-  }
-
-  // K^T, V^T as B operands: lane holds row kw + 16kb + l16, dims 32c + 8g ..
-  Frag<T> kf[NB][Tr::kDC], vf[NB][Tr::kDC];
-#pragma unroll
-  for (int kb = 0; kb < NB; ++kb) {
-    const int row = kw + 16 * kb + l16;
-#pragma unroll
-    for (int c = 0; c < Tr::kDC; ++c) {
-      if (row < nrows) {
-        kf[kb][c] = lds_frag_row<T>(kbase + (int64_t)row * kstride + 32 * c + 8 * g);
-        vf[kb][c] = lds_frag_row<T>(vbase + (int64_t)row * vstride + 32 * c + 8 * g);
-      } else {
-        zero_frag(kf[kb][c]);
-        zero_frag(vf[kb][c]);
-      }
-    }
-  }
-  f32x4 dka[Tr::kDB][NB], dva[Tr::kDB][NB];
-#pragma unroll
-  for (int db = 0; db < Tr::kDB; ++db)
-#pragma unroll
-    for (int kb = 0; kb < NB; ++kb) dka[db][kb] = dva[db][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // Query range of the workgroup and of this wave.
-  const bool active = kw < nrows;
-  int q_lo, q_hi, wq_lo, wq_hi;
-  if (GLOB) {
-    const int c_lo = chunk * a.chunk_len;
-    const int c_hi = min(S, c_lo + a.chunk_len);
-    q_lo = max(c_lo, glob_row_first_query(k0, W, rpb));
-    q_hi = c_hi;
-    wq_lo = active ? max(c_lo, glob_row_first_query(kw, W, rpb)) : S;
-    wq_hi = c_hi;
-    // no query of this chunk sees the tile's rows: gsum_kernel skips the
-    // chunk for them (with a single chunk the zeros are written instead)
-    if (q_hi <= q_lo && a.nchunk > 1) return;
-  } else {
-    q_lo = k0;
-    q_hi = min(S, k0 + Tr::kBK - 1 + W);
-    wq_lo = kw;
-    wq_hi = min(S, kw + Tr::kKW - 1 + W);
-  }
-  const int k_last = min(kw + Tr::kKW, nrows) - 1;
-  const float c2 = a.scale * kLog2e;
-  TileStage<T, D, Tr::kBQ, Tr::kThreads> stq, sto;
-
-  for (int j = 0; j < grp; ++j) {
-    const int h = hk * grp + j;
-    const int bh = b * a.Hq + h;
-    const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
-    const T* dop =
-        static_cast<const T*>(a.dout) + b * a.dosb + h * a.dosh + (int64_t)dc.off * a.doss;
-    const float* lse = a.lse + (int64_t)bh * a.S + dc.off;
-    const float* delta = a.delta + (int64_t)bh * a.S + dc.off;
-    for (int ts = q_lo; ts < q_hi; ts += Tr::kBQ) {
-      stq.load(qp, a.qss, ts, 0, q_hi, tid);
-      sto.load(dop, a.doss, ts, 0, q_hi, tid);
-      __syncthreads();
-      stq.template store_rows<Tr::kLD>(sQ, tid);
-      stq.template store_cols<Tr::kLDTQ>(sQt, tid);
-      sto.template store_rows<Tr::kLD>(sO, tid);
-      sto.template store_cols<Tr::kLDTQ>(sOt, tid);
-      if (tid < Tr::kBQ) {
-        const int qabs = ts + tid;
-        const bool ok = qabs < q_hi;
-        sL[tid] = ok ? lse[qabs] * kLog2e : 0.f;
-        sDl[tid] = ok ? delta[qabs] : 0.f;
-        if (GLOB) sGl[tid] = ok ? glob_prefix(qabs, W, rpb) : 0;
-      }
-      __syncthreads();
-      const int t_last = min(ts + Tr::kBQ, q_hi) - 1;
-      if (active && t_last >= wq_lo && ts < wq_hi) {
-        bool full;
-        if (GLOB)
-          full = ts + Tr::kBQ <= q_hi && glob_prefix(ts, W, rpb) > k_last;
-        else
-          full = ts >= k_last && ts + Tr::kBQ - 1 - W + 1 <= kw && ts + Tr::kBQ <= q_hi;
-        if (full)
-          dkdv_tile<T, D, NB, GLOB, false>(sQ, sO, sQt, sOt, sL, sDl, sGl, kf, vf, dka, dva, c2,
-                                           l16, g, ts, kw, W, q_hi);
-        else
-          dkdv_tile<T, D, NB, GLOB, true>(sQ, sO, sQt, sOt, sL, sDl, sGl, kf, vf, dka, dva, c2,
-                                          l16, g, ts, kw, W, q_hi);
-      }
-    }
-  }
-
-  // Epilogue. Lane owns key row kw + 16kb + l16, dims 16db + 4g .. +4.
-  if (GLOB) {
-    float* part = a.gpart + part_row(dc, chunk, nbh, bhk, 0) * 2 * D;
-#pragma unroll
-    for (int kb = 0; kb < NB; ++kb) {
-      const int row = kw + 16 * kb + l16;
-      if (row >= nrows) continue;
-      float* pk = part + (int64_t)row * 2 * D;
-#pragma unroll
-      for (int db = 0; db < Tr::kDB; ++db) {
-        *reinterpret_cast<f32x4*>(pk + 16 * db + 4 * g) = dka[db][kb] * a.scale;
-        *reinterpret_cast<f32x4*>(pk + D + 16 * db + 4 * g) = dva[db][kb];
-      }
-    }
-    return;
-  }
-  T* dkp = static_cast<T*>(a.dk) + b * a.dksb + hk * a.dksh + (int64_t)dc.off * a.dkss;
-  T* dvp = static_cast<T*>(a.dv) + b * a.dvsb + hk * a.dvsh + (int64_t)dc.off * a.dvss;
-  const float rsc = (relay && a.rscale) ? a.rscale[hk] : 1.f;
-#pragma unroll
-  for (int kb = 0; kb < NB; ++kb) {
-    const int j = kw + 16 * kb + l16;
-    if (j >= S) continue;
-#pragma unroll
-    for (int db = 0; db < Tr::kDB; ++db) dka[db][kb] *= a.scale;
-    // Global rows whose source is row j: the strided row of its block and
-    // any relay row selected from it (reference scatter, core.py:2767-2815).
-    const int rblk = j / W;
-    int grow[5];
-    float gsc[5];
-    int nm = 0;
-    if (j == rblk * W) {
-      grow[nm] = rblk * rpb;
-      gsc[nm++] = 1.f;
-    }
-    if (relay) {
-      const int32_t* src = a.src + ((int64_t)bhk * a.NB + dc.bofs + rblk) * a.top_k;
-      for (int t = 0; t < a.top_k; ++t) {
-        if (src[t] == j) {
-          grow[nm] = rblk * rpb + 1 + t;
-          gsc[nm++] = rsc;
-        }
-      }
-    }
-    // the chunk partials of the global rows are summed into chunk 0
-    for (int m = 0; m < nm; ++m) {
-      const float* pk = a.gpart + part_row(dc, 0, nbh, bhk, grow[m]) * 2 * D;
-#pragma unroll
-      for (int db = 0; db < Tr::kDB; ++db) {
-        dka[db][kb] += *reinterpret_cast<const f32x4*>(pk + 16 * db + 4 * g) * gsc[m];
-        dva[db][kb] += *reinterpret_cast<const f32x4*>(pk + D + 16 * db + 4 * g) * gsc[m];
-      }
-    }
-#pragma unroll
-    for (int db = 0; db < Tr::kDB; ++db) {
-      store4<T>(dkp + (int64_t)j * a.dkss + 16 * db + 4 * g, dka[db][kb], 1.f);
-      store4<T>(dvp + (int64_t)j * a.dvss + 16 * db + 4 * g, dva[db][kb], 1.f);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 3b. Chunk partials of the global rows summed into chunk 0, in chunk order
+// 3. Chunk partials of the global rows summed into chunk 0, in chunk order
 // (one float4 per thread; work items: the documents' rows x 2D / 4 / 256).
 // Only chunks with a query that sees the row are read.
 // ---------------------------------------------------------------------------
@@ -651,33 +151,6 @@ __global__ __launch_bounds__(1024) void dalpha_kernel(BwdArgs a) {
 // computed; transposed operands (K^T for dQ, Q^T and dO^T for dK/dV) are
 // read with ds_read_b64_tr_b16 from the same row-major tiles.
 // ---------------------------------------------------------------------------
-// Lane offsets; at D = 256 the upper half of a row lies 256 bytes behind the
-// lower half (the swizzle permutes 16 chunks): an immediate of the read.
-template <int D>
-struct LaneOffs {
-  static constexpr int kD = D < 128 ? D : 128;
-  int row[kD / 32];  // row fragment, chunk 4c + g, row lane%16
-  int tr[kD / 16];   // transposed fragment, columns 16 db ..
-  __device__ __forceinline__ int row_at(int c) const {
-    return row[c % (kD / 32)] + c / (kD / 32) * 256;
-  }
-  __device__ __forceinline__ int tr_at(int db) const {
-    return tr[db % (kD / 16)] + db / (kD / 16) * 256;
-  }
-};
-
-template <int D>
-__device__ __forceinline__ LaneOffs<D> lane_offs(int lane) {
-  using Tile = SwzTile<D, 64>;
-  LaneOffs<D> o;
-  const int g = lane >> 4;
-#pragma unroll
-  for (int c = 0; c < o.kD / 32; ++c) o.row[c] = Tile::row_lane_off(lane, 4 * c + g);
-#pragma unroll
-  for (int db = 0; db < o.kD / 16; ++db) o.tr[db] = Tile::tr_lane_off(lane, 16 * db);
-  return o;
-}
-
 // Query-centric dQ for QB blocks of 16 queries per wave against one BN-key
 // tile, in 32-key halves: S = K . Q^T and dP - Delta = V . dO^T - Delta (key
 // on rows; the products accumulate onto -Delta, so no subtraction per
@@ -857,7 +330,8 @@ void dq2_kernel(BwdArgs a) {
   };
   issue(0, stage0[0]);
 
-  const LaneOffs<D> lo = lane_offs<D>(lane);
+  LaneOffs<D> lo;
+  lo.init(lane);
   Frag<T> qf[QB][D / 32], df[QB][D / 32];
   int qi[QB];
   float lse2[QB], ndl[QB];
@@ -1041,7 +515,8 @@ void dq_wide_kernel(BwdArgs a) {
   issue_k(0, sK0);
   issue_v(0);
 
-  const LaneOffs<D> lo = lane_offs<D>(lane);
+  LaneOffs<D> lo;
+  lo.init(lane);
   // Delta = rowsum(O * dO) of the wave's queries, stored negated with
   // -lse * log2(e) for the dK/dV kernels (see dq2_kernel). Rows past the
   // document read its last row; their results are never stored.
@@ -1113,6 +588,80 @@ void dq_wide_kernel(BwdArgs a) {
   T* row = static_cast<T*>(a.dq) + b * a.dqsb + h * a.dqsh + (int64_t)(dc.off + qi) * a.dqss;
 #pragma unroll
   for (int db = 0; db < D / 16; ++db) store4<T>(row + 16 * db + 4 * g, dqa[db][0], a.scale);
+}
+
+// Epilogues of the dK/dV kernels: lane (l16, g) owns key row kw + 16kb + l16,
+// dims 16db + 4g .. +4 of each block. Global rows: the chunk's fp32 partial.
+template <int D, int KB>
+__device__ __forceinline__ void write_part(const BwdArgs& a, const Doc& dc, int chunk, int nbh,
+                                           int bhk, int kw, int nrows, int l16, int g,
+                                           const f32x4 (&dka)[D / 16][KB],
+                                           const f32x4 (&dva)[D / 16][KB]) {
+  float* part = a.gpart + part_row(dc, chunk, nbh, bhk, 0) * 2 * D;
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int row = kw + 16 * kb + l16;
+    if (row >= nrows) continue;
+    float* pk = part + (int64_t)row * 2 * D;
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) {
+      *reinterpret_cast<f32x4*>(pk + 16 * db + 4 * g) = dka[db][kb] * a.scale;
+      *reinterpret_cast<f32x4*>(pk + D + 16 * db + 4 * g) = dva[db][kb];
+    }
+  }
+}
+
+// Local rows: dK/dV of row j, with the global rows whose source is row j (the
+// strided row of its block and any relay row selected from it; reference
+// scatter, core.py:2767-2815).
+template <typename T, int D, int KB>
+__device__ __forceinline__ void write_local(const BwdArgs& a, const Doc& dc, int nbh, int b, int hk,
+                                            int kw, int l16, int g, f32x4 (&dka)[D / 16][KB],
+                                            f32x4 (&dva)[D / 16][KB]) {
+  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+  const bool relay = rpb > 1;
+  const int bhk = b * a.Hkv + hk;
+  T* dkp = static_cast<T*>(a.dk) + b * a.dksb + hk * a.dksh + (int64_t)dc.off * a.dkss;
+  T* dvp = static_cast<T*>(a.dv) + b * a.dvsb + hk * a.dvsh + (int64_t)dc.off * a.dvss;
+  const float rsc = (relay && a.rscale) ? a.rscale[hk] : 1.f;
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int j = kw + 16 * kb + l16;
+    if (j >= S) continue;
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) dka[db][kb] *= a.scale;
+    const int rblk = j / W;
+    int grow[5];
+    float gsc[5];
+    int nm = 0;
+    if (j == rblk * W) {
+      grow[nm] = rblk * rpb;
+      gsc[nm++] = 1.f;
+    }
+    if (relay) {
+      const int32_t* src = a.src + ((int64_t)bhk * a.NB + dc.bofs + rblk) * a.top_k;
+      for (int t = 0; t < a.top_k; ++t) {
+        if (src[t] == j) {
+          grow[nm] = rblk * rpb + 1 + t;
+          gsc[nm++] = rsc;
+        }
+      }
+    }
+    // the chunk partials of the global rows are summed into chunk 0
+    for (int m = 0; m < nm; ++m) {
+      const float* pk = a.gpart + part_row(dc, 0, nbh, bhk, grow[m]) * 2 * D;
+#pragma unroll
+      for (int db = 0; db < D / 16; ++db) {
+        dka[db][kb] += *reinterpret_cast<const f32x4*>(pk + 16 * db + 4 * g) * gsc[m];
+        dva[db][kb] += *reinterpret_cast<const f32x4*>(pk + D + 16 * db + 4 * g) * gsc[m];
+      }
+    }
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) {
+      store4<T>(dkp + (int64_t)j * a.dkss + 16 * db + 4 * g, dka[db][kb], 1.f);
+      store4<T>(dvp + (int64_t)j * a.dvss + 16 * db + 4 * g, dva[db][kb], 1.f);
+    }
+  }
 }
 
 // Key-centric dK/dV: each wave owns KB blocks of 16 key rows (rows of k/v,
@@ -1324,7 +873,8 @@ void dkdv2_kernel(BwdArgs a) {
   const int fq = Fill::lane_off(wave & (FW - 1), lane, qbytes);
   const int fo = Fill::lane_off(wave & (FW - 1), lane, obytes);
 
-  const LaneOffs<D> lo = lane_offs<D>(lane);
+  LaneOffs<D> lo;
+  lo.init(lane);
   Frag<T> kf[KB][D / 32], vf[KB][D / 32];
   int qmin[KB], qmax[KB];
   unsigned qspan[KB];
@@ -1451,62 +1001,422 @@ void dkdv2_kernel(BwdArgs a) {
     if (it + 1 < ntot) step(std::integral_constant<int, 1>{}, it + 1);
   }
 
+  if (GLOB)
+    write_part<D, KB>(a, dc, chunk, nbh, bhk, kw, nrows, l16, g, dka, dva);
+  else
+    write_local<T, D, KB>(a, dc, nbh, b, hk, kw, l16, g, dka, dva);
+}
+
+// ---------------------------------------------------------------------------
+// fp32 backward: dq2 and dkdv2 with every operand split in three bf16 pieces
+// (Split). 4 waves of 16 queries (dQ) or 16 key rows (dK/dV), whose own
+// operands stay split in registers; 32-row tiles of K and V (Q and dO) are
+// staged through registers and split once per workgroup, up to D = 64 in two
+// LDS stages with one barrier per tile; dS and P are split in registers.
+// Against the fp32-MFMA kernels before them (dQ with the separate Delta pass /
+// global rows / local rows), H=8: S=32768 D=64 527 / 554 / 467 -> 320 / 308 /
+// 238 us, D=128 1246 / 1600 / 1041 -> 695 / 711 / 452 us, S=4096 D=64 59 / 49 /
+// 42 -> 30 / 30 / 21 us; H=4 S=8192 D=256 194 / 207 / 146 -> 156 / 140 / 121 us.
+// ---------------------------------------------------------------------------
+constexpr int kF32Waves = 4, kF32BN = 32;
+
+template <int D, bool MASK>
+__device__ __forceinline__ void dq_f32_tile(const char* tK, const char* tV, const LaneOffs<D>& lo,
+                                            const Split (&qf)[D / 32], const Split (&df)[D / 32],
+                                            f32x4 (&dqa)[D / 16], float lse2, float ndl, float c2,
+                                            int g, const TileMask<1>& mk) {
+  using Stage = SplitStage<D, kF32BN, 64 * kF32Waves>;
+  using Tile = typename Stage::Tile;
+  f32x4 sc[2], dp[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    sc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    dp[h] = f32x4{ndl, ndl, ndl, ndl};
+  }
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    Split kf[2], vf[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      kf[h] = Stage::row_frag(tK + h * Tile::kBlk16 + lo.row_at(c));
+      vf[h] = Stage::row_frag(tV + h * Tile::kBlk16 + lo.row_at(c));
+    }
+    // consecutive MFMAs go to different accumulators
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        sc[h] = mma(sc[h], kf[h].p[split_a(t)], qf[c].p[split_b(t)]);
+        dp[h] = mma(dp[h], vf[h].p[split_a(t)], df[c].p[split_b(t)]);
+      }
+  }
+  float ds[8];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float x = fmaf(sc[h][r], c2, -lse2);
+      if (MASK && !mk.ok(16 * h + 4 * g + r, 0)) x = -__builtin_huge_valf();
+      ds[4 * h + r] = __builtin_amdgcn_exp2f(x) * dp[h][r];
+    }
+  const Split dsf = split8<true>(ds);
+#pragma unroll
+  for (int db = 0; db < D / 16; db += 2) {
+    Split kt[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) kt[e] = Stage::tr_frag(tK + lo.tr_at(db + e));
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        dqa[db + e] = mma(dqa[db + e], kt[e].p[split_a(t)], dsf.p[split_b(t)]);
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2)))
+void dq_f32_kernel(BwdArgs a) {
+  constexpr int NW = kF32Waves, BN = kF32BN, kBM = 16 * NW;
+  constexpr int kStages = D <= 64 ? 2 : 1;
+  using Stage = SplitStage<D, BN, 64 * NW>;
+  __shared__ __attribute__((aligned(1024))) char lds[kStages][2][Stage::kBytes];  // K, V
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int nbh = a.B * a.Hq;
+  const int bh = blockIdx.x % nbh;
+  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
+  const int b = bh / a.Hq, h = bh % a.Hq;
+  const int hk = h / (a.Hq / a.Hkv);
+  const int m0 = tile * kBM;
+  const int q0 = m0 + wave * 16;
+  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+
+  const float* qp = static_cast<const float*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
+  const float* dop =
+      static_cast<const float*>(a.dout) + b * a.dosb + h * a.dosh + (int64_t)dc.off * a.doss;
+  const float* opp = static_cast<const float*>(a.o) + b * a.osb + h * a.osh + (int64_t)dc.off * a.oss;
+  const float* kp = static_cast<const float*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
+  const float* vp = static_cast<const float*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
+  const int64_t row_bh = (int64_t)bh * a.S + dc.off;
+  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
+  const float* gkp = static_cast<const float*>(a.gk) + gbase;
+  const float* gvp = static_cast<const float*>(a.gv) + gbase;
+
+  const int lo_k = max(0, m0 - W + 1);
+  const int hi = min(S, m0 + kBM);
+  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int nloc = (hi - lo_k + BN - 1) / BN;
+  const int nglob = (gmax + BN - 1) / BN;
+  const int ntot = nloc + nglob;
+  // global tiles first, then the local window from its highest tile down
+  auto row0 = [&](int it) { return it >= nglob ? lo_k + (nloc - 1 - (it - nglob)) * BN : it * BN; };
+  Stage stk, stv;
+  auto load = [&](int it) {
+    if (it >= nglob) {
+      stk.load(kp, a.kss, row0(it), hi, tid);
+      stv.load(vp, a.vss, row0(it), hi, tid);
+    } else {
+      stk.load(gkp, D, row0(it), gmax, tid);
+      stv.load(gvp, D, row0(it), gmax, tid);
+    }
+  };
+  auto store = [&](int it) {
+    char(&dst)[2][Stage::kBytes] = lds[kStages == 2 ? it & 1 : 0];
+    stk.store(dst[0], tid);
+    stv.store(dst[1], tid);
+  };
+  load(0);
+
+  LaneOffs<D> lo;
+  lo.init(lane);
+  // Delta = rowsum(O * dO) of the wave's queries, stored negated with
+  // -lse * log2(e) for the dK/dV kernels (see dq2_kernel). Rows past the
+  // document read its last row; their results are never stored.
+  Split qf[D / 32], df[D / 32];
+  const int qi = q0 + l16;
+  const int qr = min(qi, S - 1);
+  const bool ok = qi < S;
+  const float lse2 = ok ? a.lse[row_bh + qr] * kLog2e : 0.f;
+  float od = 0.f;
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    qf[c] = load_split(qp + (int64_t)qr * a.qss + 32 * c + 8 * g);
+    const float* pd = dop + (int64_t)qr * a.doss + 32 * c + 8 * g;
+    const float* po = opp + (int64_t)qr * a.oss + 32 * c + 8 * g;
+    float xd[8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f32x4 d4 = reinterpret_cast<const f32x4*>(pd)[i], o4 = reinterpret_cast<const f32x4*>(po)[i];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        xd[4 * i + r] = d4[r];
+        od = fmaf(o4[r], d4[r], od);
+      }
+    }
+    df[c] = split8<true>(xd);
+  }
+  od += __shfl_xor(od, 16);
+  od += __shfl_xor(od, 32);
+  if (ok && g == 0) {
+    a.delta[row_bh + qi] = -od;
+    a.nlse2[row_bh + qi] = -lse2;
+  }
+  const float c2 = a.scale * kLog2e;
+  f32x4 dqa[D / 16];
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) dqa[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool active = q0 < S;
+  const int q_last = min(q0 + 16, S) - 1;
+  const int w_lo = max(0, q0 - W + 1);
+  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
+  const int glen = glob_prefix(qi, W, rpb);
+
+  store(0);
+  __syncthreads();
+  for (int it = 0; it < ntot; ++it) {
+    if (it + 1 < ntot) load(it + 1);
+    const char(&cur)[2][Stage::kBytes] = lds[kStages == 2 ? it & 1 : 0];
+    const bool loc = it >= nglob;
+    const int ts = row0(it);
+    if (active && (loc ? (ts <= q_last && ts + BN - 1 >= w_lo) : ts < wg_hi)) {
+      const bool full = loc ? (ts >= q_last - W + 1 && ts + BN - 1 <= q0) : ts + BN <= wg_lo;
+      TileMask<1> mk;
+      mk.hi[0] = loc ? qi - ts : glen - 1 - ts;
+      mk.span[0] = loc ? (unsigned)(W - 1) : 0x7fffffffu;
+      if (full)
+        dq_f32_tile<D, false>(cur[0], cur[1], lo, qf, df, dqa, lse2, -od, c2, g, mk);
+      else
+        dq_f32_tile<D, true>(cur[0], cur[1], lo, qf, df, dqa, lse2, -od, c2, g, mk);
+    }
+    if (kStages == 1) __syncthreads();  // every wave is done with this tile
+    if (it + 1 < ntot) store(it + 1);
+    __syncthreads();
+  }
+
+  if (!active || qi >= S) return;
+  float* row = static_cast<float*>(a.dq) + b * a.dqsb + h * a.dqsh + (int64_t)(dc.off + qi) * a.dqss;
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) store4<float>(row + 16 * db + 4 * g, dqa[db], a.scale);
+}
+
+// A key row sees the queries [qmin, qmin + qspan] (see dkdv2_kernel).
+template <int D, bool MASK, bool SUM>
+__device__ __forceinline__ void dkdv_f32_tile(const char* tQ, const char* tO, const float* sL,
+                                              const float* sDl, const LaneOffs<D>& lo,
+                                              const Split (&kf)[D / 32], const Split (&vf)[D / 32],
+                                              f32x4 (&dka)[D / 16][1], f32x4 (&dva)[D / 16][1],
+                                              float c2, int g, int q_off, unsigned qspan) {
+  using Stage = SplitStage<D, kF32BN, 64 * kF32Waves>;
+  using Tile = typename Stage::Tile;
+  f32x4 sc[2], dp[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    sc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    dp[h] = *reinterpret_cast<const f32x4*>(sDl + 16 * h + 4 * g);
+  }
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    Split qa[2], oa[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      qa[h] = Stage::row_frag(tQ + h * Tile::kBlk16 + lo.row_at(c));
+      oa[h] = Stage::row_frag(tO + h * Tile::kBlk16 + lo.row_at(c));
+    }
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        sc[h] = mma(sc[h], qa[h].p[split_a(t)], kf[c].p[split_b(t)]);
+        dp[h] = mma(dp[h], oa[h].p[split_a(t)], vf[c].p[split_b(t)]);
+      }
+  }
+  float p[8], ds[8];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const f32x4 nlq = *reinterpret_cast<const f32x4*>(sL + 16 * h + 4 * g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float x = fmaf(sc[h][r], c2, nlq[r]);
+      if (MASK && (unsigned)(16 * h + r + q_off) > qspan) x = -__builtin_huge_valf();
+      p[4 * h + r] = __builtin_amdgcn_exp2f(x);
+      ds[4 * h + r] = p[4 * h + r] * dp[h][r];
+    }
+  }
+  const Split pf = split8<false>(p), sf = split8<true>(ds);
+  // SUM (global rows): a tile's six products are summed from zero and added
+  // once. A row of the first blocks sums over thousands of queries, where six
+  // roundings of the long sum per tile would show (dK at S = 131072: relative
+  // error 1.4e-6; 5.2e-7 so; the fp32 MFMA's 1.2e-6). A local row's sum is
+  // short.
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) {
+    const Split ot = Stage::tr_frag(tO + lo.tr_at(db));
+    const Split qt = Stage::tr_frag(tQ + lo.tr_at(db));
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 tv = SUM ? zero : dva[db][0], tk = SUM ? zero : dka[db][0];
+#pragma unroll
+    for (int t = 0; t < 6; ++t) {
+      tv = mma(tv, ot.p[split_a(t)], pf.p[split_b(t)]);
+      tk = mma(tk, qt.p[split_a(t)], sf.p[split_b(t)]);
+    }
+    dva[db][0] = SUM ? dva[db][0] + tv : tv;
+    dka[db][0] = SUM ? dka[db][0] + tk : tk;
+  }
+}
+
+// At D = 128 the global-row kernel needs 350 registers: one wave per SIMD and
+// two LDS stages (at 256 registers it spills 82: 835 us against 761, B=1 H=8
+// S=32768); the local one keeps 256 (24 spilled) and two workgroups per CU.
+template <int D, bool GLOB>
+constexpr bool kF32OneWave = D > 128 || (GLOB && D == 128);
+
+template <int D, bool GLOB>
+__global__ __launch_bounds__(64 * kF32Waves)
+__attribute__((amdgpu_waves_per_eu(kF32OneWave<D, GLOB> ? 1 : 2)))
+void dkdv_f32_kernel(BwdArgs a) {
+  constexpr int NW = kF32Waves, kBK = 16 * NW, kBQ = kF32BN;
+  constexpr int kStages = D <= 64 || (GLOB && D == 128) ? 2 : 1;
+  using Stage = SplitStage<D, kBQ, 64 * NW>;
+  __shared__ __attribute__((aligned(1024))) char lds[kStages][2][Stage::kBytes];  // Q, dO
+  __shared__ __attribute__((aligned(16))) float sld[kStages][2][kBQ];  // -lse log2(e), -Delta
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int nbh = a.B * a.Hkv;
+  const int bhk = blockIdx.x % nbh;
+  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const int nck = GLOB ? num_chunks(dc.len, a.chunk_len) : 1;
+  const int tile = GLOB ? dc.item / nck : dc.item;
+  const int chunk = GLOB ? dc.item - tile * nck : 0;
+  const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
+  const int grp = a.Hq / a.Hkv;
+  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+  const int nrows = GLOB ? doc_rows(S, W, rpb) : S;  // keys: global rows or rows
+  const int k0 = tile * kBK;
+  const int kw = k0 + wave * 16;
+
+  const float *kbase, *vbase;
+  int64_t kstride, vstride;
   if (GLOB) {
-    float* part = a.gpart + part_row(dc, chunk, nbh, bhk, 0) * 2 * D;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      const int row = kw + 16 * kb + l16;
-      if (row >= nrows) continue;
-      float* pk = part + (int64_t)row * 2 * D;
-#pragma unroll
-      for (int db = 0; db < D / 16; ++db) {
-        *reinterpret_cast<f32x4*>(pk + 16 * db + 4 * g) = dka[db][kb] * a.scale;
-        *reinterpret_cast<f32x4*>(pk + D + 16 * db + 4 * g) = dva[db][kb];
-      }
-    }
-    return;
+    const int64_t gb = ((int64_t)bhk * a.G + dc.gofs) * D;
+    kbase = static_cast<const float*>(a.gk) + gb;
+    vbase = static_cast<const float*>(a.gv) + gb;
+    kstride = vstride = D;
+  } else {
+    kbase = static_cast<const float*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
+    vbase = static_cast<const float*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
+    kstride = a.kss;
+    vstride = a.vss;
   }
-  T* dkp = static_cast<T*>(a.dk) + b * a.dksb + hk * a.dksh + (int64_t)dc.off * a.dkss;
-  T* dvp = static_cast<T*>(a.dv) + b * a.dvsb + hk * a.dvsh + (int64_t)dc.off * a.dvss;
-  const float rsc = (relay && a.rscale) ? a.rscale[hk] : 1.f;
-#pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
-    const int j = kw + 16 * kb + l16;
-    if (j >= S) continue;
-#pragma unroll
-    for (int db = 0; db < D / 16; ++db) dka[db][kb] *= a.scale;
-    const int rblk = j / W;
-    int grow[5];
-    float gsc[5];
-    int nm = 0;
-    if (j == rblk * W) {
-      grow[nm] = rblk * rpb;
-      gsc[nm++] = 1.f;
-    }
-    if (relay) {
-      const int32_t* src = a.src + ((int64_t)bhk * a.NB + dc.bofs + rblk) * a.top_k;
-      for (int t = 0; t < a.top_k; ++t) {
-        if (src[t] == j) {
-          grow[nm] = rblk * rpb + 1 + t;
-          gsc[nm++] = rsc;
-        }
-      }
-    }
-    // the chunk partials of the global rows are summed into chunk 0
-    for (int m = 0; m < nm; ++m) {
-      const float* pk = a.gpart + part_row(dc, 0, nbh, bhk, grow[m]) * 2 * D;
-#pragma unroll
-      for (int db = 0; db < D / 16; ++db) {
-        dka[db][kb] += *reinterpret_cast<const f32x4*>(pk + 16 * db + 4 * g) * gsc[m];
-        dva[db][kb] += *reinterpret_cast<const f32x4*>(pk + D + 16 * db + 4 * g) * gsc[m];
-      }
-    }
-#pragma unroll
-    for (int db = 0; db < D / 16; ++db) {
-      store4<T>(dkp + (int64_t)j * a.dkss + 16 * db + 4 * g, dka[db][kb], 1.f);
-      store4<T>(dvp + (int64_t)j * a.dvss + 16 * db + 4 * g, dva[db][kb], 1.f);
-    }
+
+  // queries of the workgroup
+  int q_lo, q_hi;
+  if (GLOB) {
+    const int c_lo = chunk * a.chunk_len;
+    q_hi = min(S, c_lo + a.chunk_len);
+    q_lo = max(c_lo, glob_row_first_query(k0, W, rpb));
+    // see dkdv2_kernel
+    if (q_hi <= q_lo && a.nchunk > 1) return;
+  } else {
+    q_lo = k0;
+    q_hi = min(S, k0 + kBK - 1 + W);
   }
+  const int ntile_q = q_hi > q_lo ? (q_hi - q_lo + kBQ - 1) / kBQ : 0;
+  const int ntot = ntile_q * grp;
+
+  LaneOffs<D> lo;
+  lo.init(lane);
+  const int row = kw + l16;
+  const int rr = min(row, nrows - 1);  // rows past the last one see no query
+  Split kf[D / 32], vf[D / 32];
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c) {
+    kf[c] = load_split(kbase + (int64_t)rr * kstride + 32 * c + 8 * g);
+    vf[c] = load_split(vbase + (int64_t)rr * vstride + 32 * c + 8 * g);
+  }
+  int qmin = GLOB ? (row < nrows ? glob_row_first_query(row, W, rpb) : S) : row;
+  const int qmax = GLOB ? q_hi - 1 : min(row + W, q_hi) - 1;
+  // an empty interval gets a qmin no query reaches
+  const unsigned qspan = qmax >= qmin ? (unsigned)(qmax - qmin) : 0u;
+  if (qmax < qmin) qmin = 1 << 30;
+  f32x4 dka[D / 16][1], dva[D / 16][1];
+#pragma unroll
+  for (int db = 0; db < D / 16; ++db) dka[db][0] = dva[db][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const bool active = kw < nrows;
+  const int k_last = min(kw + 16, nrows) - 1;
+  // queries this wave can see at all, and those every row of it sees
+  const int wq_lo = GLOB ? (active ? max(q_lo, glob_row_first_query(kw, W, rpb)) : S) : kw;
+  const int wq_hi = GLOB ? q_hi : min(q_hi, kw + 15 + W);
+  const int full_lo = GLOB ? (active ? glob_row_first_query(k_last, W, rpb) : S) : k_last;
+  const int full_hi = GLOB ? q_hi : kw + W;  // exclusive
+  const float c2 = a.scale * kLog2e;
+
+  // tiles run head by head of the kv group
+  Stage stq, sto;
+  float st_l = 0.f, st_d = 0.f;
+  int ld_j = 0, ld_t = 0;  // next tile to load
+  auto load = [&]() {
+    const int hq = hk * grp + ld_j;
+    const int ts = q_lo + ld_t * kBQ;
+    stq.load(static_cast<const float*>(a.q) + b * a.qsb + hq * a.qsh + (int64_t)dc.off * a.qss,
+             a.qss, ts, q_hi, tid);
+    sto.load(static_cast<const float*>(a.dout) + b * a.dosb + hq * a.dosh + (int64_t)dc.off * a.doss,
+             a.doss, ts, q_hi, tid);
+    if (tid < kBQ) {
+      const int64_t q = ((int64_t)b * a.Hq + hq) * a.S + dc.off + min(ts + tid, q_hi - 1);
+      st_l = a.nlse2[q];
+      st_d = a.delta[q];
+    }
+    if (++ld_t == ntile_q) {
+      ld_t = 0;
+      ++ld_j;
+    }
+  };
+  auto store = [&](int it) {
+    const int st = kStages == 2 ? it & 1 : 0;
+    stq.store(lds[st][0], tid);
+    sto.store(lds[st][1], tid);
+    if (tid < kBQ) {
+      sld[st][0][tid] = st_l;
+      sld[st][1][tid] = st_d;
+    }
+  };
+  if (ntot > 0) {
+    load();
+    store(0);
+  }
+  __syncthreads();
+  int cu_t = 0;  // query tile being computed
+  for (int it = 0; it < ntot; ++it) {
+    if (it + 1 < ntot) load();
+    const int st = kStages == 2 ? it & 1 : 0;
+    const int ts = q_lo + cu_t * kBQ;
+    if (++cu_t == ntile_q) cu_t = 0;
+    const int t_last = min(ts + kBQ, q_hi) - 1;
+    if (active && t_last >= wq_lo && ts < wq_hi) {
+      const bool full = ts >= full_lo && ts + kBQ <= full_hi && ts + kBQ <= q_hi;
+      const int q_off = ts + 4 * g - qmin;
+      if (full)
+        dkdv_f32_tile<D, false, GLOB>(lds[st][0], lds[st][1], sld[st][0], sld[st][1], lo, kf, vf, dka,
+                                dva, c2, g, q_off, qspan);
+      else
+        dkdv_f32_tile<D, true, GLOB>(lds[st][0], lds[st][1], sld[st][0], sld[st][1], lo, kf, vf, dka,
+                               dva, c2, g, q_off, qspan);
+    }
+    if (kStages == 1) __syncthreads();  // every wave is done with this tile
+    if (it + 1 < ntot) store(it + 1);
+    __syncthreads();
+  }
+  if (GLOB)
+    write_part<D, 1>(a, dc, chunk, nbh, bhk, kw, nrows, l16, g, dka, dva);
+  else
+    write_local<float, D, 1>(a, dc, nbh, b, hk, kw, l16, g, dka, dva);
 }
 
 // dK/dV workgroups: waves of 16 key rows (no register file spill into AGPR
@@ -1577,33 +1487,20 @@ bool narrow_glob(const BwdArgs& a) {
   return most <= kNarrowMaxRows<D>;
 }
 
-// The gfx950-tiled kernels (dq2 and dq_wide, dkdv2) serve fp16/bf16, the
-// generic kernels fp32.
-template <typename T, int D>
-constexpr bool kTiledBwd = sizeof(T) == 2;
-template <int D>
-constexpr int kGenericNB = D > 128 ? 1 : 2;
-
 template <typename T, int D>
 hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
-  constexpr bool kTiled = kTiledBwd<T, D>;
-  constexpr int NB = kGenericNB<D>;
-  using Tr = BwdTraits<T, D, NB>;
-  constexpr int kRows = 256 / (D / 8);
-  // tiled path: dq2_kernel computes Delta for its own queries and stores
-  // -Delta (with -lse * log2(e)) for the dK/dV kernels
-  if (!kTiled && a.group == 0)
-    hipLaunchKernelGGL((delta_kernel<T, D>), dim3((a.S + kRows - 1) / kRows, a.B * a.Hq),
-                       dim3(256), 0, st, a);
+  constexpr bool kF32 = sizeof(T) == 4;
   // work items per document: query tiles (dQ), global-row tiles x query
   // chunks (global dK/dV), key tiles (local dK/dV), each of its kernel's
   // workgroup size
   BwdArgs aq = a, ag = a, al = a;
-  constexpr int kQM = !kTiled ? Tr::kBM : D > 128 ? 16 * kWideWaves : 16 * kDqWaves * kDqQB;  // dQ queries per workgroup
+  constexpr int kQM = kF32 ? 16 * kF32Waves : D > 128 ? 16 * kWideWaves : 16 * kDqWaves * kDqQB;  // dQ queries per workgroup
   set_items(aq.docs, [&](int d) { return (a.docs.len[d] + kQM - 1) / kQM; });
-  const bool narrow = kTiled && narrow_glob<D>(a);
-  const int kGK = !kTiled ? Tr::kBK : narrow ? 16 * kNarrowWaves : 16 * kDkdvGlobWaves<D> * kDkdvKB;
-  constexpr int kLK = kTiled ? 16 * kDkdvLocalWaves * kDkdvLocalKB<D> : Tr::kBK;
+  const bool narrow = !kF32 && narrow_glob<D>(a);
+  const int kGK = kF32     ? 16 * kF32Waves
+                  : narrow ? 16 * kNarrowWaves
+                           : 16 * kDkdvGlobWaves<D> * kDkdvKB;  // rows per workgroup
+  constexpr int kLK = kF32 ? 16 * kF32Waves : 16 * kDkdvLocalWaves * kDkdvLocalKB<D>;
   set_items(ag.docs, [&](int d) {
     return (doc_rows(a.docs.len[d], a.docs.W[d], a.docs.rpb[d]) + kGK - 1) / kGK *
            num_chunks(a.docs.len[d], a.chunk_len);
@@ -1613,28 +1510,29 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   const int nl = al.docs.item0[a.docs.n];
   // one document, D = 128 and a head count that is not a multiple of 8: the
   // dQ and local dK/dV kernels run in the XCD-aware order (as the forward)
-  const bool xq = kTiled && D == 128 && a.docs.n == 1 && (a.B * a.Hq) % 8 != 0;
-  const bool xl = kTiled && D == 128 && a.docs.n == 1 && (a.B * a.Hkv) % 8 != 0;
+  const bool xq = !kF32 && D == 128 && a.docs.n == 1 && (a.B * a.Hq) % 8 != 0;
+  const bool xl = !kF32 && D == 128 && a.docs.n == 1 && (a.B * a.Hkv) % 8 != 0;
   aq.xcd_nt = xq ? nq : 0;
   al.xcd_nt = xl ? nl : 0;
   const int gq = xq ? xcd_grid(a.B * a.Hq, nq) : nq * a.B * a.Hq;
   const int gl = xl ? xcd_grid(a.B * a.Hkv, nl) : nl * a.B * a.Hkv;
-  if constexpr (kTiled) {
+  if constexpr (kF32) {
+    hipLaunchKernelGGL((dq_f32_kernel<D>), dim3(gq), dim3(64 * kF32Waves), 0, st, aq);
+    hipLaunchKernelGGL((dkdv_f32_kernel<D, true>), dim3(ng * a.B * a.Hkv), dim3(64 * kF32Waves), 0,
+                       st, ag);
+  } else {
     if constexpr (D > 128)
       hipLaunchKernelGGL((dq_wide_kernel<T, D>), dim3(gq), dim3(64 * kWideWaves), 0, st, aq);
     else
       hipLaunchKernelGGL((dq2_kernel<T, D, kDqWaves, kDqQB, kDqBN, kDqWPE>), dim3(gq),
                          dim3(64 * kDqWaves), 0, st, aq);
+    // (at D = 256 the one geometry has 64 rows)
     if (D <= 128 && narrow)
       hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kNarrowWaves, kDkdvKB, kNarrowBQ>),
                          dim3(ng * a.B * a.Hkv), dim3(64 * kNarrowWaves), 0, st, ag);
     else
       hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kDkdvGlobWaves<D>, kDkdvKB, kDkdvGlobBQ<D>>),
                          dim3(ng * a.B * a.Hkv), dim3(64 * kDkdvGlobWaves<D>), 0, st, ag);
-  } else {
-    hipLaunchKernelGGL((dq_kernel<T, D, NB>), dim3(nq * a.B * a.Hq), dim3(256), 0, st, aq);
-    hipLaunchKernelGGL((dkdv_kernel<T, D, NB, true>), dim3(ng * a.B * a.Hkv), dim3(256), 0, st,
-                       ag);
   }
   if (a.nchunk > 1) {
     BwdArgs as = a;
@@ -1645,12 +1543,11 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
                        0, st, as);
   }
   if (a.dalpha) hipLaunchKernelGGL((dalpha_kernel<T, D>), dim3(a.Hkv), dim3(1024), 0, st, a);
-  if constexpr (kTiled)
+  if constexpr (kF32)
+    hipLaunchKernelGGL((dkdv_f32_kernel<D, false>), dim3(gl), dim3(64 * kF32Waves), 0, st, al);
+  else
     hipLaunchKernelGGL((dkdv2_kernel<T, D, false, kDkdvLocalWaves, kDkdvLocalKB<D>, kDkdvLocalBQ>),
                        dim3(gl), dim3(64 * kDkdvLocalWaves), 0, st, al);
-  else
-    hipLaunchKernelGGL((dkdv_kernel<T, D, NB, false>), dim3(nl * a.B * a.Hkv), dim3(256), 0, st,
-                       al);
   return hipGetLastError();
 }
 
@@ -1686,7 +1583,7 @@ ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len,
   //   B=1 H=8 D=64 S=16384: 32 (64 was 10% slower)
   // (D = 256: 64 rows per 4-wave workgroup, two workgroups per CU by their
   // 66 KB of LDS)
-  const int rows = D > 128    ? BwdTraits<f16, 256, 1>::kBK
+  const int rows = D > 128    ? 16 * kDkdvGlobWaves<256> * kDkdvKB
                    : D == 128 ? 16 * kDkdvGlobWaves<128> * kDkdvKB
                               : 16 * kDkdvGlobWaves<64> * kDkdvKB;
   const int slots = (cus > 0 ? cus : 256) * (D == 128 ? 1 : 2);
@@ -1741,7 +1638,7 @@ ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len,
 }
 
 size_t bwd_workspace_layout(int D, int B, int Hq, int Hkv, int S, int64_t part_rows) {
-  // Delta (2-byte path: -Delta) and -lse * log2(e) per query, then the chunk
+  // -Delta and -lse * log2(e) per query, then the chunk
   // partials
   const size_t delta = (((size_t)B * Hq * S * 4) + 255) / 256 * 256;
   const size_t part = (size_t)part_rows * B * Hkv * 2 * D * 4;
@@ -1750,15 +1647,14 @@ size_t bwd_workspace_layout(int D, int B, int Hq, int Hkv, int S, int64_t part_r
 
 bool bwd_tile_config(int dtype, int D, int out[9]) {
   if (dtype < 0 || dtype > 2 || (D != 32 && D != 64 && D != 128 && D != 256)) return false;
-  if (D == 256) {
-    using Tr = BwdTraits<f16, 256, 1>;  // the same geometry for every dtype
-    const int waves = Tr::kThreads / 64;
-    const int v[9] = {waves, Tr::kBM, Tr::kBN, waves, Tr::kBK, Tr::kBQ, waves, Tr::kBK, Tr::kBQ};
+  if (dtype == 2) {
+    constexpr int w = kF32Waves, r = 16 * kF32Waves, n = kF32BN;
+    const int v[9] = {w, r, n, w, r, n, w, r, n};
     for (int i = 0; i < 9; ++i) out[i] = v[i];
-  } else if (dtype == 2) {
-    using Tr = BwdTraits<float, 128>;
-    const int waves = Tr::kThreads / 64;
-    const int v[9] = {waves, Tr::kBM, Tr::kBN, waves, Tr::kBK, Tr::kBQ, waves, Tr::kBK, Tr::kBQ};
+  } else if (D == 256) {
+    const int v[9] = {kWideWaves,      16 * kWideWaves,                     kWideBN,
+                      kDkdvGlobWaves<256>, 16 * kDkdvGlobWaves<256> * kDkdvKB, kDkdvGlobBQ<256>,
+                      kDkdvLocalWaves, 16 * kDkdvLocalWaves * kDkdvLocalKB<256>, kDkdvLocalBQ};
     for (int i = 0; i < 9; ++i) out[i] = v[i];
   } else {
     const int gw = D == 128 ? kDkdvGlobWaves<128> : kDkdvGlobWaves<64>;

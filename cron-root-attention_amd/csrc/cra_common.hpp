@@ -2,7 +2,7 @@
 // fragments, LDS tile staging and the sqrt(N) index geometry.
 //
 // MFMA shape used everywhere: v_mfma_f32_16x16x32_{f16,bf16} (fp32 inputs:
-// eight v_mfma_f32_16x16x4_f32). Register layout of one wave (64 lanes),
+// six of them, see Split). Register layout of one wave (64 lanes),
 // l16 = lane % 16, g = lane / 16:
 //   A operand (16 x 32):  lane holds A[row = l16][k = kappa(g, s)], s = 0..7
 //   B operand (32 x 16):  lane holds B[k = kappa(g, s)][col = l16]
@@ -44,14 +44,6 @@ __device__ __forceinline__ f32x4 mma(f32x4 c, const Frag<bf16>& a, const Frag<bf
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a.w[0]),
                                                  __builtin_bit_cast(bf16x8, b.w[0]), c, 0, 0, 0);
 }
-__device__ __forceinline__ f32x4 mma(f32x4 c, const Frag<float>& a, const Frag<float>& b) {
-  const float* pa = reinterpret_cast<const float*>(a.w);
-  const float* pb = reinterpret_cast<const float*>(b.w);
-#pragma unroll
-  for (int s = 0; s < 8; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[s], pb[s], c, 0, 0, 0);
-  return c;
-}
-
 // Element conversions (round to nearest even, as torch's .to(dtype)).
 template <typename T>
 __device__ __forceinline__ T from_f32(float x);
@@ -65,25 +57,19 @@ __device__ __forceinline__ float from_f32<float>(float x) { return x; }
 template <typename T>
 __device__ __forceinline__ float to_f32(T x) { return (float)x; }
 
-// Packs eight fp32 values into a fragment of T (pairwise conversions, round
-// to nearest even).
+// Packs eight fp32 values into a fragment of a 2-byte T (pairwise conversions,
+// round to nearest even).
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef f16 f16x2 __attribute__((ext_vector_type(2)));
 typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
 template <typename T>
 __device__ __forceinline__ Frag<T> pack8(const float (&v)[8]) {
+  typedef T t2 __attribute__((ext_vector_type(2)));
   Frag<T> f;
-  if constexpr (sizeof(T) == 2) {
-    typedef T t2 __attribute__((ext_vector_type(2)));
-    uint32_t* w = reinterpret_cast<uint32_t*>(f.w);
+  uint32_t* w = reinterpret_cast<uint32_t*>(f.w);
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-      w[s] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v[2 * s], v[2 * s + 1]}, t2));
-  } else {
-    T* e = reinterpret_cast<T*>(f.w);
-#pragma unroll
-    for (int s = 0; s < 8; ++s) e[s] = from_f32<T>(v[s]);
-  }
+  for (int s = 0; s < 4; ++s)
+    w[s] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v[2 * s], v[2 * s + 1]}, t2));
   return f;
 }
 
@@ -98,87 +84,6 @@ __device__ __forceinline__ Frag<T> lds_frag_row(const T* p) {
   for (int i = 0; i < Frag<T>::kWords; ++i) f.w[i] = reinterpret_cast<const uint4*>(p)[i];
   return f;
 }
-
-// Two runs of four consecutive elements (kappa of a C-built fragment).
-template <typename T>
-__device__ __forceinline__ Frag<T> lds_frag_2x4(const T* p0, const T* p1) {
-  Frag<T> f;
-  if constexpr (sizeof(T) == 2) {
-    uint2 a = *reinterpret_cast<const uint2*>(p0);
-    uint2 b = *reinterpret_cast<const uint2*>(p1);
-    f.w[0] = make_uint4(a.x, a.y, b.x, b.y);
-  } else {
-    f.w[0] = *reinterpret_cast<const uint4*>(p0);
-    f.w[1] = *reinterpret_cast<const uint4*>(p1);
-  }
-  return f;
-}
-
-// ---------------------------------------------------------------------------
-// Cooperative staging of ROWS x D tiles from HBM into LDS.
-// Each thread owns RPT consecutive rows of one 8-element column group; the
-// global reads are 16-byte vectors, consecutive threads read consecutive
-// 16-byte pieces of a row. Rows outside [row_lo, row_hi) read as zero.
-// ---------------------------------------------------------------------------
-template <typename T, int D, int ROWS, int NT>
-struct TileStage {
-  static constexpr int kColGroups = D / 8;
-  static constexpr int kRowGroups = (NT / kColGroups) < ROWS ? NT / kColGroups : ROWS;
-  static constexpr int kRPT = ROWS / kRowGroups;  // rows per thread
-  static_assert(kRPT >= 1 && kRowGroups * kRPT == ROWS, "tile/thread mismatch");
-  static constexpr int kWords = Frag<T>::kWords;
-  uint4 r[kRPT][kWords];
-
-  // Threads beyond kRowGroups * kColGroups hold no rows.
-  __device__ __forceinline__ static bool owner(int tid) { return tid < kRowGroups * kColGroups; }
-
-  __device__ __forceinline__ void load(const T* base, int64_t row_stride, int row0, int row_lo,
-                                       int row_hi, int tid) {
-    const int cg = tid % kColGroups;
-    const int rg = tid / kColGroups;
-#pragma unroll
-    for (int i = 0; i < kRPT; ++i) {
-      const int row = row0 + rg * kRPT + i;
-      if (owner(tid) && row >= row_lo && row < row_hi) {
-        const uint4* src = reinterpret_cast<const uint4*>(base + (int64_t)row * row_stride + cg * 8);
-#pragma unroll
-        for (int w = 0; w < kWords; ++w) r[i][w] = src[w];
-      } else {
-#pragma unroll
-        for (int w = 0; w < kWords; ++w) r[i][w] = make_uint4(0, 0, 0, 0);
-      }
-    }
-  }
-
-  // Row-major copy: tile[row][d], row stride LD elements.
-  template <int LD>
-  __device__ __forceinline__ void store_rows(T* tile, int tid) const {
-    if (!owner(tid)) return;
-    const int cg = tid % kColGroups;
-    const int rg = tid / kColGroups;
-#pragma unroll
-    for (int i = 0; i < kRPT; ++i) {
-      uint4* dst = reinterpret_cast<uint4*>(tile + (rg * kRPT + i) * LD + cg * 8);
-#pragma unroll
-      for (int w = 0; w < kWords; ++w) dst[w] = r[i][w];
-    }
-  }
-
-  // Transposed copy: tile_t[d][row], row stride LDT elements.
-  template <int LDT>
-  __device__ __forceinline__ void store_cols(T* tile_t, int tid) const {
-    if (!owner(tid)) return;
-    const int cg = tid % kColGroups;
-    const int rg = tid / kColGroups;
-    const T* e = reinterpret_cast<const T*>(r);  // e[i*8 + j]: row i, column j
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      T* dst = tile_t + (cg * 8 + j) * LDT + rg * kRPT;
-#pragma unroll
-      for (int i = 0; i < kRPT; ++i) dst[i] = e[i * 8 + j];
-    }
-  }
-};
 
 // ---------------------------------------------------------------------------
 // sqrt(N) geometry (reference core.py:957, 1038-1061, 1112-1117).
@@ -345,6 +250,142 @@ struct SwzTile {
     const uint2 uy = __builtin_bit_cast(uint2, y);
     f.w[0] = make_uint4(ux.x, ux.y, uy.x, uy.y);
     return f;
+  }
+};
+
+// ---------------------------------------------------------------------------
+// fp32 operands on the bf16 matrix core. A float's 24-bit significand is cut
+// into three bf16 pieces of 8 bits, x = hi + mid + lo exactly (each piece the
+// truncated rest, so nothing rounds or overflows; below 2^-110 the last bits
+// fall under the smallest bf16). A product takes the six piece products down
+// to 2^-16 of it; the three left out are at most 2^-23 of |x y| together, a
+// quarter of that on average, where one fp32 multiply-add rounds by up to
+// 2^-24. Six 16x16x32 MFMAs (16 cycles each) stand for eight 16x16x4 fp32 ones
+// (32 cycles each), and round the sum six times where those did eight times:
+// against fp64 every output is nearer than with the fp32 MFMA (relative error
+// of o, dq, dk, dv at B=1 H=8 S=4096 D=64: 2.9, 3.9, 3.5, 3.4e-7 against 3.4,
+// 4.6, 4.7, 4.5e-7; H=4 S=131072: 5.4, 6.4, 5.5, 5.3e-7 against 5.8, 6.8, 12,
+// 12e-7; the same order at D = 32, 128 and 256). An infinite x is kept in the piece that meets only the
+// other operand's hi, so that infinity times a number stays infinite.
+// ---------------------------------------------------------------------------
+struct Split {
+  Frag<bf16> p[3];  // hi, mid, lo
+};
+
+// INF: x may be infinite.
+template <bool INF>
+__device__ __forceinline__ Split split8(const float (&x)[8]) {
+  Split f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    uint32_t h[2], m[2], l[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float v = x[2 * w + i];
+      const bool inf = INF && __builtin_isinf(v);
+      h[i] = inf ? 0u : __float_as_uint(v) & 0xffff0000u;
+      const float r = v - __uint_as_float(h[i]);
+      m[i] = inf ? 0u : __float_as_uint(r) & 0xffff0000u;
+      l[i] = __float_as_uint(r - __uint_as_float(m[i]));
+    }
+    // the high halves of two words
+    reinterpret_cast<uint32_t*>(f.p[0].w)[w] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
+    reinterpret_cast<uint32_t*>(f.p[1].w)[w] = __builtin_amdgcn_perm(m[1], m[0], 0x07060302u);
+    reinterpret_cast<uint32_t*>(f.p[2].w)[w] = __builtin_amdgcn_perm(l[1], l[0], 0x07060302u);
+  }
+  return f;
+}
+
+// Piece pairs of a product, the small ones first.
+__device__ __forceinline__ constexpr int split_a(int t) { return t == 0 ? 2 : t == 2 || t == 3 ? 1 : 0; }
+__device__ __forceinline__ constexpr int split_b(int t) { return t == 1 ? 2 : t == 2 || t == 4 ? 1 : 0; }
+// t:      0 1 2 3 4 5
+// a, b:   lo.hi hi.lo mid.mid mid.hi hi.mid hi.hi
+
+// ROWS x D tile of fp32 rows as three planes of SwzTile, filled through
+// registers by NT threads: load() issues the reads, store() splits and writes.
+template <int D, int ROWS, int NT>
+struct SplitStage {
+  using Tile = SwzTile<D, ROWS>;
+  static constexpr int kBytes = 3 * Tile::kBytes;
+  static constexpr int kRowGroups = NT / Tile::kCPR < ROWS ? NT / Tile::kCPR : ROWS;
+  static constexpr int kRPT = ROWS / kRowGroups;  // rows per thread
+  static_assert(kRowGroups * kRPT == ROWS, "tile/thread mismatch");
+  uint4 r[kRPT][2];
+
+  __device__ __forceinline__ void load(const float* base, int64_t row_stride, int row0, int row_hi,
+                                       int tid) {
+    const int cg = tid % Tile::kCPR, rg = tid / Tile::kCPR;
+#pragma unroll
+    for (int i = 0; i < kRPT; ++i) {
+      const int row = row0 + i * kRowGroups + rg;
+      if (rg < kRowGroups && row < row_hi) {
+        const uint4* src = reinterpret_cast<const uint4*>(base + (int64_t)row * row_stride + cg * 8);
+        r[i][0] = src[0];
+        r[i][1] = src[1];
+      } else {
+        r[i][0] = r[i][1] = make_uint4(0, 0, 0, 0);
+      }
+    }
+  }
+  __device__ __forceinline__ void store(char* lds, int tid) const {
+    const int cg = tid % Tile::kCPR, rg = tid / Tile::kCPR;
+    if (rg >= kRowGroups) return;
+#pragma unroll
+    for (int i = 0; i < kRPT; ++i) {
+      const Split f = split8<true>(*reinterpret_cast<const float(*)[8]>(&r[i][0]));
+      char* dst = lds + Tile::off(i * kRowGroups + rg, cg);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(dst + k * Tile::kBytes) = f.p[k].w[0];
+    }
+  }
+
+  __device__ __forceinline__ static Split row_frag(const char* p) {
+    Split f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) f.p[k] = Tile::template row_frag_at<bf16>(p + k * Tile::kBytes);
+    return f;
+  }
+  __device__ __forceinline__ static Split tr_frag(const char* p) {
+    Split f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const char* q = p + k * Tile::kBytes;
+      f.p[k] = Tile::template tr_frag_at<bf16>(q, q + Tile::kBlk16);
+    }
+    return f;
+  }
+};
+
+// Eight floats of a row, split.
+__device__ __forceinline__ Split load_split(const float* p) {
+  float x[8];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    *reinterpret_cast<uint4*>(&x[4 * i]) = reinterpret_cast<const uint4*>(p)[i];
+  return split8<true>(x);
+}
+
+// Lane offsets into the swizzled tiles. The swizzle permutes 16 chunks (256
+// bytes) of a row, so at D = 256 the upper half of a row is 256 bytes behind
+// the lower half: an immediate of the read, no further register.
+template <int D>
+struct LaneOffs {
+  static constexpr int kD = D < 128 ? D : 128;
+  int row[kD / 32];  // row fragment, chunk 4c + g, row lane%16
+  int tr[kD / 16];   // transposed fragment, columns 16 db ..
+  __device__ __forceinline__ void init(int lane) {
+    using Tile = SwzTile<D, 64>;
+#pragma unroll
+    for (int c = 0; c < kD / 32; ++c) row[c] = Tile::row_lane_off(lane, 4 * c + (lane >> 4));
+#pragma unroll
+    for (int db = 0; db < kD / 16; ++db) tr[db] = Tile::tr_lane_off(lane, 16 * db);
+  }
+  __device__ __forceinline__ int row_at(int c) const {
+    return row[c % (kD / 32)] + c / (kD / 32) * 256;
+  }
+  __device__ __forceinline__ int tr_at(int db) const {
+    return tr[db % (kD / 16)] + db / (kD / 16) * 256;
   }
 };
 

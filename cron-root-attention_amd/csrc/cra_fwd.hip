@@ -14,8 +14,8 @@
 // (core.py:1028), l sums the rounded P of the 2-byte types.
 //
 // Mapping: one workgroup = 4 waves = 128 consecutive queries of one (b, h);
-// each wave owns 32 queries. K/V tiles of 64 rows (32 for fp32) are staged in
-// LDS, K row-major and V transposed. S^T = K . Q^T puts a query on lane%16 so
+// each wave owns 32 queries. K/V tiles of 64 rows (32 for fp32) are staged
+// row-major in LDS. S^T = K . Q^T puts a query on lane%16 so
 // the per-query softmax state is lane-local; O^T = V^T . P^T consumes P^T
 // straight from the S^T registers. Tiles are launched heaviest first (work
 // per query grows with i) and consecutive workgroups are different heads of
@@ -31,106 +31,109 @@ namespace cra {
 
 namespace {
 
-// Geometry of the generic forward (fwd_kernel: the fp32 path, and every
-// dtype at head dim 256). NB = 16-query blocks per wave: two below D = 256,
-// one at D = 256 (two would hold 256 VGPRs of accumulators and Q operands).
-template <typename T, int D, int NB = 2>
-struct FwdTraits {
-  static constexpr int kWaves = 4;
-  static constexpr int kThreads = 64 * kWaves;
-  static constexpr int kQW = 16 * NB;                // queries per wave
-  static constexpr int kBM = kWaves * kQW;           // queries per workgroup
-  static constexpr int kBN = (sizeof(T) == 4 || D > 128) ? 32 : 64;  // key rows per LDS tile
-  static constexpr int kKB = kBN / 16;               // 16-row key blocks
-  static constexpr int kKC = kBN / 32;               // 32-row key chunks
-  static constexpr int kDC = D / 32;                 // 32-wide head-dim chunks
-  static constexpr int kDB = D / 16;                 // 16-wide head-dim blocks
-  static constexpr int kLD = D + 16 / (int)sizeof(T);  // row-major tile stride
-  static constexpr int kLDT = kBN + 4;               // transposed tile stride
-};
+// ---------------------------------------------------------------------------
+// fp32 forward: the mapping of fwd2 (below) with every operand split in three
+// bf16 pieces (Split): Q in registers, K and V tiles of 32 rows as three
+// planes in LDS, staged through registers (the split happens there, once per
+// workgroup), P split in registers. 4 waves of 16 QB queries; up to D = 64
+// two LDS stages, one barrier per tile. The running maximum is raised lazily
+// as in fwd2 (an fp32 P keeps its precision at any magnitude). Bound by
+// the matrix core and the splits' VALU work about equally (per wave and 32-key
+// tile at D = 64: 96 MFMAs, 1536 cycles, beside about 300 VALU). Against the
+// fp32-MFMA kernel before it (V transposed by LDS writes, one stage): H=8
+// S=32768 D=64 362 -> 236 us, D=128 968 -> 615 us, S=4096 D=64 45 -> 31 us,
+// H=4 S=8192 D=256 149 -> 120 us.
+// ---------------------------------------------------------------------------
+constexpr float kSumMaxF32 = 32768.f;
+constexpr int kF32Waves = 4, kF32BN = 32;
+template <int D>
+constexpr int kF32QB = D > 128 ? 1 : 2;  // 16-query blocks per wave
 
-// One key tile against the wave's 16 * NB queries: S^T, masked online
-// softmax, O^T += V^T P^T. `valid(key_offset, qb)` says whether tile row
-// key_offset is in the set of query block qb's lane query.
-template <typename T, int D, int NB, bool MASK, typename Valid>
-__device__ __forceinline__ void attend_tile(const T* sK, const T* sVt,
-                                            const Frag<T> (&qf)[NB][FwdTraits<T, D, NB>::kDC],
-                                            f32x4 (&acc)[FwdTraits<T, D, NB>::kDB][NB],
-                                            float (&m_run)[NB], float (&l_run)[NB], float c2,
-                                            int l16, int g, Valid valid) {
-  using Tr = FwdTraits<T, D, NB>;
-  f32x4 s[Tr::kKB][NB];
+template <int D, int QB, bool MASK>
+__device__ __forceinline__ void attend_f32(const char* tK, const char* tV, const LaneOffs<D>& lo,
+                                           const Split (&qf)[QB][D / 32], f32x4 (&acc)[D / 16][QB],
+                                           float (&m_run)[QB], float (&l_run)[QB], float c2, int g,
+                                           const TileMask<QB>& mk) {
+  using Stage = SplitStage<D, kF32BN, 64 * kF32Waves>;
+  using Tile = typename Stage::Tile;
+  f32x4 s[2][QB];
 #pragma unroll
-  for (int kb = 0; kb < Tr::kKB; ++kb) {
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int qb = 0; qb < NB; ++qb) s[kb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int qb = 0; qb < QB; ++qb) s[h][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < Tr::kDC; ++c) {
-      const Frag<T> kf = lds_frag_row<T>(sK + (16 * kb + l16) * Tr::kLD + 32 * c + 8 * g);
+  for (int c = 0; c < D / 32; ++c) {
+    Split kf[2];
 #pragma unroll
-      for (int qb = 0; qb < NB; ++qb) s[kb][qb] = mma(s[kb][qb], kf, qf[qb][c]);
-    }
+    for (int h = 0; h < 2; ++h) kf[h] = Stage::row_frag(tK + h * Tile::kBlk16 + lo.row_at(c));
+    // consecutive MFMAs go to different accumulators
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+          s[h][qb] = mma(s[h][qb], kf[h].p[split_a(t)], qf[qb][c].p[split_b(t)]);
   }
-  Frag<T> pf[Tr::kKC][NB];
+  Split pf[QB];
 #pragma unroll
-  for (int qb = 0; qb < NB; ++qb) {
-    float t[Tr::kKB][4];
-    float mx = -__builtin_huge_valf();
+  for (int qb = 0; qb < QB; ++qb) {
+    float pv[8], ps = 0.f;
 #pragma unroll
-    for (int kb = 0; kb < Tr::kKB; ++kb) {
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float x = s[kb][qb][r] * c2;
-        if (MASK && !valid(16 * kb + 4 * g + r, qb)) x = -__builtin_huge_valf();
-        t[kb][r] = x;
-        mx = fmaxf(mx, x);
+        if (MASK && !mk.ok(16 * h + 4 * g + r, qb)) s[h][qb][r] = -__builtin_huge_valf();
+        pv[4 * h + r] = __builtin_amdgcn_exp2f(fmaf(s[h][qb][r], c2, -m_run[qb]));
+        ps += pv[4 * h + r];
       }
+    if (__any(!(ps <= kSumMaxF32))) {
+      float mx = -__builtin_huge_valf();
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[h][qb][r]);
+      const float m_new = fmaxf(m_run[qb], group_max(mx * c2));
+      const float mu = m_new == -__builtin_huge_valf() ? 0.f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f(m_run[qb] - mu);
+      l_run[qb] *= alpha;
+#pragma unroll
+      for (int db = 0; db < D / 16; ++db) acc[db][qb] *= alpha;
+      m_run[qb] = m_new;
+      ps = 0.f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          pv[4 * h + r] = __builtin_amdgcn_exp2f(fmaf(s[h][qb][r], c2, -mu));
+          ps += pv[4 * h + r];
+        }
     }
-    mx = group_max(mx);
-    const float m_new = fmaxf(m_run[qb], mx);
-    const float m_use = m_new == -__builtin_huge_valf() ? 0.f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f(m_run[qb] - m_use);
-    float psum = 0.f;
-#pragma unroll
-    for (int kb = 0; kb < Tr::kKB; ++kb) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = __builtin_amdgcn_exp2f(t[kb][r] - m_use);
-        t[kb][r] = p;
-        psum += p;
-      }
-    }
-    l_run[qb] = l_run[qb] * alpha + psum;
-    m_run[qb] = m_new;
-#pragma unroll
-    for (int db = 0; db < Tr::kDB; ++db) acc[db][qb] *= alpha;
-#pragma unroll
-    for (int kc = 0; kc < Tr::kKC; ++kc) {
-      const float v8[8] = {t[2 * kc][0],     t[2 * kc][1],     t[2 * kc][2],     t[2 * kc][3],
-                           t[2 * kc + 1][0], t[2 * kc + 1][1], t[2 * kc + 1][2], t[2 * kc + 1][3]};
-      pf[kc][qb] = pack8<T>(v8);
-    }
+    l_run[qb] += ps;
+    pf[qb] = split8<false>(pv);
   }
 #pragma unroll
-  for (int db = 0; db < Tr::kDB; ++db) {
-    const T* row = sVt + (16 * db + l16) * Tr::kLDT;
+  for (int db = 0; db < D / 16; db += 2) {
+    Split vt[2];
 #pragma unroll
-    for (int kc = 0; kc < Tr::kKC; ++kc) {
-      const Frag<T> vf = lds_frag_2x4<T>(row + 32 * kc + 4 * g, row + 32 * kc + 16 + 4 * g);
+    for (int e = 0; e < 2; ++e) vt[e] = Stage::tr_frag(tV + lo.tr_at(db + e));
 #pragma unroll
-      for (int qb = 0; qb < NB; ++qb) acc[db][qb] = mma(acc[db][qb], vf, pf[kc][qb]);
-    }
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+          acc[db + e][qb] = mma(acc[db + e][qb], vt[e].p[split_a(t)], pf[qb].p[split_b(t)]);
   }
 }
 
-// At D = 256 the 2-byte forward fits 2 waves per SIMD (at most 256 VGPRs).
-template <typename T, int D, int NB>
-__global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(D > 128 && sizeof(T) == 2 ? 2 : 1)))
-void fwd_kernel(FwdArgs a) {
-  using Tr = FwdTraits<T, D, NB>;
-  __shared__ __attribute__((aligned(16))) T sK[Tr::kBN * Tr::kLD];
-  __shared__ __attribute__((aligned(16))) T sVt[D * Tr::kLDT];
+template <int D, int QB>
+__global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(D > 64 ? 1 : 2)))
+void fwd_f32_kernel(FwdArgs a) {
+  constexpr int NW = kF32Waves, BN = kF32BN, kQW = 16 * QB, kBM = NW * kQW;
+  constexpr int kStages = D <= 64 ? 2 : 1;
+  using Stage = SplitStage<D, BN, 64 * NW>;
+  __shared__ __attribute__((aligned(1024))) char lds[kStages][2][Stage::kBytes];  // K, V
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -138,129 +141,116 @@ void fwd_kernel(FwdArgs a) {
   const int nbh = a.B * a.Hq;
   const int bh = blockIdx.x % nbh;
   const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
-  const int tile = (dc.len + Tr::kBM - 1) / Tr::kBM - 1 - dc.item;  // heaviest first
+  const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
   const int b = bh / a.Hq, h = bh % a.Hq;
   const int hk = h / (a.Hq / a.Hkv);
-  const int m0 = tile * Tr::kBM;
-  const int q0 = m0 + wave * Tr::kQW;
+  const int m0 = tile * kBM;
+  const int q0 = m0 + wave * kQW;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
 
-  const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
-  const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
-  const T* vp = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
-  float* lse = a.lse + (int64_t)bh * a.S + dc.off;
+  const float* qp = static_cast<const float*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
+  const float* kp = static_cast<const float*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
+  const float* vp = static_cast<const float*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
   const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
-  const T* gkp = static_cast<const T*>(a.gk) + gbase;
-  const T* gvp = static_cast<const T*>(a.gv) + gbase;
+  const float* gkp = static_cast<const float*>(a.gk) + gbase;
+  const float* gvp = static_cast<const float*>(a.gv) + gbase;
 
-  // Q as the B operand of S^T = K . Q^T: lane holds q[qi][32c + 8g .. +8].
-  Frag<T> qf[NB][Tr::kDC];
-  int qi[NB];
-#pragma unroll
-  for (int qb = 0; qb < NB; ++qb) {
-    qi[qb] = q0 + 16 * qb + l16;
-#pragma unroll
-    for (int c = 0; c < Tr::kDC; ++c) {
-      if (qi[qb] < S) {
-        qf[qb][c] = lds_frag_row<T>(qp + (int64_t)qi[qb] * a.qss + 32 * c + 8 * g);
-      } else {
-#pragma unroll
-        for (int w = 0; w < Frag<T>::kWords; ++w) qf[qb][c].w[w] = make_uint4(0, 0, 0, 0);
-      }
+  const int lo_k = max(0, m0 - W + 1);
+  const int hi = min(S, m0 + kBM);
+  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int nloc = (a.phases & 1) ? (hi - lo_k + BN - 1) / BN : 0;
+  const int nglob = (a.phases & 2) ? (gmax + BN - 1) / BN : 0;
+  const int ntot = nloc + nglob;
+  // global tiles first, then the local window from its highest tile down
+  auto row0 = [&](int it) { return it >= nglob ? lo_k + (nloc - 1 - (it - nglob)) * BN : it * BN; };
+  Stage stk, stv;
+  auto load = [&](int it) {
+    if (it >= nglob) {
+      stk.load(kp, a.kss, row0(it), hi, tid);
+      stv.load(vp, a.vss, row0(it), hi, tid);
+    } else {
+      stk.load(gkp, D, row0(it), gmax, tid);
+      stv.load(gvp, D, row0(it), gmax, tid);
     }
-  }
+  };
+  if (ntot > 0) load(0);
 
-  const float c2 = a.scale * kLog2e;
-  float m_run[NB], l_run[NB];
-  f32x4 acc[Tr::kDB][NB];
+  LaneOffs<D> lo;
+  lo.init(lane);
+  Split qf[QB][D / 32];
+  int qi[QB];
+  float m_run[QB], l_run[QB];
+  f32x4 acc[D / 16][QB];
 #pragma unroll
-  for (int qb = 0; qb < NB; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
+    qi[qb] = q0 + 16 * qb + l16;
+    const int qr = min(qi[qb], S - 1);  // queries past the document are never stored
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c)
+      qf[qb][c] = load_split(qp + (int64_t)qr * a.qss + 32 * c + 8 * g);
     m_run[qb] = -__builtin_huge_valf();
     l_run[qb] = 0.f;
 #pragma unroll
-    for (int db = 0; db < Tr::kDB; ++db) acc[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < D / 16; ++db) acc[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-
+  const float c2 = a.scale * kLog2e;
   const bool active = q0 < S;
-  const int q_last = min(q0 + Tr::kQW, S) - 1;
-  TileStage<T, D, Tr::kBN, Tr::kThreads> stk, stv;
-
-  // ---- phase 1: local window -------------------------------------------
-  const int lo = max(0, m0 - W + 1);
-  const int hi = min(S, m0 + Tr::kBM);
+  const int q_last = min(q0 + kQW, S) - 1;
   const int w_lo = max(0, q0 - W + 1);
-  const int hi_loc = (a.phases & 1) ? hi : lo;
-  for (int ts = lo; ts < hi_loc; ts += Tr::kBN) {
-    stk.load(kp, a.kss, ts, 0, hi, tid);
-    stv.load(vp, a.vss, ts, 0, hi, tid);
-    __syncthreads();
-    stk.template store_rows<Tr::kLD>(sK, tid);
-    stv.template store_cols<Tr::kLDT>(sVt, tid);
-    __syncthreads();
-    if (active && ts <= q_last && ts + Tr::kBN - 1 >= w_lo) {
-      const bool full = ts >= q_last - W + 1 && ts + Tr::kBN - 1 <= q0;
-      auto valid = [&](int ko, int qb) {
-        const int j = ts + ko;
-        return j <= qi[qb] && j >= qi[qb] - W + 1;
-      };
-      if (full)
-        attend_tile<T, D, NB, false>(sK, sVt, qf, acc, m_run, l_run, c2, l16, g, valid);
-      else
-        attend_tile<T, D, NB, true>(sK, sVt, qf, acc, m_run, l_run, c2, l16, g, valid);
-    }
-  }
-
-  // ---- phase 2+3: prefix of the packed strided/relay rows ---------------
-  const int gmax = glob_prefix(hi - 1, W, rpb);
   const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
   const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
-  int glen[NB];
+  int glen[QB];
 #pragma unroll
-  for (int qb = 0; qb < NB; ++qb) glen[qb] = glob_prefix(qi[qb], W, rpb);
-  const int g_end = (a.phases & 2) ? gmax : 0;
-  for (int ts = 0; ts < g_end; ts += Tr::kBN) {
-    stk.load(gkp, D, ts, 0, gmax, tid);
-    stv.load(gvp, D, ts, 0, gmax, tid);
-    __syncthreads();
-    stk.template store_rows<Tr::kLD>(sK, tid);
-    stv.template store_cols<Tr::kLDT>(sVt, tid);
-    __syncthreads();
-    if (active && ts < wg_hi) {
-      auto valid = [&](int ko, int qb) { return ts + ko < glen[qb]; };
-      if (ts + Tr::kBN <= wg_lo)
-        attend_tile<T, D, NB, false>(sK, sVt, qf, acc, m_run, l_run, c2, l16, g, valid);
+  for (int qb = 0; qb < QB; ++qb) glen[qb] = glob_prefix(qi[qb], W, rpb);
+
+  auto store = [&](int it) {
+    char(&dst)[2][Stage::kBytes] = lds[kStages == 2 ? it & 1 : 0];
+    stk.store(dst[0], tid);
+    stv.store(dst[1], tid);
+  };
+  if (ntot > 0) store(0);
+  __syncthreads();
+  for (int it = 0; it < ntot; ++it) {
+    if (it + 1 < ntot) load(it + 1);
+    const char(&cur)[2][Stage::kBytes] = lds[kStages == 2 ? it & 1 : 0];
+    const bool loc = it >= nglob;
+    const int ts = row0(it);
+    if (active && (loc ? (ts <= q_last && ts + BN - 1 >= w_lo) : ts < wg_hi)) {
+      const bool full = loc ? (ts >= q_last - W + 1 && ts + BN - 1 <= q0) : ts + BN <= wg_lo;
+      TileMask<QB> mk;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        mk.hi[qb] = loc ? qi[qb] - ts : glen[qb] - 1 - ts;
+        mk.span[qb] = loc ? (unsigned)(W - 1) : 0x7fffffffu;
+      }
+      if (full)
+        attend_f32<D, QB, false>(cur[0], cur[1], lo, qf, acc, m_run, l_run, c2, g, mk);
       else
-        attend_tile<T, D, NB, true>(sK, sVt, qf, acc, m_run, l_run, c2, l16, g, valid);
+        attend_f32<D, QB, true>(cur[0], cur[1], lo, qf, acc, m_run, l_run, c2, g, mk);
     }
+    if (kStages == 1) __syncthreads();  // every wave is done with this tile
+    if (it + 1 < ntot) store(it + 1);
+    __syncthreads();
   }
 
-  // ---- epilogue: O = acc / l, LSE = (m + log2 l) ln 2 ---------------------
-  T* op = static_cast<T*>(a.o) + b * a.osb + h * a.osh + (int64_t)dc.off * a.oss;
+  float* op = static_cast<float*>(a.o) + b * a.osb + h * a.osh + (int64_t)dc.off * a.oss;
+  float* lse = a.lse + (int64_t)bh * a.S + dc.off;
 #pragma unroll
-  for (int qb = 0; qb < NB; ++qb) {
-    const float l = group_sum(l_run[qb]);
+  for (int qb = 0; qb < QB; ++qb) {
+    const float l = fmaxf(group_sum(l_run[qb]), 1e-6f);
     if (!active || qi[qb] >= S) continue;
-    const float inv = 1.f / fmaxf(l, 1e-6f);
-    T* orow = op + (int64_t)qi[qb] * a.oss;
+    const float inv = 1.f / l;
+    float* orow = op + (int64_t)qi[qb] * a.oss;
 #pragma unroll
-    for (int db = 0; db < Tr::kDB; ++db) {
-      T e[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) e[r] = from_f32<T>(acc[db][qb][r] * inv);
-      if constexpr (sizeof(T) == 2) {
-        *reinterpret_cast<uint2*>(orow + 16 * db + 4 * g) = *reinterpret_cast<const uint2*>(e);
-      } else {
-        *reinterpret_cast<uint4*>(orow + 16 * db + 4 * g) = *reinterpret_cast<const uint4*>(e);
-      }
-    }
-    if (g == 0)
-      lse[qi[qb]] = (m_run[qb] + __builtin_amdgcn_logf(fmaxf(l, 1e-6f))) * kLn2;
+    for (int db = 0; db < D / 16; ++db)
+      *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * g) = acc[db][qb] * inv;
+    if (g == 0) lse[qi[qb]] = (m_run[qb] + __builtin_amdgcn_logf(l)) * kLn2;
   }
 }
 
 // ---------------------------------------------------------------------------
-// fp16/bf16 forward. Same mapping as fwd_kernel (4 waves x 32 queries), but
-// K/V tiles (64 rows) are double-buffered in swizzled LDS, filled with
+// fp16/bf16 forward: 4 waves x 32 queries. K/V tiles (64 rows) are
+// double-buffered in swizzled LDS, filled with
 // global_load_lds while the previous tile is computed, V^T operands come from
 // ds_read_b64_tr_b16 on the row-major V tile, each tile is processed in two
 // 32-key halves, and the running max is raised only when the rounded
@@ -276,29 +266,8 @@ void fwd_kernel(FwdArgs a) {
 #define CRA_FWD_PF 3
 #endif
 
-// Lane offsets into the swizzled tiles. The swizzle permutes 16 chunks (256
-// bytes) of a row, so at D = 256 the upper half of a row is 256 bytes behind
-// the lower half: an immediate of the read, no further register.
-template <int D>
-struct Fwd2Lane {
-  static constexpr int kD = D < 128 ? D : 128;
-  int k[kD / 32];   // K row fragment, chunk 4c + g, row lane%16
-  int v[kD / 16];   // V^T fragment, columns 16 db ..
-  __device__ __forceinline__ void init(int lane) {
-    using Tile = SwzTile<D, 64>;
-#pragma unroll
-    for (int c = 0; c < kD / 32; ++c) k[c] = Tile::row_lane_off(lane, 4 * c + (lane >> 4));
-#pragma unroll
-    for (int db = 0; db < kD / 16; ++db) v[db] = Tile::tr_lane_off(lane, 16 * db);
-  }
-  __device__ __forceinline__ int k_at(int c) const { return k[c % (kD / 32)] + c / (kD / 32) * 256; }
-  __device__ __forceinline__ int v_at(int db) const {
-    return v[db % (kD / 16)] + db / (kD / 16) * 256;
-  }
-};
-
 template <typename T, int D, int BN, int QB>
-__device__ __forceinline__ void tile_scores(const char* tK, const Fwd2Lane<D>& lo,
+__device__ __forceinline__ void tile_scores(const char* tK, const LaneOffs<D>& lo,
                                             const Frag<T> (&qf)[QB][D / 32], int kc,
                                             f32x4 (&s)[2][QB]) {
   using Tile = SwzTile<D, BN>;
@@ -309,7 +278,7 @@ __device__ __forceinline__ void tile_scores(const char* tK, const Fwd2Lane<D>& l
   // each MFMA's accumulator was last written four MFMAs earlier (key block
   // major, two apart, measured 0.5% slower).
   auto k_frag = [&](int t) {
-    return Tile::template row_frag_at<T>(tK + (2 * kc + t % 2) * Tile::kBlk16 + lo.k_at(t / 2));
+    return Tile::template row_frag_at<T>(tK + (2 * kc + t % 2) * Tile::kBlk16 + lo.row_at(t / 2));
   };
   constexpr int PF = CRA_FWD_PF < NK ? CRA_FWD_PF : NK;
   Frag<T> kf[PF + 1];
@@ -332,12 +301,12 @@ __device__ __forceinline__ void tile_scores(const char* tK, const Fwd2Lane<D>& l
 // O^T += V^T . P^T for 32-key half kh: transposed V fragments read
 // CRA_FWD_PF steps ahead of the MFMAs that use them.
 template <typename T, int D, int BN, int QB>
-__device__ __forceinline__ void pv_half(const char* tV, int kh, const Fwd2Lane<D>& lo,
+__device__ __forceinline__ void pv_half(const char* tV, int kh, const LaneOffs<D>& lo,
                                         const Frag<T> (&pf)[QB], f32x4 (&acc)[D / 16][QB]) {
   using Tile = SwzTile<D, BN>;
   constexpr int NDB = D / 16;
   auto tr_v = [&](int db) {
-    const char* pa = tV + (2 * kh) * Tile::kBlk16 + lo.v_at(db);
+    const char* pa = tV + (2 * kh) * Tile::kBlk16 + lo.tr_at(db);
     return Tile::template tr_frag_at<T>(pa, pa + Tile::kBlk16);
   };
   constexpr int PF = CRA_FWD_PF < NDB ? CRA_FWD_PF : NDB;
@@ -438,7 +407,7 @@ __device__ __forceinline__ void half_rescale(f32x4 (&s)[2][QB], int qb, float c2
 // previous half's PV MFMAs beside each half's exponentials, in one basic
 // block, so matrix and vector work can overlap.
 template <typename T, int D, int BN, bool MASK>
-__device__ __forceinline__ void attend_tile2(const char* tK, const char* tV, const Fwd2Lane<D>& lo,
+__device__ __forceinline__ void attend_tile2(const char* tK, const char* tV, const LaneOffs<D>& lo,
                                              const Frag<T> (&qf)[2][D / 32],
                                              f32x4 (&acc)[D / 16][2], float (&m_run)[2],
                                              float (&l_run)[2], float c2, int g,
@@ -472,7 +441,7 @@ __device__ __forceinline__ void attend_tile2(const char* tK, const char* tV, con
 // key visible to any of the wave's queries (window and prefix edges).
 template <typename T, int D, int BN>
 __device__ __forceinline__ void attend_half(const char* tK, const char* tV, int kc,
-                                            const Fwd2Lane<D>& lo, const Frag<T> (&qf)[2][D / 32],
+                                            const LaneOffs<D>& lo, const Frag<T> (&qf)[2][D / 32],
                                             f32x4 (&acc)[D / 16][2], float (&m_run)[2],
                                             float (&l_run)[2], float c2, int g,
                                             const TileMask<2>& mk, const Frag<T>& one) {
@@ -571,7 +540,7 @@ __device__ __forceinline__ void fwd2_item(const FwdArgs& a, const int item, FwdS
   };
   issue(0, stage0[0]);
 
-  Fwd2Lane<D> lo;
+  LaneOffs<D> lo;
   lo.init(lane);
   Frag<T> qf[2][D / 32];
   int qi[2];
@@ -767,7 +736,7 @@ void fwd_wide_kernel(FwdArgs a) {
   };
   if (ntot > 0) issue_k(0);
 
-  Fwd2Lane<D> lo;
+  LaneOffs<D> lo;
   lo.init(lane);
   Frag<T> qf[1][D / 32];
   const int qi = q0 + l16;
@@ -864,78 +833,80 @@ hipError_t resident_slots(K kern, int threads, int* out) {
 // measured 4% slower at D = 128: the wider local window adds key tiles.
 constexpr int kFwdWaves = 4;
 
-// Head dim 256: 16 queries per wave, 64 per workgroup; the 2-byte types on
-// fwd_wide_kernel, fp32 on the generic kernel. A persistent request runs the
-// same tiled kernel (the work-queue form is built for fwd2 only; the results
+// Kernels that take one grid for every order of work: fp32 (every head dim)
+// and the 2-byte types at head dim 256. A persistent request runs the same
+// tiled kernel there (the work-queue form is built for fwd2 only; the results
 // are the same function of the inputs).
+hipError_t launch_f32(int D, const FwdArgs& a, hipStream_t st) {
+  FwdArgs b = a;
+  auto go = [&](auto dc) {
+    constexpr int Dc = decltype(dc)::value;
+    constexpr int kBM = 16 * kF32Waves * kF32QB<Dc>;
+    set_items(b.docs, [&](int d) { return (b.docs.len[d] + kBM - 1) / kBM; });
+    const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq);
+    hipLaunchKernelGGL((fwd_f32_kernel<Dc, kF32QB<Dc>>), grid, dim3(64 * kF32Waves), 0, st, b);
+  };
+  switch (D) {
+    case 32: go(std::integral_constant<int, 32>{}); break;
+    case 64: go(std::integral_constant<int, 64>{}); break;
+    case 128: go(std::integral_constant<int, 128>{}); break;
+    case 256: go(std::integral_constant<int, 256>{}); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_wide(const FwdArgs& a, hipStream_t st) {
-  using Tr = FwdTraits<T, 256, 1>;
-  static_assert(Tr::kBM == 16 * kWideWaves, "one workgroup size at head dim 256");
+  constexpr int kBM = 16 * kWideWaves;
   FwdArgs b = a;
-  set_items(b.docs, [&](int d) { return (b.docs.len[d] + Tr::kBM - 1) / Tr::kBM; });
+  set_items(b.docs, [&](int d) { return (b.docs.len[d] + kBM - 1) / kBM; });
   const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq);
-  if constexpr (sizeof(T) == 2)
-    hipLaunchKernelGGL((fwd_wide_kernel<T, 256>), grid, dim3(Tr::kThreads), 0, st, b);
-  else
-    hipLaunchKernelGGL((fwd_kernel<T, 256, 1>), grid, dim3(Tr::kThreads), 0, st, b);
+  hipLaunchKernelGGL((fwd_wide_kernel<T, 256>), grid, dim3(64 * kWideWaves), 0, st, b);
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_T(int D, const FwdArgs& a, hipStream_t st) {
   if (D == 256) return launch_wide<T>(a, st);
-  if constexpr (sizeof(T) == 2) {
-    FwdArgs b = a;
-    constexpr int kBM = 32 * kFwdWaves;
-    set_items(b.docs, [&](int d) { return (b.docs.len[d] + kBM - 1) / kBM; });
-    const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq), block(64 * kFwdWaves);
-    // one document, D = 128 and a head count that is not a multiple of 8:
-    // XCD-aware order (measured 2.5-5% faster at D = 128; at D = 64, with
-    // 45% less HBM traffic, 0.5% faster to 3.6% slower)
-    const bool xcd = b.docs.n == 1 && (b.B * b.Hq) % 8 != 0 && D == 128;
-    FwdArgs bx = b;
-    bx.xcd_nt = xcd ? b.docs.item0[1] : 0;
-    const dim3 xgrid(xcd ? xcd_grid(b.B * b.Hq, b.docs.item0[1]) : grid.x);
-    hipError_t qerr = hipSuccess;
-    auto go = [&](auto dc) {
-      constexpr int Dc = decltype(dc)::value;
-      if (a.work_counter && a.phases == 3) {
-        // one round of resident workgroups: CUs x workgroups per CU
-        auto kern = fwd2_persistent_kernel<T, Dc, kFwdWaves>;
-        int slots = 0;
-        qerr = resident_slots<T, Dc>(kern, 64 * kFwdWaves, &slots);
-        if (qerr != hipSuccess) return;
-        const int items = (int)grid.x;
-        const dim3 pgrid(std::max(1, std::min(items, slots)));
-        hipLaunchKernelGGL(kern, pgrid, block, 0, st, b);
-        return;
-      }
-      switch (a.phases) {
-        case 1: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 1>), xgrid, block, 0, st, bx); break;
-        case 2: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 2>), xgrid, block, 0, st, bx); break;
-        default: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 3>), xgrid, block, 0, st, bx);
-      }
-    };
-    switch (D) {
-      case 32: go(std::integral_constant<int, 32>{}); break;
-      case 64: go(std::integral_constant<int, 64>{}); break;
-      case 128: go(std::integral_constant<int, 128>{}); break;
-      default: return hipErrorInvalidValue;
+  FwdArgs b = a;
+  constexpr int kBM = 32 * kFwdWaves;
+  set_items(b.docs, [&](int d) { return (b.docs.len[d] + kBM - 1) / kBM; });
+  const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq), block(64 * kFwdWaves);
+  // one document, D = 128 and a head count that is not a multiple of 8:
+  // XCD-aware order (measured 2.5-5% faster at D = 128; at D = 64, with
+  // 45% less HBM traffic, 0.5% faster to 3.6% slower)
+  const bool xcd = b.docs.n == 1 && (b.B * b.Hq) % 8 != 0 && D == 128;
+  FwdArgs bx = b;
+  bx.xcd_nt = xcd ? b.docs.item0[1] : 0;
+  const dim3 xgrid(xcd ? xcd_grid(b.B * b.Hq, b.docs.item0[1]) : grid.x);
+  hipError_t qerr = hipSuccess;
+  auto go = [&](auto dc) {
+    constexpr int Dc = decltype(dc)::value;
+    if (a.work_counter && a.phases == 3) {
+      // one round of resident workgroups: CUs x workgroups per CU
+      auto kern = fwd2_persistent_kernel<T, Dc, kFwdWaves>;
+      int slots = 0;
+      qerr = resident_slots<T, Dc>(kern, 64 * kFwdWaves, &slots);
+      if (qerr != hipSuccess) return;
+      const int items = (int)grid.x;
+      const dim3 pgrid(std::max(1, std::min(items, slots)));
+      hipLaunchKernelGGL(kern, pgrid, block, 0, st, b);
+      return;
     }
-    if (qerr != hipSuccess) return qerr;
-  } else {
-    FwdArgs b = a;
-    constexpr int kBM = FwdTraits<T, 128, 2>::kBM;
-    set_items(b.docs, [&](int d) { return (b.docs.len[d] + kBM - 1) / kBM; });
-    const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq);
-    switch (D) {
-      case 32: hipLaunchKernelGGL((fwd_kernel<T, 32, 2>), grid, dim3(256), 0, st, b); break;
-      case 64: hipLaunchKernelGGL((fwd_kernel<T, 64, 2>), grid, dim3(256), 0, st, b); break;
-      case 128: hipLaunchKernelGGL((fwd_kernel<T, 128, 2>), grid, dim3(256), 0, st, b); break;
-      default: return hipErrorInvalidValue;
+    switch (a.phases) {
+      case 1: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 1>), xgrid, block, 0, st, bx); break;
+      case 2: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 2>), xgrid, block, 0, st, bx); break;
+      default: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 3>), xgrid, block, 0, st, bx);
     }
+  };
+  switch (D) {
+    case 32: go(std::integral_constant<int, 32>{}); break;
+    case 64: go(std::integral_constant<int, 64>{}); break;
+    case 128: go(std::integral_constant<int, 128>{}); break;
+    default: return hipErrorInvalidValue;
   }
+  if (qerr != hipSuccess) return qerr;
   return hipGetLastError();
 }
 
@@ -944,12 +915,11 @@ hipError_t launch_T(int D, const FwdArgs& a, hipStream_t st) {
 
 bool fwd_tile_config(int dtype, int D, int out[3]) {
   if (dtype < 0 || dtype > 2 || (D != 32 && D != 64 && D != 128 && D != 256)) return false;
-  if (D == 256) {
-    using Tr = FwdTraits<f16, 256, 1>;  // the same geometry for every dtype
-    out[0] = Tr::kWaves; out[1] = Tr::kBM; out[2] = Tr::kBN;
+  if (D == 256 && dtype != 2) {
+    out[0] = kWideWaves; out[1] = 16 * kWideWaves; out[2] = kWideBN;
   } else if (dtype == 2) {
-    using Tr = FwdTraits<float, 128>;
-    out[0] = Tr::kWaves; out[1] = Tr::kBM; out[2] = Tr::kBN;
+    out[0] = kF32Waves; out[1] = 16 * kF32Waves * (D == 256 ? kF32QB<256> : kF32QB<128>);
+    out[2] = kF32BN;
   } else {
     out[0] = kFwdWaves; out[1] = 32 * kFwdWaves; out[2] = 64;
   }
@@ -960,7 +930,7 @@ hipError_t launch_fwd(int dtype, int D, const FwdArgs& a, hipStream_t st) {
   switch (dtype) {
     case 0: return launch_T<f16>(D, a, st);
     case 1: return launch_T<bf16>(D, a, st);
-    case 2: return launch_T<float>(D, a, st);
+    case 2: return launch_f32(D, a, st);
   }
   return hipErrorInvalidValue;
 }

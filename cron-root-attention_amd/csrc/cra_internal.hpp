@@ -153,8 +153,8 @@ struct BwdArgs {
   void* dq;
   void* dk;
   void* dv;
-  float* delta;    // [B, Hq, S] rowsum(o * do); 2-byte path: stored negated
-  float* nlse2;    // [B, Hq, S] 2-byte path: -lse * log2(e)
+  float* delta;    // [B, Hq, S] -rowsum(o * do)
+  float* nlse2;    // [B, Hq, S] -lse * log2(e)
   float* gpart;    // fp32 partial dK/dV of the global rows (part_row)
   float* dalpha;   // [Hkv] or null
   int64_t qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, osb, osh, oss;
@@ -166,7 +166,7 @@ struct BwdArgs {
   float scale;
   int chunk_len;   // queries per chunk of the global-row kernel
   int nchunk;      // most query chunks of a document
-  int group;       // 0: first launch of a call (fp32: computes Delta; writes dalpha);
+  int group;       // 0: first launch of a call (writes dalpha);
                    // later document groups of the call add to dalpha
   int xcd_nt;      // > 0: XCD-aware order (xcd_item) over this many tiles per head
   Docs docs;       // items: set by the launcher per kernel
