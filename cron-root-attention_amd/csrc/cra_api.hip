@@ -224,7 +224,9 @@ cra::Docs group_table(const Plan& pl, int g) {
     t.off[i] = pl.off[d];
     t.len[i] = pl.len[d];
     t.W[i] = pl.W[d];
+    t.dW[i] = cra::fast_div(pl.W[d]);
     t.rpb[i] = pl.rpb[d];
+    t.drpb[i] = cra::fast_div(pl.rpb[d]);
     t.gofs[i] = pl.gofs[d];
     t.bofs[i] = pl.bofs[d];
   }

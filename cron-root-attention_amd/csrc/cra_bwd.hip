@@ -49,12 +49,6 @@ __device__ __forceinline__ void store4(T* p, const f32x4& v, float mul) {
     *reinterpret_cast<uint4*>(p) = *reinterpret_cast<const uint4*>(e);
 }
 
-// First query that sees packed global row gr (inverse of glob_prefix).
-__host__ __device__ inline int glob_row_first_query(int gr, int W, int rpb) {
-  const int r = gr / rpb;
-  return (gr - r * rpb) == 0 ? r * W + W : (r + 1) * W + W - 1;
-}
-
 // ---------------------------------------------------------------------------
 // 3. Chunk partials of the global rows summed into chunk 0, in chunk order
 // (one float4 per thread; work items: the documents' rows x 2D / 4 / 256).
@@ -64,19 +58,20 @@ __host__ __device__ inline int glob_row_first_query(int gr, int W, int rpb) {
 // chunk is read again and left out): one at a time, the sum is a chain of
 // memory latencies
 constexpr int kGsumU = 8;
-template <int D>
-__global__ __launch_bounds__(256) void gsum_kernel(BwdArgs a) {
+template <int D, int ND>
+__global__ __launch_bounds__(256) void gsum_kernel(BwdArgsT<ND> a) {
   constexpr int kVec = 2 * D / 4;  // float4 per row (dK and dV)
   const int nbh = a.B * a.Hkv;
-  const int bhk = blockIdx.x % nbh;
-  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const KvHead hd = kv_head(a, blockIdx.x);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bhk = hd.bhk;
   const int rows = doc_rows(dc.len, dc.W, dc.rpb);
   const int e = dc.item * 256 + (int)threadIdx.x;
   if (e >= rows * kVec) return;
   // Chunks [c_lo, c_hi) hold queries that see the row; the global-row
   // kernel wrote no partial for the others (their workgroups had no query
   // that sees the tile), so they are skipped rather than read.
-  const int first = glob_row_first_query(e / kVec, dc.W, dc.rpb);
+  const int first = glob_row_first_query(e / kVec, dc);
   const int c_lo = first / a.chunk_len;
   const int c_hi = first < dc.len ? num_chunks(dc.len, a.chunk_len) : c_lo;
   float* p0 = a.gpart + part_row(dc, 0, nbh, bhk, 0) * 2 * D + 4 * (int64_t)e;
@@ -258,9 +253,9 @@ __device__ __forceinline__ void dq2_tile(const char* tK, const char* tV, const L
 
 // NW waves of QB blocks of 16 queries each cover the workgroup's
 // 16 * NW * QB queries; key tiles of BN rows; at least WPE waves per SIMD.
-template <typename T, int D, int NW, int QB, int BN, int WPE>
+template <typename T, int D, int NW, int QB, int BN, int WPE, int ND>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE)))
-void dq2_kernel(BwdArgs a) {
+void dq2_kernel(BwdArgsT<ND> a) {
   using Tile = SwzTile<D, BN>;
   constexpr int kQW = 16 * QB, kBM = NW * kQW, kBN = BN;
   // Two pipeline stages as separate LDS objects (see fwd2_kernel).
@@ -276,11 +271,10 @@ void dq2_kernel(BwdArgs a) {
     item = xcd_item(item, nbh, a.xcd_nt);
     if (item < 0) return;  // padding block
   }
-  const int bh = item % nbh;
-  const Doc dc = find_doc(a.docs, item / nbh);
+  const QHead hd = q_head(a, item);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bh = hd.bh, b = hd.b, h = hd.h, hk = hd.hk;
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
-  const int b = bh / a.Hq, h = bh % a.Hq;
-  const int hk = h / (a.Hq / a.Hkv);
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * kQW;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -299,7 +293,7 @@ void dq2_kernel(BwdArgs a) {
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
-  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int gmax = glob_prefix(hi - 1, dc);
   const int nloc = (hi - lo_k + kBN - 1) / kBN;
   // global tiles first: their first fill is an L2 hit; then the local
   // window from its highest key tile down, in step with the neighbouring
@@ -388,11 +382,11 @@ void dq2_kernel(BwdArgs a) {
   const bool active = q0 < S;
   const int q_last = min(q0 + kQW, S) - 1;
   const int w_lo = max(0, q0 - W + 1);
-  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
-  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
+  const int wg_lo = active ? glob_prefix(q0, dc) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, dc) : 0;
   int glen[QB];
 #pragma unroll
-  for (int qb = 0; qb < QB; ++qb) glen[qb] = glob_prefix(qi[qb], W, rpb);
+  for (int qb = 0; qb < QB; ++qb) glen[qb] = glob_prefix(qi[qb], dc);
 
   // Local and global tiles share one body (parameters chosen per tile); the
   // loop is unrolled over the two stages.
@@ -450,9 +444,9 @@ void dq2_kernel(BwdArgs a) {
 // dq_kernel (tiles through registers, V and K^T stored transposed by 2-byte
 // LDS writes, one stage) took 478 us and delta_kernel before it 46 us.
 constexpr int kWideWaves = 4, kWideBN = 32;
-template <typename T, int D>
+template <typename T, int D, int ND>
 __global__ __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(2)))
-void dq_wide_kernel(BwdArgs a) {
+void dq_wide_kernel(BwdArgsT<ND> a) {
   constexpr int NW = kWideWaves, BN = kWideBN, kBM = 16 * NW;
   using Tile = SwzTile<D, BN>;
   __shared__ __attribute__((aligned(1024))) char sK0[Tile::kBytes];
@@ -462,12 +456,10 @@ void dq_wide_kernel(BwdArgs a) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int nbh = a.B * a.Hq;
-  const int bh = blockIdx.x % nbh;
-  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const QHead hd = q_head(a, blockIdx.x);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bh = hd.bh, b = hd.b, h = hd.h, hk = hd.hk;
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
-  const int b = bh / a.Hq, h = bh % a.Hq;
-  const int hk = h / (a.Hq / a.Hkv);
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * 16;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -485,7 +477,7 @@ void dq_wide_kernel(BwdArgs a) {
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
-  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int gmax = glob_prefix(hi - 1, dc);
   const int nloc = (hi - lo_k + BN - 1) / BN;
   const int nglob = (gmax + BN - 1) / BN;
   const int ntot = nloc + nglob;
@@ -551,9 +543,9 @@ void dq_wide_kernel(BwdArgs a) {
   const bool active = q0 < S;
   const int q_last = min(q0 + 16, S) - 1;
   const int w_lo = max(0, q0 - W + 1);
-  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
-  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
-  const int glen = glob_prefix(qi, W, rpb);
+  const int wg_lo = active ? glob_prefix(q0, dc) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, dc) : 0;
+  const int glen = glob_prefix(qi, dc);
 
   auto step = [&](auto buf_c, int it) {
     char(&cur)[Tile::kBytes] = decltype(buf_c)::value ? sK1 : sK0;
@@ -593,7 +585,7 @@ void dq_wide_kernel(BwdArgs a) {
 // Epilogues of the dK/dV kernels: lane (l16, g) owns key row kw + 16kb + l16,
 // dims 16db + 4g .. +4 of each block. Global rows: the chunk's fp32 partial.
 template <int D, int KB>
-__device__ __forceinline__ void write_part(const BwdArgs& a, const Doc& dc, int chunk, int nbh,
+__device__ __forceinline__ void write_part(const BwdCommon& a, const Doc& dc, int chunk, int nbh,
                                            int bhk, int kw, int nrows, int l16, int g,
                                            const f32x4 (&dka)[D / 16][KB],
                                            const f32x4 (&dva)[D / 16][KB]) {
@@ -615,7 +607,7 @@ __device__ __forceinline__ void write_part(const BwdArgs& a, const Doc& dc, int 
 // strided row of its block and any relay row selected from it; reference
 // scatter, core.py:2767-2815).
 template <typename T, int D, int KB>
-__device__ __forceinline__ void write_local(const BwdArgs& a, const Doc& dc, int nbh, int b, int hk,
+__device__ __forceinline__ void write_local(const BwdCommon& a, const Doc& dc, int nbh, int b, int hk,
                                             int kw, int l16, int g, f32x4 (&dka)[D / 16][KB],
                                             f32x4 (&dva)[D / 16][KB]) {
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -630,6 +622,8 @@ __device__ __forceinline__ void write_local(const BwdArgs& a, const Doc& dc, int
     if (j >= S) continue;
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) dka[db][kb] *= a.scale;
+    // (a plain division: with div_by the D = 64 local kernel, at its register
+    // cap, spills 21 and is 45% slower)
     const int rblk = j / W;
     int grow[5];
     float gsc[5];
@@ -797,10 +791,10 @@ __device__ __forceinline__ void dkdv2_tile(const char* tQ, const char* tO, const
 // with 32-query tiles (66 KB of LDS, two per CU). B=1 H=8 S=32768 fp16:
 // global rows 215 us, local 306 us; dkdv_kernel (one LDS stage, transposed
 // tiles written by 2-byte LDS stores) took 720 and 638 us.
-template <typename T, int D, bool GLOB, int NW, int KB, int BQ>
+template <typename T, int D, bool GLOB, int NW, int KB, int BQ, int ND>
 __global__ __launch_bounds__(64 * NW)
 __attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : GLOB && D < 128 ? 4 : 3)))
-void dkdv2_kernel(BwdArgs a) {
+void dkdv2_kernel(BwdArgsT<ND> a) {
   using Tile = SwzTile<D, BQ>;
   constexpr int kKW = 16 * KB, kBK = NW * kKW, kBQ = BQ;
   static_assert(BQ == 32 || BQ == 64 || BQ == 128, "query tile rows");
@@ -820,17 +814,16 @@ void dkdv2_kernel(BwdArgs a) {
     item = xcd_item(item, nbh, a.xcd_nt);
     if (item < 0) return;  // padding block
   }
-  const int bhk = item % nbh;
-  const int rest = item / nbh;
-  const Doc dc = find_doc(a.docs, rest);
+  const KvHead hd = kv_head(a, item);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bhk = hd.bhk, b = hd.b, hk = hd.hk;
   const int nck = GLOB ? num_chunks(dc.len, a.chunk_len) : 1;
   const int tile = GLOB ? dc.item / nck : dc.item;
   const int chunk = GLOB ? dc.item - tile * nck : 0;
-  const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
   const int grp = a.Hq / a.Hkv;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
   const bool relay = rpb > 1;
-  const int nrows = GLOB ? (S + W - 1) / W * rpb : S;  // keys: global rows or rows
+  const int nrows = GLOB ? doc_rows(S, W, rpb) : S;  // keys: global rows or rows
   const int k0 = tile * kBK;
   const int kw = k0 + wave * kKW;
 
@@ -855,7 +848,7 @@ void dkdv2_kernel(BwdArgs a) {
   if (GLOB) {
     const int c_lo = chunk * a.chunk_len;
     q_hi = min(S, c_lo + a.chunk_len);
-    q_lo = max(c_lo, glob_row_first_query(k0, W, rpb));
+    q_lo = max(c_lo, glob_row_first_query(k0, dc));
     // no query of this chunk sees the tile's rows: gsum_kernel skips the
     // chunk for them (with a single chunk the zeros are written instead)
     if (q_hi <= q_lo && a.nchunk > 1) return;
@@ -883,7 +876,7 @@ void dkdv2_kernel(BwdArgs a) {
     const int row = kw + 16 * kb + l16;
     // query rows at or past q_hi load as zeros: excluded
     if (GLOB) {
-      qmin[kb] = row < nrows ? glob_row_first_query(row, W, rpb) : S;
+      qmin[kb] = row < nrows ? glob_row_first_query(row, dc) : S;
       qmax[kb] = q_hi - 1;
     } else {
       qmin[kb] = row;
@@ -913,9 +906,9 @@ void dkdv2_kernel(BwdArgs a) {
   const bool active = kw < nrows;
   const int k_last = min(kw + kKW, nrows) - 1;
   // queries this wave can see at all
-  const int wq_lo = GLOB ? (active ? max(q_lo, glob_row_first_query(kw, W, rpb)) : S) : kw;
+  const int wq_lo = GLOB ? (active ? max(q_lo, glob_row_first_query(kw, dc)) : S) : kw;
   const int wq_hi = GLOB ? q_hi : min(q_hi, kw + kKW - 1 + W);
-  const int full_lo = GLOB ? (active ? glob_row_first_query(k_last, W, rpb) : S) : k_last;
+  const int full_lo = GLOB ? (active ? glob_row_first_query(k_last, dc) : S) : k_last;
   const int full_hi = GLOB ? q_hi : kw + W;  // exclusive
   const float c2 = a.scale * kLog2e;
 
@@ -1073,9 +1066,9 @@ __device__ __forceinline__ void dq_f32_tile(const char* tK, const char* tV, cons
   }
 }
 
-template <int D>
+template <int D, int ND>
 __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2)))
-void dq_f32_kernel(BwdArgs a) {
+void dq_f32_kernel(BwdArgsT<ND> a) {
   constexpr int NW = kF32Waves, BN = kF32BN, kBM = 16 * NW;
   constexpr int kStages = D <= 64 ? 2 : 1;
   using Stage = SplitStage<D, BN, 64 * NW>;
@@ -1084,12 +1077,10 @@ void dq_f32_kernel(BwdArgs a) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int nbh = a.B * a.Hq;
-  const int bh = blockIdx.x % nbh;
-  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const QHead hd = q_head(a, blockIdx.x);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bh = hd.bh, b = hd.b, h = hd.h, hk = hd.hk;
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
-  const int b = bh / a.Hq, h = bh % a.Hq;
-  const int hk = h / (a.Hq / a.Hkv);
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * 16;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -1107,7 +1098,7 @@ void dq_f32_kernel(BwdArgs a) {
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
-  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int gmax = glob_prefix(hi - 1, dc);
   const int nloc = (hi - lo_k + BN - 1) / BN;
   const int nglob = (gmax + BN - 1) / BN;
   const int ntot = nloc + nglob;
@@ -1171,9 +1162,9 @@ void dq_f32_kernel(BwdArgs a) {
   const bool active = q0 < S;
   const int q_last = min(q0 + 16, S) - 1;
   const int w_lo = max(0, q0 - W + 1);
-  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
-  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
-  const int glen = glob_prefix(qi, W, rpb);
+  const int wg_lo = active ? glob_prefix(q0, dc) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, dc) : 0;
+  const int glen = glob_prefix(qi, dc);
 
   store(0);
   __syncthreads();
@@ -1274,10 +1265,10 @@ __device__ __forceinline__ void dkdv_f32_tile(const char* tQ, const char* tO, co
 template <int D, bool GLOB>
 constexpr bool kF32OneWave = D > 128 || (GLOB && D == 128);
 
-template <int D, bool GLOB>
+template <int D, bool GLOB, int ND>
 __global__ __launch_bounds__(64 * kF32Waves)
 __attribute__((amdgpu_waves_per_eu(kF32OneWave<D, GLOB> ? 1 : 2)))
-void dkdv_f32_kernel(BwdArgs a) {
+void dkdv_f32_kernel(BwdArgsT<ND> a) {
   constexpr int NW = kF32Waves, kBK = 16 * NW, kBQ = kF32BN;
   constexpr int kStages = D <= 64 || (GLOB && D == 128) ? 2 : 1;
   using Stage = SplitStage<D, kBQ, 64 * NW>;
@@ -1288,12 +1279,12 @@ void dkdv_f32_kernel(BwdArgs a) {
   const int lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int nbh = a.B * a.Hkv;
-  const int bhk = blockIdx.x % nbh;
-  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const KvHead hd = kv_head(a, blockIdx.x);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bhk = hd.bhk, b = hd.b, hk = hd.hk;
   const int nck = GLOB ? num_chunks(dc.len, a.chunk_len) : 1;
   const int tile = GLOB ? dc.item / nck : dc.item;
   const int chunk = GLOB ? dc.item - tile * nck : 0;
-  const int b = bhk / a.Hkv, hk = bhk % a.Hkv;
   const int grp = a.Hq / a.Hkv;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
   const int nrows = GLOB ? doc_rows(S, W, rpb) : S;  // keys: global rows or rows
@@ -1319,7 +1310,7 @@ void dkdv_f32_kernel(BwdArgs a) {
   if (GLOB) {
     const int c_lo = chunk * a.chunk_len;
     q_hi = min(S, c_lo + a.chunk_len);
-    q_lo = max(c_lo, glob_row_first_query(k0, W, rpb));
+    q_lo = max(c_lo, glob_row_first_query(k0, dc));
     // see dkdv2_kernel
     if (q_hi <= q_lo && a.nchunk > 1) return;
   } else {
@@ -1339,7 +1330,7 @@ void dkdv_f32_kernel(BwdArgs a) {
     kf[c] = load_split(kbase + (int64_t)rr * kstride + 32 * c + 8 * g);
     vf[c] = load_split(vbase + (int64_t)rr * vstride + 32 * c + 8 * g);
   }
-  int qmin = GLOB ? (row < nrows ? glob_row_first_query(row, W, rpb) : S) : row;
+  int qmin = GLOB ? (row < nrows ? glob_row_first_query(row, dc) : S) : row;
   const int qmax = GLOB ? q_hi - 1 : min(row + W, q_hi) - 1;
   // an empty interval gets a qmin no query reaches
   const unsigned qspan = qmax >= qmin ? (unsigned)(qmax - qmin) : 0u;
@@ -1351,9 +1342,9 @@ void dkdv_f32_kernel(BwdArgs a) {
   const bool active = kw < nrows;
   const int k_last = min(kw + 16, nrows) - 1;
   // queries this wave can see at all, and those every row of it sees
-  const int wq_lo = GLOB ? (active ? max(q_lo, glob_row_first_query(kw, W, rpb)) : S) : kw;
+  const int wq_lo = GLOB ? (active ? max(q_lo, glob_row_first_query(kw, dc)) : S) : kw;
   const int wq_hi = GLOB ? q_hi : min(q_hi, kw + 15 + W);
-  const int full_lo = GLOB ? (active ? glob_row_first_query(k_last, W, rpb) : S) : k_last;
+  const int full_lo = GLOB ? (active ? glob_row_first_query(k_last, dc) : S) : k_last;
   const int full_hi = GLOB ? q_hi : kw + W;  // exclusive
   const float c2 = a.scale * kLog2e;
 
@@ -1516,38 +1507,54 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   al.xcd_nt = xl ? nl : 0;
   const int gq = xq ? xcd_grid(a.B * a.Hq, nq) : nq * a.B * a.Hq;
   const int gl = xl ? xcd_grid(a.B * a.Hkv, nl) : nl * a.B * a.Hkv;
-  if constexpr (kF32) {
-    hipLaunchKernelGGL((dq_f32_kernel<D>), dim3(gq), dim3(64 * kF32Waves), 0, st, aq);
-    hipLaunchKernelGGL((dkdv_f32_kernel<D, true>), dim3(ng * a.B * a.Hkv), dim3(64 * kF32Waves), 0,
-                       st, ag);
-  } else {
-    if constexpr (D > 128)
-      hipLaunchKernelGGL((dq_wide_kernel<T, D>), dim3(gq), dim3(64 * kWideWaves), 0, st, aq);
+  const dim3 qgrid(gq), ggrid(ng * a.B * a.Hkv), lgrid(gl);
+  by_docs(aq, [&](const auto& x) {
+    constexpr int ND = std::decay_t<decltype(x)>::kDocs;
+    if constexpr (kF32)
+      hipLaunchKernelGGL((dq_f32_kernel<D, ND>), qgrid, dim3(64 * kF32Waves), 0, st, x);
+    else if constexpr (D > 128)
+      hipLaunchKernelGGL((dq_wide_kernel<T, D, ND>), qgrid, dim3(64 * kWideWaves), 0, st, x);
     else
-      hipLaunchKernelGGL((dq2_kernel<T, D, kDqWaves, kDqQB, kDqBN, kDqWPE>), dim3(gq),
-                         dim3(64 * kDqWaves), 0, st, aq);
-    // (at D = 256 the one geometry has 64 rows)
-    if (D <= 128 && narrow)
-      hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kNarrowWaves, kDkdvKB, kNarrowBQ>),
-                         dim3(ng * a.B * a.Hkv), dim3(64 * kNarrowWaves), 0, st, ag);
-    else
-      hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kDkdvGlobWaves<D>, kDkdvKB, kDkdvGlobBQ<D>>),
-                         dim3(ng * a.B * a.Hkv), dim3(64 * kDkdvGlobWaves<D>), 0, st, ag);
-  }
+      hipLaunchKernelGGL((dq2_kernel<T, D, kDqWaves, kDqQB, kDqBN, kDqWPE, ND>), qgrid,
+                         dim3(64 * kDqWaves), 0, st, x);
+  });
+  by_docs(ag, [&](const auto& x) {
+    constexpr int ND = std::decay_t<decltype(x)>::kDocs;
+    if constexpr (kF32) {
+      hipLaunchKernelGGL((dkdv_f32_kernel<D, true, ND>), ggrid, dim3(64 * kF32Waves), 0, st, x);
+    } else {
+      if constexpr (D <= 128) {  // (at D = 256 the one geometry has 64 rows)
+        if (narrow) {
+          hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kNarrowWaves, kDkdvKB, kNarrowBQ, ND>),
+                             ggrid, dim3(64 * kNarrowWaves), 0, st, x);
+          return;
+        }
+      }
+      hipLaunchKernelGGL((dkdv2_kernel<T, D, true, kDkdvGlobWaves<D>, kDkdvKB, kDkdvGlobBQ<D>, ND>),
+                         ggrid, dim3(64 * kDkdvGlobWaves<D>), 0, st, x);
+    }
+  });
   if (a.nchunk > 1) {
     BwdArgs as = a;
     set_items(as.docs, [&](int d) {
       return (doc_rows(a.docs.len[d], a.docs.W[d], a.docs.rpb[d]) * (2 * D / 4) + 255) / 256;
     });
-    hipLaunchKernelGGL((gsum_kernel<D>), dim3(as.docs.item0[a.docs.n] * a.B * a.Hkv), dim3(256),
-                       0, st, as);
+    by_docs(as, [&](const auto& x) {
+      constexpr int ND = std::decay_t<decltype(x)>::kDocs;
+      hipLaunchKernelGGL((gsum_kernel<D, ND>), dim3(x.docs.item0[x.docs.n] * a.B * a.Hkv),
+                         dim3(256), 0, st, x);
+    });
   }
   if (a.dalpha) hipLaunchKernelGGL((dalpha_kernel<T, D>), dim3(a.Hkv), dim3(1024), 0, st, a);
-  if constexpr (kF32)
-    hipLaunchKernelGGL((dkdv_f32_kernel<D, false>), dim3(gl), dim3(64 * kF32Waves), 0, st, al);
-  else
-    hipLaunchKernelGGL((dkdv2_kernel<T, D, false, kDkdvLocalWaves, kDkdvLocalKB<D>, kDkdvLocalBQ>),
-                       dim3(gl), dim3(64 * kDkdvLocalWaves), 0, st, al);
+  by_docs(al, [&](const auto& x) {
+    constexpr int ND = std::decay_t<decltype(x)>::kDocs;
+    if constexpr (kF32)
+      hipLaunchKernelGGL((dkdv_f32_kernel<D, false, ND>), lgrid, dim3(64 * kF32Waves), 0, st, x);
+    else
+      hipLaunchKernelGGL(
+          (dkdv2_kernel<T, D, false, kDkdvLocalWaves, kDkdvLocalKB<D>, kDkdvLocalBQ, ND>), lgrid,
+          dim3(64 * kDkdvLocalWaves), 0, st, x);
+  });
   return hipGetLastError();
 }
 
@@ -1609,7 +1616,7 @@ ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len,
     for (int d = 0; d < n; ++d) {
       const int g = doc_rows(len[d], W[d], rpb[d]);
       for (int t = 0; t < g; t += 64)
-        sweeps += std::max(0, len[d] - glob_row_first_query(t, W[d], rpb[d]));
+        sweeps += std::max(0, len[d] - (t / rpb[d] + 1) * W[d]);
     }
     sweeps *= (double)B * Hkv;
     const double pieces = 3.0 * (cus > 0 ? cus : 256);
@@ -1667,7 +1674,9 @@ bool bwd_tile_config(int dtype, int D, int out[9]) {
   return true;
 }
 
-hipError_t launch_bwd(int dtype, int D, const BwdArgs& a, hipStream_t st) {
+hipError_t launch_bwd(int dtype, int D, const BwdArgs& args, hipStream_t st) {
+  BwdArgs a = args;
+  set_divs(a);
   switch (dtype) {
     case 0: return launch_T<f16>(D, a, st);
     case 1: return launch_T<bf16>(D, a, st);

@@ -85,17 +85,6 @@ __device__ __forceinline__ Frag<T> lds_frag_row(const T* p) {
   return f;
 }
 
-// ---------------------------------------------------------------------------
-// sqrt(N) geometry (reference core.py:957, 1038-1061, 1112-1117).
-// ---------------------------------------------------------------------------
-// Length of the global-row prefix query i attends to. With relay each W-block
-// contributes rpb = 1 + top_k rows (strided row first); without, rpb = 1.
-__device__ __forceinline__ int glob_prefix(int i, int W, int rpb) {
-  const int a = max(i - W + 1, 0);
-  const int f = a / W;
-  return rpb * f + ((a - f * W) != 0 ? 1 : 0);
-}
-
 // Cross-lane helpers on the 4 lane groups of a wave (lanes l, l^16, l^32, l^48).
 __device__ __forceinline__ float group_max(float x) {
   x = fmaxf(x, __shfl_xor(x, 16));

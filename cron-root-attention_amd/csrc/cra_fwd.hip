@@ -127,9 +127,9 @@ __device__ __forceinline__ void attend_f32(const char* tK, const char* tV, const
   }
 }
 
-template <int D, int QB>
+template <int D, int QB, int ND>
 __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(D > 64 ? 1 : 2)))
-void fwd_f32_kernel(FwdArgs a) {
+void fwd_f32_kernel(FwdArgsT<ND> a) {
   constexpr int NW = kF32Waves, BN = kF32BN, kQW = 16 * QB, kBM = NW * kQW;
   constexpr int kStages = D <= 64 ? 2 : 1;
   using Stage = SplitStage<D, BN, 64 * NW>;
@@ -138,12 +138,10 @@ void fwd_f32_kernel(FwdArgs a) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int nbh = a.B * a.Hq;
-  const int bh = blockIdx.x % nbh;
-  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const QHead hd = q_head(a, blockIdx.x);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bh = hd.bh, b = hd.b, h = hd.h, hk = hd.hk;
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
-  const int b = bh / a.Hq, h = bh % a.Hq;
-  const int hk = h / (a.Hq / a.Hkv);
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * kQW;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -157,7 +155,7 @@ void fwd_f32_kernel(FwdArgs a) {
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
-  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int gmax = glob_prefix(hi - 1, dc);
   const int nloc = (a.phases & 1) ? (hi - lo_k + BN - 1) / BN : 0;
   const int nglob = (a.phases & 2) ? (gmax + BN - 1) / BN : 0;
   const int ntot = nloc + nglob;
@@ -197,11 +195,11 @@ void fwd_f32_kernel(FwdArgs a) {
   const bool active = q0 < S;
   const int q_last = min(q0 + kQW, S) - 1;
   const int w_lo = max(0, q0 - W + 1);
-  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
-  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
+  const int wg_lo = active ? glob_prefix(q0, dc) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, dc) : 0;
   int glen[QB];
 #pragma unroll
-  for (int qb = 0; qb < QB; ++qb) glen[qb] = glob_prefix(qi[qb], W, rpb);
+  for (int qb = 0; qb < QB; ++qb) glen[qb] = glob_prefix(qi[qb], dc);
 
   auto store = [&](int it) {
     char(&dst)[2][Stage::kBytes] = lds[kStages == 2 ? it & 1 : 0];
@@ -473,8 +471,8 @@ using FwdStage = char[2][SwzTile<D, 64>::kBytes];  // K and V tiles of one pipel
 
 // One work item (a 128-query tile of one (b, h); items numbered heaviest
 // first, consecutive items on different heads) with its LDS stages.
-template <typename T, int D, int NW, int PH>
-__device__ __forceinline__ void fwd2_item(const FwdArgs& a, const int item, FwdStage<D>& stage0,
+template <typename T, int D, int NW, int PH, int ND>
+__device__ __forceinline__ void fwd2_item(const FwdArgsT<ND>& a, const int item, FwdStage<D>& stage0,
                                           FwdStage<D>& stage1) {
   constexpr int BN = 64;
   using Tile = SwzTile<D, BN>;
@@ -483,12 +481,10 @@ __device__ __forceinline__ void fwd2_item(const FwdArgs& a, const int item, FwdS
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int nbh = a.B * a.Hq;
-  const int bh = item % nbh;
-  const Doc dc = find_doc(a.docs, item / nbh);
+  const QHead hd = q_head(a, item);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bh = hd.bh, b = hd.b, h = hd.h, hk = hd.hk;
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
-  const int b = bh / a.Hq, h = bh % a.Hq;
-  const int hk = h / (a.Hq / a.Hkv);
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * kQW;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -503,7 +499,7 @@ __device__ __forceinline__ void fwd2_item(const FwdArgs& a, const int item, FwdS
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
-  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int gmax = glob_prefix(hi - 1, dc);
   const int nloc = (PH & 1) ? (hi - lo_k + kBN - 1) / kBN : 0;
   // Global tiles come first: every workgroup of the head reads them, so the
   // first fill (issued before anything can hide it) is an L2 hit, and the
@@ -565,9 +561,9 @@ __device__ __forceinline__ void fwd2_item(const FwdArgs& a, const int item, FwdS
   const bool active = q0 < S;
   const int q_last = min(q0 + kQW, S) - 1;
   const int w_lo = max(0, q0 - W + 1);
-  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
-  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
-  const int glen[2] = {glob_prefix(qi[0], W, rpb), glob_prefix(qi[1], W, rpb)};
+  const int wg_lo = active ? glob_prefix(q0, dc) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, dc) : 0;
+  const int glen[2] = {glob_prefix(qi[0], dc), glob_prefix(qi[1], dc)};
 
   const Frag<T> one = ones_frag<T>();
   // Local and global tiles share one body (parameters chosen per tile); the
@@ -632,9 +628,9 @@ __device__ __forceinline__ void fwd2_item(const FwdArgs& a, const int item, FwdS
 // Two pipeline stages as separate LDS objects, each selected at compile
 // time: the compiler can then tell the fill of one stage from reads of the
 // other and does not wait for the fill before those reads.
-template <typename T, int D, int NW, int PH>
+template <typename T, int D, int NW, int PH, int ND>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 3)))
-void fwd2_kernel(FwdArgs a) {
+void fwd2_kernel(FwdArgsT<ND> a) {
   __shared__ __attribute__((aligned(1024))) FwdStage<D> stage0;
   __shared__ __attribute__((aligned(1024))) FwdStage<D> stage1;
   int item = (int)blockIdx.x;
@@ -642,7 +638,7 @@ void fwd2_kernel(FwdArgs a) {
     item = xcd_item(item, a.B * a.Hq, a.xcd_nt);
     if (item < 0) return;  // padding block
   }
-  fwd2_item<T, D, NW, PH>(a, item, stage0, stage1);
+  fwd2_item<T, D, NW, PH, ND>(a, item, stage0, stage1);
 }
 
 // Persistent form (use_persistent; the reference's work-queue kernel,
@@ -652,7 +648,7 @@ void fwd2_kernel(FwdArgs a) {
 // counter passes the item count.
 template <typename T, int D, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 3)))
-void fwd2_persistent_kernel(FwdArgs a) {
+void fwd2_persistent_kernel(FwdArgsT<1> a) {
   __shared__ __attribute__((aligned(1024))) FwdStage<D> stage0;
   __shared__ __attribute__((aligned(1024))) FwdStage<D> stage1;
   __shared__ int next_item;
@@ -663,7 +659,7 @@ void fwd2_persistent_kernel(FwdArgs a) {
     const int item = next_item;
     __syncthreads();  // read before the next overwrite
     if (item >= n_items) break;
-    fwd2_item<T, D, NW, 3>(a, item, stage0, stage1);
+    fwd2_item<T, D, NW, 3, 1>(a, item, stage0, stage1);
   }
 }
 
@@ -677,9 +673,9 @@ void fwd2_persistent_kernel(FwdArgs a) {
 // S=32768 fp16: 214 us (562 effective TFLOP/s); fwd_kernel (tiles through
 // registers, V stored transposed by 2-byte LDS writes) took 470 us.
 constexpr int kWideWaves = 4, kWideBN = 32;
-template <typename T, int D>
+template <typename T, int D, int ND>
 __global__ __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(3)))
-void fwd_wide_kernel(FwdArgs a) {
+void fwd_wide_kernel(FwdArgsT<ND> a) {
   constexpr int NW = kWideWaves, BN = kWideBN, kBM = 16 * NW;
   using Tile = SwzTile<D, BN>;
   __shared__ __attribute__((aligned(1024))) char sK[Tile::kBytes];
@@ -688,12 +684,10 @@ void fwd_wide_kernel(FwdArgs a) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int nbh = a.B * a.Hq;
-  const int bh = blockIdx.x % nbh;
-  const Doc dc = find_doc(a.docs, (int)(blockIdx.x / nbh));
+  const QHead hd = q_head(a, blockIdx.x);
+  const Doc dc = find_doc(a.docs, hd.rest);
+  const int bh = hd.bh, b = hd.b, h = hd.h, hk = hd.hk;
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
-  const int b = bh / a.Hq, h = bh % a.Hq;
-  const int hk = h / (a.Hq / a.Hkv);
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * 16;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
@@ -707,7 +701,7 @@ void fwd_wide_kernel(FwdArgs a) {
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
-  const int gmax = glob_prefix(hi - 1, W, rpb);
+  const int gmax = glob_prefix(hi - 1, dc);
   const int nloc = (a.phases & 1) ? (hi - lo_k + BN - 1) / BN : 0;
   const int nglob = (a.phases & 2) ? (gmax + BN - 1) / BN : 0;
   const int ntot = nloc + nglob;
@@ -753,9 +747,9 @@ void fwd_wide_kernel(FwdArgs a) {
   const bool active = q0 < S;
   const int q_last = min(q0 + 16, S) - 1;
   const int w_lo = max(0, q0 - W + 1);
-  const int wg_lo = active ? glob_prefix(q0, W, rpb) : 0;
-  const int wg_hi = active ? glob_prefix(q_last, W, rpb) : 0;
-  const int glen = glob_prefix(qi, W, rpb);
+  const int wg_lo = active ? glob_prefix(q0, dc) : 0;
+  const int wg_hi = active ? glob_prefix(q_last, dc) : 0;
+  const int glen = glob_prefix(qi, dc);
   const Frag<T> one = ones_frag<T>();
 
   for (int it = 0; it < ntot; ++it) {
@@ -844,7 +838,10 @@ hipError_t launch_f32(int D, const FwdArgs& a, hipStream_t st) {
     constexpr int kBM = 16 * kF32Waves * kF32QB<Dc>;
     set_items(b.docs, [&](int d) { return (b.docs.len[d] + kBM - 1) / kBM; });
     const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq);
-    hipLaunchKernelGGL((fwd_f32_kernel<Dc, kF32QB<Dc>>), grid, dim3(64 * kF32Waves), 0, st, b);
+    by_docs(b, [&](const auto& x) {
+      constexpr int ND = std::decay_t<decltype(x)>::kDocs;
+      hipLaunchKernelGGL((fwd_f32_kernel<Dc, kF32QB<Dc>, ND>), grid, dim3(64 * kF32Waves), 0, st, x);
+    });
   };
   switch (D) {
     case 32: go(std::integral_constant<int, 32>{}); break;
@@ -862,7 +859,10 @@ hipError_t launch_wide(const FwdArgs& a, hipStream_t st) {
   FwdArgs b = a;
   set_items(b.docs, [&](int d) { return (b.docs.len[d] + kBM - 1) / kBM; });
   const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq);
-  hipLaunchKernelGGL((fwd_wide_kernel<T, 256>), grid, dim3(64 * kWideWaves), 0, st, b);
+  by_docs(b, [&](const auto& x) {
+    constexpr int ND = std::decay_t<decltype(x)>::kDocs;
+    hipLaunchKernelGGL((fwd_wide_kernel<T, 256, ND>), grid, dim3(64 * kWideWaves), 0, st, x);
+  });
   return hipGetLastError();
 }
 
@@ -883,22 +883,31 @@ hipError_t launch_T(int D, const FwdArgs& a, hipStream_t st) {
   hipError_t qerr = hipSuccess;
   auto go = [&](auto dc) {
     constexpr int Dc = decltype(dc)::value;
-    if (a.work_counter && a.phases == 3) {
-      // one round of resident workgroups: CUs x workgroups per CU
-      auto kern = fwd2_persistent_kernel<T, Dc, kFwdWaves>;
-      int slots = 0;
-      qerr = resident_slots<T, Dc>(kern, 64 * kFwdWaves, &slots);
-      if (qerr != hipSuccess) return;
-      const int items = (int)grid.x;
-      const dim3 pgrid(std::max(1, std::min(items, slots)));
-      hipLaunchKernelGGL(kern, pgrid, block, 0, st, b);
-      return;
-    }
-    switch (a.phases) {
-      case 1: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 1>), xgrid, block, 0, st, bx); break;
-      case 2: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 2>), xgrid, block, 0, st, bx); break;
-      default: hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 3>), xgrid, block, 0, st, bx);
-    }
+    by_docs(bx, [&](const auto& x) {
+      constexpr int ND = std::decay_t<decltype(x)>::kDocs;
+      if constexpr (ND == 1) {
+        // one document: also the persistent and the phase-restricted forms
+        if (a.work_counter && a.phases == 3) {
+          // one round of resident workgroups: CUs x workgroups per CU
+          auto kern = fwd2_persistent_kernel<T, Dc, kFwdWaves>;
+          int slots = 0;
+          qerr = resident_slots<T, Dc>(kern, 64 * kFwdWaves, &slots);
+          if (qerr != hipSuccess) return;
+          const dim3 pgrid(std::max(1, std::min((int)grid.x, slots)));
+          hipLaunchKernelGGL(kern, pgrid, block, 0, st, x);
+          return;
+        }
+        if (a.phases == 1) {
+          hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 1, 1>), xgrid, block, 0, st, x);
+          return;
+        }
+        if (a.phases == 2) {
+          hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 2, 1>), xgrid, block, 0, st, x);
+          return;
+        }
+      }
+      hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 3, ND>), xgrid, block, 0, st, x);
+    });
   };
   switch (D) {
     case 32: go(std::integral_constant<int, 32>{}); break;
@@ -926,7 +935,9 @@ bool fwd_tile_config(int dtype, int D, int out[3]) {
   return true;
 }
 
-hipError_t launch_fwd(int dtype, int D, const FwdArgs& a, hipStream_t st) {
+hipError_t launch_fwd(int dtype, int D, const FwdArgs& args, hipStream_t st) {
+  FwdArgs a = args;
+  set_divs(a);
   switch (dtype) {
     case 0: return launch_T<f16>(D, a, st);
     case 1: return launch_T<bf16>(D, a, st);

@@ -15,6 +15,8 @@
 // reproduce it bit for bit: each lane sums the squares of its 8 consecutive
 // elements left to right (no fused multiply-add), then the D/8 lane partials
 // are combined by a butterfly p += p[lane ^ off], off = D/16 .. 1.
+#include <type_traits>
+
 #include "cra_common.hpp"
 #include "cra_internal.hpp"
 
@@ -38,8 +40,8 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t x, int off) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-template <typename T, int D>
-__global__ __launch_bounds__(256) void build_global_kernel(GlobalArgs a) {
+template <typename T, int D, int ND>
+__global__ __launch_bounds__(256) void build_global_kernel(GlobalArgsT<ND> a) {
   constexpr int kLPR = D / 8;        // lanes per row
   constexpr int kNRG = 256 / kLPR;   // row groups per workgroup
   constexpr int kW16 = Frag<T>::kWords;
@@ -194,11 +196,18 @@ hipError_t launch_T(int D, const GlobalArgs& args, int B, hipStream_t st) {
   GlobalArgs a = args;  // work items: the W-blocks of each document
   set_items(a.docs, [&](int d) { return (a.docs.len[d] + a.docs.W[d] - 1) / a.docs.W[d]; });
   dim3 grid(a.docs.item0[a.docs.n], B * a.Hkv);
+  auto go = [&](auto dc) {
+    constexpr int Dc = decltype(dc)::value;
+    by_docs(a, [&](const auto& x) {
+      constexpr int ND = std::decay_t<decltype(x)>::kDocs;
+      hipLaunchKernelGGL((build_global_kernel<T, Dc, ND>), grid, dim3(256), 0, st, x);
+    });
+  };
   switch (D) {
-    case 32: hipLaunchKernelGGL((build_global_kernel<T, 32>), grid, dim3(256), 0, st, a); break;
-    case 64: hipLaunchKernelGGL((build_global_kernel<T, 64>), grid, dim3(256), 0, st, a); break;
-    case 128: hipLaunchKernelGGL((build_global_kernel<T, 128>), grid, dim3(256), 0, st, a); break;
-    case 256: hipLaunchKernelGGL((build_global_kernel<T, 256>), grid, dim3(256), 0, st, a); break;
+    case 32: go(std::integral_constant<int, 32>{}); break;
+    case 64: go(std::integral_constant<int, 64>{}); break;
+    case 128: go(std::integral_constant<int, 128>{}); break;
+    case 256: go(std::integral_constant<int, 256>{}); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -13,29 +13,61 @@ namespace cra {
 // work items are numbered document by document: item0[d] is the first item
 // of document d and item0[n] the total.
 constexpr int kMaxDocs = 64;
-struct Docs {
-  int n;
-  int off[kMaxDocs];   // first row along S
-  int len[kMaxDocs];   // rows
-  int W[kMaxDocs];     // window = block size
-  int rpb[kMaxDocs];   // packed global rows per block: 1 + top_k with relay, else 1
-  int gofs[kMaxDocs];  // first packed global row
-  int bofs[kMaxDocs];  // first block (relay_src rows)
-  int pofs[kMaxDocs];  // backward: first row of the global-row partials, per (b, kv head)
-  int item0[kMaxDocs + 1];
+
+// Division of a 32-bit unsigned by a launch constant (Granlund and Montgomery,
+// "Division by Invariant Integers using Multiplication", 1994): a multiply, a
+// subtraction and two shifts where the compiler's 32-bit division is about
+// forty instructions.
+struct FastDiv {
+  uint32_t m, sh;  // multiplier; the two shifts, the second in bits 8..
 };
+inline FastDiv fast_div(uint32_t d) {
+  int l = 0;
+  while (l < 32 && (uint64_t(1) << l) < d) ++l;
+  const uint64_t m = ((((uint64_t(1) << l) - d) << 32) / d) + 1;
+  return FastDiv{(uint32_t)m, (uint32_t)((l > 0 ? 1 : 0) | (l > 1 ? l - 1 : 0) << 8)};
+}
+__host__ __device__ inline uint32_t div_by(uint32_t n, FastDiv f) {
+  const uint32_t t = (uint32_t)(((uint64_t)f.m * n) >> 32);
+  return (t + ((n - t) >> (f.sh & 0xff))) >> (f.sh >> 8);
+}
+
+template <int N>
+struct DocsT {
+  int n;
+  int off[N];   // first row along S
+  int len[N];   // rows
+  int W[N];     // window = block size
+  FastDiv dW[N];
+  int rpb[N];   // packed global rows per block: 1 + top_k with relay, else 1
+  FastDiv drpb[N];
+  int gofs[N];  // first packed global row
+  int bofs[N];  // first block (relay_src rows)
+  int pofs[N];  // backward: first row of the global-row partials, per (b, kv head)
+  int item0[N + 1];
+};
+using Docs = DocsT<kMaxDocs>;
 
 // One document, resolved for a work item.
 struct Doc {
   int off, len, W, rpb, gofs, bofs, pofs;
+  FastDiv dW, drpb;
   int item;  // work item index within the document
 };
 
-__device__ __forceinline__ Doc find_doc(const Docs& t, int item) {
+// A launch of one document (every plain call) takes a table of one: a tenth
+// of the kernel arguments, and no lookup on the way to the first load. With
+// the divisions above, each kernel of a short call is 0.5-1 us shorter (H=12
+// S=1000 D=64: forward 8.9 -> 8.4 us, dQ 10.4 -> 9.7; H=8 S=8192 forward 17.5
+// -> 17.0, global-row build 7.5 -> 6.5; B=2 H=32 S=4096 D=128 forward 77.5 ->
+// 72 us).
+template <int N>
+__device__ __forceinline__ Doc find_doc(const DocsT<N>& t, int item) {
   int d = 0;
-  for (int i = 1; i < t.n; ++i) d += item >= t.item0[i];  // item0 is non-decreasing
-  return Doc{t.off[d], t.len[d], t.W[d], t.rpb[d], t.gofs[d], t.bofs[d], t.pofs[d],
-             item - t.item0[d]};
+  if constexpr (N > 1)
+    for (int i = 1; i < t.n; ++i) d += item >= t.item0[i];  // item0 is non-decreasing
+  return Doc{t.off[d],  t.len[d],  t.W[d],  t.rpb[d],  t.gofs[d],
+             t.bofs[d], t.pofs[d], t.dW[d], t.drpb[d], item - (N > 1 ? t.item0[d] : 0)};
 }
 
 // XCD-aware work order for launches of nbh heads x nt tiles (one document)
@@ -106,7 +138,7 @@ __host__ __device__ inline int xcd_item(int block, int nbh, int nt) {
   return r * nbh + c.q0 + (p < c.r0 ? 1 : 0) + (k - xcd_before(c, nt, r));
 }
 
-struct GlobalArgs {
+struct GlobalCommon {
   const void* k;
   const void* v;
   int64_t ksb, ksh, kss, vsb, vsh, vss;
@@ -117,10 +149,16 @@ struct GlobalArgs {
   int Hkv, top_k;
   int NB;              // blocks of all documents (rows of relay_src per head)
   int64_t G;           // packed global rows of all documents, per head
-  Docs docs;           // items: W-blocks
 };
+template <int N>
+struct GlobalArgsT : GlobalCommon {
+  using Common = GlobalCommon;
+  static constexpr int kDocs = N;
+  DocsT<N> docs;  // items: W-blocks
+};
+using GlobalArgs = GlobalArgsT<kMaxDocs>;
 
-struct FwdArgs {
+struct FwdCommon {
   const void* q;
   const void* k;
   const void* v;
@@ -130,16 +168,23 @@ struct FwdArgs {
   float* lse;
   int64_t qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, osb, osh, oss;
   int B, Hq, Hkv;
+  FastDiv d_bhq, d_hq, d_bhkv, d_hkv, d_grp;  // by B * Hq, Hq, B * Hkv, Hkv, Hq / Hkv
   int S;       // rows along S of all documents (row stride of lse)
   int64_t G;   // packed global rows of all documents, per head
   float scale;
   int phases;  // bit 0: local window, bit 1: global rows
   int* work_counter;  // persistent launch: zeroed item counter, else null
   int xcd_nt;  // > 0: XCD-aware order (xcd_item) over this many tiles per head
-  Docs docs;   // items: query tiles (set by the launcher for its tile size)
 };
+template <int N>
+struct FwdArgsT : FwdCommon {
+  using Common = FwdCommon;
+  static constexpr int kDocs = N;
+  DocsT<N> docs;  // items: query tiles (set by the launcher for its tile size)
+};
+using FwdArgs = FwdArgsT<kMaxDocs>;
 
-struct BwdArgs {
+struct BwdCommon {
   const void* q;
   const void* k;
   const void* v;
@@ -160,6 +205,7 @@ struct BwdArgs {
   int64_t qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, osb, osh, oss;
   int64_t dosb, dosh, doss, dqsb, dqsh, dqss, dksb, dksh, dkss, dvsb, dvsh, dvss;
   int B, Hq, Hkv, top_k;
+  FastDiv d_bhq, d_hq, d_bhkv, d_hkv, d_grp;  // by B * Hq, Hq, B * Hkv, Hkv, Hq / Hkv
   int S;           // rows along S of all documents (row stride of lse, delta)
   int NB;          // blocks of all documents (rows of relay_src per head)
   int64_t G;       // packed global rows of all documents, per head
@@ -169,8 +215,60 @@ struct BwdArgs {
   int group;       // 0: first launch of a call (writes dalpha);
                    // later document groups of the call add to dalpha
   int xcd_nt;      // > 0: XCD-aware order (xcd_item) over this many tiles per head
-  Docs docs;       // items: set by the launcher per kernel
 };
+template <int N>
+struct BwdArgsT : BwdCommon {
+  using Common = BwdCommon;
+  static constexpr int kDocs = N;
+  DocsT<N> docs;  // items: set by the launcher per kernel
+};
+using BwdArgs = BwdArgsT<kMaxDocs>;
+
+// Calls launch(args) with the arguments over a table of one document if there
+// is one, else with the table as it is.
+template <template <int> class A, typename F>
+inline void by_docs(const A<kMaxDocs>& a, F launch) {
+  if (a.docs.n != 1) {
+    launch(a);
+    return;
+  }
+  A<1> o;
+  using Common = typename A<1>::Common;
+  static_cast<Common&>(o) = a;
+  const Docs& t = a.docs;
+  o.docs = DocsT<1>{1,           {t.off[0]},    {t.len[0]},  {t.W[0]},    {t.dW[0]}, {t.rpb[0]},
+                    {t.drpb[0]}, {t.gofs[0]},   {t.bofs[0]}, {t.pofs[0]}, {t.item0[0], t.item0[1]}};
+  launch(o);
+}
+
+template <typename A>
+inline void set_divs(A& a) {
+  a.d_bhq = fast_div(a.B * a.Hq);
+  a.d_hq = fast_div(a.Hq);
+  a.d_bhkv = fast_div(a.B * a.Hkv);
+  a.d_hkv = fast_div(a.Hkv);
+  a.d_grp = fast_div(a.Hq / a.Hkv);
+}
+
+// (batch, head) of a work item, items numbered heads first.
+struct QHead {
+  int rest, bh, b, h, hk;
+};
+template <typename A>
+__device__ __forceinline__ QHead q_head(const A& a, int item) {
+  const int rest = div_by(item, a.d_bhq), bh = item - rest * (a.B * a.Hq);
+  const int b = div_by(bh, a.d_hq), h = bh - b * a.Hq;
+  return QHead{rest, bh, b, h, (int)div_by(h, a.d_grp)};
+}
+struct KvHead {
+  int rest, bhk, b, hk;
+};
+template <typename A>
+__device__ __forceinline__ KvHead kv_head(const A& a, int item) {
+  const int rest = div_by(item, a.d_bhkv), bhk = item - rest * (a.B * a.Hkv);
+  const int b = div_by(bhk, a.d_hkv);
+  return KvHead{rest, bhk, b, bhk - b * a.Hkv};
+}
 
 // Number the work items document by document: count(d) items for document d.
 template <typename F>
@@ -196,6 +294,21 @@ __host__ __device__ inline int num_chunks(int len, int chunk_len) {
 
 // Packed global rows of a document.
 __host__ __device__ inline int doc_rows(int len, int W, int rpb) { return (len + W - 1) / W * rpb; }
+
+// sqrt(N) geometry (reference core.py:957, 1038-1061, 1112-1117): length of the
+// global-row prefix query i attends to. With relay each W-block contributes
+// rpb = 1 + top_k rows (strided row first); without, rpb = 1.
+__device__ __forceinline__ int glob_prefix(int i, const Doc& dc) {
+  const int a = i - dc.W + 1 > 0 ? i - dc.W + 1 : 0;
+  const int f = div_by(a, dc.dW);
+  return dc.rpb * f + ((a - f * dc.W) != 0 ? 1 : 0);
+}
+
+// First query that sees packed global row gr (inverse of glob_prefix).
+__device__ __forceinline__ int glob_row_first_query(int gr, const Doc& dc) {
+  const int r = div_by(gr, dc.drpb);
+  return (gr - r * dc.rpb) == 0 ? r * dc.W + dc.W : (r + 1) * dc.W + dc.W - 1;
+}
 
 // Partial dK/dV of global row `row` of a document from query chunk `chunk`:
 // row index into gpart ([2, D] each). A document's partials are
