@@ -368,6 +368,7 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   a.NB = (int)pl.NB;
   a.G = pl.G;
   a.scale = p->scale;
+  a.cus = device_cus();
   a.chunk_len = chunks.chunk_len;
   a.nchunk = chunks.nchunk;
   // workspace carve-up: delta and nlse2 [B*Hq*S] fp32 each, then the

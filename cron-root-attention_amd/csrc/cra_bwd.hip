@@ -1452,30 +1452,46 @@ constexpr int kDkdvLocalBQ = 32;
 
 // The global-row kernel's second geometry: 4-wave workgroups of 64 rows with
 // 32-query tiles (the local kernel's: 33 KB of LDS, 3 workgroups per CU at
-// D = 128), for problems of few packed rows. A workgroup of 192 rows then
-// leaves most waves without a visible row in the early chunks (at G = 192
-// all rows are one tile, and half of its wave slots idle), and one workgroup
-// per CU makes the last round coarse; against that, 64-row tiles sweep the
-// queries once per 64 rows. Kernel time, 192-row / 64-row workgroups, D = 128
-// (H: query / kv heads):
-//   B=2 H=32/32 S=4096   (G =  192)   72 /   51 us
-//   B=1 H=16/4  S=16000  (G =  381)  112 /   82 us
-//   B=1 H=16/16 S=32768  (G =  546)  210 /  213 us;  H=32/4  516 / 402 us
-//   B=1 H=16/16 S=65536  (G =  768)  557 /  523 us
-//   B=1 H=16/16 S=131072 (G = 1086) 1373 / 1550 us
-// Below D = 128 the first geometry is 128 rows with two workgroups per CU
-// and loses less: H=8 S=16384 (G = 384) 31 / 27 us, H=12 S=8192 (G = 273)
-// 20.6 / 21.1, S=32768 (G = 546) 96 / 96, S=65536 (G = 768) 227 / 242 us.
-constexpr int kNarrowWaves = 4, kNarrowBQ = 32;
-template <int D>
-constexpr int kNarrowMaxRows = D > 128 ? 0 : D == 128 ? 768 : 384;
+// D = 128). It is finer: where the wide workgroups (192 rows at D = 128, 128
+// below) are fewer than two rounds of the CUs their last round leaves the chip
+// half idle, and rows padded to a wide tile, or not yet visible to a chunk,
+// idle their waves. Against that, 64-row tiles sweep the queries once per 64
+// rows. Kernel time, wide / 64-row workgroups (wide workgroups in the launch;
+// H: query / kv heads; G: packed rows):
+//   D=128  B=2 H=32/32 S=4096  (384; G = 192)   72 /   51 us
+//          B=1 H=16/4  S=16000 (384; G = 381)  112 /   82 us
+//          B=1 H=16/16 S=16384 (384; G = 384)  109 /   84 us
+//          B=2 H=32/32 S=16384 (384; G = 384)  277 /  266 us
+//          B=1 H=32/4  S=32768 (384; G = 546)  516 /  402 us
+//          B=8 H=32/32 S=2048  (512; G =  45)   66 /   59 us
+//          B=8 H=32/32 S=4096  (512; G = 192)  166 /  206 us
+//          B=4 H=32/32 S=8192  (512; G = 273)  192 /  224 us
+//          B=4 H=32/8  S=32768 (576; G = 546) 1712 / 1720 us
+//          B=2 H=32/32 S=65536 (2816; G = 768) 2051 / 2520 us
+//   D=64   B=8 H=32/32 S=2048  (512; G =  45)   31 /   27 us
+//          B=4 H=32/32 S=8192  (768; G = 273)  126 /  128 us
+//          B=8 H=32/8  S=8192  (768; G = 273)  267 /  278 us
+//          B=1 H=12/12 S=65536 (792; G = 768)  227 /  242 us
+// So: the 64-row workgroups for launches of fewer than two wide workgroups
+// per CU (up to 768 rows, the most that was measured), and where the rows
+// padded to wide tiles are at least twice those padded to 64.
+constexpr int kNarrowWaves = 4, kNarrowBQ = 32, kNarrowMaxRows = 768;
 
 template <int D>
 bool narrow_glob(const BwdArgs& a) {
+  constexpr int kWide = 16 * kDkdvGlobWaves<D> * kDkdvKB, kNarrow = 16 * kNarrowWaves;
+  int64_t items = 0, wide = 0, narrow = 0;
   int most = 0;
-  for (int d = 0; d < a.docs.n; ++d)
-    most = std::max(most, doc_rows(a.docs.len[d], a.docs.W[d], a.docs.rpb[d]));
-  return most <= kNarrowMaxRows<D>;
+  for (int d = 0; d < a.docs.n; ++d) {
+    const int rows = doc_rows(a.docs.len[d], a.docs.W[d], a.docs.rpb[d]);
+    const int chunks = num_chunks(a.docs.len[d], a.chunk_len);
+    const int tiles = (rows + kWide - 1) / kWide;
+    most = std::max(most, rows);
+    items += (int64_t)tiles * chunks * a.B * a.Hkv;
+    wide += (int64_t)tiles * kWide * chunks;
+    narrow += (int64_t)(rows + kNarrow - 1) / kNarrow * kNarrow * chunks;
+  }
+  return D <= 128 && ((items < 2 * a.cus && most <= kNarrowMaxRows) || wide >= 2 * narrow);
 }
 
 template <typename T, int D>

@@ -210,6 +210,7 @@ struct BwdCommon {
   int NB;          // blocks of all documents (rows of relay_src per head)
   int64_t G;       // packed global rows of all documents, per head
   float scale;
+  int cus;         // compute units of the device (launch rules)
   int chunk_len;   // queries per chunk of the global-row kernel
   int nchunk;      // most query chunks of a document
   int group;       // 0: first launch of a call (writes dalpha);

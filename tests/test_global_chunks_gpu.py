@@ -24,11 +24,13 @@ def _check(grads, ref, dtype):
 
 
 @pytest.mark.parametrize("S,W,D,Hq,Hkv,dtype", [
-    (2048, 8, 128, 2, 2, F16),    # 768 rows: the last 64-row problem at D = 128
+    (2048, 8, 128, 2, 2, F16),    # 768 rows: the last 64-row problem of few workgroups
     (2049, 8, 128, 2, 2, F16),    # 771 rows: 192-row workgroups
     (700, 11, 128, 4, 2, BF16),   # 192 rows, grouped heads: three full 64-row tiles
-    (1024, 8, 64, 2, 2, F16),     # 384 rows: the last 64-row problem below D = 128
-    (1025, 8, 64, 2, 1, BF16),    # 387 rows: 128-row workgroups
+    (2048, 8, 64, 2, 2, F16),     # 768 rows below D = 128
+    (2049, 8, 64, 2, 1, BF16),    # 771 rows below D = 128: 128-row workgroups
+    (300, 9, 128, 256, 256, F16),  # 102 rows, two wide workgroups per CU: 192-row workgroups
+    (400, 20, 128, 128, 64, F16), # 60 rows: one 64-row tile
     (65, 65, 32, 1, 1, F16),      # one block: no query sees a global row
 ])
 def test_row_limits(S, W, D, Hq, Hkv, dtype):
