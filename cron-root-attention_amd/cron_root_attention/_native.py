@@ -98,6 +98,7 @@ _D = ctypes.POINTER(CraDocs)
 _SIGNATURES = {
     "cra_supported_head_dim": (ctypes.c_int, [ctypes.c_int32]),
     "cra_global_rows": (ctypes.c_int64, [_P]),
+    "cra_reads_global_rows": (ctypes.c_int, [_P, CraTensor, CraTensor]),
     "cra_build_global": (ctypes.c_int, [_P, CraTensor, CraTensor, ctypes.c_void_p, ctypes.c_void_p,
                                         ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     "cra_fwd": (ctypes.c_int, [_P, CraTensor, CraTensor, CraTensor, ctypes.c_void_p,
@@ -278,6 +279,15 @@ def global_rows(p: CraProblem) -> int:
             _raise(E_INVALID, "cra_global_rows")
         n = _sizes[key] = int(n)
     return n
+
+
+def reads_global_rows(p: CraProblem, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether cra_fwd / cra_bwd read the packed rows (else they take the
+    global rows from k and v, and build_global need not run)."""
+    n = load_library().cra_reads_global_rows(ctypes.byref(p), tensor_arg(k), tensor_arg(v))
+    if n < 0:
+        _raise(E_INVALID, "cra_reads_global_rows")
+    return bool(n)
 
 
 def build_global(p: CraProblem, k: torch.Tensor, v: torch.Tensor,

@@ -178,8 +178,12 @@ class CronRootAttentionV14Function(torch.autograd.Function):
                             1.0 / math.sqrt(D))
         rscale = _relay_scale(relay_log_scale, relay_on, q, Hkv)
         st = torch.cuda.current_stream(q.device).cuda_stream
-        gk, gv, src = _native.build_global(p, kp, vp, rscale, stream=st)
-        if use_persistent and not relay_on:   # the reference's persistent path (core.py:3548)
+        persistent = use_persistent and not relay_on  # the reference's path (core.py:3548)
+        if persistent or _native.reads_global_rows(p, kp, vp):
+            gk, gv, src = _native.build_global(p, kp, vp, rscale, stream=st)
+        else:  # the kernels read the global rows in kp and vp: nothing is packed
+            gk, gv, src = kp, vp, None
+        if persistent:
             o, lse = _native.forward_persistent(p, qp, kp, vp, gk, gv, stream=st)
         else:
             o, lse = _native.forward(p, qp, kp, vp, gk, gv, stream=st)

@@ -211,6 +211,16 @@ int plan_varlen(const cra_problem* p, const cra_docs* d, Plan* pl) {
   return CRA_OK;
 }
 
+// One document without relay, k and v of one row stride: its global rows are
+// rows r * W of k and v, and the kernels read them there. Their tiles are addressed with 32-bit offsets up
+// to 64 rows of W past the last one, so strides for which that could wrap keep
+// the packed rows.
+bool direct_rows(const cra_problem* p, const Plan& pl, const cra_tensor& k, const cra_tensor& v) {
+  if (pl.n != 1 || pl.any_relay) return false;
+  const int64_t step = k.ss * elem_size(p->dtype);
+  return k.ss == v.ss && k.ss >= 0 && (pl.len[0] + 64 * (int64_t)pl.W[0]) * step < ((int64_t)1 << 32);
+}
+
 int num_groups(const Plan& pl) { return (pl.n + cra::kMaxDocs - 1) / cra::kMaxDocs; }
 
 // Kernel-argument table of document group g (up to kMaxDocs documents, in
@@ -310,6 +320,9 @@ int fwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   a.scale = p->scale;
   a.phases = phase_mask;
   a.work_counter = work_counter;
+  // (the persistent and the phase-restricted kernels take packed rows only)
+  a.direct = !work_counter && phase_mask == (CRA_PHASE_LOCAL | CRA_PHASE_GLOBAL) &&
+             direct_rows(p, pl, k, v);
   for (int g = 0; g < num_groups(pl); ++g) {
     a.docs = group_table(pl, g);
     hipError_t e = cra::launch_fwd(p->dtype, p->D, a, (hipStream_t)stream);
@@ -369,6 +382,7 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   a.G = pl.G;
   a.scale = p->scale;
   a.cus = device_cus();
+  a.direct = direct_rows(p, pl, k, v);
   a.chunk_len = chunks.chunk_len;
   a.nchunk = chunks.nchunk;
   // workspace carve-up: delta and nlse2 [B*Hq*S] fp32 each, then the
@@ -446,6 +460,12 @@ int32_t cra_abi_version(void) { return CRA_ABI_VERSION; }
 int64_t cra_global_rows(const cra_problem* p) {
   if (check_problem(p)) return -1;
   return num_blocks(p) * rows_per_block(p);
+}
+
+int cra_reads_global_rows(const cra_problem* p, cra_tensor k, cra_tensor v) {
+  Plan pl;
+  if (plan_plain(p, &pl)) return -1;
+  return direct_rows(p, pl, k, v) ? 0 : 1;
 }
 
 int cra_build_global(const cra_problem* p, cra_tensor k, cra_tensor v, void* glob_k, void* glob_v,

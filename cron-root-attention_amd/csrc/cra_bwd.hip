@@ -253,7 +253,7 @@ __device__ __forceinline__ void dq2_tile(const char* tK, const char* tV, const L
 
 // NW waves of QB blocks of 16 queries each cover the workgroup's
 // 16 * NW * QB queries; key tiles of BN rows; at least WPE waves per SIMD.
-template <typename T, int D, int NW, int QB, int BN, int WPE, int ND>
+template <typename T, int D, int NW, int QB, int BN, int WPE, int ND, bool DIR = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE)))
 void dq2_kernel(BwdArgsT<ND> a) {
   using Tile = SwzTile<D, BN>;
@@ -287,9 +287,7 @@ void dq2_kernel(BwdArgsT<ND> a) {
   const float* lse = a.lse + (int64_t)bh * a.S + dc.off;
   float* delta = a.delta + (int64_t)bh * a.S + dc.off;
   float* nlse2 = a.nlse2 + (int64_t)bh * a.S + dc.off;
-  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
-  const T* gkp = static_cast<const T*>(a.gk) + gbase;
-  const T* gvp = static_cast<const T*>(a.gv) + gbase;
+  const GlobRows gr = glob_rows<T, D>(a, dc, b, hk, kp, vp, DIR);
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
@@ -303,14 +301,15 @@ void dq2_kernel(BwdArgsT<ND> a) {
   // Buffer resources over the rows this workgroup may read (local rows below
   // hi, global rows below gmax): loads past them return zeros.
   using Fill = typename Tile::template Fill<NW>;
-  const int kbytes = (int)(a.kss * 2), vbytes = (int)(a.vss * 2);
+  const int kbytes = (int)(a.kss * 2), vbytes = DIR ? kbytes : (int)(a.vss * 2);
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(kp, (uint32_t)((hi - 1) * kbytes + D * 2));
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(vp, (uint32_t)((hi - 1) * vbytes + D * 2));
-  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gkp, (uint32_t)(gmax * D * 2));
-  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gvp, (uint32_t)(gmax * D * 2));
+  const int gkb = (int)gr.kstep, gvb = (int)gr.vstep;
+  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gr.k, gmax > 0 ? (uint32_t)((gmax - 1) * gkb + D * 2) : 0);
+  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gr.v, gmax > 0 ? (uint32_t)((gmax - 1) * gvb + D * 2) : 0);
   const int fk = Fill::lane_off(wave, lane, kbytes);
   const int fv = Fill::lane_off(wave, lane, vbytes);
-  const int fg = Fill::lane_off(wave, lane, D * 2);
+  const int fgk = Fill::lane_off(wave, lane, gkb), fgv = Fill::lane_off(wave, lane, gvb);
   auto issue = [&](int it, char* dst) {
     if (it >= nglob) {
       const int ts = lo_k + (nloc - 1 - (it - nglob)) * kBN;
@@ -318,8 +317,8 @@ void dq2_kernel(BwdArgsT<ND> a) {
       Fill::load(dst + Tile::kBytes, rv, fv, vbytes, ts, wave);
     } else {
       const int ts = it * kBN;
-      Fill::load(dst, rgk, fg, D * 2, ts, wave);
-      Fill::load(dst + Tile::kBytes, rgv, fg, D * 2, ts, wave);
+      Fill::load(dst, rgk, fgk, gkb, ts, wave);
+      Fill::load(dst + Tile::kBytes, rgv, fgv, gvb, ts, wave);
     }
   };
   issue(0, stage0[0]);
@@ -444,7 +443,7 @@ void dq2_kernel(BwdArgsT<ND> a) {
 // dq_kernel (tiles through registers, V and K^T stored transposed by 2-byte
 // LDS writes, one stage) took 478 us and delta_kernel before it 46 us.
 constexpr int kWideWaves = 4, kWideBN = 32;
-template <typename T, int D, int ND>
+template <typename T, int D, int ND, bool DIR = false>
 __global__ __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(2)))
 void dq_wide_kernel(BwdArgsT<ND> a) {
   constexpr int NW = kWideWaves, BN = kWideBN, kBM = 16 * NW;
@@ -471,9 +470,7 @@ void dq_wide_kernel(BwdArgsT<ND> a) {
   const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
   const T* vp = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
   const int64_t row_bh = (int64_t)bh * a.S + dc.off;
-  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
-  const T* gkp = static_cast<const T*>(a.gk) + gbase;
-  const T* gvp = static_cast<const T*>(a.gv) + gbase;
+  const GlobRows gr = glob_rows<T, D>(a, dc, b, hk, kp, vp, DIR);
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
@@ -482,27 +479,28 @@ void dq_wide_kernel(BwdArgsT<ND> a) {
   const int nglob = (gmax + BN - 1) / BN;
   const int ntot = nloc + nglob;
   using Fill = typename Tile::template Fill<NW>;
-  const int kbytes = (int)(a.kss * 2), vbytes = (int)(a.vss * 2);
+  const int kbytes = (int)(a.kss * 2), vbytes = DIR ? kbytes : (int)(a.vss * 2);
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(kp, (uint32_t)((hi - 1) * kbytes + D * 2));
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(vp, (uint32_t)((hi - 1) * vbytes + D * 2));
-  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gkp, (uint32_t)(gmax * D * 2));
-  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gvp, (uint32_t)(gmax * D * 2));
+  const int gkb = (int)gr.kstep, gvb = (int)gr.vstep;
+  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gr.k, gmax > 0 ? (uint32_t)((gmax - 1) * gkb + D * 2) : 0);
+  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gr.v, gmax > 0 ? (uint32_t)((gmax - 1) * gvb + D * 2) : 0);
   const int fk = Fill::lane_off(wave, lane, kbytes);
   const int fv = Fill::lane_off(wave, lane, vbytes);
-  const int fg = Fill::lane_off(wave, lane, D * 2);
+  const int fgk = Fill::lane_off(wave, lane, gkb), fgv = Fill::lane_off(wave, lane, gvb);
   // global tiles first, then the local window from its highest tile down
   auto row0 = [&](int it) { return it >= nglob ? lo_k + (nloc - 1 - (it - nglob)) * BN : it * BN; };
   auto issue_k = [&](int it, char* dst) {
     if (it >= nglob)
       Fill::load(dst, rk, fk, kbytes, row0(it), wave);
     else
-      Fill::load(dst, rgk, fg, D * 2, row0(it), wave);
+      Fill::load(dst, rgk, fgk, gkb, row0(it), wave);
   };
   auto issue_v = [&](int it) {
     if (it >= nglob)
       Fill::load(sV, rv, fv, vbytes, row0(it), wave);
     else
-      Fill::load(sV, rgv, fg, D * 2, row0(it), wave);
+      Fill::load(sV, rgv, fgv, gvb, row0(it), wave);
   };
   issue_k(0, sK0);
   issue_v(0);
@@ -830,17 +828,16 @@ void dkdv2_kernel(BwdArgsT<ND> a) {
   const T* kbase;
   const T* vbase;
   int64_t kstride, vstride;
+  kbase = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
+  vbase = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
+  kstride = a.kss;
+  vstride = a.vss;
   if (GLOB) {
-    const int64_t gb = ((int64_t)bhk * a.G + dc.gofs) * D;
-    kbase = static_cast<const T*>(a.gk) + gb;
-    vbase = static_cast<const T*>(a.gv) + gb;
-    kstride = D;
-    vstride = D;
-  } else {
-    kbase = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
-    vbase = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
-    kstride = a.kss;
-    vstride = a.vss;
+    const GlobRows gr = glob_rows<T, D>(a, dc, b, hk, kbase, vbase, a.direct);
+    kbase = (const T*)gr.k;
+    vbase = (const T*)gr.v;
+    kstride = gr.kstep / (int)sizeof(T);
+    vstride = gr.vstep / (int)sizeof(T);
   }
 
   // query interval of the workgroup; per-key intervals for the masks
@@ -1092,9 +1089,8 @@ void dq_f32_kernel(BwdArgsT<ND> a) {
   const float* kp = static_cast<const float*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
   const float* vp = static_cast<const float*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
   const int64_t row_bh = (int64_t)bh * a.S + dc.off;
-  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
-  const float* gkp = static_cast<const float*>(a.gk) + gbase;
-  const float* gvp = static_cast<const float*>(a.gv) + gbase;
+  const GlobRows gr = glob_rows<float, D>(a, dc, b, hk, kp, vp, a.direct);
+  const float *gkp = (const float*)gr.k, *gvp = (const float*)gr.v;
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
@@ -1110,8 +1106,8 @@ void dq_f32_kernel(BwdArgsT<ND> a) {
       stk.load(kp, a.kss, row0(it), hi, tid);
       stv.load(vp, a.vss, row0(it), hi, tid);
     } else {
-      stk.load(gkp, D, row0(it), gmax, tid);
-      stv.load(gvp, D, row0(it), gmax, tid);
+      stk.load(gkp, gr.kstep / 4, row0(it), gmax, tid);
+      stv.load(gvp, gr.vstep / 4, row0(it), gmax, tid);
     }
   };
   auto store = [&](int it) {
@@ -1293,16 +1289,16 @@ void dkdv_f32_kernel(BwdArgsT<ND> a) {
 
   const float *kbase, *vbase;
   int64_t kstride, vstride;
+  kbase = static_cast<const float*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
+  vbase = static_cast<const float*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
+  kstride = a.kss;
+  vstride = a.vss;
   if (GLOB) {
-    const int64_t gb = ((int64_t)bhk * a.G + dc.gofs) * D;
-    kbase = static_cast<const float*>(a.gk) + gb;
-    vbase = static_cast<const float*>(a.gv) + gb;
-    kstride = vstride = D;
-  } else {
-    kbase = static_cast<const float*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
-    vbase = static_cast<const float*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
-    kstride = a.kss;
-    vstride = a.vss;
+    const GlobRows gr = glob_rows<float, D>(a, dc, b, hk, kbase, vbase, a.direct);
+    kbase = (const float*)gr.k;
+    vbase = (const float*)gr.v;
+    kstride = gr.kstep / (int)sizeof(float);
+    vstride = gr.vstep / (int)sizeof(float);
   }
 
   // queries of the workgroup
@@ -1528,11 +1524,15 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
     constexpr int ND = std::decay_t<decltype(x)>::kDocs;
     if constexpr (kF32)
       hipLaunchKernelGGL((dq_f32_kernel<D, ND>), qgrid, dim3(64 * kF32Waves), 0, st, x);
-    else if constexpr (D > 128)
-      hipLaunchKernelGGL((dq_wide_kernel<T, D, ND>), qgrid, dim3(64 * kWideWaves), 0, st, x);
     else
-      hipLaunchKernelGGL((dq2_kernel<T, D, kDqWaves, kDqQB, kDqBN, kDqWPE, ND>), qgrid,
-                         dim3(64 * kDqWaves), 0, st, x);
+      dispatch_direct<ND>(a.direct, [&](auto dir) {
+        constexpr bool DIR = decltype(dir)::value;
+        if constexpr (D > 128)
+          hipLaunchKernelGGL((dq_wide_kernel<T, D, ND, DIR>), qgrid, dim3(64 * kWideWaves), 0, st, x);
+        else
+          hipLaunchKernelGGL((dq2_kernel<T, D, kDqWaves, kDqQB, kDqBN, kDqWPE, ND, DIR>), qgrid,
+                             dim3(64 * kDqWaves), 0, st, x);
+      });
   });
   by_docs(ag, [&](const auto& x) {
     constexpr int ND = std::decay_t<decltype(x)>::kDocs;

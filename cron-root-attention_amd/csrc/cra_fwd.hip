@@ -149,9 +149,8 @@ void fwd_f32_kernel(FwdArgsT<ND> a) {
   const float* qp = static_cast<const float*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
   const float* kp = static_cast<const float*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
   const float* vp = static_cast<const float*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
-  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
-  const float* gkp = static_cast<const float*>(a.gk) + gbase;
-  const float* gvp = static_cast<const float*>(a.gv) + gbase;
+  const GlobRows gr = glob_rows<float, D>(a, dc, b, hk, kp, vp, a.direct);
+  const float *gkp = (const float*)gr.k, *gvp = (const float*)gr.v;
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
@@ -167,8 +166,8 @@ void fwd_f32_kernel(FwdArgsT<ND> a) {
       stk.load(kp, a.kss, row0(it), hi, tid);
       stv.load(vp, a.vss, row0(it), hi, tid);
     } else {
-      stk.load(gkp, D, row0(it), gmax, tid);
-      stv.load(gvp, D, row0(it), gmax, tid);
+      stk.load(gkp, gr.kstep / 4, row0(it), gmax, tid);
+      stv.load(gvp, gr.vstep / 4, row0(it), gmax, tid);
     }
   };
   if (ntot > 0) load(0);
@@ -471,7 +470,7 @@ using FwdStage = char[2][SwzTile<D, 64>::kBytes];  // K and V tiles of one pipel
 
 // One work item (a 128-query tile of one (b, h); items numbered heaviest
 // first, consecutive items on different heads) with its LDS stages.
-template <typename T, int D, int NW, int PH, int ND>
+template <typename T, int D, int NW, int PH, int ND, bool DIR>
 __device__ __forceinline__ void fwd2_item(const FwdArgsT<ND>& a, const int item, FwdStage<D>& stage0,
                                           FwdStage<D>& stage1) {
   constexpr int BN = 64;
@@ -493,9 +492,7 @@ __device__ __forceinline__ void fwd2_item(const FwdArgsT<ND>& a, const int item,
   const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
   const T* vp = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
   float* lse = a.lse + (int64_t)bh * a.S + dc.off;
-  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
-  const T* gkp = static_cast<const T*>(a.gk) + gbase;
-  const T* gvp = static_cast<const T*>(a.gv) + gbase;
+  const GlobRows gr = glob_rows<T, D>(a, dc, b, hk, kp, vp, DIR);
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
@@ -515,14 +512,15 @@ __device__ __forceinline__ void fwd2_item(const FwdArgsT<ND>& a, const int item,
   // hi, global rows below gmax): loads past them return zeros. 32-bit
   // offsets, uniform bases.
   using Fill = typename Tile::template Fill<NW>;
-  const int kbytes = (int)(a.kss * 2), vbytes = (int)(a.vss * 2);
+  const int kbytes = (int)(a.kss * 2), vbytes = DIR ? kbytes : (int)(a.vss * 2);
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(kp, (uint32_t)((hi - 1) * kbytes + D * 2));
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(vp, (uint32_t)((hi - 1) * vbytes + D * 2));
-  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gkp, (uint32_t)(gmax * D * 2));
-  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gvp, (uint32_t)(gmax * D * 2));
+  const int gkb = (int)gr.kstep, gvb = (int)gr.vstep;
+  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gr.k, gmax > 0 ? (uint32_t)((gmax - 1) * gkb + D * 2) : 0);
+  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gr.v, gmax > 0 ? (uint32_t)((gmax - 1) * gvb + D * 2) : 0);
   const int fk = Fill::lane_off(wave, lane, kbytes);
   const int fv = Fill::lane_off(wave, lane, vbytes);
-  const int fg = Fill::lane_off(wave, lane, D * 2);
+  const int fgk = Fill::lane_off(wave, lane, gkb), fgv = Fill::lane_off(wave, lane, gvb);
   auto issue = [&](int it, char* dst) {
     if (it >= nglob) {
       const int ts = lo_k + (nloc - 1 - (it - nglob)) * kBN;
@@ -530,8 +528,8 @@ __device__ __forceinline__ void fwd2_item(const FwdArgsT<ND>& a, const int item,
       Fill::load(dst + Tile::kBytes, rv, fv, vbytes, ts, wave);
     } else {
       const int ts = it * kBN;
-      Fill::load(dst, rgk, fg, D * 2, ts, wave);
-      Fill::load(dst + Tile::kBytes, rgv, fg, D * 2, ts, wave);
+      Fill::load(dst, rgk, fgk, gkb, ts, wave);
+      Fill::load(dst + Tile::kBytes, rgv, fgv, gvb, ts, wave);
     }
   };
   issue(0, stage0[0]);
@@ -628,7 +626,7 @@ __device__ __forceinline__ void fwd2_item(const FwdArgsT<ND>& a, const int item,
 // Two pipeline stages as separate LDS objects, each selected at compile
 // time: the compiler can then tell the fill of one stage from reads of the
 // other and does not wait for the fill before those reads.
-template <typename T, int D, int NW, int PH, int ND>
+template <typename T, int D, int NW, int PH, int ND, bool DIR = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 3)))
 void fwd2_kernel(FwdArgsT<ND> a) {
   __shared__ __attribute__((aligned(1024))) FwdStage<D> stage0;
@@ -638,7 +636,7 @@ void fwd2_kernel(FwdArgsT<ND> a) {
     item = xcd_item(item, a.B * a.Hq, a.xcd_nt);
     if (item < 0) return;  // padding block
   }
-  fwd2_item<T, D, NW, PH, ND>(a, item, stage0, stage1);
+  fwd2_item<T, D, NW, PH, ND, DIR>(a, item, stage0, stage1);
 }
 
 // Persistent form (use_persistent; the reference's work-queue kernel,
@@ -659,7 +657,7 @@ void fwd2_persistent_kernel(FwdArgsT<1> a) {
     const int item = next_item;
     __syncthreads();  // read before the next overwrite
     if (item >= n_items) break;
-    fwd2_item<T, D, NW, 3, 1>(a, item, stage0, stage1);
+    fwd2_item<T, D, NW, 3, 1, false>(a, item, stage0, stage1);
   }
 }
 
@@ -673,7 +671,7 @@ void fwd2_persistent_kernel(FwdArgsT<1> a) {
 // S=32768 fp16: 214 us (562 effective TFLOP/s); fwd_kernel (tiles through
 // registers, V stored transposed by 2-byte LDS writes) took 470 us.
 constexpr int kWideWaves = 4, kWideBN = 32;
-template <typename T, int D, int ND>
+template <typename T, int D, int ND, bool DIR = false>
 __global__ __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(3)))
 void fwd_wide_kernel(FwdArgsT<ND> a) {
   constexpr int NW = kWideWaves, BN = kWideBN, kBM = 16 * NW;
@@ -695,9 +693,7 @@ void fwd_wide_kernel(FwdArgsT<ND> a) {
   const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
   const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
   const T* vp = static_cast<const T*>(a.v) + b * a.vsb + hk * a.vsh + (int64_t)dc.off * a.vss;
-  const int64_t gbase = ((int64_t)(b * a.Hkv + hk) * a.G + dc.gofs) * D;
-  const T* gkp = static_cast<const T*>(a.gk) + gbase;
-  const T* gvp = static_cast<const T*>(a.gv) + gbase;
+  const GlobRows gr = glob_rows<T, D>(a, dc, b, hk, kp, vp, DIR);
 
   const int lo_k = max(0, m0 - W + 1);
   const int hi = min(S, m0 + kBM);
@@ -706,27 +702,28 @@ void fwd_wide_kernel(FwdArgsT<ND> a) {
   const int nglob = (a.phases & 2) ? (gmax + BN - 1) / BN : 0;
   const int ntot = nloc + nglob;
   using Fill = typename Tile::template Fill<NW>;
-  const int kbytes = (int)(a.kss * 2), vbytes = (int)(a.vss * 2);
+  const int kbytes = (int)(a.kss * 2), vbytes = DIR ? kbytes : (int)(a.vss * 2);
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(kp, (uint32_t)((hi - 1) * kbytes + D * 2));
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(vp, (uint32_t)((hi - 1) * vbytes + D * 2));
-  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gkp, (uint32_t)(gmax * D * 2));
-  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gvp, (uint32_t)(gmax * D * 2));
+  const int gkb = (int)gr.kstep, gvb = (int)gr.vstep;
+  const __amdgpu_buffer_rsrc_t rgk = make_rsrc(gr.k, gmax > 0 ? (uint32_t)((gmax - 1) * gkb + D * 2) : 0);
+  const __amdgpu_buffer_rsrc_t rgv = make_rsrc(gr.v, gmax > 0 ? (uint32_t)((gmax - 1) * gvb + D * 2) : 0);
   const int fk = Fill::lane_off(wave, lane, kbytes);
   const int fv = Fill::lane_off(wave, lane, vbytes);
-  const int fg = Fill::lane_off(wave, lane, D * 2);
+  const int fgk = Fill::lane_off(wave, lane, gkb), fgv = Fill::lane_off(wave, lane, gvb);
   // global tiles first, then the local window from its highest tile down
   auto row0 = [&](int it) { return it >= nglob ? lo_k + (nloc - 1 - (it - nglob)) * BN : it * BN; };
   auto issue_k = [&](int it) {
     if (it >= nglob)
       Fill::load(sK, rk, fk, kbytes, row0(it), wave);
     else
-      Fill::load(sK, rgk, fg, D * 2, row0(it), wave);
+      Fill::load(sK, rgk, fgk, gkb, row0(it), wave);
   };
   auto issue_v = [&](int it) {
     if (it >= nglob)
       Fill::load(sV, rv, fv, vbytes, row0(it), wave);
     else
-      Fill::load(sV, rgv, fg, D * 2, row0(it), wave);
+      Fill::load(sV, rgv, fgv, gvb, row0(it), wave);
   };
   if (ntot > 0) issue_k(0);
 
@@ -861,7 +858,10 @@ hipError_t launch_wide(const FwdArgs& a, hipStream_t st) {
   const dim3 grid(b.docs.item0[b.docs.n] * b.B * b.Hq);
   by_docs(b, [&](const auto& x) {
     constexpr int ND = std::decay_t<decltype(x)>::kDocs;
-    hipLaunchKernelGGL((fwd_wide_kernel<T, 256, ND>), grid, dim3(64 * kWideWaves), 0, st, x);
+    dispatch_direct<ND>(a.direct, [&](auto dir) {
+      hipLaunchKernelGGL((fwd_wide_kernel<T, 256, ND, decltype(dir)::value>), grid,
+                         dim3(64 * kWideWaves), 0, st, x);
+    });
   });
   return hipGetLastError();
 }
@@ -895,6 +895,10 @@ hipError_t launch_T(int D, const FwdArgs& a, hipStream_t st) {
           if (qerr != hipSuccess) return;
           const dim3 pgrid(std::max(1, std::min((int)grid.x, slots)));
           hipLaunchKernelGGL(kern, pgrid, block, 0, st, x);
+          return;
+        }
+        if (a.direct) {
+          hipLaunchKernelGGL((fwd2_kernel<T, Dc, kFwdWaves, 3, 1, true>), xgrid, block, 0, st, x);
           return;
         }
         if (a.phases == 1) {

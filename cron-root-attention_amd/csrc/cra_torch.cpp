@@ -30,6 +30,7 @@ namespace {
 
 struct Api {
   decltype(&cra_global_rows) global_rows = nullptr;
+  decltype(&cra_reads_global_rows) reads_global = nullptr;
   decltype(&cra_build_global) build_global = nullptr;
   decltype(&cra_fwd) fwd = nullptr;
   decltype(&cra_bwd_workspace_bytes) ws_bytes = nullptr;
@@ -58,6 +59,7 @@ void bind(std::string path) {
   TORCH_CHECK(h != nullptr, "cannot load ", path, ": ", dlerror());
   Api api;
   resolve(h, path, "cra_global_rows", api.global_rows);
+  resolve(h, path, "cra_reads_global_rows", api.reads_global);
   resolve(h, path, "cra_build_global", api.build_global);
   resolve(h, path, "cra_fwd", api.fwd);
   resolve(h, path, "cra_bwd_workspace_bytes", api.ws_bytes);
@@ -133,26 +135,42 @@ void* stream_of(const at::Tensor& t) {
   return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
-// Forward launches: packed global rows (one allocation for K and V rows),
-// relay source rows, then the three-phase forward. Returns o, lse, the packed
-// rows and the relay source rows (undefined without relay).
+// Addresses of the packed K and V rows; without them (the kernels take the
+// global rows from k and v) k's own address stands in, which is not read.
+std::pair<const char*, const char*> glob_ptrs(const at::Tensor& gkv, const at::Tensor& k) {
+  if (!gkv.defined()) {
+    const char* p = static_cast<const char*>(k.data_ptr());
+    return {p, p};
+  }
+  const char* p = static_cast<const char*>(gkv.data_ptr());
+  return {p, p + gkv.numel() / 2 * gkv.element_size()};
+}
+
+// Forward launches: packed global rows (one allocation for K and V rows) and
+// relay source rows where the kernels read them, then the three-phase forward.
+// Returns o, lse, the packed rows and the relay source rows (either may be
+// undefined). At S = 512 the packing was 3 of the call's 12 us on the GPU.
 std::array<at::Tensor, 4> run_forward(const cra_problem& p, const at::Tensor& q,
                                       const at::Tensor& k, const at::Tensor& v) {
   const Api& a = api();
   void* st = stream_of(q);
-  const int64_t G = a.global_rows(&p);
-  TORCH_CHECK(G >= 0, "cra_global_rows: invalid problem");
-  at::Tensor gkv = at::empty({2, p.B, p.H_kv, G, p.D}, k.options());
-  char* gk = static_cast<char*>(gkv.data_ptr());
-  char* gv = gk + (int64_t)p.B * p.H_kv * G * p.D * k.element_size();
-  at::Tensor src;
-  if (p.relay) {
-    const int64_t nb = (p.S + p.W - 1) / p.W;
-    src = at::empty({p.B, p.H_kv, nb * p.top_k}, k.options().dtype(at::kInt));
+  const int reads = a.reads_global(&p, targ(k), targ(v));
+  TORCH_CHECK(reads >= 0, "cra_reads_global_rows: invalid problem");
+  at::Tensor gkv, src;
+  if (reads) {
+    const int64_t G = a.global_rows(&p);
+    TORCH_CHECK(G >= 0, "cra_global_rows: invalid problem");
+    gkv = at::empty({2, p.B, p.H_kv, G, p.D}, k.options());
+    if (p.relay) {
+      const int64_t nb = (p.S + p.W - 1) / p.W;
+      src = at::empty({p.B, p.H_kv, nb * p.top_k}, k.options().dtype(at::kInt));
+    }
+    char* gk = static_cast<char*>(gkv.data_ptr());
+    check(a.build_global(&p, targ(k), targ(v), gk, gk + gkv.numel() / 2 * gkv.element_size(),
+                         p.relay ? src.data_ptr<int32_t>() : nullptr, nullptr, st),
+          "cra_build_global");
   }
-  check(a.build_global(&p, targ(k), targ(v), gk, gv,
-                       p.relay ? src.data_ptr<int32_t>() : nullptr, nullptr, st),
-        "cra_build_global");
+  const auto [gk, gv] = glob_ptrs(gkv, k);
   at::Tensor o = at::empty(q.sizes(), q.options());
   at::Tensor lse = at::empty({p.B, p.H_q, p.S}, q.options().dtype(at::kFloat));
   check(a.fwd(&p, targ(q), targ(k), targ(v), gk, gv, targ(o), lse.data_ptr<float>(), st),
@@ -212,8 +230,7 @@ class CraAttention : public torch::autograd::Function<CraAttention> {
     at::Tensor dv = at::empty(v.sizes(), v.options());
     const size_t nws = a.ws_bytes(&p);
     at::Tensor ws = at::empty({(int64_t)std::max<size_t>(nws, 256)}, q.options().dtype(at::kByte));
-    const char* gk = static_cast<const char*>(gkv.data_ptr());
-    const char* gv = gk + gkv.numel() / 2 * gkv.element_size();
+    const auto [gk, gv] = glob_ptrs(gkv, k);
     check(a.bwd(&p, targ(q), targ(k), targ(v), targ(o), targ(dout), lse.data_ptr<float>(), gk,
                 gv, p.relay ? src.data_ptr<int32_t>() : nullptr, nullptr, targ(dq), targ(dk),
                 targ(dv), nullptr, ws.data_ptr(), (size_t)ws.numel(), st),

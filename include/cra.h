@@ -81,6 +81,15 @@ int cra_supported_head_dim(int32_t D);
  * (1+top_k)*floor(ls/W) + (ls % W != 0) (relay) or ceil(ls/W) (no relay). */
 int64_t cra_global_rows(const cra_problem* p);
 
+/* Whether cra_fwd and cra_bwd read the packed global rows for this problem
+ * and these k and v: 1 if so, 0 if they take them from k and v in place (no
+ * relay: row r is row r * W of k and v; k and v of one row stride, within
+ * 32-bit offsets). At 0
+ * cra_build_global need not run: glob_k and glob_v must still be non-NULL and
+ * 16-byte aligned, and are not read by cra_fwd and cra_bwd (cra_fwd_persistent
+ * and a single phase of cra_fwd_phases always read them). -1: invalid problem. */
+int cra_reads_global_rows(const cra_problem* p, cra_tensor k, cra_tensor v);
+
 /* Builds the packed global rows and the relay source rows.
  *   k, v:       [B, H_kv, S, D]
  *   glob_k/v:   contiguous [B, H_kv, cra_global_rows(p), D], dtype of k
