@@ -283,6 +283,20 @@ def cron_root_attention_v14(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                                               relay_log_scale, relay_top_k)
 
 
+@torch.compiler.disable
+def _layer_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                     kv_groups: int = 1) -> torch.Tensor:
+    """The op as a layer calls it on its own projections: the same values, the
+    output (and the gradients of q, k, v) as [B, H, S, D] views of [B, S, H, D]
+    buffers, so that the reshapes to and from the projections copy nothing.
+    Calls that do not go to the C++ operator give the op's contiguous output."""
+    if q.device.type != "cpu" and _native.attention_op() is not None:
+        plan = _op_plan(q, k, v, False, kv_groups, 2)
+        if plan is not None:
+            return torch.ops.cra.layer_attention(q, k, v, *plan)
+    return cron_root_attention_v14(q, k, v, kv_groups=kv_groups)
+
+
 _OP_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
 
 

@@ -27,7 +27,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .core import cron_root_attention_v14
+from .core import _layer_attention, cron_root_attention_v14
 
 # (mode, head_dim, smallest B*H the row applies to) -> smallest swept S from
 # which the sqrt(N) op beats SDPA at every larger swept S.
@@ -126,7 +126,12 @@ class CronRootAttentionHybrid(nn.Module):
         q = self.q_proj(x).view(B, S, self.n_heads, self.head_dim).transpose(1, 2)
         k = self.k_proj(x).view(B, S, self.n_heads, self.head_dim).transpose(1, 2)
         v = self.v_proj(x).view(B, S, self.n_heads, self.head_dim).transpose(1, 2)
-        out = cron_root_attention_hybrid(q, k, v, backend="auto", threshold=self.threshold)
+        training = torch.is_grad_enabled() and q.requires_grad
+        if dispatch_backend(S, self.head_dim, training, B * self.n_heads,
+                            self.threshold) == "cron_root":
+            out = _layer_attention(q, k, v)
+        else:
+            out = F.scaled_dot_product_attention(q, k, v, is_causal=True)
         out = out.transpose(1, 2).contiguous().view(B, S, D)
         out = self.o_proj(out)
         if self.dropout > 0 and self.training:

@@ -1,5 +1,6 @@
 // Torch operator binding of libcra_hip.so (include/cra.h) with its autograd
-// in C++: torch.ops.cra.attention(q, k, v, window, relay, top_k, scale).
+// in C++: torch.ops.cra.attention(q, k, v, window, relay, top_k, scale), and
+// layer_attention, the same over [B, S, H, D] buffers.
 //
 // It serves the common call of cron_root_attention_v14 (reference
 // core.py:3767-3797) -- GPU tensors, head dim 32/64/128/256, no
@@ -146,12 +147,21 @@ std::pair<const char*, const char*> glob_ptrs(const at::Tensor& gkv, const at::T
   return {p, p + gkv.numel() / 2 * gkv.element_size()};
 }
 
+// A [B, H, S, D] tensor like t: contiguous, or with bshd a view of a
+// contiguous [B, S, H, D] one, the layout a projection takes and gives. A layer
+// that asks for it saves the copies between the two: at B=1 S=16000 H=16/4
+// D=128 one of the output (50 us) and one of each of dq, dk, dv (50 + 2 x 17).
+at::Tensor empty_bhsd(const at::Tensor& t, bool bshd) {
+  if (!bshd) return at::empty(t.sizes(), t.options());
+  return at::empty({t.size(0), t.size(2), t.size(1), t.size(3)}, t.options()).transpose(1, 2);
+}
+
 // Forward launches: packed global rows (one allocation for K and V rows) and
 // relay source rows where the kernels read them, then the three-phase forward.
 // Returns o, lse, the packed rows and the relay source rows (either may be
 // undefined). At S = 512 the packing was 3 of the call's 12 us on the GPU.
 std::array<at::Tensor, 4> run_forward(const cra_problem& p, const at::Tensor& q,
-                                      const at::Tensor& k, const at::Tensor& v) {
+                                      const at::Tensor& k, const at::Tensor& v, bool bshd) {
   const Api& a = api();
   void* st = stream_of(q);
   const int reads = a.reads_global(&p, targ(k), targ(v));
@@ -171,7 +181,7 @@ std::array<at::Tensor, 4> run_forward(const cra_problem& p, const at::Tensor& q,
           "cra_build_global");
   }
   const auto [gk, gv] = glob_ptrs(gkv, k);
-  at::Tensor o = at::empty(q.sizes(), q.options());
+  at::Tensor o = empty_bhsd(q, bshd);
   at::Tensor lse = at::empty({p.B, p.H_q, p.S}, q.options().dtype(at::kFloat));
   check(a.fwd(&p, targ(q), targ(k), targ(v), gk, gv, targ(o), lse.data_ptr<float>(), st),
         "cra_fwd");
@@ -200,16 +210,17 @@ class CraAttention : public torch::autograd::Function<CraAttention> {
  public:
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q_in,
                             const at::Tensor& k_in, const at::Tensor& v_in, int64_t window,
-                            bool relay, int64_t top_k, double scale) {
+                            bool relay, int64_t top_k, double scale, bool bshd) {
     check_inputs(q_in, k_in, v_in);
     const at::Tensor q = ready(q_in), k = ready(k_in), v = ready(v_in);
     const cra_problem p = make_problem(q, k, window, relay, top_k, scale);
-    auto r = run_forward(p, q, k, v);
+    auto r = run_forward(p, q, k, v, bshd);
     ctx->save_for_backward({q, k, v, r[0], r[1], r[2], r[3]});
     ctx->saved_data["window"] = window;
     ctx->saved_data["relay"] = relay;
     ctx->saved_data["top_k"] = top_k;
     ctx->saved_data["scale"] = scale;
+    ctx->saved_data["bshd"] = bshd;
     return r[0];
   }
 
@@ -225,9 +236,8 @@ class CraAttention : public torch::autograd::Function<CraAttention> {
     if (!kernel_ready(dout)) dout = dout.contiguous();
     const Api& a = api();
     void* st = stream_of(q);
-    at::Tensor dq = at::empty(q.sizes(), q.options());
-    at::Tensor dk = at::empty(k.sizes(), k.options());
-    at::Tensor dv = at::empty(v.sizes(), v.options());
+    const bool bshd = ctx->saved_data["bshd"].toBool();
+    at::Tensor dq = empty_bhsd(q, bshd), dk = empty_bhsd(k, bshd), dv = empty_bhsd(v, bshd);
     const size_t nws = a.ws_bytes(&p);
     at::Tensor ws = at::empty({(int64_t)std::max<size_t>(nws, 256)}, q.options().dtype(at::kByte));
     const auto [gk, gv] = glob_ptrs(gkv, k);
@@ -235,22 +245,24 @@ class CraAttention : public torch::autograd::Function<CraAttention> {
                 gv, p.relay ? src.data_ptr<int32_t>() : nullptr, nullptr, targ(dq), targ(dk),
                 targ(dv), nullptr, ws.data_ptr(), (size_t)ws.numel(), st),
           "cra_bwd");
-    return {dq, dk, dv, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
+    return {dq, dk, dv, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
   }
 };
 
+template <bool BSHD>
 at::Tensor attention_autograd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                               int64_t window, bool relay, int64_t top_k, double scale) {
-  return CraAttention::apply(q, k, v, window, relay, top_k, scale);
+  return CraAttention::apply(q, k, v, window, relay, top_k, scale, BSHD);
 }
 
 // Below autograd (inference mode, or tensors without autograd keys): the
 // forward launches alone.
+template <bool BSHD>
 at::Tensor attention_forward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                              int64_t window, bool relay, int64_t top_k, double scale) {
   check_inputs(q, k, v);
   const at::Tensor qr = ready(q), kr = ready(k), vr = ready(v);
-  return run_forward(make_problem(qr, kr, window, relay, top_k, scale), qr, kr, vr)[0];
+  return run_forward(make_problem(qr, kr, window, relay, top_k, scale), qr, kr, vr, BSHD)[0];
 }
 
 }  // namespace
@@ -260,8 +272,18 @@ TORCH_LIBRARY(cra, m) {
   m.def(
       "attention(Tensor q, Tensor k, Tensor v, int window, bool relay, int top_k, float scale)"
       " -> Tensor");
+  // the output and the gradients as [B, H, S, D] views of [B, S, H, D] buffers
+  m.def(
+      "layer_attention(Tensor q, Tensor k, Tensor v, int window, bool relay, int top_k,"
+      " float scale) -> Tensor");
 }
 
-TORCH_LIBRARY_IMPL(cra, Autograd, m) { m.impl("attention", &attention_autograd); }
+TORCH_LIBRARY_IMPL(cra, Autograd, m) {
+  m.impl("attention", &attention_autograd<false>);
+  m.impl("layer_attention", &attention_autograd<true>);
+}
 
-TORCH_LIBRARY_IMPL(cra, CUDA, m) { m.impl("attention", &attention_forward); }
+TORCH_LIBRARY_IMPL(cra, CUDA, m) {
+  m.impl("attention", &attention_forward<false>);
+  m.impl("layer_attention", &attention_forward<true>);
+}
