@@ -1469,8 +1469,10 @@ constexpr int kDkdvLocalBQ = 32;
 //          B=8 H=32/8  S=8192  (768; G = 273)  267 /  278 us
 //          B=1 H=12/12 S=65536 (792; G = 768)  227 /  242 us
 // So: the 64-row workgroups for launches of fewer than two wide workgroups
-// per CU (up to 768 rows, the most that was measured), and where the rows
-// padded to wide tiles are at least twice those padded to 64.
+// per CU (up to 768 rows, the most that was measured), and where the documents'
+// rows padded to wide tiles are at least 1.75 times those padded to 64: one
+// document of up to 64 rows, or packed ones with many short among them (16 of 1
+// to 9001 tokens, H=16/4 D=128: 2.0 times, 97 / 76 us).
 constexpr int kNarrowWaves = 4, kNarrowBQ = 32, kNarrowMaxRows = 768;
 
 template <int D>
@@ -1484,10 +1486,10 @@ bool narrow_glob(const BwdArgs& a) {
     const int tiles = (rows + kWide - 1) / kWide;
     most = std::max(most, rows);
     items += (int64_t)tiles * chunks * a.B * a.Hkv;
-    wide += (int64_t)tiles * kWide * chunks;
-    narrow += (int64_t)(rows + kNarrow - 1) / kNarrow * kNarrow * chunks;
+    wide += (int64_t)tiles * kWide;
+    narrow += (int64_t)(rows + kNarrow - 1) / kNarrow * kNarrow;
   }
-  return D <= 128 && ((items < 2 * a.cus && most <= kNarrowMaxRows) || wide >= 2 * narrow);
+  return D <= 128 && ((items < 2 * a.cus && most <= kNarrowMaxRows) || 4 * wide >= 7 * narrow);
 }
 
 template <typename T, int D>

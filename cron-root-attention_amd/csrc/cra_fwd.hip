@@ -423,10 +423,17 @@ __device__ __forceinline__ void attend_tile2(const char* tK, const char* tV, con
       half_exp<T, MASK, 2>(s[kc], kc, qb, c2, m_run[qb], g, mk, one, pn[qb], ps[qb]);
     if (kc > 0) pv_half<T, D, BN, 2>(tV, kc - 1, lo, pf, acc);  // beside this half's exponentials
     if (kc + 1 < kHalves) tile_scores<T, D, BN, 2>(tK, lo, qf, kc + 1, s[kc + 1]);
+    // one branch for both query blocks (a branch each measured 0.5% slower:
+    // forward kernel at H=16 S=131072 D=128 1207 against 1201 us, at H=12
+    // S=32768 D=64 87.2 against 86.5 us)
+    if (__any(!(ps[0] <= kSumMax) || !(ps[1] <= kSumMax))) {
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb)
+        if (__any(!(ps[qb] <= kSumMax)))
+          half_rescale<T, D, 2>(s[kc], qb, c2, acc, m_run, l_run, one, pn[qb], ps[qb]);
+    }
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      if (__any(!(ps[qb] <= kSumMax)))
-        half_rescale<T, D, 2>(s[kc], qb, c2, acc, m_run, l_run, one, pn[qb], ps[qb]);
       l_run[qb] += ps[qb];
       pf[qb] = pn[qb];
     }
@@ -450,12 +457,14 @@ __device__ __forceinline__ void attend_half(const char* tK, const char* tV, int 
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb)
     half_exp<T, true, 2>(s, kc, qb, c2, m_run[qb], g, mk, one, pf[qb], ps[qb]);
+  if (__any(!(ps[0] <= kSumMax) || !(ps[1] <= kSumMax))) {
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
-    if (__any(!(ps[qb] <= kSumMax)))
-      half_rescale<T, D, 2>(s, qb, c2, acc, m_run, l_run, one, pf[qb], ps[qb]);
-    l_run[qb] += ps[qb];
+    for (int qb = 0; qb < 2; ++qb)
+      if (__any(!(ps[qb] <= kSumMax)))
+        half_rescale<T, D, 2>(s, qb, c2, acc, m_run, l_run, one, pf[qb], ps[qb]);
   }
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb) l_run[qb] += ps[qb];
   pv_half<T, D, BN, 2>(tV, kc, lo, pf, acc);
 }
 

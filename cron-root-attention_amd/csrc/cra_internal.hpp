@@ -66,8 +66,15 @@ struct Doc {
 template <int N>
 __device__ __forceinline__ Doc find_doc(const DocsT<N>& t, int item) {
   int d = 0;
-  if constexpr (N > 1)
-    for (int i = 1; i < t.n; ++i) d += item >= t.item0[i];  // item0 is non-decreasing
+  if constexpr (N > 1) {
+    // the last d with item0[d] <= item (item0 is non-decreasing): a search
+    // of log2(n) dependent loads, not a scan of n
+    int hi = t.n - 1;
+    while (d < hi) {
+      const int mid = (d + hi + 1) >> 1;
+      if (item >= t.item0[mid]) d = mid; else hi = mid - 1;
+    }
+  }
   return Doc{t.off[d],  t.len[d],  t.W[d],  t.rpb[d],  t.gofs[d],
              t.bofs[d], t.pofs[d], t.dW[d], t.drpb[d], item - (N > 1 ? t.item0[d] : 0)};
 }
