@@ -244,7 +244,7 @@ cra::Docs group_table(const Plan& pl, int g) {
 }
 
 cra::ChunkPlan chunk_plan(const cra_problem* p, const Plan& pl) {
-  return cra::plan_chunks(p->D, p->B, p->H_kv, pl.n, pl.len.data(), pl.W.data(), pl.rpb.data(),
+  return cra::plan_chunks(p->D, p->B, p->H_q, p->H_kv, pl.n, pl.len.data(), pl.W.data(), pl.rpb.data(),
                           device_cus());
 }
 

@@ -1589,7 +1589,7 @@ hipError_t launch_T(int D, const BwdArgs& a, hipStream_t st) {
 
 }  // namespace
 
-ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len,
+ChunkPlan plan_chunks(int D, int B, int Hq, int Hkv, int n, const int* len,
                       const int* W, const int* rpb, int cus) {
   // Query chunks of the global-row kernel: each document's query range is
   // cut into chunks of chunk_len queries (a multiple of 64), one
@@ -1653,9 +1653,20 @@ ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len,
   int64_t nc = (3 * slots + 2 * base - 1) / (2 * base);  // 1.5 rounds of workgroups
   const int64_t by_len = (max_len + 6143) / 6144;
   if (nc < by_len) nc = by_len;
-  const int64_t max_nc = (max_len + 255) / 256;
+  // At least 256 queries a chunk, counted over the heads of the kv group: a
+  // workgroup sweeps its chunk once per head of the group, and with few kv
+  // heads the chunks are all the workgroups there are. Global-row kernel with
+  // 256 queries of each head / of all: B=2 H=16/2 S=2048 D=64 37 / 12 us, B=1
+  // H=8/1 S=4096 D=128 51 / 18, H=32/4 S=8192 D=128 95 / 66, H=32/8 S=2000
+  // D=128 26 / 11, fp32 H=8/2 S=3000 D=64 67 / 27 us.
+  const int grp = Hq / Hkv;
+  const int64_t max_nc = ((int64_t)max_len * grp + 255) / 256;
   if (nc > max_nc) nc = max_nc;
   if (nc < 1) nc = 1;
+  if (grp > 1) {  // (with one head per kv head 64-query rounding can leave the last chunks empty)
+    c.chunk_len = chunk_len_for(max_len, (int)nc);
+    nc = num_chunks(max_len, c.chunk_len);
+  }
   c.nchunk = (int)nc;
   c.chunk_len = chunk_len_for(max_len, c.nchunk);
   c.part_rows = nc * doc_rows(len[0], W[0], rpb[0]);

@@ -383,7 +383,7 @@ struct ChunkPlan {
   int nchunk;         // most chunks of a document
   int64_t part_rows;  // partial rows per (b, kv head), all documents
 };
-ChunkPlan plan_chunks(int D, int B, int Hkv, int n, const int* len, const int* W,
+ChunkPlan plan_chunks(int D, int B, int Hq, int Hkv, int n, const int* len, const int* W,
                       const int* rpb, int cus);
 // Workspace of the backward: Delta and -lse*log2(e), [B*Hq*S] fp32 each
 // (rounded up to 256 bytes), then the partials, part_rows * B * Hkv rows of

@@ -31,6 +31,8 @@ def _check(grads, ref, dtype):
     (2049, 8, 64, 2, 1, BF16),    # 771 rows below D = 128: 128-row workgroups
     (300, 9, 128, 256, 256, F16),  # 102 rows, two wide workgroups per CU: 192-row workgroups
     (400, 20, 128, 128, 64, F16), # 60 rows: one 64-row tile
+    (330, 19, 64, 8, 1, F16),     # grouped heads: chunks of 64 queries, the last of 10
+    (256, 16, 128, 16, 2, BF16),  # grouped heads: exact chunks of 64 queries
     (65, 65, 32, 1, 1, F16),      # one block: no query sees a global row
 ])
 def test_row_limits(S, W, D, Hq, Hkv, dtype):
