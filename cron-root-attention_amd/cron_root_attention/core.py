@@ -182,11 +182,12 @@ class CronRootAttentionV14Function(torch.autograd.Function):
         if persistent or _native.reads_global_rows(p, kp, vp):
             gk, gv, src = _native.build_global(p, kp, vp, rscale, stream=st)
         else:  # the kernels read the global rows in kp and vp: nothing is packed
-            gk, gv, src = kp, vp, None
+            gk = gv = src = None
         if persistent:
             o, lse = _native.forward_persistent(p, qp, kp, vp, gk, gv, stream=st)
         else:
-            o, lse = _native.forward(p, qp, kp, vp, gk, gv, stream=st)
+            o, lse = _native.forward(p, qp, kp, vp, kp if gk is None else gk,
+                                     vp if gv is None else gv, stream=st)
         ctx.problem = p
         ctx.D = D
         ctx.has_alpha = relay_log_scale is not None and relay_on
@@ -200,6 +201,10 @@ class CronRootAttentionV14Function(torch.autograd.Function):
         p = ctx.problem
         D = ctx.D
         dop = _kernel_ready(_pad_d(do.to(qp.dtype), p.D))
+        if gk is None:
+            if _native.reads_global_rows(p, kp, vp):  # layouts changed by a saved-tensor hook
+                kp, vp = kp.contiguous(), vp.contiguous()
+            gk, gv = kp, vp
         dq, dk, dv, dalpha = _native.backward(p, qp, kp, vp, o, dop, lse, gk, gv, src, rscale,
                                               ctx.has_alpha)
         if p.D != D:

@@ -227,8 +227,8 @@ class CraAttention : public torch::autograd::Function<CraAttention> {
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
     const auto s = ctx->get_saved_variables();
-    const at::Tensor &q = s[0], &k = s[1], &v = s[2], &o = s[3], &lse = s[4], &gkv = s[5],
-                     &src = s[6];
+    const at::Tensor &q = s[0], &o = s[3], &lse = s[4], &gkv = s[5], &src = s[6];
+    at::Tensor k = s[1], v = s[2];
     const cra_problem p =
         make_problem(q, k, ctx->saved_data["window"].toInt(), ctx->saved_data["relay"].toBool(),
                      ctx->saved_data["top_k"].toInt(), ctx->saved_data["scale"].toDouble());
@@ -236,6 +236,12 @@ class CraAttention : public torch::autograd::Function<CraAttention> {
     if (!kernel_ready(dout)) dout = dout.contiguous();
     const Api& a = api();
     void* st = stream_of(q);
+    if (!gkv.defined() && a.reads_global(&p, targ(k), targ(v)) != 0) {
+      // nothing was packed, and a saved-tensor hook gave k and v back in
+      // layouts that would need it
+      k = k.contiguous();
+      v = v.contiguous();
+    }
     const bool bshd = ctx->saved_data["bshd"].toBool();
     at::Tensor dq = empty_bhsd(q, bshd), dk = empty_bhsd(k, bshd), dv = empty_bhsd(v, bshd);
     const size_t nws = a.ws_bytes(&p);

@@ -49,3 +49,26 @@ def test_against_packed_and_oracle(B, Hq, Hkv, S, D, dtype, bshd):
             continue
         assert rel_fro(t, ref[name]) <= TOL_GRAD[dtype], name
 
+
+@pytest.mark.parametrize("D", [64, 80])   # the C++ operator, the Python Function
+def test_saved_tensor_hooks_may_change_layouts(D):
+    """Nothing is packed in the forward; a hook then gives v back with another
+    row stride than k's, for which the kernels would read packed rows."""
+    q, k, v, do = (t.to(DEV) for t in inputs(1, 2, 2, 300, D, F16, seed=5))
+    x = [t.requires_grad_(True) for t in (q, k, v)]
+    want = torch.autograd.grad(cra.cron_root_attention(*x), x, do)
+    seen = []
+
+    def unpack(t):
+        if t.dim() == 4 and t.shape[2] == 300:
+            seen.append(t)
+            if len(seen) == 3:  # q, k, v, ...: v as a [B, S, H, D] buffer
+                return t.transpose(1, 2).contiguous().transpose(1, 2)
+        return t
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        o = cra.cron_root_attention(*x)
+    got = torch.autograd.grad(o, x, do)
+    assert len(seen) >= 3
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
