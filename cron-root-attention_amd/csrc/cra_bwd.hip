@@ -1492,6 +1492,21 @@ bool narrow_glob(const BwdArgs& a) {
   return D <= 128 && ((items < 2 * a.cus && most <= kNarrowMaxRows) || 4 * wide >= 7 * narrow);
 }
 
+// Below D = 128 a local workgroup takes 128 keys, 32 a wave; where that gives
+// no more than one workgroup per CU it takes 64, 16 a wave: the chip has room
+// for twice the workgroups, and each is shorter. Local kernel, 128 / 64 keys
+// (128-key workgroups in the launch): B=2 H=16/2 S=2048 D=64 (64) 39 / 21.5
+// us, H=16/2 S=1000 (16) 34 / 16.6, H=12 S=1000 (96) 9.7 / 7.0, H=8 S=4096
+// (256) 12.3 / 10.4, H=16/4 S=8192 (256) 29 / 24, H=12 S=8192 (768) 22.7 / 26.5.
+template <int D>
+bool half_local_tiles(const BwdArgs& a) {
+  if (kDkdvLocalKB<D> == 1) return false;
+  constexpr int kKeys = 16 * kDkdvLocalWaves * kDkdvLocalKB<D>;
+  int64_t items = 0;
+  for (int d = 0; d < a.docs.n; ++d) items += (a.docs.len[d] + kKeys - 1) / kKeys;
+  return items * a.B * a.Hkv <= a.cus;
+}
+
 template <typename T, int D>
 hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   constexpr bool kF32 = sizeof(T) == 4;
@@ -1505,7 +1520,8 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
   const int kGK = kF32     ? 16 * kF32Waves
                   : narrow ? 16 * kNarrowWaves
                            : 16 * kDkdvGlobWaves<D> * kDkdvKB;  // rows per workgroup
-  constexpr int kLK = kF32 ? 16 * kF32Waves : 16 * kDkdvLocalWaves * kDkdvLocalKB<D>;
+  const bool half_local = !kF32 && half_local_tiles<D>(a);
+  const int kLK = kF32 ? 16 * kF32Waves : 16 * kDkdvLocalWaves * (half_local ? 1 : kDkdvLocalKB<D>);
   set_items(ag.docs, [&](int d) {
     return (doc_rows(a.docs.len[d], a.docs.W[d], a.docs.rpb[d]) + kGK - 1) / kGK *
            num_chunks(a.docs.len[d], a.chunk_len);
@@ -1568,6 +1584,9 @@ hipError_t launch_TD(const BwdArgs& a, hipStream_t st) {
     constexpr int ND = std::decay_t<decltype(x)>::kDocs;
     if constexpr (kF32)
       hipLaunchKernelGGL((dkdv_f32_kernel<D, false, ND>), lgrid, dim3(64 * kF32Waves), 0, st, x);
+    else if (half_local)
+      hipLaunchKernelGGL((dkdv2_kernel<T, D, false, kDkdvLocalWaves, 1, kDkdvLocalBQ, ND>), lgrid,
+                         dim3(64 * kDkdvLocalWaves), 0, st, x);
     else
       hipLaunchKernelGGL(
           (dkdv2_kernel<T, D, false, kDkdvLocalWaves, kDkdvLocalKB<D>, kDkdvLocalBQ, ND>), lgrid,

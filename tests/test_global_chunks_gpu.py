@@ -33,6 +33,9 @@ def _check(grads, ref, dtype):
     (400, 20, 128, 128, 64, F16), # 60 rows: one 64-row tile
     (330, 19, 64, 8, 1, F16),     # grouped heads: chunks of 64 queries, the last of 10
     (256, 16, 128, 16, 2, BF16),  # grouped heads: exact chunks of 64 queries
+    (300, 9, 64, 256, 256, F16),  # more 128-key local workgroups than CUs
+    (129, 12, 32, 512, 256, BF16),
+    (129, 12, 64, 4, 1, F16),     # fewer: 64-key ones, the last of one key
     (65, 65, 32, 1, 1, F16),      # one block: no query sees a global row
 ])
 def test_row_limits(S, W, D, Hq, Hkv, dtype):
