@@ -146,6 +146,13 @@ __global__ __launch_bounds__(1024) void dalpha_kernel(BwdArgs a) {
 // computed; transposed operands (K^T for dQ, Q^T and dO^T for dK/dV) are
 // read with ds_read_b64_tr_b16 from the same row-major tiles.
 // ---------------------------------------------------------------------------
+// At D = 256 Delta is subtracted from the finished dP, one rounding of the
+// difference: accumulating onto -Delta (below D = 256, one operation less per
+// element) rounds every partial sum at Delta's magnitude, over twice the
+// products.
+template <int D>
+constexpr bool kSubDelta = D > 128;
+
 // Query-centric dQ for QB blocks of 16 queries per wave against one BN-key
 // tile, in 32-key halves: S = K . Q^T and dP - Delta = V . dO^T - Delta (key
 // on rows; the products accumulate onto -Delta, so no subtraction per
@@ -179,7 +186,8 @@ __device__ __forceinline__ void dq2_ds(const char* tK, const char* tV, int kc,
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       sc[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      dp[qb] = f32x4{ndl[qb], ndl[qb], ndl[qb], ndl[qb]};
+      const float d0 = kSubDelta<D> ? 0.f : ndl[qb];
+      dp[qb] = f32x4{d0, d0, d0, d0};
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -200,7 +208,8 @@ __device__ __forceinline__ void dq2_ds(const char* tK, const char* tV, int kc,
       for (int qb = 0; qb < QB; ++qb) {
         float x = fmaf(sc[qb][r], c2, -lse2[qb]);
         if (MASK && !mk.ok(ko, qb)) x = -__builtin_huge_valf();
-        ds[h][qb][r] = __builtin_amdgcn_exp2f(x) * dp[qb][r];
+        ds[h][qb][r] =
+            __builtin_amdgcn_exp2f(x) * (kSubDelta<D> ? dp[qb][r] + ndl[qb] : dp[qb][r]);
       }
     }
   }
@@ -439,9 +448,9 @@ void dq2_kernel(BwdArgsT<ND> a) {
 // tile at a time and K two, 48 KB of LDS per workgroup: the next K arrives
 // during this tile's S and dP, the next V during its K^T . dS^T. Bound by
 // LDS reads (one K, V or K^T fragment per MFMA: at most about 60% MFMA-busy)
-// and 2 waves per SIMD (216 VGPRs). B=1 H=8 S=32768 fp16: 318 us, where
-// dq_kernel (tiles through registers, V and K^T stored transposed by 2-byte
-// LDS writes, one stage) took 478 us and delta_kernel before it 46 us.
+// and 2 waves per SIMD (211 VGPRs). B=1 H=8 S=32768 bf16: 340 us; with tiles
+// through registers and V and K^T stored transposed by 2-byte LDS writes, one
+// stage, it took 479 us and a Delta pass before it 46 us.
 constexpr int kWideWaves = 4, kWideBN = 32;
 template <typename T, int D, int ND, bool DIR = false>
 __global__ __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(2)))
@@ -488,16 +497,16 @@ void dq_wide_kernel(BwdArgsT<ND> a) {
   const int fk = Fill::lane_off(wave, lane, kbytes);
   const int fv = Fill::lane_off(wave, lane, vbytes);
   const int fgk = Fill::lane_off(wave, lane, gkb), fgv = Fill::lane_off(wave, lane, gvb);
-  // global tiles first, then the local window from its highest tile down
-  auto row0 = [&](int it) { return it >= nglob ? lo_k + (nloc - 1 - (it - nglob)) * BN : it * BN; };
+  // the local window, then the global rows, as the forward
+  auto row0 = [&](int it) { return it < nloc ? lo_k + it * BN : (it - nloc) * BN; };
   auto issue_k = [&](int it, char* dst) {
-    if (it >= nglob)
+    if (it < nloc)
       Fill::load(dst, rk, fk, kbytes, row0(it), wave);
     else
       Fill::load(dst, rgk, fgk, gkb, row0(it), wave);
   };
   auto issue_v = [&](int it) {
-    if (it >= nglob)
+    if (it < nloc)
       Fill::load(sV, rv, fv, vbytes, row0(it), wave);
     else
       Fill::load(sV, rgv, fgv, gvb, row0(it), wave);
@@ -515,7 +524,7 @@ void dq_wide_kernel(BwdArgsT<ND> a) {
   const int qr = min(qi, S - 1);
   const bool ok = qi < S;
   const float lse2[1] = {ok ? a.lse[row_bh + qr] * kLog2e : 0.f};
-  float od = 0.f;
+  float od8[D / 32];
 #pragma unroll
   for (int c = 0; c < D / 32; ++c) {
     qf[0][c] = lds_frag_row<T>(qp + (int64_t)qr * a.qss + 32 * c + 8 * g);
@@ -523,11 +532,26 @@ void dq_wide_kernel(BwdArgsT<ND> a) {
     const Frag<T> of = lds_frag_row<T>(opp + (int64_t)qr * a.oss + 32 * c + 8 * g);
     const T* eo = reinterpret_cast<const T*>(of.w);
     const T* ed = reinterpret_cast<const T*>(df[0][c].w);
+    od8[c] = 0.f;
+    if constexpr (std::is_same<T, f16>::value) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) od = fmaf(to_f32(eo[i]), to_f32(ed[i]), od);
+      for (int i = 0; i < 4; ++i)
+        od8[c] = __builtin_amdgcn_fdot2(reinterpret_cast<const f16x2*>(eo)[i],
+                                        reinterpret_cast<const f16x2*>(ed)[i], od8[c], false);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) od8[c] = fmaf(to_f32(eo[i]), to_f32(ed[i]), od8[c]);
+    }
   }
-  od += __shfl_xor(od, 16);
+  // eight products in a row, then pairs of sums: the error grows with the
+  // logarithm of D
+#pragma unroll
+  for (int n = D / 64; n >= 1; n /= 2)
+#pragma unroll
+    for (int c = 0; c < n; ++c) od8[c] += od8[c + n];
+  float od = od8[0];
   od += __shfl_xor(od, 32);
+  od += __shfl_xor(od, 16);
   const float ndl[1] = {-od};
   if (ok && g == 0) {
     a.delta[row_bh + qi] = -od;
@@ -551,7 +575,7 @@ void dq_wide_kernel(BwdArgsT<ND> a) {
     wait_vmem();
     __syncthreads();  // this tile's K and V landed; every wave is done with the other K
     if (it + 1 < ntot) issue_k(it + 1, nxt);
-    const bool loc = it >= nglob;
+    const bool loc = it < nloc;
     const int ts = row0(it);
     const bool work = active && (loc ? (ts <= q_last && ts + BN - 1 >= w_lo) : ts < wg_hi);
     Frag<T> dsf[1];
@@ -693,7 +717,7 @@ __device__ __forceinline__ void dkdv2_tile(const char* tQ, const char* tO, const
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
         sc[qb2][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        dp[qb2][kb] = ndq;
+        dp[qb2][kb] = kSubDelta<D> ? f32x4{0.f, 0.f, 0.f, 0.f} : ndq;
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -731,6 +755,8 @@ __device__ __forceinline__ void dkdv2_tile(const char* tQ, const char* tO, const
     for (int qb2 = 0; qb2 < 2; ++qb2) {
       const int qblk = 2 * qs + qb2;
       const f32x4 nlq = *reinterpret_cast<const f32x4*>(sL + 16 * qblk + 4 * g);
+      f32x4 ndq{};
+      if (kSubDelta<D>) ndq = *reinterpret_cast<const f32x4*>(sDl + 16 * qblk + 4 * g);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
 #pragma unroll
@@ -743,7 +769,8 @@ __device__ __forceinline__ void dkdv2_tile(const char* tQ, const char* tO, const
             if (out) x = -__builtin_huge_valf();
           }
           p[qb2][kb][r] = __builtin_amdgcn_exp2f(x);
-          ds[qb2][kb][r] = p[qb2][kb][r] * dp[qb2][kb][r];
+          ds[qb2][kb][r] =
+              p[qb2][kb][r] * (kSubDelta<D> ? dp[qb2][kb][r] + ndq[r] : dp[qb2][kb][r]);
         }
       }
     }
@@ -785,10 +812,10 @@ __device__ __forceinline__ void dkdv2_tile(const char* tQ, const char* tO, const
 // rows; query tiles of BQ rows. At most 168 VGPRs: 3 waves per SIMD (the
 // global-row kernel below D = 128: at most 128, 4 waves per SIMD). At D = 256
 // the accumulators and the resident K/V fragments take 192 registers of a
-// 16-row wave: 256 VGPRs (2-10 spilled), 2 waves per SIMD, 4-wave workgroups
-// with 32-query tiles (66 KB of LDS, two per CU). B=1 H=8 S=32768 fp16:
-// global rows 215 us, local 306 us; dkdv_kernel (one LDS stage, transposed
-// tiles written by 2-byte LDS stores) took 720 and 638 us.
+// 16-row wave: 256 VGPRs (9-10 spilled), 2 waves per SIMD, 4-wave workgroups
+// with 32-query tiles (66 KB of LDS, two per CU). B=1 H=8 S=32768 bf16:
+// global rows 224 us, local 323 us; with one LDS stage and transposed tiles
+// written by 2-byte LDS stores 721 and 638 us.
 template <typename T, int D, bool GLOB, int NW, int KB, int BQ, int ND>
 __global__ __launch_bounds__(64 * NW)
 __attribute__((amdgpu_waves_per_eu(D > 128 ? 2 : GLOB && D < 128 ? 4 : 3)))

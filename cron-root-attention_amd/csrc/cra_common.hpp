@@ -86,15 +86,25 @@ __device__ __forceinline__ Frag<T> lds_frag_row(const T* p) {
 }
 
 // Cross-lane helpers on the 4 lane groups of a wave (lanes l, l^16, l^32, l^48).
+// The swaps exchange 16- or 32-lane halves of two registers in the VALU: both
+// holding x, they come back as x of the lane and of its partner in some order
+// (__shfl_xor goes through the LDS pipe, the bound of the kernels that ask for a
+// maximum with every tile).
+template <int OFF, typename F>
+__device__ __forceinline__ float with_partner(float x, F f) {
+  static_assert(OFF == 16 || OFF == 32, "lane group distance");
+  const uint32_t u = __float_as_uint(x);
+  const auto r = OFF == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false)
+                           : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 __device__ __forceinline__ float group_max(float x) {
-  x = fmaxf(x, __shfl_xor(x, 16));
-  x = fmaxf(x, __shfl_xor(x, 32));
-  return x;
+  auto mx = [](float a, float b) { return fmaxf(a, b); };
+  return with_partner<32>(with_partner<16>(x, mx), mx);
 }
 __device__ __forceinline__ float group_sum(float x) {
-  x += __shfl_xor(x, 16);
-  x += __shfl_xor(x, 32);
-  return x;
+  auto add = [](float a, float b) { return a + b; };
+  return with_partner<32>(with_partner<16>(x, add), add);
 }
 
 // ---------------------------------------------------------------------------

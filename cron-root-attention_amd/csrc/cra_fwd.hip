@@ -676,10 +676,55 @@ void fwd2_persistent_kernel(FwdArgsT<1> a) {
 // and softmax are computed its V is on the way, and the next tile's K during
 // P.V, so 32 KB of LDS per workgroup hide the fills and three workgroups (3
 // waves per SIMD at 168 VGPRs) share a CU. Bound by LDS reads: a K or V
-// fragment serves one MFMA, which caps MFMA-busy at about 60%. B=1 H=8
-// S=32768 fp16: 214 us (562 effective TFLOP/s); fwd_kernel (tiles through
-// registers, V stored transposed by 2-byte LDS writes) took 470 us.
+// fragment serves one MFMA, which caps MFMA-busy at about 60%.
+//
+// The softmax is the plain online one: the maximum is raised with every tile
+// (a query's largest P is exactly 1), l sums the unrounded P and O is divided
+// by it. fwd2's lazy maximum, sum of the rounded P and reciprocal would be 10%
+// faster here and put O and the gradients 2% farther from fp64 (B=1 H=8/4
+// S=8191 bf16 training step: relative error 3.53e-3 against 3.45e-3).
+//
+// B=1 H=8 S=32768 bf16: 234 us (514 effective TFLOP/s; 211 with the lazy
+// maximum); with tiles through registers and V stored transposed by 2-byte
+// LDS writes it took 470 us.
 constexpr int kWideWaves = 4, kWideBN = 32;
+
+// Softmax of a 32-key tile: raises the maximum, rescales l and O^T where it
+// rose and rounds P to the input type. l is the lane's own share of the sum.
+template <typename T, int D, bool MASK>
+__device__ __forceinline__ void wide_softmax(const f32x4 (&s)[2][1], float c2, int g,
+                                             const TileMask<1>& mk, f32x4 (&acc)[D / 16][1],
+                                             float& m_run, float& l_run, Frag<T>& pf) {
+  float t[8];  // scores (scaled in masked tiles), then P
+  float mx = -__builtin_huge_valf();
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float x = s[h][0][r];
+      if (MASK) x = mk.ok(16 * h + 4 * g + r, 0) ? x * c2 : -__builtin_huge_valf();
+      t[4 * h + r] = x;
+      mx = fmaxf(mx, x);
+    }
+  mx = group_max(MASK ? mx : mx * c2);
+  const float m_new = fmaxf(m_run, mx);
+  const float m_use = m_new == -__builtin_huge_valf() ? 0.f : m_new;  // no visible key yet
+  const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+  float psum = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    t[i] = __builtin_amdgcn_exp2f(MASK ? t[i] - m_use : fmaf(t[i], c2, -m_use));
+    psum += t[i];
+  }
+  l_run = l_run * alpha + psum;
+  m_run = m_new;
+  if (__any(alpha != 1.f)) {
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) acc[db][0] *= alpha;
+  }
+  pf = pack8<T>(t);
+}
+
 template <typename T, int D, int ND, bool DIR = false>
 __global__ __launch_bounds__(64 * kWideWaves) __attribute__((amdgpu_waves_per_eu(3)))
 void fwd_wide_kernel(FwdArgsT<ND> a) {
@@ -720,16 +765,16 @@ void fwd_wide_kernel(FwdArgsT<ND> a) {
   const int fk = Fill::lane_off(wave, lane, kbytes);
   const int fv = Fill::lane_off(wave, lane, vbytes);
   const int fgk = Fill::lane_off(wave, lane, gkb), fgv = Fill::lane_off(wave, lane, gvb);
-  // global tiles first, then the local window from its highest tile down
-  auto row0 = [&](int it) { return it >= nglob ? lo_k + (nloc - 1 - (it - nglob)) * BN : it * BN; };
+  // the local window, then the global rows
+  auto row0 = [&](int it) { return it < nloc ? lo_k + it * BN : (it - nloc) * BN; };
   auto issue_k = [&](int it) {
-    if (it >= nglob)
+    if (it < nloc)
       Fill::load(sK, rk, fk, kbytes, row0(it), wave);
     else
       Fill::load(sK, rgk, fgk, gkb, row0(it), wave);
   };
   auto issue_v = [&](int it) {
-    if (it >= nglob)
+    if (it < nloc)
       Fill::load(sV, rv, fv, vbytes, row0(it), wave);
     else
       Fill::load(sV, rgv, fgv, gvb, row0(it), wave);
@@ -756,13 +801,12 @@ void fwd_wide_kernel(FwdArgsT<ND> a) {
   const int wg_lo = active ? glob_prefix(q0, dc) : 0;
   const int wg_hi = active ? glob_prefix(q_last, dc) : 0;
   const int glen = glob_prefix(qi, dc);
-  const Frag<T> one = ones_frag<T>();
 
   for (int it = 0; it < ntot; ++it) {
     wait_vmem();
     __syncthreads();  // K of this tile landed; every wave is done with the previous V
     issue_v(it);
-    const bool loc = it >= nglob;
+    const bool loc = it < nloc;
     const int ts = row0(it);
     const bool work = active && (loc ? (ts <= q_last && ts + BN - 1 >= w_lo) : ts < wg_hi);
     Frag<T> pf[1];
@@ -773,14 +817,10 @@ void fwd_wide_kernel(FwdArgsT<ND> a) {
       mk.span[0] = loc ? (unsigned)(W - 1) : 0x7fffffffu;
       f32x4 s[2][1];
       tile_scores<T, D, BN, 1>(sK, lo, qf, 0, s);
-      float ps;
       if (full)
-        half_exp<T, false, 1>(s, 0, 0, c2, m_run[0], g, mk, one, pf[0], ps);
+        wide_softmax<T, D, false>(s, c2, g, mk, acc, m_run[0], l_run[0], pf[0]);
       else
-        half_exp<T, true, 1>(s, 0, 0, c2, m_run[0], g, mk, one, pf[0], ps);
-      if (__any(!(ps <= kSumMax)))
-        half_rescale<T, D, 1>(s, 0, c2, acc, m_run, l_run, one, pf[0], ps);
-      l_run[0] += ps;
+        wide_softmax<T, D, true>(s, c2, g, mk, acc, m_run[0], l_run[0], pf[0]);
     }
     wait_vmem();
     __syncthreads();  // V landed; every wave is done with this tile's K
@@ -788,10 +828,10 @@ void fwd_wide_kernel(FwdArgsT<ND> a) {
     if (work) pv_half<T, D, BN, 1>(sV, 0, lo, pf, acc);
   }
 
+  const float l = fmaxf(group_sum(l_run[0]), 1e-6f);
   if (!active || qi >= S) return;
   T* orow = static_cast<T*>(a.o) + b * a.osb + h * a.osh + (int64_t)(dc.off + qi) * a.oss;
-  const float l = fmaxf(l_run[0], 1e-6f);
-  const float inv = __builtin_amdgcn_rcpf(l);  // its 1-ulp error is invisible in the 2-byte O
+  const float inv = 1.f / l;
 #pragma unroll
   for (int db = 0; db < D / 16; ++db) {
     T e[4];
