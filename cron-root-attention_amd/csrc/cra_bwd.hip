@@ -443,6 +443,18 @@ void dq2_kernel(BwdArgsT<ND> a) {
   }
 }
 
+// Delta of the lane's query from sums of eight products, chunk c of the lane's
+// group in x[c]: by pairs, so that the error grows with the logarithm of D.
+template <int D>
+__device__ __forceinline__ float delta_sum(float (&x)[D / 32]) {
+#pragma unroll
+  for (int n = D / 64; n >= 1; n /= 2)
+#pragma unroll
+    for (int c = 0; c < n; ++c) x[c] += x[c + n];
+  x[0] += __shfl_xor(x[0], 32);
+  return x[0] + __shfl_xor(x[0], 16);
+}
+
 // dQ of the 2-byte types at head dim 256: 4 waves of 16 queries (Q, dO and dQ
 // take 128 registers of a wave per 16 queries), 32-key tiles. V is staged one
 // tile at a time and K two, 48 KB of LDS per workgroup: the next K arrives
@@ -543,15 +555,7 @@ void dq_wide_kernel(BwdArgsT<ND> a) {
       for (int i = 0; i < 8; ++i) od8[c] = fmaf(to_f32(eo[i]), to_f32(ed[i]), od8[c]);
     }
   }
-  // eight products in a row, then pairs of sums: the error grows with the
-  // logarithm of D
-#pragma unroll
-  for (int n = D / 64; n >= 1; n /= 2)
-#pragma unroll
-    for (int c = 0; c < n; ++c) od8[c] += od8[c + n];
-  float od = od8[0];
-  od += __shfl_xor(od, 32);
-  od += __shfl_xor(od, 16);
+  const float od = delta_sum<D>(od8);
   const float ndl[1] = {-od};
   if (ok && g == 0) {
     a.delta[row_bh + qi] = -od;
@@ -1029,7 +1033,8 @@ void dkdv2_kernel(BwdArgsT<ND> a) {
 // (Split). 4 waves of 16 queries (dQ) or 16 key rows (dK/dV), whose own
 // operands stay split in registers; 32-row tiles of K and V (Q and dO) are
 // staged through registers and split once per workgroup, up to D = 64 in two
-// LDS stages with one barrier per tile; dS and P are split in registers.
+// LDS stages with one barrier per tile; dS and P are split in registers. Delta
+// is subtracted from the finished dP, as at D = 256 in 2 bytes (kSubDelta).
 // Against the fp32-MFMA kernels before them (dQ with the separate Delta pass /
 // global rows / local rows), H=8: S=32768 D=64 527 / 554 / 467 -> 320 / 308 /
 // 238 us, D=128 1246 / 1600 / 1041 -> 695 / 711 / 452 us, S=4096 D=64 59 / 49 /
@@ -1044,11 +1049,10 @@ __device__ __forceinline__ void dq_f32_tile(const char* tK, const char* tV, cons
                                             int g, const TileMask<1>& mk) {
   using Stage = SplitStage<D, kF32BN, 64 * kF32Waves>;
   using Tile = typename Stage::Tile;
-  f32x4 sc[2], dp[2];
+  f32x4 sc[2], dp[2], sl[2], dl[2];  // sl, dl: the small products (kSmallApart)
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    sc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dp[h] = f32x4{ndl, ndl, ndl, ndl};
+    sc[h] = dp[h] = sl[h] = dl[h] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 #pragma unroll
   for (int c = 0; c < D / 32; ++c) {
@@ -1063,9 +1067,18 @@ __device__ __forceinline__ void dq_f32_tile(const char* tK, const char* tV, cons
     for (int t = 0; t < 6; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        sc[h] = mma(sc[h], kf[h].p[split_a(t)], qf[c].p[split_b(t)]);
-        dp[h] = mma(dp[h], vf[h].p[split_a(t)], df[c].p[split_b(t)]);
+        f32x4& s_ = t < kSmallApart<D> ? sl[h] : sc[h];
+        f32x4& d_ = t < kSmallApart<D> ? dl[h] : dp[h];
+        s_ = mma(s_, kf[h].p[split_a(t)], qf[c].p[split_b(t)]);
+        d_ = mma(d_, vf[h].p[split_a(t)], df[c].p[split_b(t)]);
       }
+  }
+  if (kSmallApart<D> > 0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      sc[h] += sl[h];
+      dp[h] += dl[h];
+    }
   }
   float ds[8];
 #pragma unroll
@@ -1074,7 +1087,7 @@ __device__ __forceinline__ void dq_f32_tile(const char* tK, const char* tV, cons
     for (int r = 0; r < 4; ++r) {
       float x = fmaf(sc[h][r], c2, -lse2);
       if (MASK && !mk.ok(16 * h + 4 * g + r, 0)) x = -__builtin_huge_valf();
-      ds[4 * h + r] = __builtin_amdgcn_exp2f(x) * dp[h][r];
+      ds[4 * h + r] = __builtin_amdgcn_exp2f(x) * (dp[h][r] + ndl);
     }
   const Split dsf = split8<true>(ds);
 #pragma unroll
@@ -1090,8 +1103,11 @@ __device__ __forceinline__ void dq_f32_tile(const char* tK, const char* tV, cons
   }
 }
 
+// (D = 64: at most 168 registers, three workgroups per CU; at 170 and two it
+// took 1249 us against 1039 at B=1 H=4 S=131072)
 template <int D, int ND>
-__global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2)))
+__global__ __launch_bounds__(64 * kF32Waves)
+__attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : D > 64 ? 2 : 3)))
 void dq_f32_kernel(BwdArgsT<ND> a) {
   constexpr int NW = kF32Waves, BN = kF32BN, kBM = 16 * NW;
   constexpr int kStages = D <= 64 ? 2 : 1;
@@ -1154,26 +1170,26 @@ void dq_f32_kernel(BwdArgsT<ND> a) {
   const int qr = min(qi, S - 1);
   const bool ok = qi < S;
   const float lse2 = ok ? a.lse[row_bh + qr] * kLog2e : 0.f;
-  float od = 0.f;
+  float od8[D / 32];
 #pragma unroll
   for (int c = 0; c < D / 32; ++c) {
     qf[c] = load_split(qp + (int64_t)qr * a.qss + 32 * c + 8 * g);
     const float* pd = dop + (int64_t)qr * a.doss + 32 * c + 8 * g;
     const float* po = opp + (int64_t)qr * a.oss + 32 * c + 8 * g;
     float xd[8];
+    od8[c] = 0.f;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const f32x4 d4 = reinterpret_cast<const f32x4*>(pd)[i], o4 = reinterpret_cast<const f32x4*>(po)[i];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         xd[4 * i + r] = d4[r];
-        od = fmaf(o4[r], d4[r], od);
+        od8[c] = fmaf(o4[r], d4[r], od8[c]);
       }
     }
     df[c] = split8<true>(xd);
   }
-  od += __shfl_xor(od, 16);
-  od += __shfl_xor(od, 32);
+  const float od = delta_sum<D>(od8);
   if (ok && g == 0) {
     a.delta[row_bh + qi] = -od;
     a.nlse2[row_bh + qi] = -lse2;
@@ -1226,11 +1242,10 @@ __device__ __forceinline__ void dkdv_f32_tile(const char* tQ, const char* tO, co
                                               float c2, int g, int q_off, unsigned qspan) {
   using Stage = SplitStage<D, kF32BN, 64 * kF32Waves>;
   using Tile = typename Stage::Tile;
-  f32x4 sc[2], dp[2];
+  f32x4 sc[2], dp[2], sl[2], dl[2];  // sl, dl: the small products (kSmallApart)
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    sc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dp[h] = *reinterpret_cast<const f32x4*>(sDl + 16 * h + 4 * g);
+    sc[h] = dp[h] = sl[h] = dl[h] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 #pragma unroll
   for (int c = 0; c < D / 32; ++c) {
@@ -1244,28 +1259,42 @@ __device__ __forceinline__ void dkdv_f32_tile(const char* tQ, const char* tO, co
     for (int t = 0; t < 6; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        sc[h] = mma(sc[h], qa[h].p[split_a(t)], kf[c].p[split_b(t)]);
-        dp[h] = mma(dp[h], oa[h].p[split_a(t)], vf[c].p[split_b(t)]);
+        f32x4& s_ = t < kSmallApart<D> ? sl[h] : sc[h];
+        f32x4& d_ = t < kSmallApart<D> ? dl[h] : dp[h];
+        s_ = mma(s_, qa[h].p[split_a(t)], kf[c].p[split_b(t)]);
+        d_ = mma(d_, oa[h].p[split_a(t)], vf[c].p[split_b(t)]);
       }
+  }
+  if (kSmallApart<D> > 0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      sc[h] += sl[h];
+      dp[h] += dl[h];
+    }
   }
   float p[8], ds[8];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const f32x4 nlq = *reinterpret_cast<const f32x4*>(sL + 16 * h + 4 * g);
+    const f32x4 ndq = *reinterpret_cast<const f32x4*>(sDl + 16 * h + 4 * g);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float x = fmaf(sc[h][r], c2, nlq[r]);
       if (MASK && (unsigned)(16 * h + r + q_off) > qspan) x = -__builtin_huge_valf();
       p[4 * h + r] = __builtin_amdgcn_exp2f(x);
-      ds[4 * h + r] = p[4 * h + r] * dp[h][r];
+      ds[4 * h + r] = p[4 * h + r] * (dp[h][r] + ndq[r]);
     }
   }
   const Split pf = split8<false>(p), sf = split8<true>(ds);
   // SUM (global rows): a tile's six products are summed from zero and added
   // once. A row of the first blocks sums over thousands of queries, where six
   // roundings of the long sum per tile would show (dK at S = 131072: relative
-  // error 1.4e-6; 5.2e-7 so; the fp32 MFMA's 1.2e-6). A local row's sum is
-  // short.
+  // error 1.4e-6, and 5.6e-7 so; the fp32 MFMA's 9.5e-7). A local row sums over
+  // W queries of each head of its kv group: added up straight its error stays
+  // below the fp32 MFMA's with the longest sums too (H=32/1 S=131072 D=64, 11.6K
+  // queries: dK 2.1e-6 against 3.4e-6; H=16/1 S=65536 D=128 1.2e-6 against
+  // 1.7e-6), and per-tile sums would take the D = 128 kernel, at its register
+  // cap, 7% longer for a sixth less of it.
 #pragma unroll
   for (int db = 0; db < D / 16; ++db) {
     const Split ot = Stage::tr_frag(tO + lo.tr_at(db));

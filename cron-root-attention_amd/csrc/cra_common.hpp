@@ -254,43 +254,62 @@ struct SwzTile {
 
 // ---------------------------------------------------------------------------
 // fp32 operands on the bf16 matrix core. A float's 24-bit significand is cut
-// into three bf16 pieces of 8 bits, x = hi + mid + lo exactly (each piece the
-// truncated rest, so nothing rounds or overflows; below 2^-110 the last bits
-// fall under the smallest bf16). A product takes the six piece products down
-// to 2^-16 of it; the three left out are at most 2^-23 of |x y| together, a
-// quarter of that on average, where one fp32 multiply-add rounds by up to
-// 2^-24. Six 16x16x32 MFMAs (16 cycles each) stand for eight 16x16x4 fp32 ones
-// (32 cycles each), and round the sum six times where those did eight times:
-// against fp64 every output is nearer than with the fp32 MFMA (relative error
-// of o, dq, dk, dv at B=1 H=8 S=4096 D=64: 2.9, 3.9, 3.5, 3.4e-7 against 3.4,
-// 4.6, 4.7, 4.5e-7; H=4 S=131072: 5.4, 6.4, 5.5, 5.3e-7 against 5.8, 6.8, 12,
-// 12e-7; the same order at D = 32, 128 and 256). An infinite x is kept in the piece that meets only the
-// other operand's hi, so that infinity times a number stays infinite.
+// into three bf16 pieces of 8 bits, x = hi + mid + lo exactly: hi and mid are
+// rounded to nearest, so mid is at most 2^-8 and lo 2^-17 of x's power of two
+// (below 2^-110 the last bits fall under the smallest bf16). A product takes
+// the six piece products down to 2^-16 of it; the three left out are at most
+// 2^-24 of |x y| together (2^-28 on average, of either sign), what one fp32
+// multiply-add rounds by. (Pieces cut off instead leave up to 2^-21, always
+// toward zero: sums of one sign lose it. dq of positive inputs at H=2 S=131072
+// D=64: relative error 1.8e-4 against 3.1e-5.) Six 16x16x32 MFMAs (16 cycles
+// each) stand for eight 16x16x4 fp32 ones (32 cycles each) and round the sum
+// six times where those did eight times. Relative error of o, dq, dk, dv
+// against fp64, x 1e-7, fp32 MFMA / this:
+//   H=8 S=4096 D=64         3.4, 4.5, 4.7, 4.5 / 2.6, 4.1, 3.7, 3.6
+//   H=4 S=4096 D=32         2.9, 4.1, 4.2, 4.3 / 2.2, 3.8, 3.3, 3.3
+//   H=4 S=4096 D=128        4.3, 5.4, 5.5, 5.2 / 3.3, 4.7, 4.4, 4.2
+//   H=4 S=8192 D=256        5.8, 6.9, 6.9, 6.5 / 2.9, 4.2, 3.9, 3.8
+//   H=2 S=131072 D=64       5.8, 6.8, 9.5, 9.3 / 5.2, 6.4, 5.7, 5.4
+//   H=32/1 S=131072 D=64    5.8, 6.8, 34, 34   / 5.1, 6.4, 21, 20
+// Inputs of one sign keep the fp32 MFMA's error up to D = 128 (H=4 S=4096
+// D=128 1.9, 127, 2.0, 1.9 / 1.7, 127, 1.9, 1.7; dq is a difference of
+// near-equal sums there) within a fifth, dk at D = 256 within a third.
+// An infinite x is kept in the piece that meets only the other operand's hi,
+// so that infinity times a number stays infinite.
 // ---------------------------------------------------------------------------
 struct Split {
   Frag<bf16> p[3];  // hi, mid, lo
 };
 
-// INF: x may be infinite.
+constexpr float kMaxBf16 = 0x1.fep127f;
+
+// INF: x may be infinite, or finite above the largest bf16 (which is its hi then).
 template <bool INF>
 __device__ __forceinline__ Split split8(const float (&x)[8]) {
+  auto pack = [](const float (&v)[2]) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v[0], v[1]}, bf16x2));
+  };
+  auto value = [](uint32_t u, int i) { return __uint_as_float(i ? u & 0xffff0000u : u << 16); };
   Split f;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
-    uint32_t h[2], m[2], l[2];
+    float v[2], c[2];
+    bool inf[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const float v = x[2 * w + i];
-      const bool inf = INF && __builtin_isinf(v);
-      h[i] = inf ? 0u : __float_as_uint(v) & 0xffff0000u;
-      const float r = v - __uint_as_float(h[i]);
-      m[i] = inf ? 0u : __float_as_uint(r) & 0xffff0000u;
-      l[i] = __float_as_uint(r - __uint_as_float(m[i]));
+      inf[i] = INF && __builtin_isinf(x[2 * w + i]);
+      v[i] = inf[i] ? 0.f : x[2 * w + i];
+      c[i] = INF ? __builtin_amdgcn_fmed3f(v[i], -kMaxBf16, kMaxBf16) : v[i];
     }
-    // the high halves of two words
-    reinterpret_cast<uint32_t*>(f.p[0].w)[w] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302u);
-    reinterpret_cast<uint32_t*>(f.p[1].w)[w] = __builtin_amdgcn_perm(m[1], m[0], 0x07060302u);
-    reinterpret_cast<uint32_t*>(f.p[2].w)[w] = __builtin_amdgcn_perm(l[1], l[0], 0x07060302u);
+    const uint32_t h = pack(c);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) v[i] -= value(h, i);
+    const uint32_t m = pack(v);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) v[i] = inf[i] ? x[2 * w + i] : v[i] - value(m, i);
+    reinterpret_cast<uint32_t*>(f.p[0].w)[w] = h;
+    reinterpret_cast<uint32_t*>(f.p[1].w)[w] = m;
+    reinterpret_cast<uint32_t*>(f.p[2].w)[w] = pack(v);
   }
   return f;
 }
@@ -300,6 +319,14 @@ __device__ __forceinline__ constexpr int split_a(int t) { return t == 0 ? 2 : t 
 __device__ __forceinline__ constexpr int split_b(int t) { return t == 1 ? 2 : t == 2 || t == 4 ? 1 : 0; }
 // t:      0 1 2 3 4 5
 // a, b:   lo.hi hi.lo mid.mid mid.hi hi.mid hi.hi
+
+// Products of the scores and dP that are summed apart from hi.hi and added at
+// the end: all but hi.hi at D = 256, whose sums over eight chunks would round 48
+// times at full magnitude (now 8). Relative error of o, dq, dk, dv at B=1 H=4
+// S=8192: 4.7, 5.9, 5.7, 5.3e-7 in one sum, 2.9, 4.2, 3.9, 3.8e-7 so, for 1-4%
+// of the kernels' time; at D = 128 a fourth less error would cost dQ 9%.
+template <int D>
+constexpr int kSmallApart = D > 128 ? 5 : 0;
 
 // ROWS x D tile of fp32 rows as three planes of SwzTile, filled through
 // registers by NT threads: load() issues the reads, store() splits and writes.
@@ -330,9 +357,22 @@ struct SplitStage {
   __device__ __forceinline__ void store(char* lds, int tid) const {
     const int cg = tid % Tile::kCPR, rg = tid / Tile::kCPR;
     if (rg >= kRowGroups) return;
+    // values above the largest bf16 are rare: tested together
+    float mx = 0.f;
+#pragma unroll
+    for (int i = 0; i < kRPT; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(reinterpret_cast<const float*>(r[i])[j]));
+    if (__any(mx > kMaxBf16))
+      store_split<true>(lds, cg, rg);
+    else
+      store_split<false>(lds, cg, rg);
+  }
+  template <bool INF>
+  __device__ __forceinline__ void store_split(char* lds, int cg, int rg) const {
 #pragma unroll
     for (int i = 0; i < kRPT; ++i) {
-      const Split f = split8<true>(*reinterpret_cast<const float(*)[8]>(&r[i][0]));
+      const Split f = split8<INF>(*reinterpret_cast<const float(*)[8]>(&r[i][0]));
       char* dst = lds + Tile::off(i * kRowGroups + rg, cg);
 #pragma unroll
       for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(dst + k * Tile::kBytes) = f.p[k].w[0];

@@ -56,11 +56,11 @@ __device__ __forceinline__ void attend_f32(const char* tK, const char* tV, const
                                            const TileMask<QB>& mk) {
   using Stage = SplitStage<D, kF32BN, 64 * kF32Waves>;
   using Tile = typename Stage::Tile;
-  f32x4 s[2][QB];
+  f32x4 s[2][QB], sl[2][QB];  // sl: the small products (kSmallApart)
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb) s[h][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int qb = 0; qb < QB; ++qb) s[h][qb] = sl[h][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int c = 0; c < D / 32; ++c) {
     Split kf[2];
@@ -72,8 +72,16 @@ __device__ __forceinline__ void attend_f32(const char* tK, const char* tV, const
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int qb = 0; qb < QB; ++qb)
-          s[h][qb] = mma(s[h][qb], kf[h].p[split_a(t)], qf[qb][c].p[split_b(t)]);
+        for (int qb = 0; qb < QB; ++qb) {
+          f32x4& s_ = t < kSmallApart<D> ? sl[h][qb] : s[h][qb];
+          s_ = mma(s_, kf[h].p[split_a(t)], qf[qb][c].p[split_b(t)]);
+        }
+  }
+  if (kSmallApart<D> > 0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) s[h][qb] += sl[h][qb];
   }
   Split pf[QB];
 #pragma unroll
