@@ -103,6 +103,8 @@ _SIGNATURES = {
                                         ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
     "cra_fwd": (ctypes.c_int, [_P, CraTensor, CraTensor, CraTensor, ctypes.c_void_p,
                                ctypes.c_void_p, CraTensor, ctypes.c_void_p, ctypes.c_void_p]),
+    "cra_fwd_inplace": (ctypes.c_int, [_P, CraTensor, CraTensor, CraTensor, CraTensor,
+                                       ctypes.c_void_p, ctypes.c_void_p]),
     "cra_fwd_phases": (ctypes.c_int, [_P, CraTensor, CraTensor, CraTensor, ctypes.c_void_p,
                                       ctypes.c_void_p, CraTensor, ctypes.c_void_p, ctypes.c_int32,
                                       ctypes.c_void_p]),
@@ -114,6 +116,9 @@ _SIGNATURES = {
                                ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                ctypes.c_void_p, CraTensor, CraTensor, CraTensor, ctypes.c_void_p,
                                ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "cra_bwd_inplace": (ctypes.c_int, [_P, CraTensor, CraTensor, CraTensor, CraTensor, CraTensor,
+                                       ctypes.c_void_p, CraTensor, CraTensor, CraTensor,
+                                       ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cra_bwd_noalloc": (ctypes.c_int, [_P, CraTensor, CraTensor, CraTensor, CraTensor, CraTensor,
                                        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                        ctypes.c_void_p, ctypes.c_void_p, CraTensor, CraTensor,
@@ -282,8 +287,8 @@ def global_rows(p: CraProblem) -> int:
 
 
 def reads_global_rows(p: CraProblem, k: torch.Tensor, v: torch.Tensor) -> bool:
-    """Whether cra_fwd / cra_bwd read the packed rows (else they take the
-    global rows from k and v, and build_global need not run)."""
+    """Whether the call needs packed rows (else forward and backward can read the
+    global rows in k and v, gk = gv = None, and build_global need not run)."""
     n = load_library().cra_reads_global_rows(ctypes.byref(p), tensor_arg(k), tensor_arg(v))
     if n < 0:
         _raise(E_INVALID, "cra_reads_global_rows")
@@ -314,12 +319,16 @@ PHASE_GLOBAL = 2
 
 def forward(p: CraProblem, q, k, v, gk, gv, phases: int = PHASE_LOCAL | PHASE_GLOBAL,
             stream: Optional[int] = None):
-    """cra_fwd (all phases) or cra_fwd_phases (a subset, for measurement)."""
+    """cra_fwd (all phases), without packed rows (gk None) cra_fwd_inplace, or
+    cra_fwd_phases (a subset, for measurement)."""
     lib = load_library()
     st = _stream(q) if stream is None else stream
     o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     lse = torch.empty(p.B, p.H_q, p.S, dtype=torch.float32, device=q.device)
-    if phases == PHASE_LOCAL | PHASE_GLOBAL:
+    if gk is None:
+        _check(lib.cra_fwd_inplace(ctypes.byref(p), tensor_arg(q), tensor_arg(k), tensor_arg(v),
+                                   tensor_arg(o), lse.data_ptr(), st), "cra_fwd_inplace")
+    elif phases == PHASE_LOCAL | PHASE_GLOBAL:
         _check(lib.cra_fwd(ctypes.byref(p), tensor_arg(q), tensor_arg(k), tensor_arg(v),
                            gk.data_ptr(), gv.data_ptr(), tensor_arg(o), lse.data_ptr(),
                            st), "cra_fwd")
@@ -352,12 +361,19 @@ def workspace_bytes(p: CraProblem) -> int:
 
 
 def backward(p: CraProblem, q, k, v, o, do, lse, gk, gv, src, relay_scale, want_dalpha: bool):
+    """cra_bwd, or without packed rows (gk None) cra_bwd_inplace."""
     lib = load_library()
     dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     dk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
     dv = torch.empty(v.shape, dtype=v.dtype, device=v.device)
     nbytes = workspace_bytes(p)
     ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=q.device)
+    if gk is None:
+        _check(lib.cra_bwd_inplace(ctypes.byref(p), tensor_arg(q), tensor_arg(k), tensor_arg(v),
+                                   tensor_arg(o), tensor_arg(do), lse.data_ptr(), tensor_arg(dq),
+                                   tensor_arg(dk), tensor_arg(dv), ws.data_ptr(), ws.numel(),
+                                   _stream(q)), "cra_bwd_inplace")
+        return dq, dk, dv, None
     dalpha = (torch.empty(p.H_kv, dtype=torch.float32, device=q.device)
               if (want_dalpha and p.relay) else None)
     rs = relay_scale.data_ptr() if (relay_scale is not None and p.relay) else None

@@ -186,8 +186,7 @@ class CronRootAttentionV14Function(torch.autograd.Function):
         if persistent:
             o, lse = _native.forward_persistent(p, qp, kp, vp, gk, gv, stream=st)
         else:
-            o, lse = _native.forward(p, qp, kp, vp, kp if gk is None else gk,
-                                     vp if gv is None else gv, stream=st)
+            o, lse = _native.forward(p, qp, kp, vp, gk, gv, stream=st)
         ctx.problem = p
         ctx.D = D
         ctx.has_alpha = relay_log_scale is not None and relay_on
@@ -201,10 +200,8 @@ class CronRootAttentionV14Function(torch.autograd.Function):
         p = ctx.problem
         D = ctx.D
         dop = _kernel_ready(_pad_d(do.to(qp.dtype), p.D))
-        if gk is None:
-            if _native.reads_global_rows(p, kp, vp):  # layouts changed by a saved-tensor hook
-                kp, vp = kp.contiguous(), vp.contiguous()
-            gk, gv = kp, vp
+        if gk is None and _native.reads_global_rows(p, kp, vp):
+            kp, vp = kp.contiguous(), vp.contiguous()  # layouts changed by a saved-tensor hook
         dq, dk, dv, dalpha = _native.backward(p, qp, kp, vp, o, dop, lse, gk, gv, src, rscale,
                                               ctx.has_alpha)
         if p.D != D:

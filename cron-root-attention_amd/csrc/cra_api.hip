@@ -212,13 +212,26 @@ int plan_varlen(const cra_problem* p, const cra_docs* d, Plan* pl) {
 }
 
 // One document without relay, k and v of one row stride: its global rows are
-// rows r * W of k and v, and the kernels read them there. Their tiles are addressed with 32-bit offsets up
-// to 64 rows of W past the last one, so strides for which that could wrap keep
-// the packed rows.
+// rows r * W of k and v, and the kernels can read them there. Their tiles are
+// addressed with 32-bit offsets up to 64 rows of W past the last one, so strides
+// for which that could wrap need packed rows.
 bool direct_rows(const cra_problem* p, const Plan& pl, const cra_tensor& k, const cra_tensor& v) {
   if (pl.n != 1 || pl.any_relay) return false;
   const int64_t step = k.ss * elem_size(p->dtype);
   return k.ss == v.ss && k.ss >= 0 && (pl.len[0] + 64 * (int64_t)pl.W[0]) * step < ((int64_t)1 << 32);
+}
+
+// The global rows of a call: packed, or read in k and v.
+int check_global_rows(const cra_problem* p, const Plan& pl, const cra_tensor& k, const cra_tensor& v,
+                      const void* glob_k, const void* glob_v, bool inplace) {
+  if (!inplace) {
+    if (int e = check_buf("glob_k", glob_k)) return e;
+    return check_buf("glob_v", glob_v);
+  }
+  if ((int64_t)p->B * p->H_kv > 65535) return fail(CRA_E_INVALID, "B*H_kv exceeds 65535");
+  if (!direct_rows(p, pl, k, v))
+    return fail(CRA_E_LAYOUT, "this call needs packed global rows (cra_reads_global_rows)");
+  return CRA_OK;
 }
 
 int num_groups(const Plan& pl) { return (pl.n + cra::kMaxDocs - 1) / cra::kMaxDocs; }
@@ -296,7 +309,8 @@ int build_global_impl(const cra_problem* p, const Plan& pl, cra_tensor k, cra_te
 
 int fwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, cra_tensor v,
              const void* glob_k, const void* glob_v, cra_tensor o, float* lse,
-             int32_t phase_mask, void* stream, int32_t* work_counter = nullptr) {
+             int32_t phase_mask, void* stream, int32_t* work_counter = nullptr,
+             bool inplace = false) {
   if (phase_mask < 1 || phase_mask > (CRA_PHASE_LOCAL | CRA_PHASE_GLOBAL))
     return fail(CRA_E_INVALID, "phase_mask must be a non-empty subset of CRA_PHASE_LOCAL | CRA_PHASE_GLOBAL");
   const int esz = elem_size(p->dtype);
@@ -306,8 +320,7 @@ int fwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   if (int e = check_tensor("o", o, esz)) return e;
   if (int e = check_span("k", k, p, esz)) return e;
   if (int e = check_span("v", v, p, esz)) return e;
-  if (int e = check_buf("glob_k", glob_k)) return e;
-  if (int e = check_buf("glob_v", glob_v)) return e;
+  if (int e = check_global_rows(p, pl, k, v, glob_k, glob_v, inplace)) return e;
   if (int e = check_buf("lse", lse)) return e;
   cra::FwdArgs a{};
   a.q = q.ptr; a.k = k.ptr; a.v = v.ptr; a.gk = glob_k; a.gv = glob_v; a.o = o.ptr; a.lse = lse;
@@ -320,9 +333,7 @@ int fwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   a.scale = p->scale;
   a.phases = phase_mask;
   a.work_counter = work_counter;
-  // (the persistent and the phase-restricted kernels take packed rows only)
-  a.direct = !work_counter && phase_mask == (CRA_PHASE_LOCAL | CRA_PHASE_GLOBAL) &&
-             direct_rows(p, pl, k, v);
+  a.direct = inplace;
   for (int g = 0; g < num_groups(pl); ++g) {
     a.docs = group_table(pl, g);
     hipError_t e = cra::launch_fwd(p->dtype, p->D, a, (hipStream_t)stream);
@@ -338,7 +349,7 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
              cra_tensor o, cra_tensor dout, const float* lse, const void* glob_k,
              const void* glob_v, const int32_t* relay_src, const float* relay_scale,
              cra_tensor dq, cra_tensor dk, cra_tensor dv, float* dalpha, void* workspace,
-             size_t workspace_bytes_given, void* stream, int nchunk_cap = 0) {
+             size_t workspace_bytes_given, void* stream, int nchunk_cap = 0, bool inplace = false) {
   const int esz = elem_size(p->dtype);
   if (int e = check_tensor("q", q, esz)) return e;
   if (int e = check_tensor("k", k, esz)) return e;
@@ -354,8 +365,7 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   if (int e = check_span("v", v, p, esz)) return e;
   if (int e = check_span("dout", dout, p, esz)) return e;
   if (int e = check_buf("lse", lse)) return e;
-  if (int e = check_buf("glob_k", glob_k)) return e;
-  if (int e = check_buf("glob_v", glob_v)) return e;
+  if (int e = check_global_rows(p, pl, k, v, glob_k, glob_v, inplace)) return e;
   if (pl.any_relay && !relay_src) return fail(CRA_E_INVALID, "relay_src is NULL with relay on");
   const cra::ChunkPlan chunks = cap_chunks(pl, chunk_plan(p, pl), nchunk_cap);
   const size_t need = workspace_bytes(p, chunks);
@@ -382,7 +392,7 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   a.G = pl.G;
   a.scale = p->scale;
   a.cus = device_cus();
-  a.direct = direct_rows(p, pl, k, v);
+  a.direct = inplace;
   a.chunk_len = chunks.chunk_len;
   a.nchunk = chunks.nchunk;
   // workspace carve-up: delta and nlse2 [B*Hq*S] fp32 each, then the
@@ -481,6 +491,14 @@ int cra_fwd(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cons
                         stream);
 }
 
+int cra_fwd_inplace(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cra_tensor o,
+                    float* lse, void* stream) {
+  Plan pl;
+  if (int e = plan_plain(p, &pl)) return e;
+  return fwd_impl(p, pl, q, k, v, nullptr, nullptr, o, lse, CRA_PHASE_LOCAL | CRA_PHASE_GLOBAL,
+                  stream, nullptr, true);
+}
+
 int cra_fwd_phases(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v,
                    const void* glob_k, const void* glob_v, cra_tensor o, float* lse,
                    int32_t phase_mask, void* stream) {
@@ -513,6 +531,15 @@ int cra_bwd(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cra_
   if (int e = plan_plain(p, &pl)) return e;
   return bwd_impl(p, pl, q, k, v, o, dout, lse, glob_k, glob_v, relay_src, relay_scale, dq, dk,
                   dv, dalpha, workspace, workspace_bytes, stream);
+}
+
+int cra_bwd_inplace(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cra_tensor o,
+                    cra_tensor dout, const float* lse, cra_tensor dq, cra_tensor dk, cra_tensor dv,
+                    void* workspace, size_t workspace_bytes, void* stream) {
+  Plan pl;
+  if (int e = plan_plain(p, &pl)) return e;
+  return bwd_impl(p, pl, q, k, v, o, dout, lse, nullptr, nullptr, nullptr, nullptr, dq, dk, dv,
+                  nullptr, workspace, workspace_bytes, stream, 0, true);
 }
 
 int cra_bwd_noalloc(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cra_tensor o,

@@ -34,8 +34,10 @@ struct Api {
   decltype(&cra_reads_global_rows) reads_global = nullptr;
   decltype(&cra_build_global) build_global = nullptr;
   decltype(&cra_fwd) fwd = nullptr;
+  decltype(&cra_fwd_inplace) fwd_inplace = nullptr;
   decltype(&cra_bwd_workspace_bytes) ws_bytes = nullptr;
   decltype(&cra_bwd) bwd = nullptr;
+  decltype(&cra_bwd_inplace) bwd_inplace = nullptr;
   decltype(&cra_strerror) strerror_ = nullptr;
   decltype(&cra_last_error) last_error = nullptr;
   decltype(&cra_abi_version) abi_version = nullptr;
@@ -63,8 +65,10 @@ void bind(std::string path) {
   resolve(h, path, "cra_reads_global_rows", api.reads_global);
   resolve(h, path, "cra_build_global", api.build_global);
   resolve(h, path, "cra_fwd", api.fwd);
+  resolve(h, path, "cra_fwd_inplace", api.fwd_inplace);
   resolve(h, path, "cra_bwd_workspace_bytes", api.ws_bytes);
   resolve(h, path, "cra_bwd", api.bwd);
+  resolve(h, path, "cra_bwd_inplace", api.bwd_inplace);
   resolve(h, path, "cra_strerror", api.strerror_);
   resolve(h, path, "cra_last_error", api.last_error);
   resolve(h, path, "cra_abi_version", api.abi_version);
@@ -136,14 +140,9 @@ void* stream_of(const at::Tensor& t) {
   return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
-// Addresses of the packed K and V rows; without them (the kernels take the
-// global rows from k and v) k's own address stands in, which is not read.
-std::pair<const char*, const char*> glob_ptrs(const at::Tensor& gkv, const at::Tensor& k) {
-  if (!gkv.defined()) {
-    const char* p = static_cast<const char*>(k.data_ptr());
-    return {p, p};
-  }
-  const char* p = static_cast<const char*>(gkv.data_ptr());
+// Addresses of the packed K and V rows.
+std::pair<char*, char*> glob_ptrs(const at::Tensor& gkv) {
+  char* p = static_cast<char*>(gkv.data_ptr());
   return {p, p + gkv.numel() / 2 * gkv.element_size()};
 }
 
@@ -157,7 +156,7 @@ at::Tensor empty_bhsd(const at::Tensor& t, bool bshd) {
 }
 
 // Forward launches: packed global rows (one allocation for K and V rows) and
-// relay source rows where the kernels read them, then the three-phase forward.
+// relay source rows where the call needs them, then the three-phase forward.
 // Returns o, lse, the packed rows and the relay source rows (either may be
 // undefined). At S = 512 the packing was 3 of the call's 12 us on the GPU.
 std::array<at::Tensor, 4> run_forward(const cra_problem& p, const at::Tensor& q,
@@ -175,16 +174,21 @@ std::array<at::Tensor, 4> run_forward(const cra_problem& p, const at::Tensor& q,
       const int64_t nb = (p.S + p.W - 1) / p.W;
       src = at::empty({p.B, p.H_kv, nb * p.top_k}, k.options().dtype(at::kInt));
     }
-    char* gk = static_cast<char*>(gkv.data_ptr());
-    check(a.build_global(&p, targ(k), targ(v), gk, gk + gkv.numel() / 2 * gkv.element_size(),
-                         p.relay ? src.data_ptr<int32_t>() : nullptr, nullptr, st),
+    const auto [gk, gv] = glob_ptrs(gkv);
+    check(a.build_global(&p, targ(k), targ(v), gk, gv, p.relay ? src.data_ptr<int32_t>() : nullptr,
+                         nullptr, st),
           "cra_build_global");
   }
-  const auto [gk, gv] = glob_ptrs(gkv, k);
   at::Tensor o = empty_bhsd(q, bshd);
   at::Tensor lse = at::empty({p.B, p.H_q, p.S}, q.options().dtype(at::kFloat));
-  check(a.fwd(&p, targ(q), targ(k), targ(v), gk, gv, targ(o), lse.data_ptr<float>(), st),
-        "cra_fwd");
+  if (reads) {
+    const auto [gk, gv] = glob_ptrs(gkv);
+    check(a.fwd(&p, targ(q), targ(k), targ(v), gk, gv, targ(o), lse.data_ptr<float>(), st),
+          "cra_fwd");
+  } else {
+    check(a.fwd_inplace(&p, targ(q), targ(k), targ(v), targ(o), lse.data_ptr<float>(), st),
+          "cra_fwd_inplace");
+  }
   return {o, lse, gkv, src};
 }
 
@@ -246,11 +250,18 @@ class CraAttention : public torch::autograd::Function<CraAttention> {
     at::Tensor dq = empty_bhsd(q, bshd), dk = empty_bhsd(k, bshd), dv = empty_bhsd(v, bshd);
     const size_t nws = a.ws_bytes(&p);
     at::Tensor ws = at::empty({(int64_t)std::max<size_t>(nws, 256)}, q.options().dtype(at::kByte));
-    const auto [gk, gv] = glob_ptrs(gkv, k);
-    check(a.bwd(&p, targ(q), targ(k), targ(v), targ(o), targ(dout), lse.data_ptr<float>(), gk,
-                gv, p.relay ? src.data_ptr<int32_t>() : nullptr, nullptr, targ(dq), targ(dk),
-                targ(dv), nullptr, ws.data_ptr(), (size_t)ws.numel(), st),
-          "cra_bwd");
+    if (gkv.defined()) {
+      const auto [gk, gv] = glob_ptrs(gkv);
+      check(a.bwd(&p, targ(q), targ(k), targ(v), targ(o), targ(dout), lse.data_ptr<float>(), gk, gv,
+                  p.relay ? src.data_ptr<int32_t>() : nullptr, nullptr, targ(dq), targ(dk),
+                  targ(dv), nullptr, ws.data_ptr(), (size_t)ws.numel(), st),
+            "cra_bwd");
+    } else {
+      check(a.bwd_inplace(&p, targ(q), targ(k), targ(v), targ(o), targ(dout),
+                          lse.data_ptr<float>(), targ(dq), targ(dk), targ(dv), ws.data_ptr(),
+                          (size_t)ws.numel(), st),
+            "cra_bwd_inplace");
+    }
     return {dq, dk, dv, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
   }
 };

@@ -81,13 +81,10 @@ int cra_supported_head_dim(int32_t D);
  * (1+top_k)*floor(ls/W) + (ls % W != 0) (relay) or ceil(ls/W) (no relay). */
 int64_t cra_global_rows(const cra_problem* p);
 
-/* Whether cra_fwd and cra_bwd read the packed global rows for this problem
- * and these k and v: 1 if so, 0 if they take them from k and v in place (no
- * relay: row r is row r * W of k and v; k and v of one row stride, within
- * 32-bit offsets). At 0
- * cra_build_global need not run: glob_k and glob_v must still be non-NULL and
- * 16-byte aligned, and are not read by cra_fwd and cra_bwd (cra_fwd_persistent
- * and a single phase of cra_fwd_phases always read them). -1: invalid problem. */
+/* Whether this problem with these k and v needs packed global rows: 1 if so, 0
+ * if cra_fwd_inplace and cra_bwd_inplace can read them in k and v (no relay:
+ * row r is row r * W; k and v of one row stride, within 32-bit offsets) and
+ * cra_build_global need not run. -1: invalid problem. */
 int cra_reads_global_rows(const cra_problem* p, cra_tensor k, cra_tensor v);
 
 /* Builds the packed global rows and the relay source rows.
@@ -112,6 +109,13 @@ int cra_build_global(const cra_problem* p, cra_tensor k, cra_tensor v, void* glo
  * (reference core.py:907-1158, launched at core.py:3588-3610). */
 int cra_fwd(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v,
             const void* glob_k, const void* glob_v, cra_tensor o, float* lse, void* stream);
+
+/* cra_fwd without packed rows, for the calls where cra_reads_global_rows is 0
+ * (else CRA_E_LAYOUT): same results as cra_fwd with the rows cra_build_global
+ * packs, bit for bit. No counterpart in the reference as an entry point; its
+ * forward reads the strided rows in place (core.py:1042-1087). */
+int cra_fwd_inplace(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cra_tensor o,
+                    float* lse, void* stream);
 
 /* cra_fwd as a persistent kernel: a grid of one round of resident
  * workgroups (CUs x workgroups per CU) that take the 128-query tiles, heaviest
@@ -157,6 +161,13 @@ int cra_bwd(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cra_
             cra_tensor dout, const float* lse, const void* glob_k, const void* glob_v,
             const int32_t* relay_src, const float* relay_scale, cra_tensor dq, cra_tensor dk,
             cra_tensor dv, float* dalpha, void* workspace, size_t workspace_bytes, void* stream);
+
+/* cra_bwd without packed rows, where cra_reads_global_rows is 0 (else
+ * CRA_E_LAYOUT): same workspace, and same results as cra_bwd with the rows
+ * cra_build_global packs, bit for bit. */
+int cra_bwd_inplace(const cra_problem* p, cra_tensor q, cra_tensor k, cra_tensor v, cra_tensor o,
+                    cra_tensor dout, const float* lse, cra_tensor dq, cra_tensor dk, cra_tensor dv,
+                    void* workspace, size_t workspace_bytes, void* stream);
 
 /* Size of the fixed device scratch of cra_bwd_noalloc, per device. */
 #define CRA_NOALLOC_SCRATCH_BYTES (64u << 20)

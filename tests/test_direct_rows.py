@@ -1,5 +1,5 @@
-"""cra_reads_global_rows: which calls read packed global rows (CPU; nothing is
-launched and no pointer is read)."""
+"""cra_reads_global_rows: which calls need packed global rows, and what the
+in-place entry points refuse (CPU; nothing is launched and no pointer is read)."""
 import ctypes
 import math
 
@@ -41,3 +41,16 @@ def test_wider_elements_halve_the_limit():
 
 def test_invalid_problem():
     assert reads(10, False, 64, W=11) == -1
+
+
+@pytest.mark.parametrize("relay,vss,hkv,code", [
+    (1, 64, 2, N.E_LAYOUT),        # relay rows are packed
+    (0, 128, 2, N.E_LAYOUT),       # k and v of different row strides
+    (0, 64, 65536, N.E_INVALID),   # the limit of cra_build_global
+])
+def test_inplace_refuses(relay, vss, hkv, code):
+    lib = N.load_library()
+    p = ctypes.byref(N.problem(1, hkv, hkv, 100, 64, 10, relay, 2, torch.float16, 0.125))
+    t, v = N.CraTensor(0x10000, 6400 * hkv, 6400, 64), N.CraTensor(0x10000, 100 * vss * hkv, 100 * vss, vss)
+    assert lib.cra_fwd_inplace(p, t, t, v, t, 0x10000, None) == code
+    assert lib.cra_bwd_inplace(p, t, t, v, t, t, 0x10000, t, t, t, 0x10000, 1 << 40, None) == code
