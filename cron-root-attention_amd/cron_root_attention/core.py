@@ -291,12 +291,25 @@ def _layer_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     """The op as a layer calls it on its own projections: the same values, the
     output (and the gradients of q, k, v) as [B, H, S, D] views of [B, S, H, D]
     buffers, so that the reshapes to and from the projections copy nothing.
+    The backward reads the output: it must not be edited in place (``_layer_op``).
     Calls that do not go to the C++ operator give the op's contiguous output."""
     if q.device.type != "cpu" and _native.attention_op() is not None:
         plan = _op_plan(q, k, v, False, kv_groups, 2)
         if plan is not None:
             return torch.ops.cra.layer_attention(q, k, v, *plan)
     return cron_root_attention_v14(q, k, v, kv_groups=kv_groups)
+
+
+def _layer_op(proj: nn.Module):
+    """The op of a layer whose output projection is ``proj``: _layer_attention
+    where ``proj`` is a plain nn.Linear, which only reads its input. A hook, a
+    subclass or another module may edit it in place, which is for a copy of the
+    output to take: the op's contiguous one, copied by the layer's reshape."""
+    mod = torch.nn.modules.module
+    plain = (type(proj) is nn.Linear and "forward" not in proj.__dict__
+             and not (proj._forward_pre_hooks or proj._forward_hooks
+                      or mod._global_forward_pre_hooks or mod._global_forward_hooks))
+    return _layer_attention if plain else cron_root_attention_v14
 
 
 _OP_DTYPES = (torch.float16, torch.bfloat16, torch.float32)

@@ -27,7 +27,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .core import _layer_attention, cron_root_attention_v14
+from .core import _layer_op, cron_root_attention_v14
 
 # (mode, head_dim, smallest B*H the row applies to) -> smallest swept S from
 # which the sqrt(N) op beats SDPA at every larger swept S.
@@ -91,17 +91,21 @@ def cron_root_attention_hybrid(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     """SDPA below ``threshold`` tokens, the sqrt(N) kernel at or above it
     (reference hybrid.py:25-64).  ``threshold=None`` picks the measured gfx950
     crossover for this head dim and for training vs inference (grad mode)."""
-    S = q.shape[2]
     if backend == "cron_root":
         return cron_root_attention_v14(q, k, v)
     if backend == "sdpa":
         return F.scaled_dot_product_attention(q, k, v, is_causal=True)
     if backend != "auto":
         raise ValueError(f"unknown backend {backend!r}")
+    return _auto(q, k, v, threshold, cron_root_attention_v14)
+
+
+def _auto(q, k, v, threshold, op):
+    """The ``"auto"`` backend with ``op`` as the sqrt(N) kernel."""
     training = torch.is_grad_enabled() and q.requires_grad
-    if dispatch_backend(S, q.shape[-1], training, q.shape[0] * q.shape[1],
+    if dispatch_backend(q.shape[2], q.shape[-1], training, q.shape[0] * q.shape[1],
                         threshold) == "cron_root":
-        return cron_root_attention_v14(q, k, v)
+        return op(q, k, v)
     return F.scaled_dot_product_attention(q, k, v, is_causal=True)
 
 
@@ -126,12 +130,7 @@ class CronRootAttentionHybrid(nn.Module):
         q = self.q_proj(x).view(B, S, self.n_heads, self.head_dim).transpose(1, 2)
         k = self.k_proj(x).view(B, S, self.n_heads, self.head_dim).transpose(1, 2)
         v = self.v_proj(x).view(B, S, self.n_heads, self.head_dim).transpose(1, 2)
-        training = torch.is_grad_enabled() and q.requires_grad
-        if dispatch_backend(S, self.head_dim, training, B * self.n_heads,
-                            self.threshold) == "cron_root":
-            out = _layer_attention(q, k, v)
-        else:
-            out = F.scaled_dot_product_attention(q, k, v, is_causal=True)
+        out = _auto(q, k, v, self.threshold, _layer_op(self.o_proj))
         out = out.transpose(1, 2).contiguous().view(B, S, D)
         out = self.o_proj(out)
         if self.dropout > 0 and self.training:

@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .core import _layer_attention
+from .core import _layer_op
 from .hybrid import dispatch_backend
 
 
@@ -70,7 +70,7 @@ class CronRootAttention(nn.Module):
             out = F.scaled_dot_product_attention(q, k, v, is_causal=True,
                                                  enable_gqa=self.kv_groups > 1)
         else:
-            out = _layer_attention(q, k, v, kv_groups=self.kv_groups)
+            out = _layer_op(self.o_proj)(q, k, v, kv_groups=self.kv_groups)
         out = out.permute(0, 2, 1, 3).reshape(B, S, self.d_model)
         return self.drop(self.o_proj(out))
 
@@ -121,7 +121,7 @@ class CronRootMultiheadAttention(nn.Module):
         B, S, E = query.shape
         qkv = F.linear(query, self.in_proj_weight, self.in_proj_bias)
         qkv = qkv.view(B, S, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4)
-        out = _layer_attention(*qkv.unbind(0))
+        out = _layer_op(self.out_proj)(*qkv.unbind(0))
         out = out.permute(0, 2, 1, 3).reshape(B, S, E)
         out = self.drop(self.out_proj(out))
         if not self.batch_first:

@@ -37,6 +37,62 @@ def test_values_and_layout(B, Hq, Hkv, S, D, dtype):
             assert t.transpose(1, 2).is_contiguous()
 
 
+def _layers():
+    yield "CronRootAttention", cra.CronRootAttention(256, 4, n_kv_heads=2), "o_proj"
+    yield "CronRootAttentionHybrid", cra.CronRootAttentionHybrid(256, 4, threshold=1), "o_proj"
+    yield "CronRootMultiheadAttention", cra.CronRootMultiheadAttention(256, 4), "out_proj"
+
+
+@pytest.mark.parametrize("how", ["pre-hook", "hook", "module", "global pre-hook"])
+def test_output_edited_in_place(how):
+    """What a hook or module on the output projection does to its input in place
+    is for the layer's copy: the backward reads the attention output."""
+    for name, layer, proj in _layers():
+        torch.manual_seed(0)
+        layer = layer.to(DEV, F16)
+        lin = getattr(layer, proj)
+        lin.requires_grad_(how != "hook")  # (the linear's weight gradient reads its input)
+        x = torch.randn(1, 300, 256, device=DEV, dtype=F16)
+        dy = torch.randn_like(x)
+
+        def step():
+            y = x.clone().requires_grad_(True)
+            out = layer(y, y, y)[0] if name == "CronRootMultiheadAttention" else layer(y)
+            return [out.detach(), *torch.autograd.grad(out, y, dy)]
+
+        def edit(m, args, *_):
+            if m is lin:
+                args[0].mul_(2)
+
+        def copy(m, args):
+            return (args[0] * 2,)
+
+        if how == "hook":  # after the product: the result is the layer's own
+            want = step()
+            lin.register_forward_hook(edit)
+            got = step()
+        else:
+            h = lin.register_forward_pre_hook(copy)
+            want = step()
+            h.remove()
+            if how == "pre-hook":
+                lin.register_forward_pre_hook(edit)
+                got = step()
+            elif how == "global pre-hook":
+                h = torch.nn.modules.module.register_module_forward_pre_hook(edit)
+                got = step()
+                h.remove()
+            else:
+                class Twice(torch.nn.Module):
+                    def forward(self, t):
+                        return t.mul_(2)
+
+                setattr(layer, proj, torch.nn.Sequential(Twice(), lin))
+                got = step()
+        for a, b in zip(got, want):
+            assert torch.equal(a, b), name
+
+
 def test_layer_gradients_reach_fused_projections():
     """CronRootMultiheadAttention: q, k, v are slices of one projection."""
     torch.manual_seed(0)
