@@ -395,6 +395,7 @@ int bwd_impl(const cra_problem* p, const Plan& pl, cra_tensor q, cra_tensor k, c
   a.direct = inplace;
   a.chunk_len = chunks.chunk_len;
   a.nchunk = chunks.nchunk;
+  a.even = chunks.even;
   // workspace carve-up: delta and nlse2 [B*Hq*S] fp32 each, then the
   // global-row partials
   char* ws = static_cast<char*>(workspace);

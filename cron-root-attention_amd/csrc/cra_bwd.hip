@@ -72,8 +72,9 @@ __global__ __launch_bounds__(256) void gsum_kernel(BwdArgsT<ND> a) {
   // kernel wrote no partial for the others (their workgroups had no query
   // that sees the tile), so they are skipped rather than read.
   const int first = glob_row_first_query(e / kVec, dc);
-  const int c_lo = first / a.chunk_len;
-  const int c_hi = first < dc.len ? num_chunks(dc.len, a.chunk_len) : c_lo;
+  const int nck = num_chunks(dc.len, a.chunk_len);
+  const int c_lo = first / doc_chunk_len<ND>(dc.len, nck, a.chunk_len);
+  const int c_hi = first < dc.len ? nck : c_lo;
   float* p0 = a.gpart + part_row(dc, 0, nbh, bhk, 0) * 2 * D + 4 * (int64_t)e;
   const int64_t cstride = (int64_t)nbh * rows * 2 * D;
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -874,8 +875,9 @@ void dkdv2_kernel(BwdArgsT<ND> a) {
   // query interval of the workgroup; per-key intervals for the masks
   int q_lo, q_hi;
   if (GLOB) {
-    const int c_lo = chunk * a.chunk_len;
-    q_hi = min(S, c_lo + a.chunk_len);
+    const int chunk_len = doc_chunk_len<ND>(S, nck, a.chunk_len);
+    const int c_lo = chunk * chunk_len;
+    q_hi = min(S, c_lo + chunk_len);
     q_lo = max(c_lo, glob_row_first_query(k0, dc));
     // no query of this chunk sees the tile's rows: gsum_kernel skips the
     // chunk for them (with a single chunk the zeros are written instead)
@@ -1360,8 +1362,9 @@ void dkdv_f32_kernel(BwdArgsT<ND> a) {
   // queries of the workgroup
   int q_lo, q_hi;
   if (GLOB) {
-    const int c_lo = chunk * a.chunk_len;
-    q_hi = min(S, c_lo + a.chunk_len);
+    const int chunk_len = doc_chunk_len<ND>(S, nck, a.chunk_len);
+    const int c_lo = chunk * chunk_len;
+    q_hi = min(S, c_lo + chunk_len);
     q_lo = max(c_lo, glob_row_first_query(k0, dc));
     // see dkdv2_kernel
     if (q_hi <= q_lo && a.nchunk > 1) return;
@@ -1510,25 +1513,38 @@ constexpr int kDkdvLocalBQ = 32;
 // idle their waves. Against that, 64-row tiles sweep the queries once per 64
 // rows. Kernel time, wide / 64-row workgroups (wide workgroups in the launch;
 // H: query / kv heads; G: packed rows):
-//   D=128  B=2 H=32/32 S=4096  (384; G = 192)   72 /   51 us
-//          B=1 H=16/4  S=16000 (384; G = 381)  112 /   82 us
-//          B=1 H=16/16 S=16384 (384; G = 384)  109 /   84 us
-//          B=2 H=32/32 S=16384 (384; G = 384)  277 /  266 us
-//          B=1 H=32/4  S=32768 (384; G = 546)  516 /  402 us
-//          B=8 H=32/32 S=2048  (512; G =  45)   66 /   59 us
-//          B=8 H=32/32 S=4096  (512; G = 192)  166 /  206 us
-//          B=4 H=32/32 S=8192  (512; G = 273)  192 /  224 us
+//   D=128  H=8/8 S=4096        (256; G = 192)   21 /   17 us
+//          B=2 H=32/32 S=4096  (384; G = 192)   65 /   48 us
+//          H=16/16 S=16384     (384; G = 384)  100 /   79 us
+//          H=8/8 S=65536       (384; G = 768)  331 /  278 us
+//          H=16/4 S=65536      (384; G = 768)  700 /  543 us
+//          B=8 H=32/32 S=2048  (512; G =  45)   69 /   59 us
+//          H=32/4 S=4096       (G = 192)        55 /   34 us
+//          B=4 H=32/32 S=8192  (512; G = 273)  200 /  219 us
+//          H=16/16 S=32768     (G = 546)       198 /  209 us
+//          H=16/16 S=65536     (704; G = 768)  537 /  513 us
 //          B=4 H=32/8  S=32768 (576; G = 546) 1712 / 1720 us
 //          B=2 H=32/32 S=65536 (2816; G = 768) 2051 / 2520 us
-//   D=64   B=8 H=32/32 S=2048  (512; G =  45)   31 /   27 us
-//          B=4 H=32/32 S=8192  (768; G = 273)  126 /  128 us
-//          B=8 H=32/8  S=8192  (768; G = 273)  267 /  278 us
-//          B=1 H=12/12 S=65536 (792; G = 768)  227 /  242 us
+//   D=64   H=8/8 S=2100        (G = 138)       9.4 /  8.2 us
+//          H=8/8 S=4096        (G = 192)      10.2 / 10.8 us
+//          H=4/4 S=8192        (G = 273)      11.7 / 12.6 us
+//          H=16/16 S=3000      (G = 165)      12.0 / 12.0 us
+//          B=8 H=32/32 S=2048  (512; G =  45)   33 /   29 us
+//          H=8/8 S=16384       (768; G = 384)   32 /   27 us
+//          H=16/16 S=16384     (768; G = 384)   51 /   45 us
+//          B=4 H=32/32 S=8192  (768; G = 273)  129 /  128 us
+//          H=8/8 S=32768       (G = 546)        67 /   71 us
+//          H=12/12 S=65536     (792; G = 768)  227 /  242 us
 // So: the 64-row workgroups for launches of fewer than two wide workgroups
 // per CU (up to 768 rows, the most that was measured), and where the documents'
-// rows padded to wide tiles are at least 1.75 times those padded to 64: one
-// document of up to 64 rows, or packed ones with many short among them (16 of 1
-// to 9001 tokens, H=16/4 D=128: 2.0 times, 97 / 76 us).
+// rows padded to wide tiles are at least 1.75 times those padded to 64 (one
+// document of up to 64 rows, packed ones with many short among them). At D = 64
+// the line is a rough one: it misses 15% at S = 16384 and gives away 6% at S =
+// 4096 and 8192 with few heads. Packed documents of up to 768 rows take them
+// too where their sweeps are cut (plan_chunks): the pieces are made for them
+// (over 190 such batches 0.86 times the wide kernel's time on average, with
+// gsum_kernel; at most 1.07 times). Uncut ones keep the wide workgroups (eight
+// documents of 4096, H=32/32 D=128: 164 / 222 us).
 constexpr int kNarrowWaves = 4, kNarrowBQ = 32, kNarrowMaxRows = 768;
 
 template <int D>
@@ -1545,7 +1561,8 @@ bool narrow_glob(const BwdArgs& a) {
     wide += (int64_t)tiles * kWide;
     narrow += (int64_t)(rows + kNarrow - 1) / kNarrow * kNarrow;
   }
-  return D <= 128 && ((items < 2 * a.cus && most <= kNarrowMaxRows) || 4 * wide >= 7 * narrow);
+  const bool few = a.docs.n > 1 ? !a.even : items < 2 * a.cus;
+  return D <= 128 && ((few && most <= kNarrowMaxRows) || 4 * wide >= 7 * narrow);
 }
 
 // Below D = 128 a local workgroup takes 128 keys, 32 a wave; where that gives
@@ -1696,24 +1713,30 @@ ChunkPlan plan_chunks(int D, int B, int Hq, int Hkv, int n, const int* len,
   const int64_t base = row_tiles * B * Hkv;
   ChunkPlan c{};
   if (n > 1) {
-    // Several documents: chunks of one length, so that a long document gets
-    // more of them than a short one. The sweeps (visible queries x heads of
-    // the kv group, per 64-row tile) are cut into about three pieces per CU,
-    // the 64-row kernel's resident workgroups. (With the same number of
-    // chunks for every document the longest document's workgroups ran alone
-    // at the end: 16 documents of 1 to 9001 tokens, H=16/4 D=128, 237 us in
-    // the global-row kernel and 7 in gsum_kernel; with this rule and 64-row
-    // tiles 78 + 12, with 0.75 / 1.5 / 2 times as many pieces 78 + 10, 74 +
-    // 14 and 82 + 20.)
+    // Several documents: pieces of about one length, so that a long document
+    // gets more of them than a short one. The sweeps (queries that see a 64-row
+    // tile, over the tiles, batches and kv heads) are cut into about three
+    // pieces per CU, the 64-row kernel's resident workgroups, unless the longest
+    // is at most 0.6 of a CU's load: those fill the chip evenly as they are, and
+    // pieces would only add partials. Global-row kernel and gsum_kernel over 226
+    // batches (1 to 131072 tokens, 2 to 200 documents, 1 to 32 kv heads) against
+    // the same number of chunks for every document, where the longest
+    // document's workgroups run alone at the end: 0.81 times the time on
+    // average (1.5, 2 and 4 pieces per CU 0.87, 0.83 and 0.83; always cut
+    // 0.82), at most 1.17 times, 3.4% of the step (16 documents of 1 to 9001
+    // tokens, H=16/4 D=128: 244 -> 91 us; six of 5000, H=32/32 D=128: uncut 204
+    // us, cut 232).
     double sweeps = 0;
+    int longest = 0;
     for (int d = 0; d < n; ++d) {
       const int g = doc_rows(len[d], W[d], rpb[d]);
+      longest = std::max(longest, len[d] - W[d]);
       for (int t = 0; t < g; t += 64)
         sweeps += std::max(0, len[d] - (t / rpb[d] + 1) * W[d]);
     }
-    sweeps *= (double)B * Hkv;
-    const double pieces = 3.0 * (cus > 0 ? cus : 256);
-    const double L = std::min(std::max(sweeps / pieces, 64.0), 6144.0);
+    sweeps *= (double)B * Hkv / (cus > 0 ? cus : 256);  // per CU
+    c.even = longest <= 0.6 * sweeps;
+    const double L = c.even ? 6144.0 : std::min(std::max(sweeps / 3, 64.0), 6144.0);
     c.chunk_len = chunk_len_for((int)L, 1);
     for (;;) {
       c.part_rows = 0;

@@ -222,8 +222,9 @@ struct BwdCommon {
   int64_t G;       // packed global rows of all documents, per head
   float scale;
   int cus;         // compute units of the device (launch rules)
-  int chunk_len;   // queries per chunk of the global-row kernel
+  int chunk_len;   // most queries per chunk of the global-row kernel
   int nchunk;      // most query chunks of a document
+  int even;        // packed documents that fill the chip evenly uncut (ChunkPlan)
   int group;       // 0: first launch of a call (writes dalpha);
                    // later document groups of the call add to dalpha
   int xcd_nt;      // > 0: XCD-aware order (xcd_item) over this many tiles per head
@@ -339,6 +340,14 @@ __host__ __device__ inline int num_chunks(int len, int chunk_len) {
   return (len + chunk_len - 1) / chunk_len;
 }
 
+// Queries per chunk of a document cut into `nck`: packed documents (ND > 1)
+// are cut evenly, so that a document a little longer than chunk_len does not
+// end in a short piece; one document's chunk_len is even already.
+template <int ND>
+__device__ __forceinline__ int doc_chunk_len(int len, int nck, int chunk_len) {
+  return ND > 1 ? chunk_len_for(len, nck) : chunk_len;
+}
+
 // Packed global rows of a document.
 __host__ __device__ inline int doc_rows(int len, int W, int rpb) { return (len + W - 1) / W * rpb; }
 
@@ -379,8 +388,9 @@ hipError_t launch_bwd(int dtype, int D, const BwdArgs& a, hipStream_t st);
 // of lengths len[], windows W[] and packed rows per block rpb[] on a device
 // with `cus` compute units.
 struct ChunkPlan {
-  int chunk_len;      // queries per chunk (multiple of 64)
+  int chunk_len;      // most queries per chunk (multiple of 64)
   int nchunk;         // most chunks of a document
+  bool even;          // packed documents that fill the chip evenly uncut
   int64_t part_rows;  // partial rows per (b, kv head), all documents
 };
 ChunkPlan plan_chunks(int D, int B, int Hq, int Hkv, int n, const int* len, const int* W,

@@ -11,7 +11,7 @@ import torch
 
 from cron_root_attention.core import _attention_with_plan, _varlen_with_plan
 from oracle import cra_oracle as O
-from tests.parity_util import BF16, DEV, F16, TOL_GRAD, inputs, rel_fro, say
+from tests.parity_util import BF16, DEV, F16, F32, TOL_GRAD, inputs, rel_fro, say
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +73,28 @@ def test_document_chunks(D, dtype, lens):
             assert rel_fro(got[2][:, :, a:b], ref["dv"]) <= TOL_GRAD[dtype]
             continue
         _check([t[:, :, a:b] for t in got], ref, dtype)
+
+
+@pytest.mark.parametrize("D,dtype,H,W,lens", [
+    (64, F16, 8, 2, (1100, 530, 270)),        # chunks of 256, 192 and 192 queries
+    (64, F32, 12, 2, (1000, 300, 260, 1)),    # 256, 192, 192 and one
+    (128, BF16, 16, 9, (70,) * 90),           # uncut, two launches of documents
+])
+def test_documents_cut_evenly(D, dtype, H, W, lens):
+    """Each document in chunks of its own even length, or none cut."""
+    say(f"documents cut evenly: D={D} {dtype} H={H} W={W} lens={lens[:4]}")
+    S = sum(lens)
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    Ws = [min(n, W) for n in lens]
+    relay = [n >= 64 for n in lens]
+    q, k, v, do = inputs(1, H, H, S, D, dtype, seed=S)
+    x = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+    o = _varlen_with_plan(*x, cu, Ws, relay)
+    got = torch.autograd.grad(o, x, do.to(DEV))
+    for i, (a, b) in list(enumerate(zip(cu, cu[1:])))[::max(1, len(lens) // 8)]:
+        part = [t[:, ::5, a:b] for t in (q, k, v, do)]
+        _, _, _, ref = O.forward_backward(*part, O.Plan(b - a, Ws[i], relay[i], 2))
+        if b - a > 1:
+            _check([t[:, ::5, a:b] for t in got], ref, dtype)
