@@ -25,8 +25,8 @@ def calibrate(H: int = 8, D: int = 64, dtype=None, S: int = 4096, verbose: bool 
 
     The reference benchmarks Triton (num_warps, num_stages) candidates here
     and returns {"fwd": (num_warps, num_stages), "bwd": (...)}. The HIP
-    kernels have one tile geometry per (dtype, D), fixed at build time; this
-    returns the same shape of dict with (waves per workgroup, LDS pipeline
+    kernels' tiles are fixed per (dtype, D) at build time (the dK/dV kernels of
+    small launches take narrower ones); this returns the same shape of dict with (waves per workgroup, LDS pipeline
     stages) of the forward and of the dQ kernel, as the library reports them
     (``cra_tile_config``; the whole geometry: ``_native.tile_config``), and,
     on a GPU, runs one forward+backward at S to load the kernels.
@@ -41,10 +41,10 @@ def calibrate(H: int = 8, D: int = 64, dtype=None, S: int = 4096, verbose: bool 
         v = _torch.randn(1, H, S, D, device=dev, dtype=dtype, requires_grad=True)
         cron_root_attention_v14(q, k, v).sum().backward()
         _torch.cuda.synchronize(dev)
-    # fp16/bf16 up to D = 128 double-buffer their streamed tiles in LDS; fp32
-    # stages one tile, and so does D = 256 (fp16/bf16: K and V in turn, each
-    # filled while the other is in use)
-    stages = 2 if (dtype != _torch.float32 and Dp <= 128) else 1
+    # double-buffered tiles in LDS where they fit: fp16/bf16 up to D = 128, fp32
+    # (three bf16 pieces an element) up to 64. Above, one stage (fp16/bf16: K and
+    # V in turn, each filled while the other is in use)
+    stages = 2 if Dp <= (64 if dtype == _torch.float32 else 128) else 1
     cfg = {"fwd": (t["fwd_waves"], stages), "bwd": (t["dq_waves"], stages)}
     if verbose:
         print(f"  H={H} D={D}: fwd {t['fwd_waves']} waves x {t['fwd_queries']} queries, "

@@ -260,10 +260,13 @@ int cra_device_info(int32_t device, cra_device_info_t* out);
 
 /* The tile geometry compiled for (dtype, D): waves per workgroup, rows per
  * workgroup (queries or key rows) and rows per streamed tile of the forward
- * and the three backward kernels. Serves calibrate(), which in the reference
- * times Triton (num_warps, num_stages) candidates per (op, H, D)
- * (_KernelAutoTuner, core.py:250-596; __init__.py:84-180); here the
- * geometry is fixed per (gfx950, dtype, D) at build time. */
+ * and the three backward kernels, as a launch that fills the chip takes them.
+ * In fp16/bf16 up to D = 128 smaller launches, and rows that would mostly be
+ * padding, take global-row dK/dV workgroups of 4 waves, 64 rows and 32-query
+ * tiles, and below D = 128 local ones of 64 keys. Serves calibrate(), which in
+ * the reference times Triton (num_warps, num_stages) candidates per (op, H, D)
+ * (_KernelAutoTuner, core.py:250-596; __init__.py:84-180); here the tiles are
+ * fixed per (gfx950, dtype, D) at build time. */
 typedef struct {
   int32_t fwd_waves, fwd_queries, fwd_key_tile;
   int32_t dq_waves, dq_queries, dq_key_tile;

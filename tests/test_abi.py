@@ -274,7 +274,7 @@ def test_tile_config_reports_compiled_geometry():
         for D in (32, 64, 128, 256):
             t = N.tile_config(dt, D)
             assert all(v > 0 for v in t.values())
-            # 32 queries per wave; 16 at D = 256 (the generic kernels' register budget)
+            # 32 queries per wave; 16 at D = 256 (the register budget)
             assert t["fwd_queries"] == (16 if D == 256 else 32) * t["fwd_waves"]
     h256 = N.tile_config(torch.bfloat16, 256)
     assert (h256["fwd_waves"], h256["fwd_queries"], h256["fwd_key_tile"]) == (4, 64, 32)
@@ -295,9 +295,18 @@ def test_tile_config_reports_compiled_geometry():
     import cron_root_attention as cra
     cfg = cra.calibrate(16, 128, verbose=False)
     assert cfg == {"fwd": (h["fwd_waves"], 2), "bwd": (h["dq_waves"], 2)}   # reference's keys
-    # the generic kernels (fp32, D = 256) stage one tile at a time
+    # D = 256 in fp16/bf16 stages one tile of K and of V at a time
     assert cra.calibrate(16, 200, dtype=torch.float16, verbose=False) == {"fwd": (4, 1),
                                                                           "bwd": (4, 1)}
+
+
+def test_calibrate_reports_the_stages_of_fp32():
+    """fp32 keeps two LDS stages of K and V up to D = 64, one above."""
+    import torch
+    import cron_root_attention as cra
+    for D, stages in ((32, 2), (48, 2), (64, 2), (80, 1), (128, 1), (256, 1)):
+        cfg = cra.calibrate(2, D, dtype=torch.float32, S=64, verbose=False)
+        assert cfg == {"fwd": (4, stages), "bwd": (4, stages)}, D
 
 
 def lib_tc_unsupported(D):
