@@ -287,7 +287,7 @@ void dq2_kernel(BwdArgsT<ND> a) {
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * kQW;
-  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+  const int S = dc.len, W = dc.W;
 
   const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
   const T* dop =
@@ -483,7 +483,7 @@ void dq_wide_kernel(BwdArgsT<ND> a) {
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * 16;
-  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+  const int S = dc.len, W = dc.W;
 
   const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
   const T* dop =
@@ -852,7 +852,6 @@ void dkdv2_kernel(BwdArgsT<ND> a) {
   const int chunk = GLOB ? dc.item - tile * nck : 0;
   const int grp = a.Hq / a.Hkv;
   const int S = dc.len, W = dc.W, rpb = dc.rpb;
-  const bool relay = rpb > 1;
   const int nrows = GLOB ? doc_rows(S, W, rpb) : S;  // keys: global rows or rows
   const int k0 = tile * kBK;
   const int kw = k0 + wave * kKW;
@@ -1038,9 +1037,9 @@ void dkdv2_kernel(BwdArgsT<ND> a) {
 // LDS stages with one barrier per tile; dS and P are split in registers. Delta
 // is subtracted from the finished dP, as at D = 256 in 2 bytes (kSubDelta).
 // Against the fp32-MFMA kernels before them (dQ with the separate Delta pass /
-// global rows / local rows), H=8: S=32768 D=64 527 / 554 / 467 -> 320 / 308 /
-// 238 us, D=128 1246 / 1600 / 1041 -> 695 / 711 / 452 us, S=4096 D=64 59 / 49 /
-// 42 -> 30 / 30 / 21 us; H=4 S=8192 D=256 194 / 207 / 146 -> 156 / 140 / 121 us.
+// global rows / local rows), H=8: S=32768 D=64 547 / 566 / 469 -> 336 / 324 /
+// 247 us, D=128 1248 / 1603 / 1040 -> 629 / 674 / 487 us, S=4096 D=64 58 / 49 /
+// 42 -> 26 / 29 / 21 us; H=4 S=8192 D=256 199 / 211 / 146 -> 147 / 148 / 120 us.
 // ---------------------------------------------------------------------------
 constexpr int kF32Waves = 4, kF32BN = 32;
 
@@ -1125,7 +1124,7 @@ void dq_f32_kernel(BwdArgsT<ND> a) {
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * 16;
-  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+  const int S = dc.len, W = dc.W;
 
   const float* qp = static_cast<const float*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
   const float* dop =
@@ -1313,9 +1312,10 @@ __device__ __forceinline__ void dkdv_f32_tile(const char* tQ, const char* tO, co
   }
 }
 
-// At D = 128 the global-row kernel needs 350 registers: one wave per SIMD and
-// two LDS stages (at 256 registers it spills 82: 835 us against 761, B=1 H=8
-// S=32768); the local one keeps 256 (24 spilled) and two workgroups per CU.
+// At D = 128 the global-row kernel needs 343 registers: one wave per SIMD and
+// two LDS stages (at 256 registers it spilled 82: 835 us against 761, B=1 H=8
+// S=32768); the local one keeps 256 (22 spilled) and two workgroups per CU. At
+// D = 256 both take the 512 of one wave per SIMD (9 and 24 spilled).
 template <int D, bool GLOB>
 constexpr bool kF32OneWave = D > 128 || (GLOB && D == 128);
 
@@ -1467,13 +1467,13 @@ void dkdv_f32_kernel(BwdArgsT<ND> a) {
 
 // dK/dV workgroups: waves of 16 key rows (no register file spill into AGPR
 // copies at D = 128; 32 rows per wave measured 14% slower). The global-row
-// kernel uses 12 waves (192 rows): at 164 VGPRs a SIMD holds 3 of its
+// kernel uses 12 waves (192 rows): at 166 VGPRs a SIMD holds 3 of its
 // waves, and one 12-wave workgroup fills them, where a second 8-wave
 // workgroup did not fit beside the first (8 waves measured 1.7% slower
 // backward, 4 waves 3% slower than 8); the local
 // kernel 4 waves (64 rows: its band of queries, 64 + W - 1, wastes fewer
 // pairs than with 128 rows; measured 7% faster). dQ workgroups: 4 waves of
-// 32 queries, 64-key tiles, 2 waves per SIMD at 246 VGPRs (each K/V
+// 32 queries, 64-key tiles, 2 waves per SIMD at 254 VGPRs (each K/V
 // fragment read from LDS serves two query blocks). 16 queries per wave
 // lose that reuse: 8 waves measured 27% slower, and with 32-key tiles at
 // 3 or 4 waves per SIMD still 5-10% slower backward at D = 128.

@@ -41,8 +41,8 @@ namespace {
 // the matrix core and the splits' VALU work about equally (per wave and 32-key
 // tile at D = 64: 96 MFMAs, 1536 cycles, beside about 300 VALU). Against the
 // fp32-MFMA kernel before it (V transposed by LDS writes, one stage): H=8
-// S=32768 D=64 362 -> 236 us, D=128 968 -> 615 us, S=4096 D=64 45 -> 31 us,
-// H=4 S=8192 D=256 149 -> 120 us.
+// S=32768 D=64 377 -> 246 us, D=128 963 -> 598 us, S=4096 D=64 45 -> 28 us,
+// H=4 S=8192 D=256 153 -> 122 us.
 // ---------------------------------------------------------------------------
 constexpr float kSumMaxF32 = 32768.f;
 constexpr int kF32Waves = 4, kF32BN = 32;
@@ -152,7 +152,7 @@ void fwd_f32_kernel(FwdArgsT<ND> a) {
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * kQW;
-  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+  const int S = dc.len, W = dc.W;
 
   const float* qp = static_cast<const float*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
   const float* kp = static_cast<const float*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
@@ -503,7 +503,7 @@ __device__ __forceinline__ void fwd2_item(const FwdArgsT<ND>& a, const int item,
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * kQW;
-  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+  const int S = dc.len, W = dc.W;
 
   const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
   const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;
@@ -750,7 +750,7 @@ void fwd_wide_kernel(FwdArgsT<ND> a) {
   const int tile = (dc.len + kBM - 1) / kBM - 1 - dc.item;  // heaviest first
   const int m0 = tile * kBM;
   const int q0 = m0 + wave * 16;
-  const int S = dc.len, W = dc.W, rpb = dc.rpb;
+  const int S = dc.len, W = dc.W;
 
   const T* qp = static_cast<const T*>(a.q) + b * a.qsb + h * a.qsh + (int64_t)dc.off * a.qss;
   const T* kp = static_cast<const T*>(a.k) + b * a.ksb + hk * a.ksh + (int64_t)dc.off * a.kss;

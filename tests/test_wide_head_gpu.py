@@ -2,8 +2,8 @@
 
 The reference takes any head dim (``BLOCK_D = triton.next_power_of_2(D)``,
 core.py:3495). This build compiles D = 256 (every dtype; D in (128, 256] is
-zero-padded to 256, scores keeping 1/sqrt(D) of the true D) on its generic
-kernels with 16 queries or keys per wave. Forward element-wise and every
+zero-padded to 256, scores keeping 1/sqrt(D) of the true D), 16 queries or
+keys per wave. Forward element-wise and every
 gradient against the oracle, as for the other head dims (tolerances in
 ``tests/parity_util.py``), at small shapes in full and at S = 32768 on
 spot rows; GQA, relay top-k, relay_log_scale and use_persistent included.
